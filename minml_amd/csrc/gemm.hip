@@ -19,6 +19,7 @@
 #include "epilogues.hpp"
 #include "gemm_launch.hpp"
 #include "gemm_stream.hpp"
+#include "gemm_direct.hpp"
 #include "gemm_dma.hpp"
 
 namespace
@@ -243,6 +244,20 @@ namespace mlhip
 		 */
 		const bool plain = (g.alpha == 1.0f) && (g.beta == 0.0f) && (g.bias == nullptr) && (g.act == ACTIVATION_LINEAR) && (g.N * esize) % 16 == 0
 				&& aligned_to(g.D, 16) && ((g.stride_c * esize) % 16 == 0) && g.dtype != DTYPE_INT8;
+		/* the same products with few rows, whose launch is all latency */
+		if (fast && g.dtype == DTYPE_FLOAT16 && vectorized && gemm_direct_applies(g.M, g.N, g.batch, k_bytes))
+		{
+			const StreamGemmArgs sg { g.A, g.B, g.D, g.M, g.N, static_cast<int>(k_bytes), g.batch, g.stride_a, g.stride_b, g.stride_c };
+			if (plain)
+				launch_gemm_direct(stream, sg, PlainStore { });
+			else
+				specialise_epilogue(make_float_epilogue<half_t>(g, true), [&](const auto &ep)
+				{
+					launch_gemm_direct(stream, sg, ep);
+				});
+			MLHIP_CHECK(hipGetLastError());
+			return;
+		}
 		if (fast && (g.stride_a != 0 || g.batch == 1)
 				&& ((plain || g.dtype == DTYPE_FLOAT16) ? stream_gemm_plain_applies(g.M, g.batch, k_bytes, esize) : stream_gemm_applies(g.M, g.batch, k_bytes)))
 		{

@@ -1,0 +1,233 @@
+/*
+ * gemm_direct.hpp — fp16 products too small to give every compute unit a streaming workgroup:  C[i] = A[i] * B[i]^T  with short K rows
+ * (the 36 Winograd products of a few positions; the dense layers and 1x1 convolutions of a few positions).
+ *
+ * Such a launch is bound by latency, not by HBM or the matrix cores: it takes one memory round trip, the bytes that the busiest compute
+ * unit must pull in, a short chain of MFMAs and the stores. The streaming kernel (gemm_stream.hpp) is the wrong shape for it: a
+ * workgroup there first brings 128 KB of B into registers, 32 rows x 32 bytes per instruction, and at one position all but 36 compute
+ * units stay idle. Here the product is cut into tiles small enough to occupy the chip, and a workgroup requests the WHOLE K extent of
+ * its rows of A and B at once by direct-to-LDS loads (8 rows x 128 bytes per instruction, whole cache lines; the same loads straight
+ * into the fragment layout, 16 half lines per instruction, took 13.9 instead of 7.1 us at 256 rows), multiplies each 128-byte piece of
+ * K as soon as it has landed (one barrier per piece), and stores its 4 consecutive outputs per lane and block directly.
+ * 16x16 MFMA blocks (v_mfma_f32_16x16x32_f16: bit-identical to the 32x32x16 form of the other engines, so that a position's result does
+ * not depend on which engine its batch takes). Two tile shapes: 64 x 64 by 8 wavefronts of 16 x 32 (many small wavefronts keep more
+ * loads in flight: 4 wavefronts of 32 x 32 take 7.05 instead of 6.66 us at 256 rows), and 32 x 32 by 4 wavefronts of 16 x 16 where
+ * 64 x 64 leaves compute units without a tile. Consecutive tiles (same matrix, same columns) lie on one XCD and share its L2.
+ *
+ * Measured, 36 products of M rows in a recorded chain, us per launch, streaming kernel -> this one: 256 -> 256 channels: M = 16
+ * (one 15x15 position) 8.9 -> 3.3, 64 9.2 -> 3.9, 256 9.1 -> 6.7, 512 13.2 -> 9.5, 1024 17.0 -> 15.1, 1616 20.4 -> 22.8;
+ * 128 -> 128 channels: 16 4.9 -> 2.4, 1024 8.5 -> 6.8, 2048 11.3 -> 10.7; 384 -> 384: 16 10.8 -> 4.0, 256 12.7 -> 13.2;
+ * one product of 256 -> 768 columns: 225 rows 9.7 -> 2.9, 1350 10.2 -> 4.7, 4000 10.1 -> 8.5.
+ */
+#ifndef MINML_AMD_GEMM_DIRECT_HPP_
+#define MINML_AMD_GEMM_DIRECT_HPP_
+
+#include "common.hpp"
+#include "gemm_stream.hpp"
+
+namespace mlhip
+{
+	template<int KB, int BLOCKS_M, int BLOCKS_N, int WAVES_M, int WAVES_N, typename Epilogue>
+	__global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void kernel_gemm_direct_nt(const half_t *A, const half_t *B, half_t *C, int M, int N, size_t stride_a,
+			size_t stride_b, size_t stride_c, unsigned int tiles_m, unsigned int tiles_n, size_t a_row_bytes, Epilogue epilogue)
+	{
+		constexpr bool PLAIN = std::is_same<Epilogue, PlainStore>::value;
+		constexpr int PIECES = KB / 128; /* 128-byte pieces of a K row */
+		constexpr int BM = 16 * BLOCKS_M * WAVES_M, BN = 16 * BLOCKS_N * WAVES_N, WAVES = WAVES_M * WAVES_N;
+		constexpr int ROW_BLOCKS = (BM + BN) / 8, PIECE_LOADS = ROW_BLOCKS / WAVES; /* 8-row blocks of a piece, all and per wavefront */
+		static_assert(KB % 128 == 0 && ROW_BLOCKS % WAVES == 0, "K rows of whole 128-byte pieces, the same number of loads for every wavefront");
+		const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+		const int wave_m = wave / WAVES_N, wave_n = wave % WAVES_N;
+		const int frag_row = lane & 15, quarter = lane >> 4;
+
+		const unsigned int id = xcd_contiguous_block_id(blockIdx.x, gridDim.x);
+		const unsigned int column_tiles = id / tiles_m; /* matrix * tiles_n + n_tile */
+		const unsigned int matrix = column_tiles / tiles_n;
+		const int m_tile = (id - column_tiles * tiles_m) * BM, n_tile = (column_tiles - matrix * tiles_n) * BN;
+		const int m0 = m_tile + wave_m * 16 * BLOCKS_M, n0 = n_tile + wave_n * 16 * BLOCKS_N;
+
+		/* lane l, register r of block (i, j): m = 16 i + l % 16, n = 16 j + 4 (l / 16) + r */
+		Epilogue local = epilogue;
+		struct Nothing
+		{
+				struct Column
+				{
+				};
+				struct Extra
+				{
+				};
+		};
+		typedef typename std::conditional<PLAIN, Nothing, Epilogue>::type Parts;
+		typename Parts::Column column[BLOCKS_N];
+		typename Parts::Extra extra[BLOCKS_M][BLOCKS_N];
+		if constexpr (!PLAIN)
+		{
+			local.D += matrix * stride_c;
+			if (local.bias != nullptr)
+				local.bias += static_cast<size_t>(matrix) * local.bias_batch_stride;
+#pragma unroll
+			for (int j = 0; j < BLOCKS_N; j++)
+			{
+				const int n = n0 + 16 * j + 4 * quarter;
+				column[j] = local.load_column(n < N ? n : 0);
+			}
+			if (local.has_extra())
+			{
+				local.C += matrix * stride_c;
+#pragma unroll
+				for (int i = 0; i < BLOCKS_M; i++)
+#pragma unroll
+					for (int j = 0; j < BLOCKS_N; j++)
+					{
+						const int n = n0 + 16 * j + 4 * quarter;
+						extra[i][j] = local.load_extra(min(m0 + 16 * i + frag_row, M - 1), n < N ? n : 0);
+					}
+			}
+		}
+
+		/* operand tiles -> LDS: [128-byte piece of K][row][128 bytes], 8 rows per instruction, the 16-byte chunks of a row swizzled */
+		extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+		const uint8_t *a_base = reinterpret_cast<const uint8_t*>(A + matrix * stride_a);
+		const uint8_t *b_base = reinterpret_cast<const uint8_t*>(B + matrix * stride_b);
+#pragma unroll
+		for (int u = 0; u < PIECES * PIECE_LOADS; u++)
+		{
+			const int block = wave + WAVES * (u % PIECE_LOADS), piece = u / PIECE_LOADS;
+			const int row = block * 8 + (lane >> 3);
+			const int chunk = ((lane & 7) ^ ((row >> 1) & 7)) * 16;
+			const uint8_t *src = (row < BM) ? a_base + static_cast<size_t>(min(m_tile + row, M - 1)) * a_row_bytes
+					: b_base + static_cast<size_t>(min(n_tile + row - BM, N - 1)) * KB;
+			__builtin_amdgcn_global_load_lds((global_ptr_t) (src + piece * 128 + chunk), (lds_ptr_t) (lds + (piece * ROW_BLOCKS + block) * 1024), 16, 0, 0);
+		}
+		float4_t acc[BLOCKS_M][BLOCKS_N];
+#pragma unroll
+		for (int i = 0; i < BLOCKS_M; i++)
+#pragma unroll
+			for (int j = 0; j < BLOCKS_N; j++)
+				acc[i][j] = float4_t { 0.0f, 0.0f, 0.0f, 0.0f };
+		int a_first[BLOCKS_M], b_first[BLOCKS_N]; /* this lane's fragment of the first k step, the others by XOR and piece */
+#pragma unroll
+		for (int i = 0; i < BLOCKS_M; i++)
+		{
+			const int row = wave_m * 16 * BLOCKS_M + 16 * i + frag_row;
+			a_first[i] = row * 128 + ((quarter ^ ((row >> 1) & 7)) * 16);
+		}
+#pragma unroll
+		for (int j = 0; j < BLOCKS_N; j++)
+		{
+			const int row = BM + wave_n * 16 * BLOCKS_N + 16 * j + frag_row;
+			b_first[j] = row * 128 + ((quarter ^ ((row >> 1) & 7)) * 16);
+		}
+		stream_static_for<2 * PIECES>([&](auto step)
+		{
+			constexpr int s = decltype(step)::value;
+			if constexpr (s % 2 == 0)
+			{ /* piece s / 2 has landed once at most the loads of the later pieces are outstanding (loads return in order) */
+				wait_vmcnt<(PIECES - 1 - s / 2) * PIECE_LOADS>();
+				barrier_no_fence();
+			}
+			uint4_t a[BLOCKS_M], b[BLOCKS_N];
+			const uint8_t *piece = lds + (s / 2) * (BM + BN) * 128;
+#pragma unroll
+			for (int i = 0; i < BLOCKS_M; i++)
+				a[i] = *reinterpret_cast<const uint4_t*>(piece + (a_first[i] ^ ((s & 1) * 64)));
+#pragma unroll
+			for (int j = 0; j < BLOCKS_N; j++)
+				b[j] = *reinterpret_cast<const uint4_t*>(piece + (b_first[j] ^ ((s & 1) * 64)));
+#pragma unroll
+			for (int i = 0; i < BLOCKS_M; i++)
+#pragma unroll
+				for (int j = 0; j < BLOCKS_N; j++)
+					acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, b[j]), __builtin_bit_cast(half8_t, a[i]), acc[i][j], 0, 0, 0);
+		});
+#pragma unroll
+		for (int i = 0; i < BLOCKS_M; i++)
+		{
+			const int m = m0 + 16 * i + frag_row;
+			if (m >= M)
+				continue;
+#pragma unroll
+			for (int j = 0; j < BLOCKS_N; j++)
+			{
+				const int n = n0 + 16 * j + 4 * quarter;
+				if (n >= N) /* N is a multiple of 4 (checked by the launcher) */
+					continue;
+				if constexpr (PLAIN)
+				{
+					Vec<half_t, 4> out;
+#pragma unroll
+					for (int e = 0; e < 4; e++)
+						out.v[e] = acc[i][j][e];
+					out.store(C + matrix * stride_c + static_cast<size_t>(m) * N + n);
+				}
+				else
+				{
+					const float vals[4] = { acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3] };
+					local.apply(m, n, vals, column[j], extra[i][j]);
+				}
+			}
+		}
+	}
+
+	template<int KB, int BLOCKS_M, int BLOCKS_N, int WAVES_M, int WAVES_N, typename Epilogue>
+	inline void launch_gemm_direct_as(hipStream_t stream, const StreamGemmArgs &g, const Epilogue &epilogue)
+	{
+		const int tiles_m = ceil_div(g.M, 16 * BLOCKS_M * WAVES_M), tiles_n = ceil_div(g.N, 16 * BLOCKS_N * WAVES_N);
+		constexpr int LDS = KB * 16 * (BLOCKS_M * WAVES_M + BLOCKS_N * WAVES_N);
+		auto kernel = kernel_gemm_direct_nt<KB, BLOCKS_M, BLOCKS_N, WAVES_M, WAVES_N, Epilogue>;
+		if (LDS > 64 * 1024)
+			ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), LDS);
+		hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned int>(tiles_m) * tiles_n * g.batch), dim3(64 * WAVES_M * WAVES_N), LDS, stream, reinterpret_cast<const half_t*>(g.A),
+				reinterpret_cast<const half_t*>(g.B), reinterpret_cast<half_t*>(g.C), g.M, g.N, g.stride_a, g.stride_b, g.stride_c, tiles_m, tiles_n,
+				g.a_row_bytes != 0 ? g.a_row_bytes : static_cast<size_t>(KB), epilogue);
+	}
+	/*
+	 * Whether this kernel takes a product: the tiles per compute unit at which it and the streaming kernel are level. Every tile fetches
+	 * its rows of A and B anew (KB * 128 bytes), where the streaming kernel fetches A once; 8 tiles of 64 KB per compute unit are level at
+	 * 512-byte rows (1024 rows x 36), and at 768-byte rows, where a tile of 96 KB is alone on its compute unit, only 2.
+	 */
+	inline bool gemm_direct_applies(int M, int N, int batch, size_t k_bytes)
+	{
+		if (!(k_bytes == 128 || k_bytes == 256 || k_bytes == 384 || k_bytes == 512 || k_bytes == 768))
+			return false;
+		const long long tiles = static_cast<long long>(ceil_div(M, 64)) * ceil_div(N, 64) * batch;
+		return tiles <= static_cast<long long>(device_compute_units()) * ((k_bytes <= 512) ? 8 : 2);
+	}
+	template<int KB, typename Epilogue>
+	inline void launch_gemm_direct_kb(hipStream_t stream, const StreamGemmArgs &g, const Epilogue &epilogue)
+	{
+		/* 64 x 64 tiles once they fill every compute unit twice: at one tile each the smaller shape is level or faster (M = 96: 4.3
+		 * against 4.9 us, M = 256: 6.9 against 6.7 us) */
+		const long long tiles = static_cast<long long>(ceil_div(g.M, 64)) * ceil_div(g.N, 64) * g.batch;
+		if (tiles >= 2LL * device_compute_units())
+			launch_gemm_direct_as<KB, 1, 2, 4, 2>(stream, g, epilogue);
+		else
+			launch_gemm_direct_as<KB, 1, 1, 2, 2>(stream, g, epilogue);
+	}
+	template<typename Epilogue>
+	inline void launch_gemm_direct(hipStream_t stream, const StreamGemmArgs &g, const Epilogue &epilogue)
+	{
+		switch (g.k_bytes)
+		{
+			case 128:
+				launch_gemm_direct_kb<128>(stream, g, epilogue);
+				break;
+			case 256:
+				launch_gemm_direct_kb<256>(stream, g, epilogue);
+				break;
+			case 384:
+				launch_gemm_direct_kb<384>(stream, g, epilogue);
+				break;
+			case 512:
+				launch_gemm_direct_kb<512>(stream, g, epilogue);
+				break;
+			case 768:
+				launch_gemm_direct_kb<768>(stream, g, epilogue);
+				break;
+			default:
+				fail_logic("HIP backend: direct GEMM: unsupported K row length");
+		}
+	}
+} /* namespace mlhip */
+
+#endif /* MINML_AMD_GEMM_DIRECT_HPP_ */

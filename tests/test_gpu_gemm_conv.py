@@ -170,6 +170,35 @@ def test_gemm_ex_streaming_shapes(ctx, dtype, k_bytes, M, N):
         assert max_abs_rel(dD.copyToHost(ctx), want) <= TOL[dtype]
 
 
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 384])
+@pytest.mark.parametrize("bt,M,N", [(1, 1, 4), (36, 16, 256), (3, 31, 36), (2, 33, 100), (36, 65, 128), (36, 130, 260), (5, 257, 64), (1, 1350, 768)])
+def test_few_rows_equal_many_rows(ctx, K, bt, M, N):
+    """fp16 products too small for the streaming kernel (32 x 32 and 64 x 64 tiles with the whole K in LDS): ragged rows and columns around
+    both tile sizes, every K row length, bare and with bias + beta * C + ReLU, against the oracle; and bit for bit the first rows of a
+    product large enough for the streaming kernel or the tile engine, because a position's result must not depend on its batch."""
+    rng = np.random.default_rng(K + bt + M + N)
+    big = 36000 // bt
+    A = random_tensor(rng, (bt, M, K), "float16", 0.3)
+    A[:, :: 7] = O.to_half(O.from_half(A[:, :: 7]) * 300.0)  # rows of another magnitude
+    Bm = random_tensor(rng, (bt, N, K), "float16", 0.3)
+    dB = ml.toDevice(ctx, Bm)
+    dC = ml.Tensor((bt, M, N), "float16")
+    dC.setall(ctx, float("nan"))
+    ml.gemmBatched(ctx, "n", "t", dC, ml.toDevice(ctx, A), dB, 1.0, 0.0)
+    few = dC.copyToHost(ctx)
+    assert max_abs_rel(few, O.gemm(A, Bm)) <= TOL["float16"]
+    many = np.zeros((bt, big, K), np.uint16)
+    many[:, :M] = A
+    dM = ml.Tensor((bt, big, N), "float16")
+    ml.gemmBatched(ctx, "n", "t", dM, ml.toDevice(ctx, many), dB, 1.0, 0.0)
+    assert np.array_equal(dM.copyToHost(ctx)[:, :M], few)
+    C, bias = random_tensor(rng, (M, N), "float16"), random_tensor(rng, (N,), "float16")
+    dD = ml.Tensor((M, N), "float16")
+    dD.setall(ctx, float("nan"))
+    ml.gemm_ex(ctx, dD, 1.1, "n", ml.toDevice(ctx, A[0]), "t", ml.toDevice(ctx, Bm[0]), 0.5, ml.toDevice(ctx, C), ml.toDevice(ctx, bias), "relu")
+    assert max_abs_rel(dD.copyToHost(ctx), O.gemm(A[0], Bm[0], alpha=1.1, beta=0.5, C=C, bias=bias, act=O.RELU)) <= TOL["float16"]
+
+
 @pytest.mark.parametrize("dtype", ["float32", "float16"])
 @pytest.mark.parametrize("N", [192, 320, 384, 448, 130, 576])
 def test_gemm_ex_tile_engine_widths(ctx, dtype, N):
