@@ -676,6 +676,188 @@ namespace
 		fused_transform_phase2<T, VEC, SLICE, THREADS, false>(g, lds_bytes);
 	}
 
+	/*
+	 * The same launch for few images. One workgroup per image and 64 channels leaves most of the chip idle there, and it is slow by itself:
+	 * a compute unit moves about one 64-byte piece per 3 clocks whatever the width of the instruction, so the 36 loads and 36 stores of 16
+	 * tiles x 128 bytes take 7000 clocks, and its four wavefronts issue the arithmetic of 16 tiles back to back (another 10000). Here a
+	 * workgroup owns ONE ROW of tiles of an image (a strip of 4 pixel rows) and 16 channels, one channel per lane. The strip's input
+	 * transform needs one more pixel row above and below: wavefront 0 runs the output transform of the strip's own tiles, wavefronts 1 and
+	 * 2 repeat that of the tile rows above and below for the one pixel row that is needed (30 of 36 loads, a third of the arithmetic). y
+	 * goes through LDS as [6][4 * tiles_w + 2][16] with zeros outside the image, so that the windows of phase 2 are read at constant
+	 * offsets. Results are bit-identical to the kernel above (same expressions), but nothing that is read may be written by the same
+	 * launch: neighbouring strips read one another's rows. 15x15 at 256 channels, one image: 7.8 -> 4.2 us, with residual and stored y
+	 * 9.4 -> 4.5 us (2 channels per lane: 4.6 / 4.9, 4: 6.2 / 6.8).
+	 */
+	constexpr int STRIP_CHANNELS = 16;
+	template<typename T, int ACT, bool HAS_EXT>
+	__global__ __launch_bounds__(192) void kernel_output_input_transform_strips(const T *__restrict__ matrices, T *output, const T *__restrict__ bias, const T *ext,
+			T *__restrict__ next_matrices, int batch_size, int height, int width, int channels, int tiles_h, int tiles_w)
+	{
+		typedef typename RawVec<T, 1>::type raw_t;
+		constexpr int SLICE = STRIP_CHANNELS;
+		extern __shared__ __attribute__((aligned(16))) uint8_t lds_bytes[];
+		T *pixels = reinterpret_cast<T*>(lds_bytes); /* [6][pitch][SLICE] */
+		const int pitch = 4 * tiles_w + 2;
+		const unsigned int slices = channels / SLICE;
+		/* the 4 slices that share 128-byte lines run on one XCD, everything else goes round the XCDs: few workgroups must spread over the chip */
+		const unsigned int lin = xcd_run_block_id(blockIdx.x, gridDim.x, 4);
+		const unsigned int strip_id = lin / slices;
+		const unsigned int slice = lin - strip_id * slices;
+		const unsigned int batch = strip_id / tiles_h;
+		const int strip = strip_id - batch * tiles_h;
+		const size_t matrix_stride = static_cast<size_t>(batch_size) * tiles_h * tiles_w * channels;
+		const size_t image_pixels = static_cast<size_t>(batch) * height * width;
+		const int channel_local = threadIdx.x & 15;
+		const unsigned int channel = slice * SLICE + channel_local;
+		const int tile_lane = threadIdx.x >> 4; /* 0 .. 11; 4 per wavefront */
+
+		/* FIRST .. FIRST + COUNT - 1: the output rows that are wanted of the tiles of `tile_row`; lds_row: where row FIRST goes */
+		const auto output_rows = [&](auto first_tag, auto count_tag, int tile_row, int lds_row) __attribute__((always_inline))
+		{
+			constexpr int FIRST = decltype(first_tag)::value, COUNT = decltype(count_tag)::value;
+			const int lane_of_wave = tile_lane & 3;
+			const int x0 = 4 * tile_row;
+			Vec<T, 1> zero;
+			zero.zero();
+			if (tile_row < 0 || tile_row >= tiles_h)
+			{ /* beyond the image: a row of zeros */
+				for (int i = lane_of_wave; i < pitch; i += 4)
+					zero.store(pixels + (lds_row * pitch + i) * SLICE + channel_local);
+				return;
+			}
+			if (lane_of_wave < COUNT)
+			{ /* the columns left and right of the image */
+				zero.store(pixels + (lds_row + lane_of_wave) * pitch * SLICE + channel_local);
+				zero.store(pixels + ((lds_row + lane_of_wave) * pitch + pitch - 1) * SLICE + channel_local);
+			}
+			T *y = (output != nullptr && COUNT == 4) ? output + image_pixels * channels + channel : nullptr;
+			const T *residual_base = HAS_EXT ? ext + image_pixels * channels + channel : nullptr;
+#pragma clang loop unroll(disable)
+			for (int tile = lane_of_wave; tile < tiles_w; tile += 4)
+			{
+				/* the position's matrix in scalar registers, the lane's place in it as a 32-bit offset; an edge row depends on 5 of the 6 rows */
+				constexpr int FIRST_ROW = (FIRST == 3) ? 1 : 0, LAST_ROW = (FIRST + COUNT == 1) ? 4 : 5;
+				const T *plane = matrices + static_cast<size_t>(batch) * tiles_h * tiles_w * channels + FIRST_ROW * 6 * matrix_stride;
+				const uint32_t place = ((tile_row * tiles_w + tile) * channels + channel) * sizeof(T);
+				raw_t raw[6][6];
+#pragma unroll
+				for (int row = FIRST_ROW; row <= LAST_ROW; row++)
+#pragma unroll
+					for (int col = 0; col < 6; col++)
+					{
+						raw[row][col] = *reinterpret_cast<const raw_t*>(reinterpret_cast<const uint8_t*>(plane) + place);
+						plane += matrix_stride;
+					}
+				if constexpr (COUNT == 1)
+#pragma unroll
+					for (int col = 0; col < 6; col++)
+						raw[(FIRST_ROW == 1) ? 0 : 5][col] = raw[1][col]; /* any value: the wanted row does not depend on it */
+				int offset[COUNT][4]; /* of the outputs within the image, clamped into it */
+				raw_t residual[COUNT][4];
+#pragma unroll
+				for (int row = 0; row < COUNT; row++)
+#pragma unroll
+					for (int col = 0; col < 4; col++)
+					{
+						offset[row][col] = (min(x0 + FIRST + row, height - 1) * width + min(4 * tile + col, width - 1)) * channels;
+						if constexpr (HAS_EXT)
+							residual[row][col] = *reinterpret_cast<const raw_t*>(residual_base + offset[row][col]);
+					}
+				Vec<T, 1> b;
+				b.zero();
+				if (bias != nullptr)
+					b.load(bias + channel);
+
+				float tmp[COUNT][6][1];
+#pragma unroll
+				for (int col = 0; col < 6; col++)
+				{
+					float line[6][1], res[4][1];
+#pragma unroll
+					for (int row = 0; row < 6; row++)
+						line[row][0] = RawVec<T, 1>::get(raw[row][col], 0);
+					output_transform_1d<1>(line, res);
+#pragma unroll
+					for (int row = 0; row < COUNT; row++)
+						tmp[row][col][0] = res[FIRST + row][0];
+				}
+#pragma unroll
+				for (int row = 0; row < COUNT; row++)
+				{
+					float res[4][1];
+					output_transform_1d<1>(tmp[row], res);
+					const bool row_inside = (x0 + FIRST + row) < height;
+#pragma unroll
+					for (int col = 0; col < 4; col++)
+					{
+						const bool inside = row_inside && (4 * tile + col) < width;
+						float t = res[col][0] + b.v[0];
+						if constexpr (HAS_EXT)
+							t = t + RawVec<T, 1>::get(residual[row][col], 0);
+						if constexpr (ACT == 1)
+							t = fmaxf(t, 0.0f);
+						Vec<T, 1> out;
+						out.v[0] = inside ? t : 0.0f;
+						out.store(pixels + ((lds_row + row) * pitch + 1 + 4 * tile + col) * SLICE + channel_local);
+						if (COUNT == 4 && y != nullptr && inside)
+							out.store(y + offset[row][col]);
+					}
+				}
+			}
+		};
+		const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+		typedef std::integral_constant<int, 0> row_0;
+		typedef std::integral_constant<int, 1> one_row;
+		if (wave == 0)
+			output_rows(row_0(), std::integral_constant<int, 4>(), strip, 1);
+		else if (wave == 1)
+			output_rows(std::integral_constant<int, 3>(), one_row(), strip - 1, 0);
+		else
+			output_rows(row_0(), one_row(), strip + 1, 5);
+		__syncthreads();
+
+#pragma clang loop unroll(disable)
+		for (int tile = tile_lane; tile < tiles_w; tile += 12)
+		{
+			const T *window = pixels + 4 * tile * SLICE + channel_local;
+			raw_t raw[6][6];
+#pragma unroll
+			for (int row = 0; row < 6; row++)
+#pragma unroll
+				for (int col = 0; col < 6; col++)
+					raw[row][col] = *reinterpret_cast<const raw_t*>(window + (row * pitch + col) * SLICE);
+			float tmp[6][6][1];
+#pragma unroll
+			for (int col = 0; col < 6; col++)
+			{
+				float line[6][1], res[6][1];
+#pragma unroll
+				for (int row = 0; row < 6; row++)
+					line[row][0] = RawVec<T, 1>::get(raw[row][col], 0);
+				input_transform_1d<1>(line, res);
+#pragma unroll
+				for (int row = 0; row < 6; row++)
+					tmp[row][col][0] = res[row][0];
+			}
+			T *plane = next_matrices + static_cast<size_t>(batch * tiles_h + strip) * tiles_w * channels + slice * SLICE;
+			const uint32_t place = (tile * channels + channel_local) * sizeof(T);
+#pragma unroll
+			for (int row = 0; row < 6; row++)
+			{
+				float res[6][1];
+				input_transform_1d<1>(tmp[row], res);
+#pragma unroll
+				for (int col = 0; col < 6; col++)
+				{
+					Vec<T, 1> out;
+					out.v[0] = res[col][0];
+					out.store(reinterpret_cast<T*>(reinterpret_cast<uint8_t*>(plane) + place));
+					plane += matrix_stride;
+				}
+			}
+		}
+	}
+
 	/* ---------------------------------------------------------------------------------------------------------------------
 	 * A whole 3x3 layer in one launch (fp16, 256 -> 256 channels, 16 tiles per image):
 	 *   V [36][T][256] x U [36][256][256]^T -> M -> output transform (+ bias, + ext, activation) -> y -> input transform -> V' [36][T][256]
@@ -1042,8 +1224,9 @@ namespace
 		}
 		MLHIP_CHECK(hipGetLastError());
 	}
-	/* fused output + next input transform: channels must be a multiple of 64 and 4-element accesses aligned */
-	template<typename T, int SLICE, int VEC, int THREADS>
+	/* fused output + next input transform: channels must be a multiple of 64 and 4-element accesses aligned; COMMON_ACT_ONLY / EXT_ALLOWED:
+	 * the caller has checked that the activation is linear or ReLU / that there is no residual, other forms are not instantiated */
+	template<typename T, int SLICE, int VEC, int THREADS, bool COMMON_ACT_ONLY, bool EXT_ALLOWED>
 	void launch_output_input(hipStream_t stream, const mlTensor_t &matrices, const mlTensor_t &bias, const mlTensor_t &ext, const mlShape_t &shape, void *output,
 			mlActivationType_t act, mlTensor_t &next)
 	{
@@ -1066,25 +1249,60 @@ namespace
 				ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), static_cast<int>(lds)); \
 			hipLaunchKernelGGL(kernel, grid, block, lds, stream, in, out, b, e, a, nxt, batch, height, width, channels, tiles_h, tiles_w); \
 		} while (0)
-		if (e != nullptr)
+		if constexpr (EXT_ALLOWED)
 		{
-			if (mode == 0)
-				MLHIP_LAUNCH_FUSED(0, true);
-			else if (mode == 1)
-				MLHIP_LAUNCH_FUSED(1, true);
-			else
-				MLHIP_LAUNCH_FUSED(2, true);
+			if (e != nullptr)
+			{
+				if (mode == 0)
+					MLHIP_LAUNCH_FUSED(0, true);
+				else if (mode == 1)
+					MLHIP_LAUNCH_FUSED(1, true);
+				else if constexpr (!COMMON_ACT_ONLY)
+					MLHIP_LAUNCH_FUSED(2, true);
+			}
 		}
-		else
+		if (e == nullptr)
 		{
 			if (mode == 0)
 				MLHIP_LAUNCH_FUSED(0, false);
 			else if (mode == 1)
 				MLHIP_LAUNCH_FUSED(1, false);
-			else
+			else if constexpr (!COMMON_ACT_ONLY)
 				MLHIP_LAUNCH_FUSED(2, false);
 		}
 #undef MLHIP_LAUNCH_FUSED
+		MLHIP_CHECK(hipGetLastError());
+	}
+	/* linear or ReLU activation; nothing the launch reads may overlap what it writes */
+	template<typename T>
+	void launch_output_input_strips(hipStream_t stream, const mlTensor_t &matrices, const mlTensor_t &bias, const mlTensor_t &ext, const mlShape_t &shape,
+			void *output, mlActivationType_t act, mlTensor_t &next)
+	{
+		const int batch = shape.dim[0], height = shape.dim[1], width = shape.dim[2], channels = shape.dim[3];
+		const int tiles_h = ceil_div(height, 4), tiles_w = ceil_div(width, 4);
+		const size_t lds = static_cast<size_t>(6) * (4 * tiles_w + 2) * STRIP_CHANNELS * sizeof(T);
+		const dim3 grid(static_cast<unsigned int>(batch) * tiles_h * (channels / STRIP_CHANNELS));
+		const T *in = ptr<const T>(matrices), *b = ptr<const T>(bias), *e = ptr<const T>(ext);
+		T *out = reinterpret_cast<T*>(output), *nxt = ptr<T>(next);
+		const bool relu = (act == ACTIVATION_RELU);
+#define MLHIP_LAUNCH_STRIPS(ACT, EXT) \
+		hipLaunchKernelGGL((kernel_output_input_transform_strips<T, ACT, EXT>), grid, dim3(192), lds, stream, in, out, b, e, nxt, batch, height, width, channels, \
+				tiles_h, tiles_w)
+		if (e != nullptr)
+		{
+			if (relu)
+				MLHIP_LAUNCH_STRIPS(1, true);
+			else
+				MLHIP_LAUNCH_STRIPS(0, true);
+		}
+		else
+		{
+			if (relu)
+				MLHIP_LAUNCH_STRIPS(1, false);
+			else
+				MLHIP_LAUNCH_STRIPS(0, false);
+		}
+#undef MLHIP_LAUNCH_STRIPS
 		MLHIP_CHECK(hipGetLastError());
 	}
 }
@@ -1317,12 +1535,47 @@ extern "C"
 			return;
 		}
 		mlTensor_t next = next_matrices;
-		/* 64-channel slices, 256 threads, two workgroups per CU. Measured alternatives that were not faster: slices of 128 or 256 channels
-		 * (longer contiguous segments) with 512 or 1024 threads, and 2-element vectors at twice the occupancy. */
+		/*
+		 * Which form, by the number of 64-channel slices of images (= workgroups of the widest form) for 256 compute units; measured, us,
+		 * without / with residual and stored y, 256 channels 15x15 fp16 (other widths, boards and fp32 agree):
+		 *   slices                              4           24          64          128          256          1024
+		 *   64 channels per workgroup        7.8 / 9.4   8.0 / 9.6   8.5 / 10.0   9.0 / 10.6  10.7 / 14.3  28.0 / 40
+		 *   32 channels                      7.3 / 9.4   7.7 / 10.1  6.1 / 7.7    6.9 / 8.8    9.7 / 17.3  38.8 / 61
+		 *   16 channels                      8.4 / 9.4  10.0 / 11.8  6.6 / 7.4    8.4 / 9.5   12.5 / 17.4  54.5 / 80
+		 *   strips of 16 channels            4.2 / 4.5   5.3 / 5.8   7.4 / 8.6   10.7 / 11.9  15.2 / 19.8  48.3 / 70
+		 * (a launch over few images is bound by what one workgroup must issue, a launch over many by memory, which wants whole 128-byte
+		 * lines; with residual the 16-channel form is ahead of the 32-channel one in fp32 and level in fp16). Measured alternatives that were
+		 * not faster for many images: slices of 128 or 256 channels with 512 or 1024 threads, and 2-element vectors at twice the occupancy.
+		 */
+		const hipStream_t stream = stream_of(context);
+		const long long slices = static_cast<long long>(output_shape.dim[0]) * (channels / 64), units = device_compute_units();
+		const bool common_act = (act == ACTIVATION_LINEAR || act == ACTIVATION_RELU);
+		/* a strip reads residual pixels and product rows that its neighbours own: nothing it reads may be written by this launch */
+		const auto overlap = [](const void *p, size_t p_bytes, const void *q, size_t q_bytes)
+		{
+			const uint8_t *a = static_cast<const uint8_t*>(p), *b = static_cast<const uint8_t*>(q);
+			return a != nullptr && b != nullptr && a < b + q_bytes && b < a + p_bytes;
+		};
+		const size_t y_bytes = volume(output_shape) * esize, m_bytes = 36 * tiles * channels * esize;
+		const bool separate = !overlap(output, y_bytes, ext.data, y_bytes) && !overlap(next.data, m_bytes, ext.data, y_bytes)
+				&& !overlap(output, y_bytes, matrices.data, m_bytes) && !overlap(next.data, m_bytes, matrices.data, m_bytes);
+		const auto launch = [&](auto zero)
+		{
+			typedef decltype(zero) T;
+			const bool strips_fit = static_cast<size_t>(6) * (4 * ceil_div(output_shape.dim[2], 4) + 2) * STRIP_CHANNELS * sizeof(T) <= 64 * 1024;
+			if (common_act && separate && strips_fit && 10 * slices <= units)
+				launch_output_input_strips<T>(stream, matrices, bias, ext, output_shape, output, act, next);
+			else if (common_act && (ext.data == nullptr) && 4 * slices > units && slices <= units)
+				launch_output_input<T, 32, 2, 256, true, false>(stream, matrices, bias, ext, output_shape, output, act, next);
+			else if (common_act && 2 * slices <= units)
+				launch_output_input<T, 16, 1, 256, true, true>(stream, matrices, bias, ext, output_shape, output, act, next);
+			else
+				launch_output_input<T, 64, 4, 256, false, true>(stream, matrices, bias, ext, output_shape, output, act, next);
+		};
 		if (matrices.dtype == DTYPE_FLOAT16)
-			launch_output_input<half_t, 64, 4, 256>(stream_of(context), matrices, bias, ext, output_shape, output, act, next);
+			launch(half_t(0));
 		else
-			launch_output_input<float, 64, 4, 256>(stream_of(context), matrices, bias, ext, output_shape, output, act, next);
+			launch(0.0f);
 	}
 	catch (...)
 	{

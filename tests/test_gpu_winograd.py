@@ -197,6 +197,36 @@ def test_fused_output_input_transform_bit_exact(ctx, dtype, shape):
     assert mismatches(dy3.copyToHost(ctx), dy2.copyToHost(ctx)) == 0
 
 
+@pytest.mark.parametrize("dtype", ["float32", "float16"])
+@pytest.mark.parametrize("shape", [(6, 15, 15, 256), (3, 17, 20, 128), (1, 1, 3, 64), (2, 5, 30, 64), (1, 3, 1100, 64), (7, 9, 11, 256), (22, 6, 5, 256),
+                                   (9, 19, 19, 512), (70, 4, 7, 256)])
+def test_fused_output_input_transform_forms(ctx, dtype, shape):
+    """The forms of the fused transform for different numbers of 64-channel slices of images: strips of one tile row (up to 25 slices;
+    several tile columns per wavefront, boards that end inside a tile, one row, too wide for the strips' LDS), 16 or 32 channels per
+    workgroup, 64. Bit for bit against the oracle; and with y written over the residual, which the strips must leave to another form."""
+    rng = np.random.default_rng(sum(shape))
+    b, h, w, c = shape
+    tiles = b * ((h + 3) // 4) * ((w + 3) // 4)
+    m, bias, ext = random_tensor(rng, (36, tiles, c), dtype), random_tensor(rng, (c,), dtype), random_tensor(rng, shape, dtype)
+    dm, db, de = ml.toDevice(ctx, m), ml.toDevice(ctx, bias), ml.toDevice(ctx, ext)
+    dv, dy = ml.Tensor((36, tiles, c), dtype), ml.Tensor(shape, dtype)
+    for with_ext, act, keep in ((False, O.RELU, False), (True, O.RELU, True), (True, O.LINEAR, False), (False, O.LINEAR, True)):
+        if not keep and (h * w + 1) * 64 * (2 if dtype == "float16" else 4) > 160 * 1024:
+            continue  # the entry point's two-kernel route
+        want_y = O.winograd_output_transform(m, shape, bias, ext if with_ext else None, act)
+        dv.setall(ctx, float("nan"))
+        dy.setall(ctx, 7.0)
+        ml.winogradOutputInputTransform(ctx, (c, 3, 3, c), dm, shape, dy if keep else None, db, de if with_ext else None, act, dv)
+        want_v = O.winograd_input_transform(want_y)
+        assert mismatches(dv.copyToHost(ctx), want_v) == 0
+        if keep:
+            assert mismatches(dy.copyToHost(ctx), want_y) == 0
+        if keep and with_ext:
+            ml.winogradOutputInputTransform(ctx, (c, 3, 3, c), dm, shape, de, db, de, act, dv)
+            assert mismatches(dv.copyToHost(ctx), want_v) == 0 and mismatches(de.copyToHost(ctx), want_y) == 0
+            de = ml.toDevice(ctx, ext)
+
+
 @pytest.mark.parametrize("case", [(32, 15, 15, True, True, O.RELU), (64, 13, 16, False, False, O.RELU), (36, 15, 15, True, False, O.LINEAR),
                                   (256, 15, 15, True, True, O.RELU), (8, 15, 15, True, True, O.RELU), (32, 19, 19, True, True, O.RELU)])
 def test_whole_layer_launch_is_bit_identical(ctx, case):
