@@ -16,6 +16,8 @@ One difference by design: kernel sizes other than 1 and 3 use the fused implicit
 point only on cuDNN builds, Conv2D.cpp:478-485) because on this backend it needs no im2row workspace; `algorithm=` overrides the choice.
 The int8 path has the reference's three-call sequence ("reference") and the single fused launch ("fused").
 """
+import math
+
 import numpy as np
 
 from . import backend as B
@@ -145,7 +147,7 @@ class Conv2D:
         """(input matrices, output matrices): views at element 0 and 36*T*Cin of the workspace (Conv2D.cpp:365-367)."""
         in_shape = get_matrices_shape(self.kernel_size, self.winograd_tile_size, (batch,) + self.input_shape[1:])
         out_shape = get_matrices_shape(self.kernel_size, self.winograd_tile_size, (batch,) + self.output_shape[1:])
-        return workspace.view(in_shape), workspace.view(out_shape, int(np.prod(in_shape)))
+        return workspace.view(in_shape), workspace.view(out_shape, math.prod(in_shape))
 
     def winograd_input(self, x, workspace):
         input_matrices, _ = self._winograd_views(x.shape[0], workspace)
@@ -168,9 +170,9 @@ class Conv2D:
         """Output transform of this layer fused with the input transform of `next_layer` (a Winograd layer on this layer's output,
         sharing the workspace): the next layer's input matrices land at element 0, where this layer's are no longer needed.
         `output` may be None when nothing else reads this layer's result."""
-        _, output_matrices = self._winograd_views(batch, workspace)
+        input_matrices, output_matrices = self._winograd_views(batch, workspace)
         next_input, _ = next_layer._winograd_views(batch, workspace)
-        if next_input.volume() > self._winograd_views(batch, workspace)[0].volume():
+        if next_input.volume() > input_matrices.volume():
             raise ValueError("the next layer's input matrices would overlap this layer's output matrices in the workspace")
         out_shape = (batch,) + self.output_shape[1:]
         ml.winogradOutputInputTransform(self.context, self.weight_shape, output_matrices, out_shape, output, self.bias, add, self.activation, next_input)

@@ -9,6 +9,7 @@ Where the reference asserts (shape / dtype / device agreement) these functions r
 the library reports errors the reference's way, by C++ exceptions across the C boundary, which cannot be caught from Python.
 """
 import ctypes
+import math
 
 import numpy as np
 
@@ -162,10 +163,7 @@ class Tensor:
         return self.shape[i]
 
     def volume(self):
-        v = 1
-        for d in self.shape:
-            v *= d
-        return v if self.shape else 0
+        return math.prod(self.shape) if self.shape else 0
 
     def firstDim(self):
         return self.shape[0]
@@ -180,13 +178,16 @@ class Tensor:
         return self.volume() == 0
 
     def view(self, shape, offset=0):
-        """Non-owning tensor over the same memory, `offset` in elements (reference: Tensor::view)."""
-        shape = tuple(int(d) for d in shape)
-        vol = int(np.prod(shape)) if shape else 0
-        if offset + vol > self.volume():
+        """Non-owning tensor over the same memory, `offset` in elements (reference: Tensor::view; hip_create_view is the same sum of
+        address and offset). A pass over a network makes several hundred of these, so they are put together field by field."""
+        shape = tuple(map(int, shape))
+        volume = math.prod(shape) if shape else 0
+        if offset + volume > self.volume():
             raise ValueError("view exceeds the tensor")
-        p = B.fn("create_view")(self.ptr, offset * B.DTYPE_SIZE[self.dtype], vol * B.DTYPE_SIZE[self.dtype])
-        return Tensor(shape, self.dtype, self.device_index, _ptr=p, _owner=self)
+        v = Tensor.__new__(Tensor)
+        v.shape, v.dtype, v.device_index, v._owner, v._owning = shape, self.dtype, self.device_index, self, False
+        v.ptr = self.ptr + offset * B.DTYPE_SIZE[self.dtype]
+        return v
 
     def reinterpretAs(self, dtype):
         """Same bytes, other element type; the last dimension is rescaled (used for the int32 view of the workspace)."""
