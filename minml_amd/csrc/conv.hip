@@ -16,6 +16,7 @@
 #include "epilogues.hpp"
 #include "gemm_launch.hpp"
 #include "gemm_dma.hpp"
+#include "conv_tiles.hpp"
 #include "conv_window.hpp"
 #include "gemm_dma_window.hpp"
 
@@ -247,8 +248,29 @@ namespace
 			a_loader.c_bytes = static_cast<int>(c_bytes);
 			a_loader.fill = 0;
 			const DenseDmaRows b_loader { reinterpret_cast<const uint8_t*>(weights), filters_out, static_cast<int>(k_bytes) };
+			ConvTileArgs tile_args = conv_tile_args(input, weights, M, filters_out, height, width, kernel_h, kernel_w, c_bytes, 0);
+			/* layers that the windowed tiles take at larger batches: K in their order, and no other engine between the two */
+			tile_args.slices_first = sizeof(T) == 2 && conv_dma_window_applies(c_bytes, filters_out, kernel_h, kernel_w, height, width);
+			const auto few_rows = [&](const auto &ep)
+			{
+				return tile_args.slices_first ? try_launch_small_tiles<T>(stream, tile_args, ep)
+						: try_launch_fewer_rows<T>(stream, a_loader, b_loader, tile_args, ep);
+			};
+			bool launched = false;
 			if constexpr (sizeof(T) == 2)
-				if (conv_dma_window_applies(c_bytes, filters_out, kernel_h, kernel_w, height, width))
+				specialise_epilogue(make_epilogue(), [&](const auto &ep)
+				{
+					launched = few_rows(ep);
+				});
+			else
+				launched = few_rows(make_epilogue());
+			if (launched)
+			{
+				MLHIP_CHECK(hipGetLastError());
+				return;
+			}
+			if constexpr (sizeof(T) == 2)
+				if (tile_args.slices_first)
 				{ /* the tiles' rows are consecutive pixels: the window of pixels they share enters LDS once per 128-byte slice of the channels */
 					specialise_epilogue(make_epilogue(), [&](const auto &ep)
 					{
@@ -267,6 +289,20 @@ namespace
 		}
 		else if (fast)
 		{
+			const ConvTileArgs tile_args = conv_tile_args(input, weights, M, filters_out, height, width, kernel_h, kernel_w, c_bytes, 0);
+			bool launched = false;
+			if constexpr (sizeof(T) == 2)
+				specialise_epilogue(make_epilogue(), [&](const auto &ep)
+				{
+					launched = try_launch_straddling<T>(stream, tile_args, ep);
+				});
+			else
+				launched = try_launch_straddling<T>(stream, tile_args, make_epilogue());
+			if (launched)
+			{
+				MLHIP_CHECK(hipGetLastError());
+				return;
+			}
 			typedef TileConfig<128, 128, 64, 2, 2> Cfg;
 			Im2RowRows<T> a_loader;
 			a_loader.base = reinterpret_cast<const T*>(input);

@@ -21,6 +21,7 @@
 #include "gemm_stream.hpp"
 #include "gemm_direct.hpp"
 #include "gemm_dma.hpp"
+#include "conv_tiles.hpp"
 
 namespace
 {
@@ -302,6 +303,18 @@ namespace mlhip
 		const DenseDmaRows dma_a { reinterpret_cast<const uint8_t*>(g.A), g.M, static_cast<int>(k_bytes) };
 		const DenseDmaRows dma_b { reinterpret_cast<const uint8_t*>(g.B), g.N, static_cast<int>(k_bytes) };
 
+		/* the same operands as the tile engine sees them, for the products whose rows are too few to fill its tiles */
+		const auto few_rows = [&](auto zero, const auto &ep)
+		{
+			typedef decltype(zero) T;
+			ConvTileArgs args = dense_tile_args(dma_a, dma_b, g.M, g.N, static_cast<int>(k_bytes));
+			args.batch = g.batch;
+			args.stride_input = g.stride_a * esize;
+			args.stride_weights = g.stride_b * esize;
+			args.stride_out = g.stride_c;
+			return try_launch_fewer_rows<T>(stream, dma_a, dma_b, args, ep);
+		};
+
 		typedef TileConfig<128, 128, 64, 2, 2> Cfg;
 		const int tiles_m = ceil_div(g.M, Cfg::BM), tiles_n = ceil_div(g.N, Cfg::BN);
 		const dim3 fast_grid(static_cast<unsigned int>(tiles_m) * tiles_n, g.batch);
@@ -323,6 +336,8 @@ namespace mlhip
 				ep.beta = g.beta;
 				ep.act = g.act;
 				ep.vectorized = vectorized;
+				if (dma && few_rows(half_t(0), ep))
+					break;
 				if (dma)
 					launch_gemm_dma<half_t>(stream, dma_a, dma_b, g.M, g.N, static_cast<int>(k_bytes), g.batch, g.stride_a * esize, g.stride_b * esize,
 							g.stride_c, ep);
@@ -352,6 +367,8 @@ namespace mlhip
 				ep.beta = g.beta;
 				ep.act = g.act;
 				ep.vectorized = vectorized;
+				if (dma && few_rows(0.0f, ep))
+					break;
 				if (dma)
 					launch_gemm_dma<float>(stream, dma_a, dma_b, g.M, g.N, static_cast<int>(k_bytes), g.batch, g.stride_a * esize, g.stride_b * esize,
 							g.stride_c, ep);
@@ -373,6 +390,8 @@ namespace mlhip
 				ep.N = g.N;
 				ep.row_stride = g.N;
 				ep.vectorized = vectorized;
+				if (dma && few_rows(int8_t(0), ep))
+					break;
 				if (dma)
 					launch_gemm_dma<int8_t>(stream, dma_a, dma_b, g.M, g.N, static_cast<int>(k_bytes), g.batch, g.stride_a * esize, g.stride_b * esize,
 							g.stride_c, ep);

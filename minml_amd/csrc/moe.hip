@@ -17,6 +17,7 @@
 #include "device_utils.hpp"
 #include "epilogues.hpp"
 #include "gemm_dma.hpp"
+#include "conv_tiles.hpp"
 #include "gemm_stream.hpp"
 
 namespace
@@ -784,6 +785,11 @@ extern "C"
 			DenseDmaRows a_loader { reinterpret_cast<const uint8_t*>(x.data), static_cast<int>(rows), static_cast<int>(k_bytes) };
 			a_loader.row_stride_bytes = static_cast<int>(static_cast<size_t>(experts) * k_bytes);
 			const DenseDmaRows b_loader { reinterpret_cast<const uint8_t*>(w.data), neurons, static_cast<int>(k_bytes) };
+			ConvTileArgs tile_args = dense_tile_args(a_loader, b_loader, static_cast<int>(rows), neurons, static_cast<int>(k_bytes));
+			tile_args.batch = experts;
+			tile_args.stride_input = k_bytes;
+			tile_args.stride_weights = static_cast<size_t>(neurons) * k_bytes;
+			tile_args.stride_out = neurons;
 			const auto launch = [&](auto zero)
 			{
 				typedef decltype(zero) T;
@@ -803,6 +809,8 @@ extern "C"
 				if constexpr (sizeof(T) == 2)
 					specialise_epilogue(ep, [&](const auto &fixed)
 					{
+						if (try_launch_small_tiles<T>(stream, tile_args, fixed))
+							return;
 						if (vectorized && stream_gemm_half_applies(static_cast<int>(rows), experts, k_bytes))
 						{
 							/* short K rows (the layer that widens 256 channels to the hidden width): the streaming kernel, whose B operand
@@ -812,11 +820,11 @@ extern "C"
 							sg.a_row_bytes = static_cast<size_t>(experts) * k_bytes;
 							launch_stream_gemm<T>(stream, sg, fixed);
 						}
-						else
+						else if (!try_launch_fewer_rows<T>(stream, a_loader, b_loader, tile_args, fixed))
 							launch_gemm_dma<T>(stream, a_loader, b_loader, static_cast<int>(rows), neurons, static_cast<int>(k_bytes), experts, k_bytes,
 									static_cast<size_t>(neurons) * k_bytes, static_cast<size_t>(neurons), fixed);
 					});
-				else
+				else if (!try_launch_fewer_rows<T>(stream, a_loader, b_loader, tile_args, ep))
 					launch_gemm_dma<T>(stream, a_loader, b_loader, static_cast<int>(rows), neurons, static_cast<int>(k_bytes), experts, k_bytes,
 							static_cast<size_t>(neurons) * k_bytes, static_cast<size_t>(neurons), ep);
 			};

@@ -16,6 +16,7 @@
 #include "gemm_core.hpp"
 #include "epilogues.hpp"
 #include "gemm_dma.hpp"
+#include "conv_tiles.hpp"
 
 #include <cmath>
 
@@ -207,13 +208,26 @@ namespace
 			a_loader.c_bytes = filters_in;
 			a_loader.fill = input_zero & 0xff; /* a 1x1 kernel never pads, so an out-of-range zero point is harmless there */
 			const DenseDmaRows b_loader { reinterpret_cast<const uint8_t*>(weights), filters_out, static_cast<int>(k_bytes) };
+			const ConvTileArgs tile_args = conv_tile_args(input, weights, M, filters_out, height, width, kernel_h, kernel_w, filters_in, a_loader.fill);
 			specialise_epilogue(ep, [&](const auto &fixed)
 			{
-				launch_gemm_dma<int8_t>(stream, a_loader, b_loader, M, filters_out, static_cast<int>(k_bytes), 1, 0, 0, 0, fixed);
+				if (!try_launch_fewer_rows<int8_t>(stream, a_loader, b_loader, tile_args, fixed))
+					launch_gemm_dma<int8_t>(stream, a_loader, b_loader, M, filters_out, static_cast<int>(k_bytes), 1, 0, 0, 0, fixed);
 			});
 		}
 		else if (fast)
 		{
+			const ConvTileArgs tile_args = conv_tile_args(input, weights, M, filters_out, height, width, kernel_h, kernel_w, filters_in, input_zero & 0xff);
+			bool launched = false;
+			specialise_epilogue(ep, [&](const auto &fixed)
+			{
+				launched = try_launch_straddling<int8_t>(stream, tile_args, fixed);
+			});
+			if (launched)
+			{
+				MLHIP_CHECK(hipGetLastError());
+				return;
+			}
 			typedef TileConfig<128, 128, 64, 2, 2> Cfg;
 			Im2RowRows<int8_t> a_loader;
 			a_loader.base = reinterpret_cast<const int8_t*>(input);

@@ -283,6 +283,32 @@ def test_fused_convolution(ctx, dtype, shape, cout, k):
     assert max_abs_rel(dy.copyToHost(ctx), O.conv2d_forward(x, wt)) <= TOL[dtype]
 
 
+@pytest.mark.parametrize("dtype", ["float32", "float16"])
+@pytest.mark.parametrize("shape,cout,k", [((1, 1, 3, 8), 4, 3), ((1, 11, 3, 16), 33, 3), ((5, 9, 7, 72), 100, 3), ((2, 4, 5, 56), 36, 2),
+                                          ((3, 19, 19, 128), 128, 3), ((1, 9, 10, 256), 260, 5), ((20, 19, 19, 24), 96, 3), ((26, 15, 15, 64), 260, 3),
+                                          ((100, 17, 15, 8), 192, 3), ((70, 19, 19, 128), 128, 3), ((300, 19, 19, 32), 128, 5), ((90, 19, 19, 64), 256, 3), ((2, 15, 15, 192), 768, 1), ((1, 7, 31, 640), 72, 1)])
+def test_convolution_of_few_positions(ctx, dtype, shape, cout, k):
+    """The small output tiles (32 x 32, 64 x 64, 128 x 64, 128 x 128) at the edges of their shapes, of K and of the rules that choose
+    them, against the oracle; and the first image bit for bit as it comes out of a smaller batch, which another tile or engine may
+    serve, down to the 256-row tiles (300 images)."""
+    rng = np.random.default_rng(cout * k + shape[0])
+    b, h, w, cin = shape
+    x = random_tensor(rng, shape, dtype)
+    wt = random_tensor(rng, (cout, k, k, cin), dtype, (2.0 / (k * k * cin)) ** 0.5)
+    bias = random_tensor(rng, (cout,), dtype)
+    add = random_tensor(rng, (b, h, w, cout), dtype)
+    dw, db = ml.toDevice(ctx, wt), ml.toDevice(ctx, bias)
+    O.set_num_threads(8)
+    dy = ml.Tensor((b, h, w, cout), dtype)
+    dy.setall(ctx, float("nan"))
+    ml.convolutionImplicitGemmForward(ctx, ml.toDevice(ctx, x), dw, dy, db, ml.toDevice(ctx, add), "relu")
+    got = dy.copyToHost(ctx)
+    assert max_abs_rel(got, O.conv2d_forward(x, wt, bias, add, O.RELU)) <= TOL[dtype]
+    one = ml.Tensor((1, h, w, cout), dtype)
+    ml.convolutionImplicitGemmForward(ctx, ml.toDevice(ctx, np.ascontiguousarray(x[:1])), dw, one, db, ml.toDevice(ctx, np.ascontiguousarray(add[:1])), "relu")
+    assert np.array_equal(one.copyToHost(ctx), got[:1])
+
+
 def test_conv_sweep_config4_shapes(ctx):
     """19x19 boards, fp16, channel widths {64,128,256,384}, kernels 1 / 3 / 5 with bias + ReLU + residual, at a batch the oracle finishes."""
     rng = np.random.default_rng(44)

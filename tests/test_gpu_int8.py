@@ -84,6 +84,36 @@ def test_int8_convolution_bit_exact(ctx, shape, cout, k, act):
         assert mismatches(dy.copyToHost(ctx), want) == 0
 
 
+@pytest.mark.parametrize("shape,cout,k", [((1, 1, 3, 16), 4, 3),  # one tile, K shorter than a ring slot, taps of one 16-byte chunk
+                                          ((1, 11, 3, 32), 33, 3),  # 33 rows and columns: one past the 32 x 32 tile; not a multiple of 4
+                                          ((5, 9, 7, 144), 100, 3),  # pieces that straddle taps, K not a whole slot
+                                          ((3, 19, 19, 128), 128, 5), ((2, 4, 5, 112), 36, 2),  # an even kernel
+                                          ((20, 19, 19, 48), 96, 3),  # 32 x 32 tiles no longer resident at once: 64 x 64
+                                          ((41, 15, 15, 128), 260, 3),  # 64 x 64, a column past a tile
+                                          ((100, 17, 15, 16), 192, 3),  # straddling and too many 64 x 64 tiles: 128 x 64
+                                          ((130, 15, 15, 128), 128, 1)])  # one piece of K, 128 x 128
+def test_int8_convolution_of_few_positions(ctx, shape, cout, k):
+    """The small output tiles against the oracle, bit for bit, at the edges of their shapes, of K and of the rules that choose them; the
+    input's zero point is not 0, so a padding tap and a piece past the end of K must read different bytes."""
+    b, h, w, cin = shape
+    rng = np.random.default_rng(cout * k + b)
+    x = rng.integers(-128, 128, shape).astype(np.int8)
+    wt = rng.integers(-127, 128, (cout, k, k, cin)).astype(np.int8)
+    scales = (rng.random(cout) * 0.002 + 0.0005).astype(np.float32)
+    bias = rng.standard_normal(cout).astype(np.float32)
+    ext = rng.integers(-128, 128, (b, h, w, cout)).astype(np.int8)
+    dx, dw, ds, db, de = (ml.toDevice(ctx, a) for a in (x, wt, scales, bias, ext))
+    O.set_num_threads(8)
+    for code, act, use_ext in ((O.INT8, "relu", True), (O.FLOAT32, "linear", False), (O.INT8, "sigmoid", True)):
+        want = O.int8_conv2d_forward(x, IN_QD, wt, scales, bias, code, OUT_QD, ext if use_ext else None, EXT_QD, ml.act_of(act))
+        dy = ml.Tensor((b, h, w, cout), code)
+        ml.quantizedConvForward(ctx, dx, IN_QD, dw, ds, db, dy, OUT_QD, de if use_ext else None, EXT_QD, act)
+        if act == "sigmoid":  # the device's exponential may differ from the host's in the last bit: at most one step of the output
+            assert np.abs(dy.copyToHost(ctx).astype(np.int32) - want.astype(np.int32)).max() <= 1
+        else:
+            assert mismatches(dy.copyToHost(ctx), want) == 0
+
+
 def test_quantized_network_layer_config3(ctx):
     """Config 3's recipe on one residual-block convolution: per-output-channel symmetric int8 weights (scale = max|w| / 127), per-tensor
     symmetric activations (shift 0), int32 accumulation, requantisation with fused bias + ReLU. Quantised parameters come from the
