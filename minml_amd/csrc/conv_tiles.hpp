@@ -11,11 +11,12 @@
  * The tap of every 16-byte chunk is tracked per lane, so any channel count of whole 16-byte chunks is served, and K past its end reads
  * zeros: gemm_core.hpp's register-staged tiles, which these shapes took before, have one buffer of lookahead.
  *
- * Measured, us per launch, before -> now (tile): int8 3x3, 15x15 positions: 128 channels 9 positions 14.6 -> 5.0 (32 x 32), 32: 14.8 -> 7.2
+ * Measured, us per launch, before -> now (tile): int8 3x3, 15x15 positions: 128 channels 9 positions 14.6 -> 5.1 (32 x 32), 32: 14.8 -> 7.1
  * (64 x 64), 96: 15.7 -> 12.1, 128: 16.1 -> 12.1 (128 x 128, gemm_dma.hpp); 256 channels 9: 34.9 -> 7.3, 32: 34.1 -> 13.8, 80: 36.3 -> 25.8;
- * 96 channels 9: 18.8 -> 4.9, 256: 24.4 -> 21.3 (128 x 64), 1024: 79 -> 68; 64 channels 1024: 55 -> 33; 192 channels 1024: 217 -> 164.
+ * 96 channels 9: 18.8 -> 4.9, 256: 24.4 -> 21.3 (128 x 64), 1024: 79 -> 68; 64 channels 1024: 55 -> 33; 192 channels 1024: 217 -> 162.
  * fp16, 19x19 positions: 5x5 of 256 channels 1: 131 -> 24, 16: 133 -> 52, 64: 141 -> 112; 3x3 of 128 channels 4: 19.7 -> 6.7; 3x3 of 384
- * channels 4: 63 -> 22. fp32 3x3 of 256 channels, 19x19, 1: 541 -> 25, 8: 549 -> 55, 64: 562 -> 254.
+ * channels 4: 63 -> 22. fp32 3x3 of 256 channels, 19x19, 1: 541 -> 33, 8: 548 -> 68, 64: 560 -> 260. The order
+ * of K is a template parameter: decided at run time it cost the smallest tile 0.6 of 5.7 us.
  */
 #ifndef MINML_AMD_CONV_TILES_HPP_
 #define MINML_AMD_CONV_TILES_HPP_
@@ -126,7 +127,7 @@ namespace mlhip
 			static_assert((DISTANCE - 1) * LOADS <= 63 && LDS_BYTES <= 160 * 1024, "queue depth and LDS");
 	};
 
-	template<typename T, typename Cfg, typename Epilogue>
+	template<typename T, typename Cfg, bool SLICES_FIRST, typename Epilogue>
 	__global__ __launch_bounds__(64 * Cfg::WAVES) void kernel_conv_tiles(ConvTileArgs g, unsigned int tiles_n, Epilogue epilogue)
 	{
 		typedef Mfma16Traits<T> Traits;
@@ -182,7 +183,7 @@ namespace mlhip
 		settle();
 		const auto next_piece = [&]()
 		{
-			if (g.slices_first)
+			if constexpr (SLICES_FIRST)
 			{
 				kb += g.c_bytes;
 				if (++tap_j == g.kernel_w)
@@ -210,7 +211,7 @@ namespace mlhip
 #pragma unroll
 			for (int p = 0; p < Cfg::PIECES; p++)
 			{
-				const bool in_k = g.slices_first ? c < g.c_bytes : kb < g.k_bytes; /* past the end of K both operands read zeros */
+				const bool in_k = SLICES_FIRST ? c < g.c_bytes : kb < g.k_bytes; /* past the end of K both operands read zeros */
 				const uint8_t *padding = &dma_pad_table.bytes[in_k ? g.fill : 0][0];
 #pragma unroll
 				for (int u = 0; u < Cfg::A_LOADS; u++)
@@ -256,29 +257,26 @@ namespace mlhip
 		const auto multiply = [&](int step)
 		{
 			const uint8_t *slot = lds + (step % Cfg::SLOTS) * Cfg::SLOT_BYTES;
-			constexpr int PER_PIECE = 128 / Traits::STEP;
+			constexpr int PER_PIECE = 128 / Traits::STEP, K_STEPS = Cfg::PIECES * PER_PIECE;
+			typename Traits::Fragment a[K_STEPS][Cfg::BLOCKS_M], b[K_STEPS][Cfg::BLOCKS_N];
 #pragma unroll
-			for (int p = 0; p < Cfg::PIECES; p++)
+			for (int t = 0; t < K_STEPS; t++)
 			{
-				typename Traits::Fragment a[PER_PIECE][Cfg::BLOCKS_M], b[PER_PIECE][Cfg::BLOCKS_N];
+				const uint8_t *piece = slot + (t / PER_PIECE) * Cfg::PIECE_BYTES;
 #pragma unroll
-				for (int t = 0; t < PER_PIECE; t++)
-				{
+				for (int i = 0; i < Cfg::BLOCKS_M; i++)
+					a[t][i] = Traits::load(piece + (a_first[i] ^ ((t % PER_PIECE) * Traits::STEP)), quarter);
 #pragma unroll
-					for (int i = 0; i < Cfg::BLOCKS_M; i++)
-						a[t][i] = Traits::load(slot + p * Cfg::PIECE_BYTES + (a_first[i] ^ (t * Traits::STEP)), quarter);
+				for (int j = 0; j < Cfg::BLOCKS_N; j++)
+					b[t][j] = Traits::load(piece + (b_first[j] ^ ((t % PER_PIECE) * Traits::STEP)), quarter);
+			}
+#pragma unroll
+			for (int t = 0; t < K_STEPS; t++)
+#pragma unroll
+				for (int i = 0; i < Cfg::BLOCKS_M; i++)
 #pragma unroll
 					for (int j = 0; j < Cfg::BLOCKS_N; j++)
-						b[t][j] = Traits::load(slot + p * Cfg::PIECE_BYTES + (b_first[j] ^ (t * Traits::STEP)), quarter);
-				}
-#pragma unroll
-				for (int t = 0; t < PER_PIECE; t++)
-#pragma unroll
-					for (int i = 0; i < Cfg::BLOCKS_M; i++)
-#pragma unroll
-						for (int j = 0; j < Cfg::BLOCKS_N; j++)
-							Traits::mma(b[t][j], a[t][i], acc[i][j]);
-			}
+						Traits::mma(b[t][j], a[t][i], acc[i][j]);
 		};
 		/* step s is readable once its loads have landed in every wavefront; the same barrier frees the slot of step s - 1 */
 		int s = 0;
@@ -339,11 +337,17 @@ namespace mlhip
 	template<typename T, typename Cfg, typename Epilogue>
 	inline void launch_conv_tiles_as(hipStream_t stream, const ConvTileArgs &g, const Epilogue &epilogue)
 	{
-		auto kernel = kernel_conv_tiles<T, Cfg, Epilogue>;
-		ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), Cfg::LDS_BYTES);
-		const int tiles_m = ceil_div(g.M, Cfg::BM), tiles_n = ceil_div(g.N, Cfg::BN);
-		hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned int>(tiles_m) * tiles_n, g.batch), dim3(64 * Cfg::WAVES), Cfg::LDS_BYTES, stream, g,
-				static_cast<unsigned int>(tiles_n), epilogue);
+		const auto launch = [&](auto kernel)
+		{
+			ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), Cfg::LDS_BYTES);
+			const int tiles_m = ceil_div(g.M, Cfg::BM), tiles_n = ceil_div(g.N, Cfg::BN);
+			hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned int>(tiles_m) * tiles_n, g.batch), dim3(64 * Cfg::WAVES), Cfg::LDS_BYTES, stream, g,
+					static_cast<unsigned int>(tiles_n), epilogue);
+		};
+		if constexpr (sizeof(T) == 2) /* only fp16 layers have windowed tiles */
+			if (g.slices_first)
+				return launch(kernel_conv_tiles<T, Cfg, true, Epilogue>);
+		launch(kernel_conv_tiles<T, Cfg, false, Epilogue>);
 	}
 
 	typedef ConvTileConfig<1, 1, 2, 2, 2, 4> ConvTile32; /* 64 KB of LDS: two workgroups per compute unit */
@@ -389,7 +393,7 @@ namespace mlhip
 	 *     at K = 2304, 450 tiles: 28.4 against 38.0 us, 900 tiles: 53.5 against 43.6); at most 128 columns, where the tile is only half of
 	 *     the 256-row one, up to one per compute unit (225 tiles 12.1 against 16.1 us, 450 tiles 18.8 against 18.0)
 	 *   fp32: the matrix pipe is the limit and an idle compute unit costs most: 128 x 64 tiles while the 256-row tiles leave a quarter of
-	 *     the units idle (46208 x 128, 181 tiles of 256 x 128: 134 against 157 us; 23104 x 256, 91 tiles of 256 x 256: 254 against 562)
+	 *     the units idle (46208 x 128, 181 tiles of 256 x 128: 139 against 157 us; 23104 x 256, 91 tiles of 256 x 256: 260 against 560)
 	 */
 	template<typename T, typename ALoader, typename Epilogue>
 	inline bool try_launch_fewer_rows(hipStream_t stream, const ALoader &a_loader, const DenseDmaRows &b_loader, const ConvTileArgs &g, const Epilogue &epilogue)
