@@ -192,6 +192,7 @@ namespace
 			int table_size; /* 2 r - 1 positions per direction, 0 = no bias */
 			int table_row; /* table_size rounded up to a multiple of 4 */
 			float scale; /* 1 / sqrt(head_dim) */
+			int splits = 1; /* workgroups that share the query rows of one head */
 	};
 
 	__device__ __forceinline__ int clamp_int(int x, int lower, int upper)
@@ -258,8 +259,14 @@ namespace
 	};
 	constexpr float LOG2_E = 1.4426950408889634f;
 
-	template<typename T, int D, int BIAS>
-	__global__ __launch_bounds__(256) void kernel_attention_mfma(const T *__restrict__ input, T *__restrict__ output, const T *__restrict__ table,
+	/*
+	 * THREADS = 256 where there are more (image, head) pairs than compute units. With fewer, the launch lasts as long as one workgroup:
+	 * the staging loop and then query blocks one after the other on each wavefront. 512 threads stage in half the rounds and give every
+	 * query block of a 15x15 board a wavefront of its own, and where compute units are left over `splits` workgroups share a head, so
+	 * that no two of those wavefronts share a SIMD. Every query row is computed by the same instructions either way.
+	 */
+	template<typename T, int D, int BIAS, int THREADS>
+	__global__ __launch_bounds__(THREADS) void kernel_attention_mfma(const T *__restrict__ input, T *__restrict__ output, const T *__restrict__ table,
 			AttentionShape shape)
 	{
 		typedef AttentionLds<T, D> Lds;
@@ -281,16 +288,18 @@ namespace
 
 		/* the heads of one image run on one XCD (images go round the XCDs): their q / k / v parts are neighbouring pieces of the same
 		 * token rows, which then meet in one L2 instead of being fetched through eight */
-		const unsigned int lin = (shape.heads > 1) ? xcd_run_block_id(blockIdx.x, gridDim.x, shape.heads) : blockIdx.x;
-		const int image = lin / shape.heads;
-		const int head = lin - image * shape.heads;
+		const int per_image = shape.heads * shape.splits;
+		const unsigned int lin = (per_image > 1) ? xcd_run_block_id(blockIdx.x, gridDim.x, per_image) : blockIdx.x;
+		const int image = lin / per_image;
+		const int head = (lin - image * per_image) / shape.splits;
+		const int split = lin - image * per_image - head * shape.splits;
 		const T *tokens_base = input + static_cast<size_t>(image) * tokens * shape.token_stride + head * D;
 		const int range = (shape.table_size - 1) / 2;
 		/* scores are kept in units of ln 2 (scale and table carry the factor log2 e) so that the exponential is the hardware's exp2 */
 		const float scale = shape.scale * LOG2_E;
 
 		/* ---- stage keys, transposed values, key places and the head's table ---- */
-		for (int i = threadIdx.x; i < tokens_padded * ROW_CHUNKS; i += 256)
+		for (int i = threadIdx.x; i < tokens_padded * ROW_CHUNKS; i += THREADS)
 		{
 			const int token = i / ROW_CHUNKS;
 			const int chunk = i - token * ROW_CHUNKS;
@@ -318,7 +327,7 @@ namespace
 					*reinterpret_cast<uint32_t*>(values + (chunk * 4 + e) * value_row + token * 4) = v[e];
 			}
 		}
-		for (int i = threadIdx.x; i < tokens_padded; i += 256)
+		for (int i = threadIdx.x; i < tokens_padded; i += THREADS)
 		{
 			const int token = (i < tokens) ? i : 0; /* padding keys are masked later; they only need a harmless place */
 			const int row = token / shape.width;
@@ -331,7 +340,7 @@ namespace
 		if constexpr (BIAS != BIAS_NONE)
 		{
 			const T *head_table = table + static_cast<size_t>(head) * shape.table_size * shape.table_row;
-			for (int i = threadIdx.x; i < shape.table_size * shape.table_row; i += 256)
+			for (int i = threadIdx.x; i < shape.table_size * shape.table_row; i += THREADS)
 				bias[i] = Storage<T>::load(head_table + i) * LOG2_E;
 		}
 		__syncthreads();
@@ -342,7 +351,7 @@ namespace
 		const int half_sel = lane >> 5;
 		const int key_blocks = tokens_padded / 32;
 
-		for (int query_block = wave; query_block < key_blocks; query_block += 4)
+		for (int query_block = split * (THREADS / 64) + wave; query_block < key_blocks; query_block += shape.splits * (THREADS / 64))
 		{
 			const int query = query_block * 32 + lane_row;
 			const bool query_valid = query < tokens;
@@ -557,23 +566,32 @@ namespace
 			return false;
 		const int height = shape.tokens / shape.width;
 		const int bias = (shape.table_size == 0) ? BIAS_NONE : ((shape.table_size >= 2 * std::max(height, shape.width) - 1) ? BIAS_DIRECT : BIAS_CLAMPED);
-		const void *kernel = nullptr;
-		switch (bias)
-		{
-			case BIAS_NONE:
-				kernel = reinterpret_cast<const void*>(&kernel_attention_mfma<T, D, BIAS_NONE>);
-				break;
-			case BIAS_DIRECT:
-				kernel = reinterpret_cast<const void*>(&kernel_attention_mfma<T, D, BIAS_DIRECT>);
-				break;
-			default:
-				kernel = reinterpret_cast<const void*>(&kernel_attention_mfma<T, D, BIAS_CLAMPED>);
-				break;
-		}
-		ensure_dynamic_lds(kernel, bytes);
 		AttentionShape shape_arg = shape;
-		void *args[] = { static_cast<void*>(&input), static_cast<void*>(&output), static_cast<void*>(&table), static_cast<void*>(&shape_arg) };
-		MLHIP_CHECK(hipLaunchKernel(kernel, dim3(batch * shape.heads), dim3(256), args, bytes, stream));
+		const int units = device_compute_units();
+		const long long pairs = static_cast<long long>(batch) * shape.heads;
+		const bool few = pairs <= units;
+		if (few) /* four wavefronts with a query block each occupy a compute unit; shared as far as there are units */
+			shape_arg.splits = static_cast<int>(std::max<long long>(1, std::min<long long>((shape.tokens + 127) / 128, units / std::max<long long>(pairs, 1))));
+		const auto launch = [&](const void *kernel, int threads)
+		{
+			ensure_dynamic_lds(kernel, bytes);
+			void *args[] = { static_cast<void*>(&input), static_cast<void*>(&output), static_cast<void*>(&table), static_cast<void*>(&shape_arg) };
+			MLHIP_CHECK(hipLaunchKernel(kernel, dim3(static_cast<unsigned int>(pairs) * shape_arg.splits), dim3(threads), args, bytes, stream));
+		};
+		const auto launch_with = [&](auto bias_form)
+		{
+			constexpr int BIAS = decltype(bias_form)::value;
+			if (few)
+				launch(reinterpret_cast<const void*>(&kernel_attention_mfma<T, D, BIAS, 512>), 512);
+			else
+				launch(reinterpret_cast<const void*>(&kernel_attention_mfma<T, D, BIAS, 256>), 256);
+		};
+		if (bias == BIAS_NONE)
+			launch_with(std::integral_constant<int, BIAS_NONE>());
+		else if (bias == BIAS_DIRECT)
+			launch_with(std::integral_constant<int, BIAS_DIRECT>());
+		else
+			launch_with(std::integral_constant<int, BIAS_CLAMPED>());
 		return true;
 	}
 	template<typename T>

@@ -91,6 +91,24 @@ def test_attention_shapes(ctx, dtype, case):
     assert max_abs_rel(got, want) <= TOL[dtype]
 
 
+@pytest.mark.parametrize("dtype", ["float32", "float16"])
+@pytest.mark.parametrize("few,board,heads,dim", [(1, (15, 15), 8, 32), (6, (15, 15), 8, 32), (3, (19, 19), 2, 64), (5, (9, 9), 3, 32), (1, (4, 33), 1, 128), (100, (5, 7), 2, 32)])
+def test_attention_of_few_images_equals_many(ctx, dtype, few, board, heads, dim):
+    """With fewer (image, head) pairs than compute units a head's query rows are spread over more wavefronts and workgroups: bit for bit
+    the same rows as in a batch that has one workgroup per pair."""
+    rng = np.random.default_rng(few + heads + dim)
+    many, e, size = 600 // heads, heads * dim, 2 * max(board) - 1
+    x = random_tensor(rng, (many,) + board + (3 * e,), dtype)
+    table = ml.toDevice(ctx, random_tensor(rng, (heads, size, (size + 3) // 4 * 4), dtype))
+    results = []
+    for n in (many, few):
+        y = ml.Tensor((n,) + board + (e,), dtype)
+        y.setall(ctx, float("nan"))
+        ml.multiHeadAttentionForward(ctx, ml.toDevice(ctx, np.ascontiguousarray(x[:n])), y, table, None, None, None, heads, False)
+        results.append(y.copyToHost(ctx))
+    assert np.array_equal(results[0][:few], results[1]) and np.isfinite(O.as_float(results[1])).all()
+
+
 def test_attention_special_cases(ctx):
     """Equal keys: every output is the mean of the values. A table that forbids every offset but one: each token copies the value of
     that neighbour. Sharp rows (large logits) stay finite through the running-maximum rescaling."""
