@@ -105,6 +105,122 @@ namespace
 		}
 	}
 
+	/* what a score and its token sort by: score descending, then token ascending; the score comes back as it was */
+	template<typename T>
+	struct RoutingKey;
+	template<>
+	struct RoutingKey<float>
+	{
+			typedef uint64_t type;
+			__device__ static __forceinline__ type make(const float *score, int token)
+			{
+				return (static_cast<uint64_t>(~ascending_bits(*score)) << 32) | static_cast<uint32_t>(token);
+			}
+			__device__ static __forceinline__ int token(type key)
+			{
+				return static_cast<int>(key & 0xffffffffu);
+			}
+			__device__ static __forceinline__ float score(type key)
+			{
+				return from_ascending_bits(~static_cast<uint32_t>(key >> 32));
+			}
+	};
+	template<>
+	struct RoutingKey<half_t>
+	{
+			typedef uint32_t type; /* half the registers and exchanges; fewer than 2^16 tokens */
+			__device__ static __forceinline__ type make(const half_t *score, int token)
+			{
+				uint32_t bits = *reinterpret_cast<const uint16_t*>(score);
+				if ((bits & 0x7fffu) > 0x7c00u)
+					bits |= 0x200u; /* a NaN as the conversion to fp32 leaves it */
+				const uint32_t ascending = bits ^ ((bits & 0x8000u) ? 0xffffu : 0x8000u);
+				return ((~ascending & 0xffffu) << 16) | static_cast<uint32_t>(token);
+			}
+			__device__ static __forceinline__ int token(type key)
+			{
+				return static_cast<int>(key & 0xffffu);
+			}
+			__device__ static __forceinline__ float score(type key)
+			{
+				const uint32_t ascending = ~(key >> 16) & 0xffffu;
+				return half_bits_to_float(static_cast<uint16_t>(ascending ^ ((ascending & 0x8000u) ? 0x8000u : 0xffffu)));
+			}
+	};
+	/*
+	 * The same for up to 64 * R tokens: one WAVEFRONT per (expert, image), the keys in its registers (key i in register i / 64 of lane
+	 * i % 64). A stage of the sort exchanges with another register or another lane and needs no barrier; the workgroup form above waits
+	 * at one after each of its 36 stages (225 tokens) with one exchange per thread between them. The four wavefronts of a workgroup take
+	 * consecutive experts, whose scores lie side by side.
+	 */
+	template<typename T, int R>
+	__global__ __launch_bounds__(256) void kernel_expert_choice_routing_waves(const T *scores, T *indices_and_values, int tokens, int experts, int capacity,
+			unsigned int rows)
+	{
+		typedef RoutingKey<T> Key;
+		typedef typename Key::type key_t;
+		const int lane = threadIdx.x & 63;
+		const unsigned int row = blockIdx.x * 4 + (threadIdx.x >> 6); /* image * experts + expert */
+		if (row >= rows)
+			return;
+		const unsigned int b = row / experts, e = row - b * experts;
+		key_t keys[R];
+#pragma unroll
+		for (int r = 0; r < R; r++)
+		{
+			const int t = r * 64 + lane;
+			const key_t key = Key::make(scores + (static_cast<size_t>(b) * tokens + min(t, tokens - 1)) * experts + e, t);
+			keys[r] = (t < tokens) ? key : ~static_cast<key_t>(0);
+		}
+#pragma unroll
+		for (int k = 2; k <= 64 * R; k <<= 1)
+#pragma unroll
+			for (int j = k >> 1; j > 0; j >>= 1)
+			{
+				if (j >= 64)
+				{
+#pragma unroll
+					for (int r = 0; r < R; r++)
+						if ((r & (j / 64)) == 0)
+						{
+							const key_t a = keys[r], c = keys[r | (j / 64)];
+							const bool swap = (a > c) == (((r * 64) & k) == 0);
+							keys[r] = swap ? c : a;
+							keys[r | (j / 64)] = swap ? a : c;
+						}
+				}
+				else
+				{
+#pragma unroll
+					for (int r = 0; r < R; r++)
+					{
+						const key_t own = keys[r], other = __shfl_xor(own, j);
+						const bool ascending = ((r * 64 + lane) & k) == 0;
+						const bool keep_smaller = ((lane & j) == 0) == ascending;
+						keys[r] = ((own < other) == keep_smaller) ? own : other;
+					}
+				}
+			}
+		T *index_row = indices_and_values + ((static_cast<size_t>(b) * 2 + 0) * experts + e) * capacity;
+		T *value_row = indices_and_values + ((static_cast<size_t>(b) * 2 + 1) * experts + e) * capacity;
+#pragma unroll
+		for (int r = 0; r < R; r++)
+		{
+			const int k = r * 64 + lane;
+			if (k < capacity && k < tokens)
+			{
+				const float s = Key::score(keys[r]);
+				Storage<T>::store(index_row + k, static_cast<float>(Key::token(keys[r])));
+				Storage<T>::store(value_row + k, 1.0f / (1.0f + expf(-s)));
+			}
+		}
+		for (int k = tokens + lane; k < capacity; k += 64)
+		{
+			Storage<T>::store(index_row + k, -1.0f);
+			Storage<T>::store(value_row + k, 0.0f);
+		}
+	}
+
 	/*
 	 * One workgroup per image. Every token takes the expert with the largest score + bias (the lowest index among equals); its gate is
 	 * softmax(scores)[that expert] with the maximum of score + bias as the shift, kept in the storage type; the tokens are then sorted
@@ -587,12 +703,29 @@ extern "C"
 			return;
 		MLHIP_REQUIRE(x.data != nullptr && indices_and_values.data != nullptr && batch <= 65535, "expert_choice_routing_forward: null tensor or batch above 65535");
 		const dim3 grid(experts, batch);
+		const auto launch = [&](auto zero)
+		{
+			typedef decltype(zero) T;
+			const unsigned int rows = static_cast<unsigned int>(experts) * batch; /* at most 4096 * 65535 */
+			const auto waves = [&](auto registers)
+			{
+				hipLaunchKernelGGL((kernel_expert_choice_routing_waves<T, decltype(registers)::value>), dim3((rows + 3) / 4), dim3(256), 0, stream_of(context),
+						ptr<const T>(x), ptr<T>(indices_and_values), tokens, experts, capacity, rows);
+			};
+			if (tokens > 0 && tokens <= 64)
+				waves(std::integral_constant<int, 1>());
+			else if (tokens > 64 && tokens <= 256)
+				waves(std::integral_constant<int, 4>());
+			else if (tokens > 256 && tokens <= 512) /* boards up to 22x22 */
+				waves(std::integral_constant<int, 8>());
+			else
+				hipLaunchKernelGGL(kernel_expert_choice_routing<T>, grid, dim3(256), 0, stream_of(context), ptr<const T>(x), ptr<T>(indices_and_values),
+						tokens, experts, capacity);
+		};
 		if (x.dtype == DTYPE_FLOAT16)
-			hipLaunchKernelGGL(kernel_expert_choice_routing<half_t>, grid, dim3(256), 0, stream_of(context), ptr<const half_t>(x), ptr<half_t>(indices_and_values),
-					tokens, experts, capacity);
+			launch(half_t(0));
 		else
-			hipLaunchKernelGGL(kernel_expert_choice_routing<float>, grid, dim3(256), 0, stream_of(context), ptr<const float>(x), ptr<float>(indices_and_values),
-					tokens, experts, capacity);
+			launch(0.0f);
 		MLHIP_CHECK(hipGetLastError());
 	}
 	catch (...)

@@ -49,6 +49,32 @@ def test_expert_choice_routing(ctx, dtype, shape, capacity):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "float16"])
+@pytest.mark.parametrize("tokens,experts,capacity", [(1, 1, 3), (63, 5, 64), (64, 3, 20), (65, 8, 65), (225, 8, 56), (256, 3, 256), (257, 7, 300), (400, 8, 100),
+                                                     (512, 2, 512), (513, 2, 513)])
+def test_expert_choice_routing_order(ctx, dtype, tokens, experts, capacity):
+    """The wavefront sort at the edges of its register counts (and one token past it), against a sort of the same total order on the
+    host: scores descending by their bits, equal ones by token; many ties, infinities, zeros of both signs and NaN among them."""
+    rng = np.random.default_rng(tokens + experts)
+    values = np.array([0.0, -0.0, np.inf, -np.inf, np.nan, 1.0, 1.0, -2.5, 6e-8, 0.125], np.float32)
+    s = values[rng.integers(0, values.size, (3, 1, tokens, experts))]
+    s = np.where(rng.random(s.shape) < 0.4, rng.standard_normal(s.shape).astype(np.float32), s).astype(np.float16 if dtype == "float16" else np.float32)
+    bits = s.astype(np.float32).view(np.uint32)
+    ascending = (bits ^ np.where(bits >> 31, np.uint32(0xffffffff), np.uint32(0x80000000))).astype(np.int64)
+    iv = ml.Tensor((3, 2, experts, capacity), dtype)
+    ml.expertChoiceRoutingForward(ctx, ml.toDevice(ctx, s.view(np.uint16) if dtype == "float16" else s), iv)
+    got = iv.copyToHost(ctx)
+    index, gate = index_plane(got), gate_plane(got)
+    taken = min(tokens, capacity)
+    for b in range(3):
+        for e in range(experts):
+            order = np.argsort(-ascending[b, 0, :, e], kind="stable")[:taken]
+            assert np.array_equal(index[b, e, :taken], order) and (index[b, e, taken:] == -1).all() and (gate[b, e, taken:] == 0).all()
+            with np.errstate(over="ignore"):
+                want = 1.0 / (1.0 + np.exp(-s[b, 0, order, e].astype(np.float64)))
+            assert np.allclose(gate[b, e, :taken], want, rtol=0.0, atol=1e-6 if dtype == "float32" else 1e-3, equal_nan=True)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float16"])
 @pytest.mark.parametrize("shape,capacity", [((3, 15, 15, 8), 57), ((2, 5, 7, 6), 35), ((2, 4, 4, 3), 3), ((1, 19, 19, 16), 30)])
 def test_token_choice_routing(ctx, dtype, shape, capacity):
     rng = np.random.default_rng(sum(shape) + capacity + 1)
