@@ -1544,7 +1544,8 @@ extern "C"
 		 *   16 channels                      8.4 / 9.4  10.0 / 11.8  6.6 / 7.4    8.4 / 9.5   12.5 / 17.4  54.5 / 80
 		 *   strips of 16 channels            4.2 / 4.5   5.3 / 5.8   7.4 / 8.6   10.7 / 11.9  15.2 / 19.8  48.3 / 70
 		 * (a launch over few images is bound by what one workgroup must issue, a launch over many by memory, which wants whole 128-byte
-		 * lines; with residual the 16-channel form is ahead of the 32-channel one in fp32 and level in fp16). Measured alternatives that were
+		 * lines; with residual the 16-channel form is ahead of the 32-channel one in fp32 and level in fp16 as long as all its workgroups run
+		 * at once: 90 slices of 384 channels take 14.2 us as 360 workgroups of it, 11.8 as 90 of the widest). Measured alternatives that were
 		 * not faster for many images: slices of 128 or 256 channels with 512 or 1024 threads, and 2-element vectors at twice the occupancy.
 		 */
 		const hipStream_t stream = stream_of(context);
@@ -1565,10 +1566,10 @@ extern "C"
 			const bool strips_fit = static_cast<size_t>(6) * (4 * ceil_div(output_shape.dim[2], 4) + 2) * STRIP_CHANNELS * sizeof(T) <= 64 * 1024;
 			if (common_act && separate && strips_fit && 10 * slices <= units)
 				launch_output_input_strips<T>(stream, matrices, bias, ext, output_shape, output, act, next);
-			else if (common_act && (ext.data == nullptr) && 4 * slices > units && slices <= units)
-				launch_output_input<T, 32, 2, 256, true, false>(stream, matrices, bias, ext, output_shape, output, act, next);
-			else if (common_act && 2 * slices <= units)
+			else if (common_act && 4 * slices <= units)
 				launch_output_input<T, 16, 1, 256, true, true>(stream, matrices, bias, ext, output_shape, output, act, next);
+			else if (common_act && (ext.data != nullptr ? 2 : 1) * slices <= units)
+				launch_output_input<T, 32, 2, 256, true, true>(stream, matrices, bias, ext, output_shape, output, act, next);
 			else
 				launch_output_input<T, 64, 4, 256, false, true>(stream, matrices, bias, ext, output_shape, output, act, next);
 		};
