@@ -10,6 +10,7 @@ the library reports errors the reference's way, by C++ exceptions across the C b
 """
 import ctypes
 import math
+import operator
 
 import numpy as np
 
@@ -181,6 +182,7 @@ class Tensor:
         """Non-owning tensor over the same memory, `offset` in elements (reference: Tensor::view; hip_create_view is the same sum of
         address and offset). A pass over a network makes several hundred of these, so they are put together field by field."""
         shape = tuple(map(int, shape))
+        offset = operator.index(offset)  # an address made with a numpy integer would be one too, and no call takes such a pointer
         volume = math.prod(shape) if shape else 0
         if offset + volume > self.volume():
             raise ValueError("view exceeds the tensor")

@@ -147,6 +147,17 @@ def test_python_mirror_validates_before_calling_the_library():
         ml.quantized_scale_shift_act(ctx, FakeTensor((4, 8), "int8"), (1.0, 0.0), FakeTensor((4, 8), f32), FakeTensor((8,), f32), FakeTensor((8,), f32), "relu")
 
 
+@pytest.mark.parametrize("kind", [int, np.int64, np.uint32, np.int16])
+def test_views_take_any_integer_as_offset(kind):
+    """The offset of a view may be an integer of numpy: its address must still be one that a descriptor and a call can take."""
+    whole = ml.Tensor((8, 16), "float16", _ptr=0x7000)  # not owned: nothing is read from it or freed
+    part = whole.view((kind(2), 16), kind(48))
+    assert part.desc().data == 0x7000 + 96 and part.desc().rank == 2 and part.view((4,), kind(3)).desc().data == 0x7000 + 102
+    assert ctypes.c_void_p(part.ptr).value == 0x7000 + 96
+    with pytest.raises(ValueError):
+        whole.view((8,), kind(121))
+
+
 def test_flop_count_of_the_benchmark_network():
     """40 * 7.73e10 + 9.66e9 + 1.18e8 = 3.10e12 executed flops per batch of 1024 (benchmark configuration 2)."""
     net = ResNet.__new__(ResNet)
