@@ -398,7 +398,7 @@ namespace mlhip
 	template<typename T, typename ALoader, typename Epilogue>
 	inline bool try_launch_fewer_rows(hipStream_t stream, const ALoader &a_loader, const DenseDmaRows &b_loader, const ConvTileArgs &g, const Epilogue &epilogue)
 	{
-		if (g.batch > 65535)
+		if (g.batch > 65535 || g.k_bytes == 0) /* without taps no step of K would fetch the side inputs; the other engine's tail does */
 			return false;
 		if (try_launch_small_tiles<T>(stream, g, epilogue))
 			return true;
@@ -426,6 +426,8 @@ namespace mlhip
 	template<typename T, typename Epilogue>
 	inline bool try_launch_straddling(hipStream_t stream, const ConvTileArgs &g, const Epilogue &epilogue)
 	{
+		if (g.k_bytes == 0) /* as above */
+			return false;
 		if (try_launch_small_tiles<T>(stream, g, epilogue))
 			return true;
 		if (g.k_bytes <= 512 && tiles_of(g, 128, 64) > 4LL * device_compute_units())

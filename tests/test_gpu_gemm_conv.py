@@ -309,6 +309,31 @@ def test_convolution_of_few_positions(ctx, dtype, shape, cout, k):
     assert np.array_equal(one.copyToHost(ctx), got[:1])
 
 
+@pytest.mark.parametrize("dtype", ["float32", "float16", "int8"])
+@pytest.mark.parametrize("cin,extent", [(64, (0, 0)), (128, (0, 0)), (48, (0, 0)), (128, (3, 0)), (256, (0, 1))])
+def test_convolution_without_taps(ctx, dtype, cin, extent):
+    """A kernel of zero extent contributes nothing: what remains is act(bias + add), bit for bit as a kernel of zeros gives it."""
+    rng = np.random.default_rng(cin)
+    b, h, w, cout = 3, 9, 7, 36
+    add, results = None, []
+    if dtype == "int8":
+        x, add = (ml.toDevice(ctx, rng.integers(-128, 128, (b, h, w, c)).astype(np.int8)) for c in (cin, cout))
+        scales, bias = ml.toDevice(ctx, np.full(cout, 0.01, np.float32)), ml.toDevice(ctx, rng.standard_normal(cout).astype(np.float32))
+    else:
+        x, add = (ml.toDevice(ctx, random_tensor(rng, (b, h, w, c), dtype)) for c in (cin, cout))
+        bias = ml.toDevice(ctx, random_tensor(rng, (cout,), dtype))
+    for shape in ((cout,) + extent + (cin,), (cout, 3, 3, cin)):
+        weights, y = ml.Tensor(shape, dtype), ml.Tensor((b, h, w, cout), dtype)
+        weights.zeroall(ctx)
+        y.setall(ctx, 55)
+        if dtype == "int8":
+            ml.quantizedConvForward(ctx, x, (0.05, 0.0), weights, scales, bias, y, (0.07, 0.0), add, (0.07, 0.0), "relu")
+        else:
+            ml.convolutionImplicitGemmForward(ctx, x, weights, y, bias, add, "relu")
+        results.append(y.copyToHost(ctx))
+    assert np.array_equal(results[0], results[1]) and len(np.unique(results[0])) > 20
+
+
 def test_conv_sweep_config4_shapes(ctx):
     """19x19 boards, fp16, channel widths {64,128,256,384}, kernels 1 / 3 / 5 with bias + ReLU + residual, at a batch the oracle finishes."""
     rng = np.random.default_rng(44)
