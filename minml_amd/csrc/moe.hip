@@ -151,19 +151,18 @@ namespace
 	 * The same for up to 64 * R tokens: one WAVEFRONT per (expert, image), the keys in its registers (key i in register i / 64 of lane
 	 * i % 64). A stage of the sort exchanges with another register or another lane and needs no barrier; the workgroup form above waits
 	 * at one after each of its 36 stages (225 tokens) with one exchange per thread between them. The four wavefronts of a workgroup take
-	 * consecutive experts, whose scores lie side by side.
+	 * consecutive experts, whose scores lie side by side. Images are the grid's second dimension: one flat dimension of all pairs would
+	 * pass the 2^32 threads that a grid's dimension may have at sizes that the entry point accepts.
 	 */
 	template<typename T, int R>
-	__global__ __launch_bounds__(256) void kernel_expert_choice_routing_waves(const T *scores, T *indices_and_values, int tokens, int experts, int capacity,
-			unsigned int rows)
+	__global__ __launch_bounds__(256) void kernel_expert_choice_routing_waves(const T *scores, T *indices_and_values, int tokens, int experts, int capacity)
 	{
 		typedef RoutingKey<T> Key;
 		typedef typename Key::type key_t;
 		const int lane = threadIdx.x & 63;
-		const unsigned int row = blockIdx.x * 4 + (threadIdx.x >> 6); /* image * experts + expert */
-		if (row >= rows)
+		const int b = blockIdx.y, e = blockIdx.x * 4 + (threadIdx.x >> 6);
+		if (e >= experts)
 			return;
-		const unsigned int b = row / experts, e = row - b * experts;
 		key_t keys[R];
 #pragma unroll
 		for (int r = 0; r < R; r++)
@@ -702,15 +701,13 @@ extern "C"
 		if (batch == 0 || experts == 0 || capacity == 0)
 			return;
 		MLHIP_REQUIRE(x.data != nullptr && indices_and_values.data != nullptr && batch <= 65535, "expert_choice_routing_forward: null tensor or batch above 65535");
-		const dim3 grid(experts, batch);
 		const auto launch = [&](auto zero)
 		{
 			typedef decltype(zero) T;
-			const unsigned int rows = static_cast<unsigned int>(experts) * batch; /* at most 4096 * 65535 */
 			const auto waves = [&](auto registers)
 			{
-				hipLaunchKernelGGL((kernel_expert_choice_routing_waves<T, decltype(registers)::value>), dim3((rows + 3) / 4), dim3(256), 0, stream_of(context),
-						ptr<const T>(x), ptr<T>(indices_and_values), tokens, experts, capacity, rows);
+				hipLaunchKernelGGL((kernel_expert_choice_routing_waves<T, decltype(registers)::value>), dim3((experts + 3) / 4, batch), dim3(256), 0,
+						stream_of(context), ptr<const T>(x), ptr<T>(indices_and_values), tokens, experts, capacity);
 			};
 			if (tokens > 0 && tokens <= 64)
 				waves(std::integral_constant<int, 1>());
@@ -719,8 +716,8 @@ extern "C"
 			else if (tokens > 256 && tokens <= 512) /* boards up to 22x22 */
 				waves(std::integral_constant<int, 8>());
 			else
-				hipLaunchKernelGGL(kernel_expert_choice_routing<T>, grid, dim3(256), 0, stream_of(context), ptr<const T>(x), ptr<T>(indices_and_values),
-						tokens, experts, capacity);
+				hipLaunchKernelGGL(kernel_expert_choice_routing<T>, dim3(experts, batch), dim3(256), 0, stream_of(context), ptr<const T>(x),
+						ptr<T>(indices_and_values), tokens, experts, capacity);
 		};
 		if (x.dtype == DTYPE_FLOAT16)
 			launch(half_t(0));

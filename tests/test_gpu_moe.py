@@ -74,6 +74,23 @@ def test_expert_choice_routing_order(ctx, dtype, tokens, experts, capacity):
             assert np.allclose(gate[b, e, :taken], want, rtol=0.0, atol=1e-6 if dtype == "float32" else 1e-3, equal_nan=True)
 
 
+def test_expert_choice_routing_of_very_many_pairs(ctx):
+    """4096 experts and enough images that four (image, expert) pairs per workgroup of 256 threads pass 2^32 threads in one dimension."""
+    batch, experts = 16385, 4096
+    scores, iv = ml.Tensor((batch, 1, 2, experts), "float16"), ml.Tensor((batch, 2, experts, 1), "float16")
+    scores.setall(ctx, -1.0)
+    iv.setall(ctx, 9.0)
+    last = O.to_half(np.array([[-2.0] * experts, [0.0] * experts], np.float32))
+    scores.view((2, experts), (batch - 1) * 2 * experts).copyFromHost(ctx, last)  # the second token wins in the last image
+    ml.expertChoiceRoutingForward(ctx, scores, iv)
+    half = lambda first, count: O.from_half(iv.view((count, 2, experts), first * 2 * experts).copyToHost(ctx))
+    for first, count in ((0, 2), (8191, 3), (batch - 3, 2)):
+        got = half(first, count)
+        assert (got[:, 0] == 0.0).all() and np.allclose(got[:, 1], 1.0 / (1.0 + np.exp(1.0)), rtol=0.0, atol=1e-3)
+    got = half(batch - 1, 1)
+    assert (got[:, 0] == 1.0).all() and (got[:, 1] == 0.5).all()
+
+
 @pytest.mark.parametrize("dtype", ["float32", "float16"])
 @pytest.mark.parametrize("shape,capacity", [((3, 15, 15, 8), 57), ((2, 5, 7, 6), 35), ((2, 4, 4, 3), 3), ((1, 19, 19, 16), 30)])
 def test_token_choice_routing(ctx, dtype, shape, capacity):
