@@ -421,7 +421,8 @@ namespace mlhip
 	/*
 	 * Convolutions whose 128-byte pieces straddle taps. The register-staged 128 x 128 tiles (gemm_core.hpp) remain for K of at most 512
 	 * bytes and many tiles, where storing is most of the work and the wider tile reads its input once per 128 columns (int8, 32 -> 256
-	 * channels 3x3, 230400 pixels: 88 against 94 us; 14400 pixels: 12.6 against 9.4).
+	 * channels 3x3, 230400 pixels: 88 against 94 us; 14400 pixels: 12.6 against 9.4), and beyond 2^32 threads of these tiles, the most
+	 * that a launch can have: theirs are a quarter as many.
 	 */
 	template<typename T, typename Epilogue>
 	inline bool try_launch_straddling(hipStream_t stream, const ConvTileArgs &g, const Epilogue &epilogue)
@@ -430,7 +431,8 @@ namespace mlhip
 			return false;
 		if (try_launch_small_tiles<T>(stream, g, epilogue))
 			return true;
-		if (g.k_bytes <= 512 && tiles_of(g, 128, 64) > 4LL * device_compute_units())
+		const long long tiles = tiles_of(g, 128, 64);
+		if ((g.k_bytes <= 512 && tiles > 4LL * device_compute_units()) || tiles * 64 * ConvTile128x64::WAVES > 0xffffffffLL)
 			return false;
 		launch_conv_tiles_as<T, ConvTile128x64>(stream, g, epilogue);
 		return true;

@@ -334,6 +334,27 @@ def test_convolution_without_taps(ctx, dtype, cin, extent):
     assert np.array_equal(results[0], results[1]) and len(np.unique(results[0])) > 20
 
 
+def test_convolution_of_more_pixels_than_small_workgroups_cover(ctx):
+    """1025 boards of 1024 x 1024: 2^23 tiles of 128 x 64 outputs would be 2^32 threads, more than a launch takes, so another engine has to
+    serve the layer. A board of the middle and the last one, bit for bit as each comes out alone."""
+    batch, board, cin, cout, k = 1025, 1024, 16, 4, 5
+    rng = np.random.default_rng(9)
+    try:
+        x, y = ml.Tensor((batch, board, board, cin), "float16"), ml.Tensor((batch, board, board, cout), "float16")
+    except RuntimeError:
+        pytest.skip("43 GB of device memory are not free")
+    weights, bias = ml.toDevice(ctx, random_tensor(rng, (cout, k, k, cin), "float16", 0.05)), ml.toDevice(ctx, random_tensor(rng, (cout,), "float16"))
+    x.setall(ctx, 0.5)
+    y.setall(ctx, float("nan"))
+    one = lambda t, index: t.view((1, board, board, t.shape[3]), index * board * board * t.shape[3])
+    one(x, batch - 1).copyFromHost(ctx, random_tensor(rng, (1, board, board, cin), "float16"))
+    ml.convolutionImplicitGemmForward(ctx, x, weights, y, bias, None, "relu")
+    alone = ml.Tensor((1, board, board, cout), "float16")
+    for index in (batch // 2, batch - 1):
+        ml.convolutionImplicitGemmForward(ctx, one(x, index), weights, alone, bias, None, "relu")
+        assert mismatches(one(y, index).copyToHost(ctx), alone.copyToHost(ctx)) == 0
+
+
 def test_conv_sweep_config4_shapes(ctx):
     """19x19 boards, fp16, channel widths {64,128,256,384}, kernels 1 / 3 / 5 with bias + ReLU + residual, at a batch the oracle finishes."""
     rng = np.random.default_rng(44)
