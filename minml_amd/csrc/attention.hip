@@ -261,9 +261,12 @@ namespace
 
 	/*
 	 * THREADS = 256 where there are more (image, head) pairs than compute units. With fewer, the launch lasts as long as one workgroup:
-	 * the staging loop and then query blocks one after the other on each wavefront. 512 threads stage in half the rounds and give every
-	 * query block of a 15x15 board a wavefront of its own, and where compute units are left over `splits` workgroups share a head, so
-	 * that no two of those wavefronts share a SIMD. Every query row is computed by the same instructions either way.
+	 * the staging loop and then query blocks (of 32 rows) one after the other on each wavefront. 512 threads stage in half the rounds and
+	 * give every query block of a 15x15 board a wavefront of its own, and where compute units are left over `splits` workgroups share a
+	 * head: its query blocks are dealt out one by one, so that with two splits four wavefronts of each have one and no two of them share
+	 * a SIMD. Every query row is computed by the same instructions either way. Measured, us, 256 threads -> 512 -> 512 with splits (fp16,
+	 * 8 heads of 32 unless stated): 6 images of 15x15 15.6 -> 10.3 -> 8.7, 16 16.1 -> 11.0 -> 9.4, 32 (no split) 17.3 -> 11.8; 6 of 9x9
+	 * 6.0 -> 5.5 -> 5.4; 6 of 19x19 28.6 -> 13.7 -> 11.5; 3 heads of 128, 6 of 15x15 32.5 -> 23.3 -> 19.5; fp32 31.5 -> 24.0 -> 15.9.
 	 */
 	template<typename T, int D, int BIAS, int THREADS>
 	__global__ __launch_bounds__(THREADS) void kernel_attention_mfma(const T *__restrict__ input, T *__restrict__ output, const T *__restrict__ table,
@@ -351,7 +354,7 @@ namespace
 		const int half_sel = lane >> 5;
 		const int key_blocks = tokens_padded / 32;
 
-		for (int query_block = split * (THREADS / 64) + wave; query_block < key_blocks; query_block += shape.splits * (THREADS / 64))
+		for (int query_block = wave * shape.splits + split; query_block < key_blocks; query_block += shape.splits * (THREADS / 64))
 		{
 			const int query = query_block * 32 + lane_row;
 			const bool query_valid = query < tokens;
@@ -570,8 +573,9 @@ namespace
 		const int units = device_compute_units();
 		const long long pairs = static_cast<long long>(batch) * shape.heads;
 		const bool few = pairs <= units;
-		if (few) /* four wavefronts with a query block each occupy a compute unit; shared as far as there are units */
-			shape_arg.splits = static_cast<int>(std::max<long long>(1, std::min<long long>((shape.tokens + 127) / 128, units / std::max<long long>(pairs, 1))));
+		if (few) /* as far as there are units, and no further than two query blocks for each of them: four blocks each are slower by up to
+			9 % (3 heads of 128, 6 images of 11x11: 13.0 against 11.8 us), one block each is level (-2 to +4 %) */
+			shape_arg.splits = static_cast<int>(std::max<long long>(1, std::min<long long>((shape.tokens + 63) / 64, units / std::max<long long>(pairs, 1))));
 		const auto launch = [&](const void *kernel, int threads)
 		{
 			ensure_dynamic_lds(kernel, bytes);

@@ -92,10 +92,15 @@ def test_attention_shapes(ctx, dtype, case):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "float16"])
-@pytest.mark.parametrize("few,board,heads,dim", [(1, (15, 15), 8, 32), (6, (15, 15), 8, 32), (3, (19, 19), 2, 64), (5, (9, 9), 3, 32), (1, (4, 33), 1, 128), (100, (5, 7), 2, 32)])
+@pytest.mark.parametrize("few,board,heads,dim", [(1, (15, 15), 8, 32), (6, (15, 15), 8, 32),  # 8 query blocks over 4 workgroups
+                                                 (11, (15, 15), 8, 32),  # over 2
+                                                 (3, (19, 19), 2, 64),  # 12 over 6
+                                                 (6, (19, 19), 8, 32),  # 12 over 5: 3 3 2 2 2
+                                                 (5, (9, 9), 3, 32), (1, (4, 33), 1, 128),  # 3 over 2, 5 over 3
+                                                 (100, (5, 7), 2, 32)])  # 2, not shared
 def test_attention_of_few_images_equals_many(ctx, dtype, few, board, heads, dim):
-    """With fewer (image, head) pairs than compute units a head's query rows are spread over more wavefronts and workgroups: bit for bit
-    the same rows as in a batch that has one workgroup per pair."""
+    """With fewer (image, head) pairs than compute units (256) a head's query blocks of 32 rows are dealt out to more wavefronts and
+    workgroups: bit for bit the same rows as in a batch that has one workgroup per pair."""
     rng = np.random.default_rng(few + heads + dim)
     many, e, size = 600 // heads, heads * dim, 2 * max(board) - 1
     x = random_tensor(rng, (many,) + board + (3 * e,), dtype)
