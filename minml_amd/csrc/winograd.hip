@@ -1224,9 +1224,15 @@ namespace
 		}
 		MLHIP_CHECK(hipGetLastError());
 	}
-	/* fused output + next input transform: channels must be a multiple of 64 and 4-element accesses aligned; COMMON_ACT_ONLY / EXT_ALLOWED:
-	 * the caller has checked that the activation is linear or ReLU / that there is no residual, other forms are not instantiated */
-	template<typename T, int SLICE, int VEC, int THREADS, bool COMMON_ACT_ONLY, bool EXT_ALLOWED>
+	/* fused output + next input transform: channels must be a multiple of 64 and 4-element accesses aligned; COMMON_ACT_ONLY / RESIDUAL: what
+	 * the caller has made sure of (activation linear or ReLU; a residual given or not), other forms are not instantiated */
+	enum
+	{
+		RESIDUAL_NEVER = 0,
+		RESIDUAL_ALWAYS = 1,
+		RESIDUAL_OR_NOT = 2
+	};
+	template<typename T, int SLICE, int VEC, int THREADS, bool COMMON_ACT_ONLY, int RESIDUAL>
 	void launch_output_input(hipStream_t stream, const mlTensor_t &matrices, const mlTensor_t &bias, const mlTensor_t &ext, const mlShape_t &shape, void *output,
 			mlActivationType_t act, mlTensor_t &next)
 	{
@@ -1249,7 +1255,7 @@ namespace
 				ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), static_cast<int>(lds)); \
 			hipLaunchKernelGGL(kernel, grid, block, lds, stream, in, out, b, e, a, nxt, batch, height, width, channels, tiles_h, tiles_w); \
 		} while (0)
-		if constexpr (EXT_ALLOWED)
+		if constexpr (RESIDUAL != RESIDUAL_NEVER)
 		{
 			if (e != nullptr)
 			{
@@ -1261,14 +1267,17 @@ namespace
 					MLHIP_LAUNCH_FUSED(2, true);
 			}
 		}
-		if (e == nullptr)
+		if constexpr (RESIDUAL != RESIDUAL_ALWAYS)
 		{
-			if (mode == 0)
-				MLHIP_LAUNCH_FUSED(0, false);
-			else if (mode == 1)
-				MLHIP_LAUNCH_FUSED(1, false);
-			else if constexpr (!COMMON_ACT_ONLY)
-				MLHIP_LAUNCH_FUSED(2, false);
+			if (e == nullptr)
+			{
+				if (mode == 0)
+					MLHIP_LAUNCH_FUSED(0, false);
+				else if (mode == 1)
+					MLHIP_LAUNCH_FUSED(1, false);
+				else if constexpr (!COMMON_ACT_ONLY)
+					MLHIP_LAUNCH_FUSED(2, false);
+			}
 		}
 #undef MLHIP_LAUNCH_FUSED
 		MLHIP_CHECK(hipGetLastError());
@@ -1536,17 +1545,23 @@ extern "C"
 		}
 		mlTensor_t next = next_matrices;
 		/*
-		 * Which form, by the number of 64-channel slices of images (= workgroups of the widest form) for 256 compute units; measured, us,
-		 * without / with residual and stored y, 256 channels 15x15 fp16 (other widths, boards and fp32 agree):
-		 *   slices                              4           24          64          128          256          1024
-		 *   64 channels per workgroup        7.8 / 9.4   8.0 / 9.6   8.5 / 10.0   9.0 / 10.6  10.7 / 14.3  28.0 / 40
-		 *   32 channels                      7.3 / 9.4   7.7 / 10.1  6.1 / 7.7    6.9 / 8.8    9.7 / 17.3  38.8 / 61
-		 *   16 channels                      8.4 / 9.4  10.0 / 11.8  6.6 / 7.4    8.4 / 9.5   12.5 / 17.4  54.5 / 80
-		 *   strips of 16 channels            4.2 / 4.5   5.3 / 5.8   7.4 / 8.6   10.7 / 11.9  15.2 / 19.8  48.3 / 70
-		 * (a launch over few images is bound by what one workgroup must issue, a launch over many by memory, which wants whole 128-byte
-		 * lines; with residual the 16-channel form is ahead of the 32-channel one in fp32 and level in fp16 as long as all its workgroups run
-		 * at once: 90 slices of 384 channels take 14.2 us as 360 workgroups of it, 11.8 as 90 of the widest). Measured alternatives that were
-		 * not faster for many images: slices of 128 or 256 channels with 512 or 1024 threads, and 2-element vectors at twice the occupancy.
+		 * Which form, by the number of 64-channel slices of images (= workgroups of the widest form) for 256 compute units. Measured alone,
+		 * us, 256 channels 15x15, without / with residual and stored y:
+		 *   slices                             4            24            48            64           128           192           256
+		 *   fp16  64 channels, 256 threads  9.6 / 10.4    9.1 / 10.7    9.5 / 11.1    9.7 / 11.4  10.4 / 12.4   11.0 / 13.9   12.8 / 14.6
+		 *         32 channels               6.7 / 8.1     6.8 / 8.5     7.1 / 8.9     7.3 / 9.2    8.3 / 10.7    9.7 / 15.2   12.3 / 16.4
+		 *         16 channels               7.1 / 7.6     7.5 / 8.4     7.8 / 8.6     7.9 / 8.8   10.0 / 11.2   11.8 / 16.5   15.8 / 20.5
+		 *         strips of 16 channels     4.9 / 5.2     5.5 / 6.1     6.3 / 6.9     7.1 / 7.9    9.4 / 12.4   12.8 / 17.3   16.6 / 21.7
+		 *   fp32  64 channels, 256 threads  8.4 / 12.1    8.9 / 12.8    9.4 / 13.7    9.9 / 14.8  13.1 / 18.2   15.3 / 21.7   18.1 / 24.4
+		 *         32 channels               7.2 / 11.1    7.6 / 12.0    8.2 / 13.2    8.5 / 14.8  10.9 / 19.0   14.2 / 27.2   16.2 / 30.8
+		 *         16 channels               6.4 / 7.2     6.9 / 7.8     7.5 / 8.9     8.1 / 9.2   12.3 / 15.6   16.2 / 23.6   23.5 / 30.3
+		 *         strips of 16 channels     4.6 / 4.8     5.4 / 5.8     6.5 / 7.2     7.4 / 8.2   12.4 / 15.9   17.2 / 21.4   21.7 / 27.0
+		 * A launch over few images is bound by what one workgroup must issue, a launch over many by memory, which wants whole 128-byte lines.
+		 * Strips up to 51 slices: between the network's products (product + transform, both kinds in turn) they take 16.2 us against 17.2 of
+		 * the 32-channel form at 48 slices of 256 channels, but 18.5 against 17.9 at 64; other widths and boards cross between 51 and 72.
+		 * With residual the fp32 form of 32 channels keeps 54 registers per lane in scratch memory (15x15, 128 slices: 19.0 us, 16 channels
+		 * 15.6, 64 channels 18.2; 19x19: 32.9, 25.6, 30.2) and is not built. Measured alternatives that were not faster for many images:
+		 * slices of 128 or 256 channels with 512 or 1024 threads, and 2-element vectors at twice the occupancy.
 		 */
 		const hipStream_t stream = stream_of(context);
 		const long long slices = static_cast<long long>(output_shape.dim[0]) * (channels / 64), units = device_compute_units();
@@ -1564,14 +1579,16 @@ extern "C"
 		{
 			typedef decltype(zero) T;
 			const bool strips_fit = static_cast<size_t>(6) * (4 * ceil_div(output_shape.dim[2], 4) + 2) * STRIP_CHANNELS * sizeof(T) <= 64 * 1024;
-			if (common_act && separate && strips_fit && 10 * slices <= units)
+			constexpr bool fp32 = sizeof(T) == 4;
+			const bool residual = ext.data != nullptr;
+			if (common_act && separate && strips_fit && 5 * slices <= units)
 				launch_output_input_strips<T>(stream, matrices, bias, ext, output_shape, output, act, next);
-			else if (common_act && 4 * slices <= units)
-				launch_output_input<T, 16, 1, 256, true, true>(stream, matrices, bias, ext, output_shape, output, act, next);
-			else if (common_act && (ext.data != nullptr ? 2 : 1) * slices <= units)
-				launch_output_input<T, 32, 2, 256, true, true>(stream, matrices, bias, ext, output_shape, output, act, next);
+			else if (common_act && (residual || fp32) && (residual && fp32 ? 2 : 4) * slices <= units)
+				launch_output_input<T, 16, 1, 256, true, fp32 ? RESIDUAL_OR_NOT : RESIDUAL_ALWAYS>(stream, matrices, bias, ext, output_shape, output, act, next);
+			else if (common_act && !(residual && fp32) && (residual ? 2 : 1) * slices <= units)
+				launch_output_input<T, 32, 2, 256, true, fp32 ? RESIDUAL_NEVER : RESIDUAL_OR_NOT>(stream, matrices, bias, ext, output_shape, output, act, next);
 			else
-				launch_output_input<T, 64, 4, 256, false, true>(stream, matrices, bias, ext, output_shape, output, act, next);
+				launch_output_input<T, 64, 4, 256, false, RESIDUAL_OR_NOT>(stream, matrices, bias, ext, output_shape, output, act, next);
 		};
 		if (matrices.dtype == DTYPE_FLOAT16)
 			launch(half_t(0));

@@ -199,11 +199,13 @@ def test_fused_output_input_transform_bit_exact(ctx, dtype, shape):
 
 @pytest.mark.parametrize("dtype", ["float32", "float16"])
 @pytest.mark.parametrize("shape", [(6, 15, 15, 256), (3, 17, 20, 128), (1, 1, 3, 64), (2, 5, 30, 64), (1, 3, 1100, 64), (7, 9, 11, 256), (22, 6, 5, 256),
-                                   (9, 19, 19, 512), (70, 4, 7, 256)])
+                                   (9, 19, 19, 512), (70, 4, 7, 256), (17, 7, 10, 192), (13, 15, 15, 256), (64, 5, 6, 64), (65, 3, 9, 64), (32, 13, 4, 256),
+                                   (129, 5, 3, 64), (257, 2, 6, 64)])
 def test_fused_output_input_transform_forms(ctx, dtype, shape):
-    """The forms of the fused transform for different numbers of 64-channel slices of images: strips of one tile row (up to 25 slices;
+    """The forms of the fused transform for different numbers of 64-channel slices of images: strips of one tile row (up to 51 slices;
     several tile columns per wavefront, boards that end inside a tile, one row, too wide for the strips' LDS), 16 or 32 channels per
-    workgroup, 64. Bit for bit against the oracle; and with y written over the residual, which the strips must leave to another form."""
+    workgroup, 64, with the last slice count of each form and the first of the next (51 and 52, 64 and 65, 128 and 129, 257). Bit for bit
+    against the oracle; and with y written over the residual, which the strips must leave to another form."""
     rng = np.random.default_rng(sum(shape))
     b, h, w, c = shape
     tiles = b * ((h + 3) // 4) * ((w + 3) // 4)
