@@ -14,10 +14,11 @@
  * loads in flight: 4 wavefronts of 32 x 32 take 7.05 instead of 6.66 us at 256 rows), and 32 x 32 by 4 wavefronts of 16 x 16 where
  * 64 x 64 leaves compute units without a tile. Consecutive tiles (same matrix, same columns) lie on one XCD and share its L2.
  *
- * Measured, 36 products of M rows in a recorded chain, us per launch, streaming kernel -> this one: 256 -> 256 channels: M = 16
- * (one 15x15 position) 8.9 -> 3.3, 64 9.2 -> 3.9, 256 9.1 -> 6.7, 512 13.2 -> 9.5, 1024 17.0 -> 15.1, 1616 20.4 -> 22.8;
- * 128 -> 128 channels: 16 4.9 -> 2.4, 1024 8.5 -> 6.8, 2048 11.3 -> 10.7; 384 -> 384: 16 10.8 -> 4.0, 256 12.7 -> 13.2;
- * one product of 256 -> 768 columns: 225 rows 9.7 -> 2.9, 1350 10.2 -> 4.7, 4000 10.1 -> 8.5.
+ * Measured, 36 products of M rows in a recorded chain of nothing else, us per launch, streaming kernel (384-byte rows: tile engine) ->
+ * this one: 64 -> 64 channels: M = 16 (one 15x15 position) 4.6 -> 3.4, 1024 6.0 -> 5.5; 128 -> 128: 16 6.0 -> 3.4, 512 7.2 -> 5.7;
+ * 192 -> 192: 16 4.4 -> 3.5, 256 6.5 -> 5.1, 1024 20.0 -> 11.1, 2048 39.2 -> 20.5, 16384 202 -> 163; 256 -> 256: 16 9.8 -> 4.0,
+ * 64 10.0 -> 4.2, 256 9.7 -> 6.8, 512 14.0 -> 9.9; 384 -> 384: 16 11.4 -> 4.1, 128 12.3 -> 7.7, 256 13.7 -> 12.1. One product of 256 -> 768
+ * columns: 225 rows 9.7 -> 2.9, 1350 10.2 -> 4.7, 4000 10.1 -> 8.5.
  */
 #ifndef MINML_AMD_GEMM_DIRECT_HPP_
 #define MINML_AMD_GEMM_DIRECT_HPP_
@@ -182,25 +183,53 @@ namespace mlhip
 				g.a_row_bytes != 0 ? g.a_row_bytes : static_cast<size_t>(KB), epilogue);
 	}
 	/*
-	 * Whether this kernel takes a product: the tiles per compute unit at which it and the streaming kernel are level. Every tile fetches
-	 * its rows of A and B anew (KB * 128 bytes), where the streaming kernel fetches A once; 8 tiles of 64 KB per compute unit are level at
-	 * 512-byte rows (1024 rows x 36); at 256-byte rows the streaming kernel brings its B in half the time and is level at 4 (960 rows x 36,
-	 * 128 channels, inside a network: 8.8 against 8.2 us at best, the pass 388 against 374); and at 768-byte rows, where a tile of 96 KB is alone on its compute unit, only 2.
+	 * Whether this kernel takes a product: the 64 x 64 tiles per compute unit up to which it is not behind the kernel that would take it
+	 * otherwise. Every tile fetches its rows of A and B anew (KB * 128 bytes) where the streaming kernel fetches A once. Single products
+	 * alone, batched ones between a network's transforms, where the streaming kernel gains because it starts with the rows written last
+	 * (8 layers with weights of their own, product + transform, us per layer; alone the 36 products of 128 channels are level at 2000 rows
+	 * only). Streaming kernel / this one, and the number of tiles:
+	 *   128-byte rows  single 4: 14400 x 256 (900) 7.2 / 6.8, 20000 x 256 (1252) 7.5 / 7.9; batched 3: 15x15 1280 rows x 36 (720)
+	 *                  17.9 / 17.8, 1536 (864) 19.1 / 19.7
+	 *   256-byte rows  single 4: 1024 to 1280 tiles 0.84 of the streaming kernel's time, 1280 to 1536 level; batched 3: 15x15 512 rows x 36
+	 *                  (576) 17.3 / 16.5, 640 (720) 18.1 / 18.5, 896 (1008) 20.2 / 21.8, 19x19 625 (720) 22.7 / 22.2, 875 24.5 / 25.8
+	 *   512-byte rows  single 5.75: 5400 x 1024 (1360) 12.7 / 11.6, 23104 x 256 with residual (1444) 17.6 / 16.0, without 13.2 / 13.9,
+	 *                  24000 x 256 (1500) 13.3 / 14.3; where the streaming kernel's 128 columns are not all used, 8: 57600 x 100 (1800)
+	 *                  18.7 / 16.5; batched 7: 15x15 640 rows x 36 (1440) 27.0 / 26.6, 768 (1728) 28.0 / 29.7, 896 (2016) 28.7 / 30.9,
+	 *                  19x19 625 (1440) 31.2 / 29.5, 750 (1728) 32.9 / 31.0, 875 (2016) 34.2 / 34.2
+	 *   768-byte rows  3: 15x15 192 rows x 36 (648) 24.0 / 21.9, 256 (864) 24.3 / 24.8; single products cross at 768 to 1024
+	 *   384-byte rows  every size: the streaming kernel does not take them, and the tile engine, for whose pipeline 3 pieces of K are
+	 *                  short, is behind or level throughout (1280 rows x 36 39.4 / 28.9; alone 32768 x 36 391 / 352, single products of
+	 *                  2000 to 92000 tiles 0.55 to 0.95 of its time, below 2000 level)
 	 */
 	inline bool gemm_direct_applies(int M, int N, int batch, size_t k_bytes)
 	{
-		if (!(k_bytes == 128 || k_bytes == 256 || k_bytes == 384 || k_bytes == 512 || k_bytes == 768))
-			return false;
-		const long long tiles = static_cast<long long>(ceil_div(M, 64)) * ceil_div(N, 64) * batch;
-		return tiles <= static_cast<long long>(device_compute_units()) * ((k_bytes <= 256) ? 4 : (k_bytes <= 512) ? 8 : 2);
+		const long long tiles = static_cast<long long>(ceil_div(M, 64)) * ceil_div(N, 64) * batch, units = device_compute_units();
+		const bool batched = batch > 1;
+		switch (k_bytes)
+		{
+			case 128:
+			case 256:
+				return tiles <= (batched ? 3 : 4) * units;
+			case 384:
+				return tiles <= 0xffffffffLL / 512; /* threads that a launch can have */
+			case 512:
+				return 4 * tiles <= (batched ? 28 : (N % 128 == 0) ? 23 : 32) * units;
+			case 768:
+				return tiles <= 3 * units;
+			default:
+				return false;
+		}
 	}
 	template<int KB, typename Epilogue>
 	inline void launch_gemm_direct_kb(hipStream_t stream, const StreamGemmArgs &g, const Epilogue &epilogue)
 	{
-		/* 64 x 64 tiles once they fill every compute unit twice: at one tile each the smaller shape is level or faster (M = 96: 4.3
-		 * against 4.9 us, M = 256: 6.9 against 6.7 us) */
+		/*
+		 * 64 x 64 tiles once they fill every compute unit twice, at one tile each the smaller shape is level or faster (256 rows x 36 of 128
+		 * channels, 288 tiles: 4.5 against 4.8 us). 512-byte rows, of whose tiles two are resident: from 1.5 on (192 rows x 36 with the
+		 * transform, 432 tiles: 17.9 against 16.8 us); 768-byte rows, of which one is, not earlier (96 x 36, 432 tiles: 6.6 against 7.5 us).
+		 */
 		const long long tiles = static_cast<long long>(ceil_div(g.M, 64)) * ceil_div(g.N, 64) * g.batch;
-		if (tiles >= 2LL * device_compute_units())
+		if (2 * tiles >= (KB == 512 ? 3LL : 4LL) * device_compute_units())
 			launch_gemm_direct_as<KB, 1, 2, 4, 2>(stream, g, epilogue);
 		else
 			launch_gemm_direct_as<KB, 1, 1, 2, 2>(stream, g, epilogue);

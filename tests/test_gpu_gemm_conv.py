@@ -171,13 +171,16 @@ def test_gemm_ex_streaming_shapes(ctx, dtype, k_bytes, M, N):
 
 
 @pytest.mark.parametrize("K", [64, 128, 192, 256, 384])
-@pytest.mark.parametrize("bt,M,N", [(1, 1, 4), (36, 16, 256), (3, 31, 36), (2, 33, 100), (36, 65, 128), (36, 130, 260), (5, 257, 64), (1, 1350, 768)])
+@pytest.mark.parametrize("bt,M,N", [(1, 1, 4), (1, 1, 8), (36, 16, 256), (3, 31, 36), (2, 33, 100), (36, 65, 128), (36, 130, 260), (5, 257, 64), (1, 1350, 768),
+                                    (1, 1470, 1000), (1, 1530, 1000),  # 368 and 384 tiles of 64 x 64: where 512-byte rows change shape
+                                    (1, 1984, 1000), (1, 2040, 1000), (1, 3060, 1000)])  # 496 and 512, the other rows; 768
 def test_few_rows_equal_many_rows(ctx, K, bt, M, N):
-    """fp16 products too small for the streaming kernel (32 x 32 and 64 x 64 tiles with the whole K in LDS): ragged rows and columns around
-    both tile sizes, every K row length, bare and with bias + beta * C + ReLU, against the oracle; and bit for bit the first rows of a
-    product large enough for the streaming kernel or the tile engine, because a position's result must not depend on its batch."""
+    """fp16 products too small for the streaming kernel (32 x 32 tiles, 64 x 64 from 1.5 or 2 per compute unit, with the whole K in LDS): ragged
+    rows and columns around both tile sizes, every K row length, bare and with bias + beta * C + ReLU, against the oracle; and bit for bit
+    the first rows of a product that another kernel takes, because a position's result must not depend on its batch: with more than 2048
+    tiles of 64 x 64 the streaming kernel, for 384-byte rows (K = 192) the 64 x 64 tiles. (At most 4 columns: one kernel for all rows.)"""
     rng = np.random.default_rng(K + bt + M + N)
-    big = 36000 // bt
+    big = 64 * (2048 // (-(-N // 64) * bt) + 1)
     A = random_tensor(rng, (bt, M, K), "float16", 0.3)
     A[:, :: 7] = O.to_half(O.from_half(A[:, :: 7]) * 300.0)  # rows of another magnitude
     Bm = random_tensor(rng, (bt, N, K), "float16", 0.3)
