@@ -248,37 +248,30 @@ namespace
 			a_loader.c_bytes = static_cast<int>(c_bytes);
 			a_loader.fill = 0;
 			const DenseDmaRows b_loader { reinterpret_cast<const uint8_t*>(weights), filters_out, static_cast<int>(k_bytes) };
-			ConvTileArgs tile_args = conv_tile_args(input, weights, M, filters_out, height, width, kernel_h, kernel_w, c_bytes, 0);
-			/* layers that the windowed tiles take at larger batches: K in their order, and no other engine between the two */
-			tile_args.slices_first = sizeof(T) == 2 && conv_dma_window_applies(c_bytes, filters_out, kernel_h, kernel_w, height, width);
-			const auto few_rows = [&](const auto &ep)
-			{
-				return tile_args.slices_first ? try_launch_small_tiles<T>(stream, tile_args, ep)
-						: try_launch_fewer_rows<T>(stream, a_loader, b_loader, tile_args, ep);
-			};
+			const ConvTileArgs tile_args = conv_tile_args(input, weights, M, filters_out, height, width, kernel_h, kernel_w, c_bytes, 0);
 			bool launched = false;
 			if constexpr (sizeof(T) == 2)
+			{
+				/* the tiles' rows are consecutive pixels: the window of pixels they share enters LDS once per 128-byte slice of the channels;
+				 * for few positions small tiles that take K in the same order, and no other engine between the two */
+				const bool windowed = conv_dma_window_applies(c_bytes, filters_out, kernel_h, kernel_w, height, width);
 				specialise_epilogue(make_epilogue(), [&](const auto &ep)
 				{
-					launched = few_rows(ep);
+					launched = windowed ? try_launch_small_tiles<T, true>(stream, tile_args, ep) : try_launch_fewer_rows<T>(stream, a_loader, b_loader, tile_args, ep);
+					if (windowed && !launched)
+					{
+						launch_conv_dma_window<T>(stream, input, weights, M, filters_out, height, width, kernel_h, static_cast<int>(c_bytes), 0u, ep);
+						launched = true;
+					}
 				});
+			}
 			else
-				launched = few_rows(make_epilogue());
+				launched = try_launch_fewer_rows<T>(stream, a_loader, b_loader, tile_args, make_epilogue());
 			if (launched)
 			{
 				MLHIP_CHECK(hipGetLastError());
 				return;
 			}
-			if constexpr (sizeof(T) == 2)
-				if (tile_args.slices_first)
-				{ /* the tiles' rows are consecutive pixels: the window of pixels they share enters LDS once per 128-byte slice of the channels */
-					specialise_epilogue(make_epilogue(), [&](const auto &ep)
-					{
-						launch_conv_dma_window<T>(stream, input, weights, M, filters_out, height, width, kernel_h, static_cast<int>(c_bytes), 0u, ep);
-					});
-					MLHIP_CHECK(hipGetLastError());
-					return;
-				}
 			if constexpr (sizeof(T) == 2) /* the fp16 hot path gets its epilogue's common cases fixed at compile time */
 				specialise_epilogue(make_epilogue(), [&](const auto &ep)
 				{

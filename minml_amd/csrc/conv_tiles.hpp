@@ -108,7 +108,6 @@ namespace mlhip
 			int c_bytes, k_bytes; /* c_bytes: a multiple of 16 */
 			int fill; /* padding byte, 0..255 */
 			size_t pixel_bytes; /* between consecutive pixels: c_bytes, or more where several matrices lie side by side */
-			bool slices_first = false; /* K in the order of gemm_dma_window.hpp (128 bytes of the channels over all taps, then the next 128) instead of tap by tap; c_bytes a multiple of 128 */
 			int batch = 1; /* matrices: grid's second dimension, with the distances between their operands (bytes) and results (elements) */
 			size_t stride_input = 0, stride_weights = 0, stride_out = 0;
 	};
@@ -127,6 +126,8 @@ namespace mlhip
 			static_assert((DISTANCE - 1) * LOADS <= 63 && LDS_BYTES <= 160 * 1024, "queue depth and LDS");
 	};
 
+	/* SLICES_FIRST: K in the order of gemm_dma_window.hpp (128 bytes of the channels over all taps, then the next 128; c_bytes a multiple of
+	 * 128) instead of tap by tap */
 	template<typename T, typename Cfg, bool SLICES_FIRST, typename Epilogue>
 	__global__ __launch_bounds__(64 * Cfg::WAVES) void kernel_conv_tiles(ConvTileArgs g, unsigned int tiles_n, Epilogue epilogue)
 	{
@@ -334,20 +335,14 @@ namespace mlhip
 			}
 	}
 
-	template<typename T, typename Cfg, typename Epilogue>
+	template<typename T, typename Cfg, bool SLICES_FIRST, typename Epilogue>
 	inline void launch_conv_tiles_as(hipStream_t stream, const ConvTileArgs &g, const Epilogue &epilogue)
 	{
-		const auto launch = [&](auto kernel)
-		{
-			ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), Cfg::LDS_BYTES);
-			const int tiles_m = ceil_div(g.M, Cfg::BM), tiles_n = ceil_div(g.N, Cfg::BN);
-			hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned int>(tiles_m) * tiles_n, g.batch), dim3(64 * Cfg::WAVES), Cfg::LDS_BYTES, stream, g,
-					static_cast<unsigned int>(tiles_n), epilogue);
-		};
-		if constexpr (sizeof(T) == 2) /* only fp16 layers have windowed tiles */
-			if (g.slices_first)
-				return launch(kernel_conv_tiles<T, Cfg, true, Epilogue>);
-		launch(kernel_conv_tiles<T, Cfg, false, Epilogue>);
+		auto kernel = kernel_conv_tiles<T, Cfg, SLICES_FIRST, Epilogue>;
+		ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), Cfg::LDS_BYTES);
+		const int tiles_m = ceil_div(g.M, Cfg::BM), tiles_n = ceil_div(g.N, Cfg::BN);
+		hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned int>(tiles_m) * tiles_n, g.batch), dim3(64 * Cfg::WAVES), Cfg::LDS_BYTES, stream, g,
+				static_cast<unsigned int>(tiles_n), epilogue);
 	}
 
 	typedef ConvTileConfig<1, 1, 2, 2, 2, 4> ConvTile32; /* 64 KB of LDS: two workgroups per compute unit */
@@ -374,14 +369,14 @@ namespace mlhip
 	 * chain: 552 tiles of 32 x 32 for 1444 x 384 at K = 6912 take 27.6 us, 138 of 64 x 64 take 21.8; 512 of them for 2025 x 256 take 7.3
 	 * against 9.8; 900 tiles of 64 x 64 for 14400 x 256 at K = 2304 take 25 against 18 us of 128 x 128 tiles, 724 of them level).
 	 */
-	template<typename T, typename Epilogue>
+	template<typename T, bool SLICES_FIRST = false, typename Epilogue>
 	inline bool try_launch_small_tiles(hipStream_t stream, const ConvTileArgs &g, const Epilogue &epilogue)
 	{
 		const int units = device_compute_units();
 		if (tiles_of(g, 32, 32) <= 2LL * units)
-			launch_conv_tiles_as<T, ConvTile32>(stream, g, epilogue);
+			launch_conv_tiles_as<T, ConvTile32, SLICES_FIRST>(stream, g, epilogue);
 		else if (tiles_of(g, 64, 64) <= 3LL * units)
-			launch_conv_tiles_as<T, ConvTile64>(stream, g, epilogue);
+			launch_conv_tiles_as<T, ConvTile64, SLICES_FIRST>(stream, g, epilogue);
 		else
 			return false;
 		return true;
@@ -407,7 +402,7 @@ namespace mlhip
 		{
 			if (tiles_of(g, 256, g.N > 128 ? 256 : g.N > 64 ? 128 : 64) * 4 > units * 3LL)
 				return false;
-			launch_conv_tiles_as<T, ConvTile128x64>(stream, g, epilogue);
+			launch_conv_tiles_as<T, ConvTile128x64, false>(stream, g, epilogue);
 			return true;
 		}
 		if constexpr (sizeof(T) < 4)
@@ -434,7 +429,7 @@ namespace mlhip
 		const long long tiles = tiles_of(g, 128, 64);
 		if ((g.k_bytes <= 512 && tiles > 4LL * device_compute_units()) || tiles * 64 * ConvTile128x64::WAVES > 0xffffffffLL)
 			return false;
-		launch_conv_tiles_as<T, ConvTile128x64>(stream, g, epilogue);
+		launch_conv_tiles_as<T, ConvTile128x64, false>(stream, g, epilogue);
 		return true;
 	}
 } /* namespace mlhip */
