@@ -6,7 +6,8 @@ implementation must move (inputs once, outputs once) and the flops / integer ops
 the two takes longer at the chip's peaks (HBM 8 TB/s; dense MFMA fp16 2.5 PFLOP/s, int8 5.0 POP/s, fp32 157.3 TFLOP/s); `frac` is the
 achieved fraction of that peak.
 
-Groups: winograd (transforms and batched GEMM at the residual-network shapes), small (the same launches at 1 to 128 positions), conv (implicit-GEMM sweep: 19x19 boards, batch 512,
+Groups: winograd (transforms and batched GEMM at the residual-network shapes), small (the same launches at 1 to 128 positions, replayed as
+a graph), conv (implicit-GEMM sweep: 19x19 boards, batch 512,
 channels 64..384, kernels 1 / 3 / 5, bias + residual + ReLU), int8 (quantised 3x3 convolution at 256 channels and its three-call form),
 misc (im2row, element-wise neighbours), heads (softmax, global average pooling, batch normalisation in inference mode), transformer
 (RMS normalisation and multi-head attention at the hybrid configuration's shape), moe (routing, gather, the two expert layers and
@@ -50,21 +51,32 @@ class Bench:
         self.rng = np.random.default_rng(7)
         self.rows = []
 
-    def time(self, fn):
+    def time(self, fn, recorded=False):
+        """recorded: ten times the repetitions, replayed as one graph; issued one by one, launches shorter than a call from Python (about
+        8 us) would be timed at that."""
         fn()
+        reps = self.reps * (10 if recorded else 1)
+        graph = ml.Graph.record(self.ctx, lambda: [fn() for _ in range(reps)]) if recorded else None
+        if recorded:
+            graph.launch()
         self.ctx.synchronize()
         start = ml.Event(self.ctx)
-        for _ in range(self.reps):
-            fn()
+        if recorded:
+            graph.launch()
+        else:
+            for _ in range(reps):
+                fn()
         end = ml.Event(self.ctx)
         self.ctx.synchronize()
-        t = ml.Event.getElapsedTime(start, end) / self.reps
+        t = ml.Event.getElapsedTime(start, end) / reps
         start.destroy()
         end.destroy()
+        if recorded:
+            graph.destroy()
         return t
 
     def row(self, group, name, shape, fn, nbytes, ops=0.0, op_type="float16"):
-        t = self.time(fn)
+        t = self.time(fn, recorded=group == "small")
         t_hbm = nbytes / PEAK["hbm"]
         t_mfma = ops / PEAK[op_type]
         bound = "hbm" if t_hbm >= t_mfma else "mfma"
