@@ -14,7 +14,7 @@
  * loads in flight: 4 wavefronts of 32 x 32 take 7.05 instead of 6.66 us at 256 rows), and 32 x 32 by 4 wavefronts of 16 x 16 where
  * 64 x 64 leaves compute units without a tile. Consecutive tiles (same matrix, same columns) lie on one XCD and share its L2.
  *
- * Measured, 36 products of M rows in a recorded chain of nothing else, us per launch, streaming kernel (384-byte rows: tile engine) ->
+ * Measured, 36 products of M rows, 8 launches replayed as one graph, us per launch, streaming kernel (384-byte rows: tile engine) ->
  * this one: 64 -> 64 channels: M = 16 (one 15x15 position) 4.6 -> 3.4, 1024 6.0 -> 5.5; 128 -> 128: 16 6.0 -> 3.4, 512 7.2 -> 5.7;
  * 192 -> 192: 16 4.4 -> 3.5, 256 6.5 -> 5.1, 1024 20.0 -> 11.1, 2048 39.2 -> 20.5, 16384 202 -> 163; 256 -> 256: 16 9.8 -> 4.0,
  * 64 10.0 -> 4.2, 256 9.7 -> 6.8, 512 14.0 -> 9.9; 384 -> 384: 16 11.4 -> 4.1, 128 12.3 -> 7.7, 256 13.7 -> 12.1. One product of 256 -> 768

@@ -1545,8 +1545,8 @@ extern "C"
 		}
 		mlTensor_t next = next_matrices;
 		/*
-		 * Which form, by the number of 64-channel slices of images (= workgroups of the widest form) for 256 compute units. Measured alone,
-		 * us, 256 channels 15x15, without / with residual and stored y:
+		 * Which form, by the number of 64-channel slices of images (= workgroups of the widest form) for 256 compute units. Measured alone
+		 * (8 launches replayed as one graph), us per launch, 256 channels 15x15, without / with residual and stored y:
 		 *   slices                             4            24            48            64           128           192           256
 		 *   fp16  64 channels, 256 threads  9.6 / 10.4    9.1 / 10.7    9.5 / 11.1    9.7 / 11.4  10.4 / 12.4   11.0 / 13.9   12.8 / 14.6
 		 *         32 channels               6.7 / 8.1     6.8 / 8.5     7.1 / 8.9     7.3 / 9.2    8.3 / 10.7    9.7 / 15.2   12.3 / 16.4
