@@ -25,6 +25,13 @@ namespace mlhip
 	 */
 	constexpr int EPILOGUE_RUNTIME = -1;
 
+	/*
+	 * How the sum is rounded is part of the result: a position must come out of every kernel that its batch may take with the same bits,
+	 * and a compiler that may contract a product and a sum decides that anew in each of them (and for each of the 4 elements). So it is
+	 * written out here: beta * C is always added by one fma; the bias by one fma where it is known at compile time that there is one, else
+	 * after alpha * acc was rounded. Both are the same for alpha = 1; launchers that choose between forms by the number of rows take care
+	 * that other factors meet one of them only.
+	 */
 	template<typename T, int ACT = EPILOGUE_RUNTIME, int WITH_C = EPILOGUE_RUNTIME, int WITH_BIAS = EPILOGUE_RUNTIME>
 	struct FloatEpilogue
 	{
@@ -90,6 +97,22 @@ namespace mlhip
 				e.bias_batch_stride = bias_batch_stride;
 				return e;
 			}
+			__device__ __forceinline__ float scaled(float acc) const
+			{
+				return acc * alpha;
+			}
+			/* alpha * acc + b */
+			__device__ __forceinline__ float scaled_plus(float acc, float b) const
+			{
+#pragma clang fp contract(off)
+				if constexpr (WITH_BIAS == 1)
+					return fmaf(acc, alpha, b);
+				else
+				{
+					const float x = acc * alpha;
+					return x + b;
+				}
+			}
 			__device__ __forceinline__ float finish(float x) const
 			{
 				const int a = activation();
@@ -145,13 +168,7 @@ namespace mlhip
 				Vec<T, 4> out;
 #pragma unroll
 				for (int e = 0; e < 4; e++)
-					out.v[e] = acc[e] * alpha;
-				if (with_bias())
-				{
-#pragma unroll
-					for (int e = 0; e < 4; e++)
-						out.v[e] += col.bias[e];
-				}
+					out.v[e] = with_bias() ? scaled_plus(acc[e], col.bias[e]) : scaled(acc[e]);
 #pragma unroll
 				for (int e = 0; e < 4; e++)
 					out.v[e] = finish(out.v[e]);
@@ -163,13 +180,7 @@ namespace mlhip
 				Vec<T, 4> out;
 #pragma unroll
 				for (int e = 0; e < 4; e++)
-					out.v[e] = acc[e] * alpha;
-				if (with_bias())
-				{
-#pragma unroll
-					for (int e = 0; e < 4; e++)
-						out.v[e] += col.bias[e];
-				}
+					out.v[e] = with_bias() ? scaled_plus(acc[e], col.bias[e]) : scaled(acc[e]);
 				if (with_c())
 				{
 					float c[4];
@@ -188,7 +199,7 @@ namespace mlhip
 					}
 #pragma unroll
 					for (int e = 0; e < 4; e++)
-						out.v[e] += beta * c[e];
+						out.v[e] = fmaf(beta, c[e], out.v[e]);
 				}
 #pragma unroll
 				for (int e = 0; e < 4; e++)
@@ -207,24 +218,25 @@ namespace mlhip
 				if (vectorized)
 				{
 					Vec<T, 4> out;
-#pragma unroll
-					for (int e = 0; e < 4; e++)
-						out.v[e] = acc[e] * alpha;
 					if (with_bias())
 					{
 						Vec<T, 4> b;
 						b.load(bias + n);
 #pragma unroll
 						for (int e = 0; e < 4; e++)
-							out.v[e] += b.v[e];
+							out.v[e] = scaled_plus(acc[e], b.v[e]);
 					}
+					else
+#pragma unroll
+						for (int e = 0; e < 4; e++)
+							out.v[e] = scaled(acc[e]);
 					if (with_c())
 					{
 						Vec<T, 4> c;
 						c.load(C + offset);
 #pragma unroll
 						for (int e = 0; e < 4; e++)
-							out.v[e] += beta * c.v[e];
+							out.v[e] = fmaf(beta, c.v[e], out.v[e]);
 					}
 #pragma unroll
 					for (int e = 0; e < 4; e++)
@@ -237,11 +249,9 @@ namespace mlhip
 					for (int e = 0; e < 4; e++)
 						if (n + e < N)
 						{
-							float x = acc[e] * alpha;
-							if (with_bias())
-								x += Storage<T>::load(bias + n + e);
+							float x = with_bias() ? scaled_plus(acc[e], Storage<T>::load(bias + n + e)) : scaled(acc[e]);
 							if (with_c())
-								x += beta * Storage<T>::load(C + offset + e);
+								x = fmaf(beta, Storage<T>::load(C + offset + e), x);
 							Storage<T>::store(D + offset + e, finish(x));
 						}
 				}

@@ -243,14 +243,16 @@ namespace mlhip
 		 * the Winograd products with a plain 16-byte store, everything else (gemm_ex, 1x1 convolutions, the int8 product) with the
 		 * fused epilogue on 4 consecutive outputs.
 		 */
-		const bool plain = (g.alpha == 1.0f) && (g.beta == 0.0f) && (g.bias == nullptr) && (g.act == ACTIVATION_LINEAR) && (g.N * esize) % 16 == 0
-				&& aligned_to(g.D, 16) && ((g.stride_c * esize) % 16 == 0) && g.dtype != DTYPE_INT8;
+		const bool sixteen = (g.N * esize) % 16 == 0 && aligned_to(g.D, 16) && ((g.stride_c * esize) % 16 == 0); /* rows of whole 16-byte stores */
+		const bool plain = (g.alpha == 1.0f) && (g.beta == 0.0f) && (g.bias == nullptr) && (g.act == ACTIVATION_LINEAR) && sixteen && g.dtype != DTYPE_INT8;
 		/* the same products with few rows, whose launch is all latency */
 		if (fast && g.dtype == DTYPE_FLOAT16 && vectorized && gemm_direct_applies(g.M, g.N, g.batch, k_bytes))
 		{
 			const StreamGemmArgs sg { g.A, g.B, g.D, g.M, g.N, static_cast<int>(k_bytes), g.batch, g.stride_a, g.stride_b, g.stride_c };
 			if (plain)
 				launch_gemm_direct(stream, sg, PlainStore { });
+			else if (g.alpha != 1.0f && (k_bytes == 384 || (g.beta == 0.0f && !sixteen))) /* the run-time form's rounding, as larger products have it */
+				launch_gemm_direct(stream, sg, make_float_epilogue<half_t>(g, true));
 			else
 				specialise_epilogue(make_float_epilogue<half_t>(g, true), [&](const auto &ep)
 				{

@@ -203,6 +203,44 @@ def test_few_rows_equal_many_rows(ctx, K, bt, M, N):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "float16"])
+@pytest.mark.parametrize("K", [64, 96, 128, 192, 256, 320, 384, 512, 1152])
+@pytest.mark.parametrize("N", [256, 100, 254])  # whole 16-byte stores, 8-byte ones, single elements
+def test_scaled_products_round_alike_at_every_size(ctx, dtype, K, N):
+    """alpha * acc + bias + beta * C with factors that are no powers of two, where contracted and separate operations differ: the first
+    rows of every size, which several kernels serve, must be the same bits, and for accumulators that are exact (small integers) those of
+    one formula: an fma for beta * C, an fma or two roundings for the bias. fp16 results round towards zero."""
+    rng = np.random.default_rng(K + N)
+    first, biggest, alpha, beta = 64, 16000, np.float32(0.7), np.float32(0.3)
+    A, Bm = rng.integers(-2, 3, (biggest, K)).astype(np.float32), rng.integers(-2, 3, (N, K)).astype(np.float32)
+    acc = A[:first] @ Bm.T
+    bias = storage(rng.standard_normal(N) * 20, dtype)
+    C = storage(np.tile(-(acc * alpha + O.as_float(bias)) / beta + rng.standard_normal(acc.shape) * 0.01, (biggest // first, 1)), dtype)  # almost cancels
+    dA, dB, dC, db = (ml.toDevice(ctx, storage(a, dtype) if a.dtype == np.float32 and a.shape[1:] == (K,) else a, dtype) for a in (A, Bm, C, bias))
+    c, b = O.as_float(C[:first]).astype(np.float64), O.as_float(bias)
+    apart, fused = (acc * alpha + b).astype(np.float32), (acc.astype(np.float64) * np.float64(alpha) + b).astype(np.float32)
+    for act, beta_used in (("linear", float(beta)), ("leaky_relu", float(beta)), ("linear", 0.0)):
+        results = []
+        for M in (first, 640, 2560, biggest):
+            dD = ml.Tensor((M, N), dtype)
+            ml.gemm_ex(ctx, dD, float(alpha), "n", dA.view((M, K)), "t", dB, beta_used, dC.view((M, N)), db, act)
+            results.append(dD.view((first, N)).copyToHost(ctx))
+        for M, other in zip((640, 2560, biggest), results[1:]):
+            assert np.array_equal(results[0], other), "%d rows, %s, beta %g" % (M, act, beta_used)
+        if act == "linear":
+            want = [storage((c * np.float64(np.float32(beta_used)) + t).astype(np.float32), dtype) for t in (apart, fused)]
+            assert any(np.array_equal(results[0], w) for w in want)
+    # the expert layer: alpha = 1, beta * C on rows in place
+    results = []
+    for M in (first, 640, 2560, biggest):
+        y = ml.Tensor((M // 32, 32, 1, N), dtype)
+        y.copyFrom(ctx, dC.view((M // 32, 32, 1, N)))
+        ml.moeForward(ctx, dA.view((M // 32, 32, 1, K)), dB.view((1, N, K)), db.view((1, N)), float(beta), y, "linear")
+        results.append(y.view((first, N)).copyToHost(ctx))
+    assert all(np.array_equal(results[0], other) for other in results[1:])
+    assert np.array_equal(results[0], storage((c * np.float64(beta) + (acc + b).astype(np.float32)).astype(np.float32), dtype))
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float16"])
 @pytest.mark.parametrize("N", [192, 320, 384, 448, 130, 576])
 def test_gemm_ex_tile_engine_widths(ctx, dtype, N):
     """K rows of 1024 bytes take the direct-to-LDS tile engine. Its tile width follows N: 256 x 192 tiles for multiples of 192 that are no
