@@ -182,7 +182,8 @@ class Tensor:
         """Non-owning tensor over the same memory, `offset` in elements (reference: Tensor::view; hip_create_view is the same sum of
         address and offset). A pass over a network makes several hundred of these, so they are put together field by field."""
         shape = tuple(map(int, shape))
-        offset = operator.index(offset)  # an address made with a numpy integer would be one too, and no call takes such a pointer
+        if type(offset) is not int:
+            offset = operator.index(offset)  # an address made with a numpy integer would be one too, and no call takes such a pointer
         volume = math.prod(shape) if shape else 0
         if offset + volume > self.volume():
             raise ValueError("view exceeds the tensor")
