@@ -189,7 +189,7 @@ class Tensor:
             raise ValueError("view exceeds the tensor")
         v = Tensor.__new__(Tensor)
         v.shape, v.dtype, v.device_index, v._owner, v._owning = shape, self.dtype, self.device_index, self, False
-        v.ptr = self.ptr + offset * B.DTYPE_SIZE[self.dtype]
+        v.ptr = self.ptr + offset * B.DTYPE_SIZE[self.dtype] if offset else self.ptr
         return v
 
     def reinterpretAs(self, dtype):
