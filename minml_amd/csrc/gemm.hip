@@ -20,6 +20,7 @@
 #include "gemm_launch.hpp"
 #include "gemm_stream.hpp"
 #include "gemm_direct.hpp"
+#include "gemm_tiles.hpp"
 #include "gemm_dma.hpp"
 #include "conv_tiles.hpp"
 
@@ -245,10 +246,20 @@ namespace mlhip
 		 */
 		const bool sixteen = (g.N * esize) % 16 == 0 && aligned_to(g.D, 16) && ((g.stride_c * esize) % 16 == 0); /* rows of whole 16-byte stores */
 		const bool plain = (g.alpha == 1.0f) && (g.beta == 0.0f) && (g.bias == nullptr) && (g.act == ACTIVATION_LINEAR) && sixteen && g.dtype != DTYPE_INT8;
-		/* the same products with few rows, whose launch is all latency */
-		if (fast && g.dtype == DTYPE_FLOAT16 && vectorized && gemm_direct_applies(g.M, g.N, g.batch, k_bytes))
+		/* the plain batched products between few rows and many, and those that no other kernel is made for */
+		const StreamGemmArgs short_rows { g.A, g.B, g.D, g.M, g.N, static_cast<int>(std::min<size_t>(k_bytes, 0x7fffffffu)), g.batch, g.stride_a, g.stride_b, g.stride_c };
+		if (fast && plain && g.batch > 1 && k_bytes <= 0x7fffffffu)
 		{
-			const StreamGemmArgs sg { g.A, g.B, g.D, g.M, g.N, static_cast<int>(k_bytes), g.batch, g.stride_a, g.stride_b, g.stride_c };
+			if ((g.dtype == DTYPE_FLOAT16) ? try_launch_gemm_tiles<half_t>(stream, short_rows) : try_launch_gemm_tiles<float>(stream, short_rows))
+			{
+				MLHIP_CHECK(hipGetLastError());
+				return;
+			}
+		}
+		/* the same products with few rows, whose launch is all latency */
+		if (fast && g.dtype == DTYPE_FLOAT16 && vectorized && gemm_direct_applies(short_rows))
+		{
+			const StreamGemmArgs &sg = short_rows;
 			if (plain)
 				launch_gemm_direct(stream, sg, PlainStore { });
 			else if (g.alpha != 1.0f && (k_bytes == 384 || (g.beta == 0.0f && !sixteen))) /* the run-time form's rounding, as larger products have it */

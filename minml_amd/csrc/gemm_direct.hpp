@@ -25,12 +25,13 @@
 
 #include "common.hpp"
 #include "gemm_stream.hpp"
+#include "gemm_tiles.hpp"
 
 namespace mlhip
 {
 	template<int KB, int BLOCKS_M, int BLOCKS_N, int WAVES_M, int WAVES_N, typename Epilogue>
 	__global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void kernel_gemm_direct_nt(const half_t *A, const half_t *B, half_t *C, int M, int N, size_t stride_a,
-			size_t stride_b, size_t stride_c, unsigned int tiles_m, unsigned int tiles_n, size_t a_row_bytes, Epilogue epilogue)
+			size_t stride_b, size_t stride_c, unsigned int tiles_m, unsigned int tiles_n, unsigned int matrices, int by_rows, size_t a_row_bytes, Epilogue epilogue)
 	{
 		constexpr bool PLAIN = std::is_same<Epilogue, PlainStore>::value;
 		constexpr int PIECES = KB / 128; /* 128-byte pieces of a K row */
@@ -42,9 +43,22 @@ namespace mlhip
 		const int frag_row = lane & 15, quarter = lane >> 4;
 
 		const unsigned int id = xcd_contiguous_block_id(blockIdx.x, gridDim.x);
-		const unsigned int column_tiles = id / tiles_m; /* matrix * tiles_n + n_tile */
-		const unsigned int matrix = column_tiles / tiles_n;
-		const int m_tile = (id - column_tiles * tiles_m) * BM, n_tile = (column_tiles - matrix * tiles_n) * BN;
+		unsigned int matrix;
+		int m_tile, n_tile;
+		if (by_rows)
+		{ /* every XCD has rows of all matrices (gemm_tiles.hpp) */
+			const unsigned int row_tile = id / tiles_n, slow = row_tile / matrices;
+			matrix = row_tile - slow * matrices;
+			m_tile = slow * BM;
+			n_tile = (id - row_tile * tiles_n) * BN;
+		}
+		else
+		{
+			const unsigned int column_tiles = id / tiles_m; /* matrix * tiles_n + n_tile */
+			matrix = column_tiles / tiles_n;
+			m_tile = (id - column_tiles * tiles_m) * BM;
+			n_tile = (column_tiles - matrix * tiles_n) * BN;
+		}
 		const int m0 = m_tile + wave_m * 16 * BLOCKS_M, n0 = n_tile + wave_n * 16 * BLOCKS_N;
 
 		/* lane l, register r of block (i, j): m = 16 i + l % 16, n = 16 j + 4 (l / 16) + r */
@@ -179,17 +193,17 @@ namespace mlhip
 		if (LDS > 64 * 1024)
 			ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), LDS);
 		hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned int>(tiles_m) * tiles_n * g.batch), dim3(64 * WAVES_M * WAVES_N), LDS, stream, reinterpret_cast<const half_t*>(g.A),
-				reinterpret_cast<const half_t*>(g.B), reinterpret_cast<half_t*>(g.C), g.M, g.N, g.stride_a, g.stride_b, g.stride_c, tiles_m, tiles_n,
+				reinterpret_cast<const half_t*>(g.B), reinterpret_cast<half_t*>(g.C), g.M, g.N, g.stride_a, g.stride_b, g.stride_c, tiles_m, tiles_n, g.batch, products_meet_in_l2(g, sizeof(half_t)),
 				g.a_row_bytes != 0 ? g.a_row_bytes : static_cast<size_t>(KB), epilogue);
 	}
 	/*
 	 * Whether this kernel takes a product: the 64 x 64 tiles per compute unit up to which it is not behind the kernel that would take it
 	 * otherwise. Every tile fetches its rows of A and B anew (KB * 128 bytes) where the streaming kernel fetches A once. Single products
-	 * alone, batched ones between a network's transforms, where the streaming kernel gains because it starts with the rows written last
-	 * (8 layers with weights of their own, product + transform, us per layer; alone the 36 products of 128 channels are level at 2000 rows
-	 * only). Streaming kernel / this one, and the number of tiles:
+	 * alone; batched ones between a network's transforms, where those that are plain go to gemm_tiles.hpp first. Streaming kernel / this one, and the
+	 * number of tiles:
 	 *   128-byte rows  single 4: 14400 x 256 (900) 7.2 / 6.8, 20000 x 256 (1252) 7.5 / 7.9; batched 3: 15x15 1280 rows x 36 (720)
-	 *                  17.9 / 17.8, 1536 (864) 19.1 / 19.7
+	 *                  17.9 / 17.8, 1536 (864) 19.1 / 19.7; by rows as long as that order is for (with transforms of the same order: 1024 rows of
+	 *                  64 channels 15.2 / 11.9, 2048 21.1 / 15.1, 4096 25.7 / 22.5)
 	 *   256-byte rows  single 4: 1024 to 1280 tiles 0.84 of the streaming kernel's time, 1280 to 1536 level; batched 3: 15x15 512 rows x 36
 	 *                  (576) 17.3 / 16.5, 640 (720) 18.1 / 18.5, 896 (1008) 20.2 / 21.8, 19x19 625 (720) 22.7 / 22.2, 875 24.5 / 25.8
 	 *   512-byte rows  single 5.75: 5400 x 1024 (1360) 12.7 / 11.6, 23104 x 256 with residual (1444) 17.6 / 16.0, without 13.2 / 13.9,
@@ -201,19 +215,20 @@ namespace mlhip
 	 *                  short, is behind or level throughout (1280 rows x 36 39.4 / 28.9; alone 32768 x 36 391 / 352, single products of
 	 *                  2000 to 92000 tiles 0.55 to 0.95 of its time, below 2000 level)
 	 */
-	inline bool gemm_direct_applies(int M, int N, int batch, size_t k_bytes)
+	inline bool gemm_direct_applies(const StreamGemmArgs &g)
 	{
-		const long long tiles = static_cast<long long>(ceil_div(M, 64)) * ceil_div(N, 64) * batch, units = device_compute_units();
-		const bool batched = batch > 1;
-		switch (k_bytes)
+		const long long tiles = static_cast<long long>(ceil_div(g.M, 64)) * ceil_div(g.N, 64) * g.batch, units = device_compute_units();
+		const bool batched = g.batch > 1;
+		switch (g.k_bytes)
 		{
 			case 128:
+				return tiles <= (batched ? 3 : 4) * units || products_meet_in_l2(g, sizeof(half_t));
 			case 256:
 				return tiles <= (batched ? 3 : 4) * units;
 			case 384:
 				return tiles <= 0xffffffffLL / 512; /* threads that a launch can have */
 			case 512:
-				return 4 * tiles <= (batched ? 28 : (N % 128 == 0) ? 23 : 32) * units;
+				return 4 * tiles <= (batched ? 28 : (g.N % 128 == 0) ? 23 : 32) * units;
 			case 768:
 				return tiles <= 3 * units;
 			default:
@@ -226,10 +241,12 @@ namespace mlhip
 		/*
 		 * 64 x 64 tiles once they fill every compute unit twice, at one tile each the smaller shape is level or faster (256 rows x 36 of 128
 		 * channels, 288 tiles: 4.5 against 4.8 us). 512-byte rows, of whose tiles two are resident: from 1.5 on (192 rows x 36 with the
-		 * transform, 432 tiles: 17.9 against 16.8 us); 768-byte rows, of which one is, not earlier (96 x 36, 432 tiles: 6.6 against 7.5 us).
+		 * transform, 432 tiles: 17.9 against 16.8 us); 768-byte rows, of which one is, not earlier (96 x 36, 432 tiles: 6.6 against 7.5 us). By rows the
+		 * loads are short and the smaller shape stays ahead to twice as many (128-byte rows, 960 rows x 36, 540 tiles, with the transform: 12.6
+		 * against 12.4 us, 1408 14.2 / 13.9, 1616 14.9 / 14.9, 3072 19.1 / 19.6).
 		 */
 		const long long tiles = static_cast<long long>(ceil_div(g.M, 64)) * ceil_div(g.N, 64) * g.batch;
-		if (2 * tiles >= (KB == 512 ? 3LL : 4LL) * device_compute_units())
+		if (2 * tiles >= (products_meet_in_l2(g, sizeof(half_t)) ? 8LL : KB == 512 ? 3LL : 4LL) * device_compute_units())
 			launch_gemm_direct_as<KB, 1, 2, 4, 2>(stream, g, epilogue);
 		else
 			launch_gemm_direct_as<KB, 1, 1, 2, 2>(stream, g, epilogue);

@@ -161,6 +161,20 @@ namespace
 	};
 
 	/*
+	 * Whether what a transform reads and writes stays in the last-level cache (256 MB) between the launches of a network: both sets of matrices
+	 * within 112 MB, which leaves room for the activations and weights beside them. Then nothing is marked non-temporal, and every XCD transforms one contiguous
+	 * eighth of the images, the rows that the product's tiles by rows read and write through the same L2 (gemm_tiles.hpp); beyond, the products
+	 * stream and the orders and hints beside the kernels below are ahead. Fused transform + product, us, images round the XCDs and non-temporal /
+	 * contiguous / contiguous and cached: fp16 128 channels 500 rows of 19x19 18.6 / 15.5 / 15.6, 1275 26.7 / 24.4 / 22.9; 256 channels 15x15 128 rows 13.2 / 12.2 /
+	 * 12.2, 640 23.9 / 22.9 / 22.9, 1616 37.3 / 37.1 / 35.9, 3072 (113 MB) 60.4 / 59.5 / 58.4, 4096 (151 MB) 72.0 / 72.0 / 75.5; with the streaming product 8192
+	 * (302 MB) 129 / 130 / 132; 384 channels 1792 rows (99 MB) 59.3 / 58.0 / 56.5, 2304 (127 MB) 69.6 / 69.6 / 74.4.
+	 */
+	inline bool matrices_stay_cached(size_t tiles, int channels, size_t element_size)
+	{
+		return 2 * 36 * tiles * channels * element_size <= (static_cast<size_t>(112) << 20);
+	}
+
+	/*
 	 * input [B][H][W][C] -> matrices [36][B*tiles_h*tiles_w][C]
 	 * All 36 loads of a tile are issued back to back, unconditionally, from coordinates clamped into the image; elements that lie outside
 	 * are replaced by zero afterwards. (A load under a bounds test would sit in its own basic block and be waited for on its own, which
@@ -247,7 +261,8 @@ namespace
 #pragma unroll
 				for (int c = 0; c < VEC; c++)
 					out.v[c] = res[col][c];
-				/* non-temporal: measured 94.2k against 88.2k positions per second on the 20-block network run as three calls per layer */
+				/* non-temporal: measured 94.2k against 88.2k positions per second on the 20-block network run as three calls per layer, and for few images too
+				 * (three calls per layer, 256 channels, 512 rows of tiles: 22.1 against 22.9 us, 1616 37.7 / 39.0) */
 				out.store_streaming(dst + static_cast<size_t>(row * 6 + col) * matrix_stride);
 			}
 		}
@@ -258,7 +273,7 @@ namespace
 	 * ACT: 0 = linear, 1 = ReLU (both fused as the reference fuses them), 2 = any other activation, selected at run time.
 	 * The 36 matrix rows and the 16 residual vectors (from clamped coordinates) are requested before any arithmetic.
 	 */
-	template<typename T, int VEC, int ACT, bool HAS_EXT>
+	template<typename T, int VEC, int ACT, bool HAS_EXT, bool CACHED>
 	__global__ __launch_bounds__(256) void kernel_output_transform_4x4_3x3(const T *__restrict__ matrices, T *output, const T *__restrict__ bias,
 			const T *ext, int act, int batch_size, int height, int width, int channels, int tiles_h, int tiles_w)
 	{
@@ -268,10 +283,10 @@ namespace
 		const unsigned int nb_of_tiles = batch_size * tiles_per_image;
 		const unsigned int total = nb_of_tiles * groups;
 
-		/* runs of 16 workgroups (64 tiles of 256 channels) per XCD, the runs going round the XCDs: measured 102 -> 92 us for the 20 x 256
+		/* for many images runs of 16 workgroups (64 tiles of 256 channels) per XCD, the runs going round the XCDs: measured 102 -> 92 us for the 20 x 256
 		 * network's layer with residual against one contiguous eighth of the tiles per XCD (the input transform is the other way round:
 		 * 63 us with contiguous eighths, 64-75 us with runs) */
-		const unsigned int block = xcd_run_block_id(blockIdx.x, gridDim.x, 16);
+		const unsigned int block = CACHED ? xcd_contiguous_block_id(blockIdx.x, gridDim.x) : xcd_run_block_id(blockIdx.x, gridDim.x, 16);
 		const unsigned int gid = block * blockDim.x + threadIdx.x;
 		if (gid >= total)
 			return;
@@ -291,7 +306,10 @@ namespace
 		for (int row = 0; row < 6; row++)
 #pragma unroll
 			for (int col = 0; col < 6; col++)
-				raw[row][col] = __builtin_nontemporal_load(reinterpret_cast<const raw_t*>(src + static_cast<size_t>(row * 6 + col) * matrix_stride));
+			{
+				const raw_t *p = reinterpret_cast<const raw_t*>(src + static_cast<size_t>(row * 6 + col) * matrix_stride);
+				raw[row][col] = CACHED ? *p : __builtin_nontemporal_load(p);
+			}
 
 		unsigned int offset[4][4]; /* element offsets of the 4x4 outputs, clamped into the image */
 #pragma unroll
@@ -310,7 +328,10 @@ namespace
 			for (int row = 0; row < 4; row++)
 #pragma unroll
 				for (int col = 0; col < 4; col++)
-					residual[row][col] = __builtin_nontemporal_load(reinterpret_cast<const raw_t*>(ext + offset[row][col]));
+				{
+					const raw_t *p = reinterpret_cast<const raw_t*>(ext + offset[row][col]);
+					residual[row][col] = CACHED ? *p : __builtin_nontemporal_load(p);
+				}
 		}
 		Vec<T, VEC> b;
 		if (bias != nullptr)
@@ -637,17 +658,17 @@ namespace
 	 * back (zero outside the image) and runs the input transform. Results are bit-identical to the two separate calls; what is saved is
 	 * the write and re-read of y through HBM (or only the re-read, when y is also needed as a later residual).
 	 */
-	template<typename T, int VEC, int SLICE, int ACT, bool HAS_EXT, int THREADS>
+	template<typename T, int VEC, int SLICE, int ACT, bool HAS_EXT, int THREADS, bool CACHED>
 		__global__ __launch_bounds__(THREADS, ((VEC <= 2) ? 1024 : 512) / THREADS) void kernel_output_input_transform_4x4_3x3(const T *__restrict__ matrices, T *output, const T *__restrict__ bias,
 			const T *ext, int act, T *__restrict__ next_matrices, int batch_size, int height, int width, int channels, int tiles_h, int tiles_w)
 	{
 		extern __shared__ __attribute__((aligned(16))) uint8_t lds_bytes[];
 		const unsigned int slices = channels / SLICE;
-		/* the slices of one image (at least 4 workgroups) run on one XCD, the images go round the XCDs: neighbouring 128-byte pieces of a
+		/* many images: the slices of one image (at least 4 workgroups) run on one XCD, the images go round the XCDs: neighbouring 128-byte pieces of a
 		 * row of the matrices are then fetched and written through the same L2 at about the same time (124-130 -> 117-121 us for the
 		 * 20 x 256 network's layer against the hardware's own order, in which consecutive workgroups sit on different XCDs) */
 		const unsigned int run = (slices >= 4) ? slices : slices * (4 / slices);
-		const unsigned int lin = xcd_run_block_id(blockIdx.x, gridDim.x, run);
+		const unsigned int lin = CACHED ? xcd_contiguous_block_id(blockIdx.x, gridDim.x) : xcd_run_block_id(blockIdx.x, gridDim.x, run);
 		const unsigned int batch = lin / slices;
 		const unsigned int tiles_per_image = tiles_h * tiles_w;
 		const size_t image_pixels = static_cast<size_t>(batch) * height * width;
@@ -667,11 +688,11 @@ namespace
 		g.tiles_w = tiles_w;
 		g.slice = lin - batch * slices;
 		/*
-		 * Cache hints, chosen by measurement on the 20-block network: the product matrices, the residual and y are non-temporal (each
+		 * Cache hints for many images, chosen by measurement on the 20-block network: the product matrices, the residual and y are non-temporal (each
 		 * is touched once here), the next layer's matrices are written cacheable, because the product that follows walks them from
 		 * the end and finds the rows written last still in the last-level cache.
 		 */
-		fused_transform_phase1<T, VEC, SLICE, ACT, HAS_EXT, THREADS, true, true>(g, lds_bytes);
+		fused_transform_phase1<T, VEC, SLICE, ACT, HAS_EXT, THREADS, !CACHED, !CACHED>(g, lds_bytes);
 		__syncthreads();
 		fused_transform_phase2<T, VEC, SLICE, THREADS, false>(g, lds_bytes);
 	}
@@ -691,7 +712,7 @@ namespace
 	constexpr int STRIP_CHANNELS = 16;
 	template<typename T, int ACT, bool HAS_EXT>
 	__global__ __launch_bounds__(192) void kernel_output_input_transform_strips(const T *__restrict__ matrices, T *output, const T *__restrict__ bias, const T *ext,
-			T *__restrict__ next_matrices, int batch_size, int height, int width, int channels, int tiles_h, int tiles_w)
+			T *__restrict__ next_matrices, int batch_size, int height, int width, int channels, int tiles_h, int tiles_w, int contiguous)
 	{
 		typedef typename RawVec<T, 1>::type raw_t;
 		constexpr int SLICE = STRIP_CHANNELS;
@@ -699,8 +720,10 @@ namespace
 		T *pixels = reinterpret_cast<T*>(lds_bytes); /* [6][pitch][SLICE] */
 		const int pitch = 4 * tiles_w + 2;
 		const unsigned int slices = channels / SLICE;
-		/* the 4 slices that share 128-byte lines run on one XCD, everything else goes round the XCDs: few workgroups must spread over the chip */
-		const unsigned int lin = xcd_run_block_id(blockIdx.x, gridDim.x, 4);
+		/* few images: the 4 slices that share 128-byte lines run on one XCD, everything else goes round the XCDs. From half an image per XCD on each has a contiguous
+		 * eighth of the images, where strips find the product rows of their neighbours (8 layers of 256 channels 15x15, strip + product, us: 2 images
+		 * 9.2 / 9.4, 4 10.0 / 9.7, 6 11.8 / 11.0, 12 15.0 / 13.8) */
+		const unsigned int lin = contiguous ? xcd_contiguous_block_id(blockIdx.x, gridDim.x) : xcd_run_block_id(blockIdx.x, gridDim.x, 4);
 		const unsigned int strip_id = lin / slices;
 		const unsigned int slice = lin - strip_id * slices;
 		const unsigned int batch = strip_id / tiles_h;
@@ -1175,8 +1198,9 @@ namespace
 	{
 		const dim3 block(256);
 		const int mode = (act == ACTIVATION_LINEAR) ? 0 : ((act == ACTIVATION_RELU) ? 1 : 2);
+		const bool cached = matrices_stay_cached(static_cast<size_t>(batch) * tiles_h * tiles_w, channels, sizeof(T));
 #define MLHIP_LAUNCH_OUTPUT(MODE, EXT) \
-		hipLaunchKernelGGL((kernel_output_transform_4x4_3x3<T, VEC, MODE, EXT>), grid, block, 0, stream, in, out, b, e, act, batch, height, width, channels, tiles_h, tiles_w)
+		hipLaunchKernelGGL((cached ? kernel_output_transform_4x4_3x3<T, VEC, MODE, EXT, true> : kernel_output_transform_4x4_3x3<T, VEC, MODE, EXT, false>), grid, block, 0, stream, in, out, b, e, act, batch, height, width, channels, tiles_h, tiles_w)
 		if (e != nullptr)
 		{
 			if (mode == 0)
@@ -1247,10 +1271,12 @@ namespace
 		const T *e = ptr<const T>(ext);
 		T *nxt = ptr<T>(next);
 		const int a = static_cast<int>(act);
+		const bool cached = matrices_stay_cached(static_cast<size_t>(batch) * tiles_h * tiles_w, channels, sizeof(T));
 		const int mode = (act == ACTIVATION_LINEAR) ? 0 : ((act == ACTIVATION_RELU) ? 1 : 2);
 #define MLHIP_LAUNCH_FUSED(MODE, EXT) \
 		do { \
-			auto kernel = kernel_output_input_transform_4x4_3x3<T, VEC, SLICE, MODE, EXT, THREADS>; \
+			auto kernel = cached ? kernel_output_input_transform_4x4_3x3<T, VEC, SLICE, MODE, EXT, THREADS, true> \
+					: kernel_output_input_transform_4x4_3x3<T, VEC, SLICE, MODE, EXT, THREADS, false>; \
 			if (lds > 64 * 1024) \
 				ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), static_cast<int>(lds)); \
 			hipLaunchKernelGGL(kernel, grid, block, lds, stream, in, out, b, e, a, nxt, batch, height, width, channels, tiles_h, tiles_w); \
@@ -1296,7 +1322,7 @@ namespace
 		const bool relu = (act == ACTIVATION_RELU);
 #define MLHIP_LAUNCH_STRIPS(ACT, EXT) \
 		hipLaunchKernelGGL((kernel_output_input_transform_strips<T, ACT, EXT>), grid, dim3(192), lds, stream, in, out, b, e, nxt, batch, height, width, channels, \
-				tiles_h, tiles_w)
+				tiles_h, tiles_w, batch >= 4)
 		if (e != nullptr)
 		{
 			if (relu)

@@ -83,6 +83,41 @@ def test_gemm_batched_nt_streaming_other_row_lengths(ctx, dtype, K, shape):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "float16"])
+@pytest.mark.parametrize("shape", [(36, 1, 8, 32), (36, 65, 72, 96), (36, 191, 40, 160), (36, 192, 136, 32), (8, 257, 264, 224), (7, 700, 392, 384), (36, 300, 384, 384),
+                                   (36, 130, 128, 192), (36, 520, 256, 256), (36, 1300, 264, 256), (36, 1040, 128, 128), (9, 4100, 72, 128)])
+def test_gemm_batched_nt_tiles(ctx, dtype, shape):
+    """Plain batched products between the direct and the streaming kernel: one row, ragged rows and columns of 64 and 128-wide tiles, K rows
+    of whole and half 128-byte pieces, grids by matrix and (at least 8 matrices of 192 rows) by rows."""
+    bt, M, N, K = shape
+    rng = np.random.default_rng(sum(shape))
+    A = random_tensor(rng, (bt, M, K), dtype, 0.5)
+    Bm = random_tensor(rng, (bt, N, K), dtype, 0.5)
+    dC = ml.Tensor((bt, M, N), dtype)
+    dC.setall(ctx, float("nan"))
+    ml.gemmBatched(ctx, "n", "t", dC, ml.toDevice(ctx, A), ml.toDevice(ctx, Bm), 1.0, 0.0)
+    assert max_abs_rel(dC.copyToHost(ctx), O.gemm(A, Bm)) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype,K,N", [("float16", 32, 256), ("float16", 64, 64), ("float16", 96, 96), ("float16", 128, 128), ("float16", 192, 192), ("float16", 256, 256),
+                                       ("float16", 384, 384), ("float32", 32, 64), ("float32", 64, 64), ("float32", 128, 128), ("float32", 192, 192)])
+def test_gemm_batched_rows_do_not_depend_on_their_number(ctx, dtype, K, N):
+    """Every kernel and grid order that a Winograd product may take by its number of rows gives the same bits for the same row."""
+    rng = np.random.default_rng(K + N)
+    most = 5200 if N <= 128 else 2700
+    A = random_tensor(rng, (36, most, K), dtype, 0.5)
+    dB = ml.toDevice(ctx, random_tensor(rng, (36, N, K), dtype, 0.5))
+    want = None
+    for M in (most, 17, 100, 210, 450, 700, 1500, 2400, 4000):
+        if M > most:
+            continue
+        dC = ml.Tensor((36, M, N), dtype)
+        ml.gemmBatched(ctx, "n", "t", dC, ml.toDevice(ctx, A[:, :M]), dB, 1.0, 0.0)
+        got = dC.copyToHost(ctx)
+        want = got if want is None else want
+        assert mismatches(got, np.ascontiguousarray(want[:, :M])) == 0, M
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float16"])
 def test_gemm_batched_more_matrices_than_one_grid_dimension_holds(ctx, dtype):
     """65535 + 5 tiny products in one call (the reference's interface has no limit on the batch); with beta and a broadcast B operand."""
     rng = np.random.default_rng(11)

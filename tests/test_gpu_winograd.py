@@ -229,6 +229,25 @@ def test_fused_output_input_transform_forms(ctx, dtype, shape):
             de = ml.toDevice(ctx, ext)
 
 
+@pytest.mark.parametrize("dtype,shape", [("float16", (157, 33, 33, 64)), ("float32", (75, 33, 33, 64)), ("float32", (111, 33, 33, 64)), ("float16", (203, 19, 19, 256)),
+                                         ("float16", (61, 19, 19, 128))])
+def test_fused_transform_where_matrices_leave_the_last_level_cache(ctx, dtype, shape):
+    """Both sides of the size from which the transforms mark their streams non-temporal and order the images round the XCDs, in the forms with
+    narrow and wide slices: the same bits as the two separate calls."""
+    b, h, w, c = shape
+    tiles = b * ((h + 3) // 4) * ((w + 3) // 4)
+    rng = np.random.default_rng(b)
+    dm = ml.toDevice(ctx, np.resize(random_tensor(rng, (1000003,), dtype), (36, tiles, c)))
+    db, de = ml.toDevice(ctx, random_tensor(rng, (c,), dtype)), ml.toDevice(ctx, np.resize(random_tensor(rng, (999983,), dtype), shape))
+    y, dv, want_y, want_v = ml.Tensor(shape, dtype), ml.Tensor((36, tiles, c), dtype), ml.Tensor(shape, dtype), ml.Tensor((36, tiles, c), dtype)
+    for ext in (None, de):
+        ml.winogradOutputTransform(ctx, (c, 3, 3, c), dm, want_y, db, ext, O.RELU)
+        ml.winogradInputTransform(ctx, (c, 3, 3, c), want_y, want_v)
+        ml.winogradOutputInputTransform(ctx, (c, 3, 3, c), dm, shape, y, db, ext, O.RELU, dv)
+        assert mismatches(y.copyToHost(ctx), want_y.copyToHost(ctx)) == 0
+        assert mismatches(dv.copyToHost(ctx), want_v.copyToHost(ctx)) == 0
+
+
 @pytest.mark.parametrize("case", [(32, 15, 15, True, True, O.RELU), (64, 13, 16, False, False, O.RELU), (36, 15, 15, True, False, O.LINEAR),
                                   (256, 15, 15, True, True, O.RELU), (8, 15, 15, True, True, O.RELU), (32, 19, 19, True, True, O.RELU)])
 def test_whole_layer_launch_is_bit_identical(ctx, case):
