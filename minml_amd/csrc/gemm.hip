@@ -250,11 +250,18 @@ namespace mlhip
 		const StreamGemmArgs short_rows { g.A, g.B, g.D, g.M, g.N, static_cast<int>(std::min<size_t>(k_bytes, 0x7fffffffu)), g.batch, g.stride_a, g.stride_b, g.stride_c };
 		if (fast && plain && g.batch > 1 && k_bytes <= 0x7fffffffu)
 		{
-			if ((g.dtype == DTYPE_FLOAT16) ? try_launch_gemm_tiles<half_t>(stream, short_rows) : try_launch_gemm_tiles<float>(stream, short_rows))
+			if (try_launch_gemm_tiles(stream, g.dtype, short_rows))
 			{
 				MLHIP_CHECK(hipGetLastError());
 				return;
 			}
+		}
+		if (fast && vectorized && k_bytes <= 0x7fffffffu
+				&& ((g.dtype == DTYPE_FLOAT16 && try_launch_gemm_tiles(stream, short_rows, make_float_epilogue<half_t>(g, true)))
+						|| (g.dtype == DTYPE_FLOAT32 && try_launch_gemm_tiles(stream, short_rows, make_float_epilogue<float>(g, true)))))
+		{
+			MLHIP_CHECK(hipGetLastError());
+			return;
 		}
 		/* the same products with few rows, whose launch is all latency */
 		if (fast && g.dtype == DTYPE_FLOAT16 && vectorized && gemm_direct_applies(short_rows))

@@ -27,200 +27,11 @@
 #define MINML_AMD_GEMM_TILES_HPP_
 
 #include "common.hpp"
+#include "epilogues.hpp"
 #include "gemm_stream.hpp"
 
 namespace mlhip
 {
-	template<typename T, int BLOCKS_M_, int BLOCKS_N_, int WAVES_M_, int WAVES_N_>
-	struct GemmTileShape
-	{
-			static constexpr int BLOCKS_M = BLOCKS_M_, BLOCKS_N = BLOCKS_N_; /* 32x32 blocks of one wavefront */
-			static constexpr int WAVES_M = WAVES_M_, WAVES_N = WAVES_N_, WAVES = WAVES_M * WAVES_N, THREADS = 64 * WAVES;
-			static constexpr int BM = 32 * BLOCKS_M * WAVES_M, BN = 32 * BLOCKS_N * WAVES_N;
-			static constexpr int SLOTS = 2, SLOT_BYTES = (BM + BN) * 128; /* 128 bytes of K of every row of A and B */
-			static constexpr int LOADS = (BM + BN) / 8 / WAVES; /* direct-to-LDS loads (8 rows x 128 bytes) per wavefront and piece */
-			static constexpr int SLAB_STRIDE = 32 * BLOCKS_N * static_cast<int>(sizeof(T)) + 16;
-			static constexpr int LDS_BYTES = SLOTS * SLOT_BYTES;
-			/* workgroups that share a compute unit: as many as the 160 KB of LDS hold, four at most */
-			static constexpr int RESIDENT = (160 * 1024 / LDS_BYTES < 4) ? 160 * 1024 / LDS_BYTES : 4;
-			static_assert((BM + BN) % (8 * WAVES) == 0, "the same number of loads for every wavefront");
-			static_assert(WAVES * 32 * SLAB_STRIDE <= LDS_BYTES, "the slots become the slabs of the store");
-	};
-
-	template<typename T, typename Shape>
-	__global__ __launch_bounds__(Shape::THREADS, Shape::RESIDENT * Shape::WAVES / 4) void kernel_gemm_tiles_nt(const T *A, const T *B, T *C, int M, int N, int k_bytes,
-			size_t stride_a, size_t stride_b, size_t stride_c, unsigned int tiles_m, unsigned int tiles_n, unsigned int matrices, int by_rows)
-	{
-		typedef MfmaTraits<T> Traits;
-		typedef typename Traits::acc_vec acc_vec;
-		constexpr int BLOCKS_M = Shape::BLOCKS_M, BLOCKS_N = Shape::BLOCKS_N, WAVES = Shape::WAVES, LOADS = Shape::LOADS;
-		const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-		const int wave_m = wave / Shape::WAVES_N, wave_n = wave % Shape::WAVES_N;
-		const int frag_row = lane & 31, half_sel = lane >> 5;
-		const int pieces = (k_bytes + 127) / 128;
-
-		/* the column tiles of one row tile are neighbours on one XCD; the row tile's matrix changes slowest or its rows do */
-		const unsigned int id = xcd_contiguous_block_id(blockIdx.x, gridDim.x);
-		const unsigned int row_tile = id / tiles_n;
-		const unsigned int slow = row_tile / (by_rows ? matrices : tiles_m);
-		const unsigned int fast = row_tile - slow * (by_rows ? matrices : tiles_m);
-		const unsigned int matrix = by_rows ? fast : slow;
-		const int m_tile = (by_rows ? slow : fast) * Shape::BM, n_tile = (id - row_tile * tiles_n) * Shape::BN;
-		const int m0 = m_tile + wave_m * 32 * BLOCKS_M, n0 = n_tile + wave_n * 32 * BLOCKS_N;
-
-		/*
-		 * Operands -> LDS slot: [row of A, then of B][128 bytes], the 16-byte chunks of a row swizzled. Rows beyond the matrix repeat its last
-		 * row. Row 8 q + 4 h + e of a block of 32 rows of B holds column 16 h + 4 q + e: a lane then ends with 16 consecutive columns.
-		 */
-		extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
-		const uint8_t *a_base = reinterpret_cast<const uint8_t*>(A + matrix * stride_a);
-		const uint8_t *b_base = reinterpret_cast<const uint8_t*>(B + matrix * stride_b);
-		const uint8_t *src[LOADS];
-		static_assert(WAVES % 2 == 0, "the swizzle of a lane is then the same in all its loads");
-		const int chunk = ((lane & 7) ^ ((4 * wave + (lane >> 4)) & 7)) * 16;
-#pragma unroll
-		for (int u = 0; u < LOADS; u++)
-		{
-			const int row = (wave + WAVES * u) * 8 + (lane >> 3);
-			const int place = row - Shape::BM;
-			const int column = (place & ~31) + 16 * ((place >> 2) & 1) + 4 * ((place >> 3) & 3) + (place & 3);
-			src[u] = ((row < Shape::BM) ? a_base + static_cast<size_t>(min(m_tile + row, M - 1)) * k_bytes
-					: b_base + static_cast<size_t>(min(n_tile + column, N - 1)) * k_bytes) + chunk;
-		}
-		/* the last piece may have 64 bytes only: the lanes beyond them repeat what lies 64 bytes before, and nobody reads it */
-		const auto request = [&](int piece, auto slot) __attribute__((always_inline))
-		{
-			const int back = (piece * 128 + 64 == k_bytes) ? (chunk & 64) : 0;
-#pragma unroll
-			for (int u = 0; u < LOADS; u++)
-			{
-				__builtin_amdgcn_global_load_lds((global_ptr_t) (src[u] - back), (lds_ptr_t) (lds + decltype(slot)::value * Shape::SLOT_BYTES + (wave + WAVES * u) * 1024), 16, 0, 0);
-				src[u] += 128;
-			}
-		};
-		request(0, std::integral_constant<int, 0>());
-		if (pieces > 1)
-			request(1, std::integral_constant<int, 1>());
-
-		acc_vec acc[BLOCKS_M][BLOCKS_N];
-#pragma unroll
-		for (int i = 0; i < BLOCKS_M; i++)
-#pragma unroll
-			for (int j = 0; j < BLOCKS_N; j++)
-#pragma unroll
-				for (int r = 0; r < 16; r++)
-					acc[i][j][r] = 0;
-		int a_first[BLOCKS_M], b_first[BLOCKS_N]; /* this lane's fragment of a slot's first k step, the others by XOR */
-#pragma unroll
-		for (int i = 0; i < BLOCKS_M; i++)
-		{
-			const int row = wave_m * 32 * BLOCKS_M + 32 * i + frag_row;
-			a_first[i] = row * 128 + ((half_sel ^ ((row >> 1) & 7)) * 16);
-		}
-#pragma unroll
-		for (int j = 0; j < BLOCKS_N; j++)
-		{
-			const int row = Shape::BM + wave_n * 32 * BLOCKS_N + 32 * j + frag_row;
-			b_first[j] = row * 128 + ((half_sel ^ ((row >> 1) & 7)) * 16);
-		}
-		const auto multiply = [&](int piece, auto slot) __attribute__((always_inline))
-		{
-			/* loads return in order: this piece has landed once at most those of the next one are outstanding */
-			if (piece + 1 < pieces)
-				wait_vmcnt<LOADS>();
-			else
-				wait_vmcnt<0>();
-			barrier_no_fence();
-			const uint8_t *base = lds + decltype(slot)::value * Shape::SLOT_BYTES;
-			const auto step = [&](int kk) __attribute__((always_inline))
-			{
-				uint4_t a[BLOCKS_M], b[BLOCKS_N];
-#pragma unroll
-				for (int i = 0; i < BLOCKS_M; i++)
-					a[i] = *reinterpret_cast<const uint4_t*>(base + (a_first[i] ^ (kk * 32)));
-#pragma unroll
-				for (int j = 0; j < BLOCKS_N; j++)
-					b[j] = *reinterpret_cast<const uint4_t*>(base + (b_first[j] ^ (kk * 32)));
-#pragma unroll
-				for (int i = 0; i < BLOCKS_M; i++)
-#pragma unroll
-					for (int j = 0; j < BLOCKS_N; j++)
-						Traits::mma(b[j], a[i], acc[i][j]);
-			};
-			step(0);
-			step(1);
-			if (piece * 128 + 64 < k_bytes)
-			{
-				step(2);
-				step(3);
-			}
-			/* everyone has read the slot before it takes the piece after the next one, or the slabs of the store */
-			wait_lgkmcnt_zero();
-			if (piece + 2 < pieces)
-			{
-				barrier_no_fence();
-				request(piece + 2, slot);
-			}
-		};
-		for (int piece = 0; piece < pieces; piece += 2)
-		{
-			multiply(piece, std::integral_constant<int, 0>());
-			if (piece + 1 < pieces)
-				multiply(piece + 1, std::integral_constant<int, 1>());
-		}
-		barrier_no_fence();
-
-		/* lane l, register r of block (i, j): m = 32 i + l % 32, n = 32 j + 16 (l / 32) + r; 32 rows at a time cross the wavefront's slab and
-		 * leave as whole rows of the sub-tile, 16 bytes per lane (N is a multiple of the vector, checked by the launcher) */
-		constexpr int E = 16 / sizeof(T), LANES_PER_ROW = 32 * BLOCKS_N / E, ROWS_PER_PASS = 64 / LANES_PER_ROW;
-		uint8_t *slab = lds + wave * 32 * Shape::SLAB_STRIDE;
-		T *out = C + matrix * stride_c;
-		const int col = (lane % LANES_PER_ROW) * E;
-#pragma unroll
-		for (int i = 0; i < BLOCKS_M; i++)
-		{
-#pragma unroll
-			for (int j = 0; j < BLOCKS_N; j++)
-#pragma unroll
-				for (int r = 0; r < 16; r += E)
-				{
-					Vec<T, E> v;
-#pragma unroll
-					for (int e = 0; e < E; e++)
-						v.v[e] = acc[i][j][r + e];
-					v.store(reinterpret_cast<T*>(slab + frag_row * Shape::SLAB_STRIDE) + 32 * j + 16 * half_sel + r);
-				}
-			wait_lgkmcnt_zero(); /* the slab is private to this wavefront */
-			__builtin_amdgcn_wave_barrier();
-#pragma unroll
-			for (int pass = 0; pass < 32 / ROWS_PER_PASS; pass++)
-			{
-				const int row = pass * ROWS_PER_PASS + lane / LANES_PER_ROW;
-				const uint4_t v = *reinterpret_cast<const uint4_t*>(slab + row * Shape::SLAB_STRIDE + col * sizeof(T));
-				const int m = m0 + 32 * i + row;
-				if (m < M && n0 + col < N)
-					*reinterpret_cast<uint4_t*>(out + static_cast<size_t>(m) * N + n0 + col) = v;
-			}
-			wait_lgkmcnt_zero();
-			__builtin_amdgcn_wave_barrier();
-		}
-	}
-
-	template<typename T, int BLOCKS_M, int BLOCKS_N, int WAVES_M, int WAVES_N>
-	inline bool try_launch_gemm_tiles_as(hipStream_t stream, const StreamGemmArgs &g, bool by_rows)
-	{
-		typedef GemmTileShape<T, BLOCKS_M, BLOCKS_N, WAVES_M, WAVES_N> Shape;
-		const int tiles_m = ceil_div(g.M, Shape::BM), tiles_n = ceil_div(g.N, Shape::BN);
-		const unsigned long long tiles = static_cast<unsigned long long>(tiles_m) * tiles_n * g.batch;
-		if (tiles > 0xffffffffULL / Shape::THREADS) /* threads that a launch can have */
-			return false;
-		auto kernel = kernel_gemm_tiles_nt<T, Shape>;
-		if (Shape::LDS_BYTES > 64 * 1024)
-			ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), Shape::LDS_BYTES);
-		hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned int>(tiles)), dim3(Shape::THREADS), Shape::LDS_BYTES, stream, reinterpret_cast<const T*>(g.A),
-				reinterpret_cast<const T*>(g.B), reinterpret_cast<T*>(g.C), g.M, g.N, g.k_bytes, g.stride_a, g.stride_b, g.stride_c, tiles_m, tiles_n, g.batch, by_rows);
-		return true;
-	}
 	/* what the products read once and write: all of A and C */
 	inline unsigned long long exchanged_bytes(const StreamGemmArgs &g, int element_size)
 	{
@@ -260,7 +71,7 @@ namespace mlhip
 	 * which the streaming kernel holds only 128 columns: 226 MB 132 / 120, with three calls per layer 280 MB 150 / 160; fp32 512-byte rows 151 MB 82.4 / 79.9, 227
 	 * 117 / 123; 64-byte rows (the stem, alone) 170 MB 32.4 / 29.3, 340 89.8 / 101; fp32 128-byte rows 85 MB 25.3 / 26.2, 149 31.0 / 33.6, 255 49.1 / 65.0.
 	 */
-	inline bool gemm_tiles_apply(const StreamGemmArgs &g, int element_size)
+	inline bool plain_gemm_tiles_apply(const StreamGemmArgs &g, int element_size)
 	{
 		const bool fp16 = element_size == 2;
 		if (g.k_bytes % 64 != 0 || (fp16 && (g.k_bytes == 128 || g.k_bytes > 768)))
@@ -298,29 +109,40 @@ namespace mlhip
 		return tiles >= fewest * device_compute_units() && exchanged_bytes(g, element_size) <= (megabytes << 20);
 	}
 	/*
-	 * Larger tiles, which fetch less, once there are enough of them. fp16 by rows, 64x64 / 128x64: 256 channels 448 rows (1008 tiles of 64x64) 18.6 / 19.2, 512
-	 * (1152) 19.8 / 19.1; 128 channels 896... 960 rows (1080) 16.1 / 16.0; 384 channels 192 rows (648) 18.9 / 19.4, 256 (864) 21.6 / 20.6. By matrix, 128x64 / 128x128:
-	 * 192 channels 2304 rows 32.8 / 35.5; 256 channels 1616 rows 37.8 / 36.7, 2304 52.2 / 51.2; 384 channels 1408 rows 58.4 / 55.1, 3072 97.5 / 95.6. fp32 stays at
-	 * 64x64: 128 channels 2048 rows 45.6 / 46.0, 256 channels 960 63.0 / 65.5, 640 46.7 / 45.8 (128x64).
+	 * The same for products with bias (+ beta * C), linear or ReLU: dense layers, 1x1 convolutions, the experts' layers. Alone, other kernel / this one, us, and
+	 * the number of 64x64 tiles:
+	 *   fp16, from 1.75 tiles per unit with rows up to 512 bytes (256 x 256: 2700 rows (172) 4.3 / 4.8, 7200 (452) 5.7 / 5.6; 128 to 768: 2700
+	 *   (516) 5.9 / 5.2), 1 up to 768 bytes (384 x 256: 7200 (452) 11.0 / 6.5; x 384: 2700 (258) 6.2 / 6.0), 0.5 up to 1024 (512 x 256: 2700 (172) 7.0 / 6.0). Rows of
+	 *   2048 bytes, for which a tile of 256 rows is the better one where there are enough, from 1 to 4 (eight experts of 1024 x 256: 912 rows
+	 *   (480) 13.4 / 10.6, 3648 (1824) 25.4 / 30.7); 1024 with a batch to 8 (512 x 1024: 912 rows (1920) 18.5 / 15.9, 3648 (7296) 43.5 / 46.4).
+	 *   Not beyond 96 MB of A, C and what is read of it where the streaming kernel takes the rows (256 x 256: 57600 rows, 88 MB with residual, 26.4 / 23.8,
+	 *   115200 (177) 41.7 / 41.7, 230400 81.5 / 105; 256 x 1024: 27797 (71) 28.7 / 28.1, 57600 (147) 48.8 / 55.1; 384 x 384 with residual: 27797 (64) 25.2 / 22.2, 57600
+	 *   (133) 39.7 / 40.1; eight experts of 256 x 1024: 3648 rows (75) 36.7 / 29.4, 7296 (149) 57.1 / 55.4, 14592 89 / 127), 180 with one column tile
+	 *   (128 x 128 with residual: 230400 rows (177) 36.4 / 34.2, 369664 (284) 50.2 / 68.8).
+	 *   fp32, rows of 256 and 512 bytes, which only the streaming kernel took: always (128 x 128: 225 rows 17.2 / 6.2, 27797 20.2 / 16.4, 230400 105 / 87).
+	 *   Others up to 4096 bytes from 0.6 (256 x 256: 900 rows (60) 6.8 / 8.8, 2700 (172) 11.8 / 9.2, 57600 87.6 / 74.5).
 	 */
-	template<typename T>
-	inline bool try_launch_gemm_tiles(hipStream_t stream, const StreamGemmArgs &g)
+	inline bool gemm_tiles_apply(const StreamGemmArgs &g, int element_size, bool reads_c)
 	{
-		if (!gemm_tiles_apply(g, sizeof(T)))
+		const long long tiles = static_cast<long long>(ceil_div(g.M, 64)) * ceil_div(g.N, 64) * g.batch, units = device_compute_units();
+		if (g.k_bytes % 64 != 0)
 			return false;
-		const bool by_rows = products_go_by_rows(g, sizeof(T));
-		if constexpr (sizeof(T) == 2)
-		{
-			const long long tiles = static_cast<long long>(ceil_div(g.M, 64)) * ceil_div(g.N, 64) * g.batch;
-			if (tiles >= (g.k_bytes >= 768 ? 3 : 4) * device_compute_units())
-			{
-				if (!by_rows && g.k_bytes >= 512)
-					return try_launch_gemm_tiles_as<T, 2, 1, 2, 4>(stream, g, false);
-				return try_launch_gemm_tiles_as<T, 2, 1, 2, 2>(stream, g, by_rows);
-			}
-		}
-		return try_launch_gemm_tiles_as<T, 1, 1, 2, 2>(stream, g, by_rows);
+		if (element_size == 4)
+			return g.k_bytes == 256 || g.k_bytes == 512 || (g.k_bytes <= 4096 && 8 * tiles >= 5 * units);
+		if (g.k_bytes == 2048)
+			return tiles >= units && tiles <= 4 * units;
+		if (g.k_bytes < 192 || g.k_bytes > 1024)
+			return false;
+		if (g.k_bytes > 768 && g.batch > 1 && tiles > 8 * units)
+			return false;
+		const bool streams = g.k_bytes == 256 || g.k_bytes == 512 || g.k_bytes == 768;
+		const unsigned long long bytes = exchanged_bytes(g, element_size) + (reads_c ? static_cast<unsigned long long>(g.batch) * g.M * g.N * element_size : 0);
+		return 4 * tiles >= (g.k_bytes <= 512 ? 7 : g.k_bytes <= 768 ? 4 : 2) * units && !(streams && bytes > ((g.N > 128 ? 96ULL : 180ULL) << 20));
 	}
+	/* false: nothing was launched. Plain batched products of fp16 or fp32; and products with bias (+ beta * C), linear or ReLU */
+	bool try_launch_gemm_tiles(hipStream_t stream, mlDataType_t dtype, const StreamGemmArgs &g);
+	bool try_launch_gemm_tiles(hipStream_t stream, const StreamGemmArgs &g, const FloatEpilogue<half_t> &epilogue);
+	bool try_launch_gemm_tiles(hipStream_t stream, const StreamGemmArgs &g, const FloatEpilogue<float> &epilogue);
 } /* namespace mlhip */
 
 #endif /* MINML_AMD_GEMM_TILES_HPP_ */

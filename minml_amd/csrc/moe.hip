@@ -19,6 +19,7 @@
 #include "gemm_dma.hpp"
 #include "conv_tiles.hpp"
 #include "gemm_stream.hpp"
+#include "gemm_tiles.hpp"
 
 namespace
 {
@@ -936,6 +937,11 @@ extern "C"
 				ep.bias_batch_stride = neurons;
 				/* the epilogue's common cases (ReLU / linear, bias present, beta = 0 or not) are fixed at compile time: with K of only a few
 				 * chunks the epilogue is most of a tile's time, and its run-time form is twice as slow */
+				StreamGemmArgs tiles { x.data, w.data, y.data, static_cast<int>(rows), neurons, static_cast<int>(k_bytes), experts,
+						static_cast<size_t>(channels), static_cast<size_t>(neurons) * channels, static_cast<size_t>(neurons) };
+				tiles.a_row_bytes = static_cast<size_t>(experts) * k_bytes;
+				if (try_launch_gemm_tiles(stream, tiles, ep))
+					return;
 				if constexpr (sizeof(T) == 2)
 					specialise_epilogue(ep, [&](const auto &fixed)
 					{

@@ -98,6 +98,28 @@ def test_gemm_batched_nt_tiles(ctx, dtype, shape):
     assert max_abs_rel(dC.copyToHost(ctx), O.gemm(A, Bm)) <= TOL[dtype]
 
 
+@pytest.mark.parametrize("dtype", ["float32", "float16"])
+@pytest.mark.parametrize("shape", [(7200, 256, 256), (2701, 776, 96), (14401, 264, 128), (7300, 392, 384), (9000, 200, 192), (2750, 264, 512), (130, 8192, 1024), (14500, 260, 256)])
+def test_gemm_ex_tiles(ctx, dtype, shape):
+    """Dense layers between few rows and many (tiles of 64x64, 128x64 and 128x128; ragged rows and columns; a width that is no multiple of 16 bytes
+    in fp16, which goes on to the other kernels), with bias, ReLU or linear, with and without a residual; a prefix of the rows, which takes
+    another kernel, gives the same bits."""
+    M, N, K = shape
+    rng = np.random.default_rng(sum(shape))
+    A, W = random_tensor(rng, (M, K), dtype, 0.5), random_tensor(rng, (N, K), dtype, 0.5)
+    C, bias = random_tensor(rng, (M, N), dtype), random_tensor(rng, (N,), dtype)
+    dA, dW, dC, db, dD = ml.toDevice(ctx, A), ml.toDevice(ctx, W), ml.toDevice(ctx, C), ml.toDevice(ctx, bias), ml.Tensor((M, N), dtype)
+    for act, beta in ((O.RELU, 0.0), (O.LINEAR, 1.0), (O.RELU, 0.5)):
+        dD.setall(ctx, float("nan"))
+        ml.gemm_ex(ctx, dD, 1.0, "n", dA, "t", dW, beta, dC if beta else None, db, act)
+        got = dD.copyToHost(ctx)
+        assert max_abs_rel(got, O.gemm(A, W, beta=beta, C=C if beta else None, bias=bias, act=act)) <= TOL[dtype]
+        for m in (1, 77):
+            few = ml.Tensor((m, N), dtype)
+            ml.gemm_ex(ctx, few, 1.0, "n", ml.toDevice(ctx, A[:m]), "t", dW, beta, ml.toDevice(ctx, C[:m]) if beta else None, db, act)
+            assert mismatches(few.copyToHost(ctx), np.ascontiguousarray(got[:m])) == 0
+
+
 @pytest.mark.parametrize("dtype,K,N", [("float16", 32, 256), ("float16", 64, 64), ("float16", 96, 96), ("float16", 128, 128), ("float16", 192, 192), ("float16", 256, 256),
                                        ("float16", 384, 384), ("float32", 32, 64), ("float32", 64, 64), ("float32", 128, 128), ("float32", 192, 192)])
 def test_gemm_batched_rows_do_not_depend_on_their_number(ctx, dtype, K, N):
