@@ -604,6 +604,236 @@ namespace mlhip
 		store.finish(acc, lds, M, epilogue);
 	}
 
+	/*
+	 * The same for tiles of 256x256 by 2 x 4 wavefronts, with the two slots divided into quarters that are refilled one by one. A 64 KB chunk of
+	 * operands takes about as long from the L2 (30 bytes per clock and compute unit) as it takes to multiply; requested as a whole once the slot
+	 * before it is free, it lands a whole transfer later, and transfer and multiplication take turns instead of overlapping. Here a chunk is multiplied
+	 * in four phases, one quarter of the wavefront's sub-tile each (64 rows x 32 columns, all four k steps):
+	 *     phase 0: A0 B0    phase 1: A0 B1    phase 2: A1 B1    phase 3: A1 B0
+	 * A0 / A1 are the first / second 64 rows of every wavefront row, B0 / B1 the first / second 32 columns of every wavefront column, 16 KB each.
+	 * Fragments are read one phase before they are multiplied, into the registers whose last use has just been issued: B1 in phase 0, A1 in
+	 * phase 1, A0 and B0 of the next chunk in phase 3. What a phase has multiplied nobody needs in LDS any more after the next barrier, so
+	 * its quarter takes the chunk after the next one: A0 and B0 in phase 1, B1 in phase 2, A1 in phase 3. Every request then has six phases
+	 * (one and a half chunks) to land, and up to 16 loads per wavefront are in flight. One barrier opens every phase; the loads that may still be outstanding
+	 * then are counted exactly. K is summed in the order of the other form: same bits.
+	 * The expert layer 1024 -> 256 of 256 positions 15x15 with 8 experts, half precision, 82.5 -> 78.2 us, 512 -> 1024 181 -> 172 us (a whole block of
+	 * such layers with its router 246 -> 231 us); single
+	 * products of 4096 to 65536 rows and 256 to 2304 bytes of K: level to -11 %. Dense operands only: with the addresses of a convolution computed between
+	 * the phases a launch that fills the chip is slower (5x5, 256 channels, 115200 pixels 539 -> 566 us; the int8 network at 1024
+	 * positions 5967 -> 6099 us, both also limited by power), and only those of less than a workgroup per unit are faster (-5 %).
+	 */
+	template<typename T, typename Cfg, typename ALoader, typename BLoader, typename Epilogue>
+	__device__ __forceinline__ void gemm_tile_dma_quarters(const ALoader &a_loader, const BLoader &b_loader, int M, int k_bytes, int m0, int n0, uint8_t *lds,
+			const Epilogue &epilogue)
+	{
+		typedef MfmaTraits<T> Traits;
+		typedef typename Traits::acc_vec acc_vec;
+		static_assert(Cfg::BM == 256 && Cfg::BN == 256 && Cfg::WAVES_M == 2 && Cfg::WAVES_N == 4 && Cfg::SLOTS == 2 && Cfg::KSTEPS == 4, "quarters of this tile shape");
+		constexpr int QUARTER_BYTES = 128 * Cfg::BKB, LOADS = 2; /* 128 rows; direct-to-LDS loads per wavefront */
+		constexpr int A0 = 0, B0 = 1, B1 = 2, A1 = 3; /* place of a quarter in its slot */
+
+		const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+		const int wave_m = wave / Cfg::WAVES_N, wave_n = wave % Cfg::WAVES_N;
+		const int chunks = k_bytes / Cfg::BKB;
+
+		typename ALoader::Row a_rows[2][LOADS];
+		typename BLoader::Row b_rows[2][LOADS];
+		const int load_chunk = ((lane & 7) ^ ((4 * wave + (lane >> 4)) & 7)) * 16; /* position 8 (wave + 8 u) + lane / 8: the same swizzle for every u */
+#pragma unroll
+		for (int h = 0; h < 2; h++)
+#pragma unroll
+			for (int u = 0; u < LOADS; u++)
+			{
+				const int place = (wave + Cfg::WAVES * u) * 8 + (lane >> 3);
+				a_rows[h][u] = a_loader.begin_row(m0 + (place >> 6) * 128 + h * 64 + (place & 63));
+				b_rows[h][u] = b_loader.begin_row(n0 + (place >> 5) * 64 + h * 32 + (place & 31));
+			}
+		typename ALoader::Step a_step = a_loader.first_step();
+		typename BLoader::Step b_step = b_loader.first_step();
+		const auto request_a = [&](int chunk, auto half) __attribute__((always_inline))
+		{
+			constexpr int h = decltype(half)::value;
+			uint8_t *dst = lds + (chunk & 1) * Cfg::SLOT_BYTES + (h == 0 ? A0 : A1) * QUARTER_BYTES;
+#pragma unroll
+			for (int u = 0; u < LOADS; u++)
+				__builtin_amdgcn_global_load_lds((global_ptr_t) a_loader.chunk(a_rows[h][u], a_step, load_chunk), (lds_ptr_t) (dst + (wave + Cfg::WAVES * u) * 1024), 16, 0, 0);
+			if (h == 1)
+				a_loader.advance(a_step);
+		};
+		const auto request_b = [&](int chunk, auto half) __attribute__((always_inline))
+		{
+			constexpr int h = decltype(half)::value;
+			uint8_t *dst = lds + (chunk & 1) * Cfg::SLOT_BYTES + (h == 0 ? B0 : B1) * QUARTER_BYTES;
+#pragma unroll
+			for (int u = 0; u < LOADS; u++)
+				__builtin_amdgcn_global_load_lds((global_ptr_t) b_loader.chunk(b_rows[h][u], b_step, load_chunk), (lds_ptr_t) (dst + (wave + Cfg::WAVES * u) * 1024), 16, 0, 0);
+			if (h == 1)
+				b_loader.advance(b_step);
+		};
+		typedef std::integral_constant<int, 0> first_half;
+		typedef std::integral_constant<int, 1> second_half;
+
+		/* lane l supplies row l % 32 of a 32-row block and the 16-byte half l / 32 of each 32-byte k step */
+		int a_frag[2], b_frag;
+#pragma unroll
+		for (int i = 0; i < 2; i++)
+		{
+			const int place = wave_m * 64 + 32 * i + (lane & 31);
+			a_frag[i] = place * Cfg::BKB + (((lane >> 5) ^ dma_swizzle(place)) * 16);
+		}
+		{
+			const int place = wave_n * 32 + (lane & 31);
+			b_frag = place * Cfg::BKB + (((lane >> 5) ^ dma_swizzle(place)) * 16);
+		}
+		uint4_t fa[2][4], fb0[4], fb1[4];
+		const auto read_a = [&](int chunk, int quarter, int kk) __attribute__((always_inline))
+		{
+			const uint8_t *src = lds + (chunk & 1) * Cfg::SLOT_BYTES + quarter * QUARTER_BYTES;
+#pragma unroll
+			for (int i = 0; i < 2; i++)
+				fa[i][kk] = *reinterpret_cast<const uint4_t*>(src + (a_frag[i] ^ (kk * 32)));
+		};
+		const auto read_b = [&](int chunk, int quarter, int kk, uint4_t (&regs)[4]) __attribute__((always_inline))
+		{
+			regs[kk] = *reinterpret_cast<const uint4_t*>(lds + (chunk & 1) * Cfg::SLOT_BYTES + quarter * QUARTER_BYTES + (b_frag ^ (kk * 32)));
+		};
+
+		acc_vec acc[Cfg::BLOCKS_M][Cfg::BLOCKS_N];
+#pragma unroll
+		for (int i = 0; i < Cfg::BLOCKS_M; i++)
+#pragma unroll
+			for (int j = 0; j < Cfg::BLOCKS_N; j++)
+#pragma unroll
+				for (int r = 0; r < 16; r++)
+					acc[i][j][r] = 0;
+
+		for (int c = 0; c < 2; c++)
+			if (c < chunks)
+			{
+				request_a(c, first_half());
+				request_b(c, first_half());
+				request_b(c, second_half());
+				request_a(c, second_half());
+			}
+		if (chunks > 1)
+			wait_vmcnt<6 * LOADS>();
+		else
+			wait_vmcnt<2 * LOADS>();
+		barrier_no_fence();
+		if (chunks > 0)
+		{
+#pragma unroll
+			for (int kk = 0; kk < 4; kk++)
+			{
+				read_a(0, A0, kk);
+				read_b(0, B0, kk, fb0);
+			}
+		}
+		SlabEpilogue<T, Cfg, Epilogue> store;
+		/* one chunk: whether there is a next one, and whether there is one after it */
+		const auto process_chunk = [&](int c, auto one_more, auto two_more) __attribute__((always_inline))
+		{
+			constexpr bool NEXT = decltype(one_more)::value, AFTER = decltype(two_more)::value;
+			const auto multiply = [&](int kk, const uint4_t (&regs)[4], auto row, auto column) __attribute__((always_inline))
+			{
+#pragma unroll
+				for (int i = 0; i < 2; i++)
+					Traits::mma(regs[kk], fa[i][kk], acc[decltype(row)::value + i][decltype(column)::value]);
+			};
+			typedef std::integral_constant<int, 0> zero;
+			typedef std::integral_constant<int, 1> one;
+			typedef std::integral_constant<int, 2> two;
+			/* phase 0. Behind B1 of this chunk: its A1, all of the next one */
+			wait_vmcnt<NEXT ? 5 * LOADS : LOADS>();
+			barrier_no_fence();
+			multiply(0, fb0, zero(), zero());
+			__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+			for (int kk = 0; kk < 4; kk++)
+				read_b(c, B1, kk, fb1);
+			__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+			for (int kk = 1; kk < 4; kk++)
+				multiply(kk, fb0, zero(), zero());
+			__builtin_amdgcn_sched_barrier(0);
+			/* phase 1. Behind A1: all of the next chunk */
+			wait_vmcnt<NEXT ? 4 * LOADS : 0>();
+			barrier_no_fence();
+			multiply(0, fb1, zero(), one());
+			__builtin_amdgcn_sched_barrier(0);
+			read_a(c, A1, 0);
+			if constexpr (AFTER)
+			{
+				request_a(c + 2, first_half());
+				request_b(c + 2, first_half());
+			}
+			__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+			for (int kk = 1; kk < 4; kk++)
+			{
+				multiply(kk, fb1, zero(), one());
+				__builtin_amdgcn_sched_barrier(0);
+				read_a(c, A1, kk);
+				__builtin_amdgcn_sched_barrier(0);
+			}
+			/* phase 2 */
+			barrier_no_fence();
+			multiply(0, fb1, two(), one());
+			__builtin_amdgcn_sched_barrier(0);
+			if constexpr (AFTER)
+				request_b(c + 2, second_half());
+			if constexpr (!NEXT)
+				store.begin(M, m0, n0, epilogue); /* the load queue is empty: the epilogue's first loads land under the last two phases */
+			__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+			for (int kk = 1; kk < 4; kk++)
+				multiply(kk, fb1, two(), one());
+			__builtin_amdgcn_sched_barrier(0);
+			/* phase 3. Behind A0 and B0 of the next chunk: its other two quarters, three of the one after it */
+			if constexpr (NEXT)
+			{
+				wait_vmcnt<AFTER ? 5 * LOADS : 2 * LOADS>();
+				barrier_no_fence();
+			}
+			multiply(0, fb0, two(), zero());
+			__builtin_amdgcn_sched_barrier(0);
+			if constexpr (NEXT)
+			{
+				read_a(c + 1, A0, 0);
+				read_b(c + 1, B0, 0, fb0);
+			}
+			if constexpr (AFTER)
+				request_a(c + 2, second_half());
+			__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+			for (int kk = 1; kk < 4; kk++)
+			{
+				multiply(kk, fb0, two(), zero());
+				__builtin_amdgcn_sched_barrier(0);
+				if constexpr (NEXT)
+				{
+					read_a(c + 1, A0, kk);
+					read_b(c + 1, B0, kk, fb0);
+				}
+				__builtin_amdgcn_sched_barrier(0);
+			}
+		};
+		int c = 0;
+		for (; c + 2 < chunks; c++)
+			process_chunk(c, std::true_type(), std::true_type());
+		if (c + 1 < chunks)
+			process_chunk(c++, std::true_type(), std::false_type());
+		if (c < chunks)
+			process_chunk(c, std::false_type(), std::false_type());
+		else
+			store.begin(M, m0, n0, epilogue);
+
+		/* the slots become the epilogue's slabs: every wavefront must have finished reading fragments */
+		__builtin_amdgcn_s_waitcnt(0xc07f);
+		barrier_no_fence();
+		store.finish(acc, lds, M, epilogue);
+	}
+
 	/* tile shapes by output width: wavefront sub-tiles of 128x128, 128x64 and 64x64 */
 	typedef DmaTileConfig<256, 256, 2, 4, 2, 2, 4> DmaTileWide;
 	typedef DmaTileConfig<256, 128, 4, 2, 2, 2, 2> DmaTileMedium;
@@ -632,7 +862,10 @@ namespace mlhip
 			if (epilogue.bias != nullptr)
 				epilogue.bias += batch * epilogue.bias_batch_stride; /* 0 unless every matrix of the batch has its own bias */
 		}
-		gemm_tile_dma<T, Cfg>(a_loader, b_loader, M, k_bytes, tile_m * Cfg::BM, tile_n * Cfg::BN, lds, epilogue);
+		if constexpr (std::is_same<Cfg, DmaTileWide>::value && std::is_same<ALoader, DenseDmaRows>::value)
+			gemm_tile_dma_quarters<T, Cfg>(a_loader, b_loader, M, k_bytes, tile_m * Cfg::BM, tile_n * Cfg::BN, lds, epilogue);
+		else
+			gemm_tile_dma<T, Cfg>(a_loader, b_loader, M, k_bytes, tile_m * Cfg::BM, tile_n * Cfg::BN, lds, epilogue);
 	}
 
 	template<typename T, typename Cfg, typename ALoader, typename Epilogue>

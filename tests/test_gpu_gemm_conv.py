@@ -758,6 +758,22 @@ def test_group_gemm(ctx, dtype, case):
     assert max_abs_rel(dC.copyToHost(ctx), want) <= TOL[dtype]
 
 
+@pytest.mark.parametrize("dtype,chunk", [("float16", 64), ("float32", 32)])
+@pytest.mark.parametrize("chunks", [1, 2, 3, 4, 5, 8])
+def test_group_gemm_wide_tiles(ctx, dtype, chunk, chunks):
+    """Every length of the 256-wide tile's pipeline (its head, the steady part, both parities of its two slots, its tail), with whole and
+    ragged tiles of rows and columns; the last bits do not depend on where in a tile a row or column lies. The operands and their sums are
+    small whole numbers, exact in every precision used: the tolerance is 0."""
+    M, N, K, groups = 300, 260, chunk * chunks, 2
+    rng = np.random.default_rng(chunks)
+    stored = O.to_half if dtype == "float16" else (lambda t: t)
+    a, b, c = (rng.integers(-1, 2, s).astype(np.float32) for s in ((M, K * groups), (N, K * groups), (M, N * groups)))
+    dC = ml.toDevice(ctx, stored(c))
+    ml.gemmGrouped(ctx, "n", "t", dC, ml.toDevice(ctx, stored(a)), ml.toDevice(ctx, stored(b)), 1.0, 1.0, groups)
+    want = np.concatenate([c[:, g * N:(g + 1) * N] + a[:, g * K:(g + 1) * K] @ b[:, g * K:(g + 1) * K].T for g in range(groups)], axis=1)
+    assert np.array_equal(dC.copyToHost(ctx), stored(want))
+
+
 def test_grouped_1x1_convolution_layer(ctx):
     """Conv2D with groups > 1 as the reference runs it (src/layers/Conv2D.cpp:339-349): grouped product, then bias and activation; against
     one dense 1x1 convolution of the oracle per group."""
