@@ -1571,23 +1571,24 @@ extern "C"
 		}
 		mlTensor_t next = next_matrices;
 		/*
-		 * Which form, by the number of 64-channel slices of images (= workgroups of the widest form) for 256 compute units. Measured alone
-		 * (8 launches replayed as one graph), us per launch, 256 channels 15x15, without / with residual and stored y:
-		 *   slices                             4            24            48            64           128           192           256
-		 *   fp16  64 channels, 256 threads  9.6 / 10.4    9.1 / 10.7    9.5 / 11.1    9.7 / 11.4  10.4 / 12.4   11.0 / 13.9   12.8 / 14.6
-		 *         32 channels               6.7 / 8.1     6.8 / 8.5     7.1 / 8.9     7.3 / 9.2    8.3 / 10.7    9.7 / 15.2   12.3 / 16.4
-		 *         16 channels               7.1 / 7.6     7.5 / 8.4     7.8 / 8.6     7.9 / 8.8   10.0 / 11.2   11.8 / 16.5   15.8 / 20.5
-		 *         strips of 16 channels     4.9 / 5.2     5.5 / 6.1     6.3 / 6.9     7.1 / 7.9    9.4 / 12.4   12.8 / 17.3   16.6 / 21.7
-		 *   fp32  64 channels, 256 threads  8.4 / 12.1    8.9 / 12.8    9.4 / 13.7    9.9 / 14.8  13.1 / 18.2   15.3 / 21.7   18.1 / 24.4
-		 *         32 channels               7.2 / 11.1    7.6 / 12.0    8.2 / 13.2    8.5 / 14.8  10.9 / 19.0   14.2 / 27.2   16.2 / 30.8
-		 *         16 channels               6.4 / 7.2     6.9 / 7.8     7.5 / 8.9     8.1 / 9.2   12.3 / 15.6   16.2 / 23.6   23.5 / 30.3
-		 *         strips of 16 channels     4.6 / 4.8     5.4 / 5.8     6.5 / 7.2     7.4 / 8.2   12.4 / 15.9   17.2 / 21.4   21.7 / 27.0
+		 * Which form, by the number of 64-channel slices of images (= workgroups of the widest form) for 256 compute units. In networks (40 layers,
+		 * transform + product, us per layer), 256 channels 15x15, without / with residual and stored y:
+		 *   slices                             32           48           64           80          128          192          256          320          404
+		 *   fp16  64 channels, 256 threads 14.6 / 16.0  16.0 / 17.2  16.9 / 18.3  17.5 / 18.9  19.6 / 21.2  22.5 / 24.7  25.1 / 28.3  29.2 / 32.8  34.3 / 37.6
+		 *         32 channels              12.6 / 14.0  13.8 / 15.2  14.7 / 16.6  15.5 / 17.8  18.0 / 20.4  21.9 / 24.4  24.4 / 27.7  27.7 / 32.4  32.4 / 39.5
+		 *         16 channels              12.7 / 13.3  14.0 / 14.6  15.1 / 16.1  16.7 / 17.8  19.2 / 20.4  23.0 / 24.9  26.3 / 29.7  29.7 / 35.7  37.3 / 42.1
+		 *         strips of 16 channels    10.9 / 11.3  12.9 / 13.4  14.0 / 14.6  14.9 / 16.4  18.0 / 20.6  22.7 / 25.9  26.8 / 31.1  30.0 / 35.3  36.0 / 42.8
+		 *   fp32  64 channels, 256 threads 24.2 / 27.9  24.3 / 29.3  28.5 / 34.4  29.4 / 34.8  39.2 / 44.9  52.5 / 58.5  65.8 / 73.0  77.7 / 85.9
+		 *         32 channels              23.2 / 28.3  22.6 / 30.6  27.1 / 35.0  28.0 / 35.7  37.7 / 46.5  51.0 / 60.3  64.5 / 75.2  76.1 / 87.6
+		 *         16 channels              22.9 / 23.5  22.9 / 23.5  27.1 / 28.2  28.5 / 30.0  38.5 / 40.1  52.0 / 55.0  65.8 / 70.1  78.5 / 83.3
+		 *         strips of 16 channels    20.7 / 21.0  20.8 / 21.7  25.5 / 26.8  26.9 / 28.2  37.7 / 40.1  51.0 / 55.0  65.1 / 70.1  77.7 / 83.3
 		 * A launch over few images is bound by what one workgroup must issue, a launch over many by memory, which wants whole 128-byte lines.
-		 * Strips up to 51 slices: between the network's products (product + transform, both kinds in turn) they take 16.2 us against 17.2 of
-		 * the 32-channel form at 48 slices of 256 channels, but 18.5 against 17.9 at 64; other widths and boards cross between 51 and 72.
-		 * With residual the fp32 form of 32 channels keeps 54 registers per lane in scratch memory (15x15, 128 slices: 19.0 us, 16 channels
-		 * 15.6, 64 channels 18.2; 19x19: 32.9, 25.6, 30.2) and is not built. Measured alternatives that were not faster for many images:
-		 * slices of 128 or 256 channels with 512 or 1024 threads, and 2-element vectors at twice the occupancy.
+		 * Strips to 85 slices in fp16 (at 96, 64 to 384 channels, -2 to +5 %) and to 96 in fp32 (-2 to -9 %; behind at 128): their repeated rows
+		 * come from the L2 of their XCD, which has the neighbouring strips. 32 channels to 320 slices (without residual 4 to 10 % ahead of 64
+		 * there, with residual -7 to +1 %; at 404 -4 to +6 %). With residual the fp32 form of 32 channels keeps 54 registers per lane in scratch
+		 * memory and is not built: 16 channels, 5 to 14 % ahead of 64 at 160 and 192 slices while the matrices stay cached, 20 % behind where
+		 * they do not. Measured alternatives that were not faster: slices of 128 or 256 channels with 512 or 1024 threads, 64 channels on
+		 * 2-element vectors, 32 channels on 512 threads or on 4-element vectors.
 		 */
 		const hipStream_t stream = stream_of(context);
 		const long long slices = static_cast<long long>(output_shape.dim[0]) * (channels / 64), units = device_compute_units();
@@ -1606,12 +1607,12 @@ extern "C"
 			typedef decltype(zero) T;
 			const bool strips_fit = static_cast<size_t>(6) * (4 * ceil_div(output_shape.dim[2], 4) + 2) * STRIP_CHANNELS * sizeof(T) <= 64 * 1024;
 			constexpr bool fp32 = sizeof(T) == 4;
-			const bool residual = ext.data != nullptr;
-			if (common_act && separate && strips_fit && 5 * slices <= units)
+			const bool residual = ext.data != nullptr, cached = matrices_stay_cached(tiles, channels, sizeof(T));
+			if (common_act && separate && strips_fit && (fp32 ? 8 * slices <= 3 * units : 3 * slices <= units))
 				launch_output_input_strips<T>(stream, matrices, bias, ext, output_shape, output, act, next);
-			else if (common_act && (residual || fp32) && (residual && fp32 ? 2 : 4) * slices <= units)
+			else if (common_act && (residual || fp32) && 4 * slices <= (residual && fp32 ? (cached ? 3 : 2) : 1) * units)
 				launch_output_input<T, 16, 1, 256, true, fp32 ? RESIDUAL_OR_NOT : RESIDUAL_ALWAYS>(stream, matrices, bias, ext, output_shape, output, act, next);
-			else if (common_act && !(residual && fp32) && (residual ? 2 : 1) * slices <= units)
+			else if (common_act && !(residual && fp32) && 4 * slices <= 5 * units)
 				launch_output_input<T, 32, 2, 256, true, fp32 ? RESIDUAL_NEVER : RESIDUAL_OR_NOT>(stream, matrices, bias, ext, output_shape, output, act, next);
 			else
 				launch_output_input<T, 64, 4, 256, false, RESIDUAL_OR_NOT>(stream, matrices, bias, ext, output_shape, output, act, next);

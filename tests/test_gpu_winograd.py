@@ -230,10 +230,11 @@ def test_fused_output_input_transform_forms(ctx, dtype, shape):
 
 
 @pytest.mark.parametrize("dtype,shape", [("float16", (157, 33, 33, 64)), ("float32", (75, 33, 33, 64)), ("float32", (111, 33, 33, 64)), ("float16", (203, 19, 19, 256)),
-                                         ("float16", (61, 19, 19, 128))])
-def test_fused_transform_where_matrices_leave_the_last_level_cache(ctx, dtype, shape):
+                                         ("float16", (61, 19, 19, 128))]
+                         + [(dtype, (slices, 7, 6, 64)) for dtype in ("float16", "float32") for slices in (85, 86, 96, 97, 192, 193, 320, 321)])
+def test_fused_transform_equals_the_separate_calls(ctx, dtype, shape):
     """Both sides of the size from which the transforms mark their streams non-temporal and order the images round the XCDs, in the forms with
-    narrow and wide slices: the same bits as the two separate calls."""
+    narrow and wide slices, and of the numbers of slices where one form ends: the same bits as the two separate calls."""
     b, h, w, c = shape
     tiles = b * ((h + 3) // 4) * ((w + 3) // 4)
     rng = np.random.default_rng(b)
