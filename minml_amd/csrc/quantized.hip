@@ -241,9 +241,14 @@ namespace
 			const uint32_t z = static_cast<uint32_t>(input_zero) & 0xffu;
 			a_loader.fill = z | (z << 8) | (z << 16) | (z << 24);
 			const int tiles_m = ceil_div(M, Cfg::BM), tiles_n = ceil_div(filters_out, Cfg::BN);
-			hipLaunchKernelGGL((kernel_int8_conv_implicit_gemm<Cfg, RequantEpilogue<OutT>>), dim3(static_cast<unsigned int>(tiles_m) * tiles_n),
-					dim3(Cfg::THREADS), 0, stream, a_loader, reinterpret_cast<const int8_t*>(weights), M, filters_out, static_cast<int>(k_bytes), ep,
-					tiles_n);
+			/* with so short a K the epilogue is most of the work: its common cases are fixed at compile time (the stem of the int8 network, 32 -> 256
+			 * channels 3x3, 230400 pixels: 93 -> 72 us) */
+			specialise_epilogue(ep, [&](const auto &fixed)
+			{
+				typedef typename std::decay<decltype(fixed)>::type Fixed;
+				hipLaunchKernelGGL((kernel_int8_conv_implicit_gemm<Cfg, Fixed>), dim3(static_cast<unsigned int>(tiles_m) * tiles_n), dim3(Cfg::THREADS), 0, stream, a_loader,
+						reinterpret_cast<const int8_t*>(weights), M, filters_out, static_cast<int>(k_bytes), fixed, tiles_n);
+			});
 		}
 		else
 		{
