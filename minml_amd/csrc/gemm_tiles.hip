@@ -187,9 +187,9 @@ namespace
 
 		/* lane l, register r of block (i, j): m = 32 i + l % 32, n = 32 j + 16 (l / 32) + r; 32 rows at a time cross the wavefront's slab and
 		 * leave as whole rows of the sub-tile, 16 bytes per lane (N is a multiple of the vector, checked by the launcher) */
-		constexpr int E = 16 / sizeof(T), LANES_PER_ROW = 32 * BLOCKS_N / E, ROWS_PER_PASS = 64 / LANES_PER_ROW;
+		constexpr int E = 16 / sizeof(T), PER_ROW = 32 * BLOCKS_N / E;
+		static_assert(PER_ROW % 2 == 0, "whole passes of 64 lanes over 32 rows");
 		uint8_t *slab = lds + wave * 32 * Shape::SLAB_STRIDE;
-		const int col = (lane % LANES_PER_ROW) * E;
 #pragma unroll
 		for (int i = 0; i < BLOCKS_M; i++)
 		{
@@ -220,9 +220,9 @@ namespace
 			wait_lgkmcnt_zero(); /* the slab is private to this wavefront */
 			__builtin_amdgcn_wave_barrier();
 #pragma unroll
-			for (int pass = 0; pass < 32 / ROWS_PER_PASS; pass++)
+			for (int pass = 0; pass < PER_ROW / 2; pass++)
 			{
-				const int row = pass * ROWS_PER_PASS + lane / LANES_PER_ROW;
+				const int row = (64 * pass + lane) / PER_ROW, col = (64 * pass + lane) % PER_ROW * E;
 				const uint4_t v = *reinterpret_cast<const uint4_t*>(slab + row * Shape::SLAB_STRIDE + col * sizeof(T));
 				const int m = m0 + 32 * i + row;
 				if (m < M && n0 + col < N)
@@ -254,6 +254,12 @@ namespace
 	 * (1152) 19.8 / 19.1; 128 channels 896... 960 rows (1080) 16.1 / 16.0; 384 channels 192 rows (648) 18.9 / 19.4, 256 (864) 21.6 / 20.6. By matrix, 128x64 / 128x128:
 	 * 192 channels 2304 rows 32.8 / 35.5; 256 channels 1616 rows 37.8 / 36.7, 2304 52.2 / 51.2; 384 channels 1408 rows 58.4 / 55.1, 3072 97.5 / 95.6. fp32 stays at
 	 * 64x64: 128 channels 2048 rows 45.6 / 46.0, 256 channels 960 63.0 / 65.5, 640 46.7 / 45.8 (128x64).
+	 * By matrix tiles of 128x192 wherever they pad the columns no more than 64 would: A is fetched once for 192 columns and twice for 384, in place of
+	 * three times by either of the others, and nothing is multiplied for padding as by 128x128 at 192. Whole networks, the tile before / this one, us: 192
+	 * channels, 10 blocks, 1616 rows 640 / 599, 4800 1401 / 1383, with three calls per layer (8 blocks) 1616 564 / 538, 6400 1540 / 1435; 384 channels, 1024 rows
+	 * 856 / 827, 1616 1225 / 1200, 2880 1957 / 1898, with three calls per layer 3248 1734 / 1679. By rows they are level or behind, with too few of
+	 * them for two rounds (8 blocks: 192 channels 768 rows 333.5 / 337.2, 384 channels 256 rows 352.2 / 356.5), and as a dense layer with its epilogue, whose
+	 * side inputs do not fit the registers beside three blocks (192 channels with residual, 184832 rows 57.7 / 67.0, 384 channels 27797 21.1 / 21.9).
 	 */
 	template<typename T>
 	bool try_launch_plain(hipStream_t stream, const StreamGemmArgs &g)
@@ -266,6 +272,8 @@ namespace
 			const long long tiles = static_cast<long long>(ceil_div(g.M, 64)) * ceil_div(g.N, 64) * g.batch;
 			if (tiles >= (g.k_bytes >= 768 ? 3 : 4) * device_compute_units())
 			{
+				if (!by_rows && ceil_div(g.N, 64) % 3 == 0)
+					return launch_as<T, 1, 3, 4, 2>(stream, g, false, PlainStore { });
 				if (!by_rows && g.k_bytes >= 512)
 					return launch_as<T, 2, 1, 2, 4>(stream, g, false, PlainStore { });
 				return launch_as<T, 2, 1, 2, 2>(stream, g, by_rows, PlainStore { });

@@ -4,7 +4,7 @@
  * for the K rows and types that have no kernel of their own (fp32; K rows of any multiple of 64 bytes).
  *
  * A streaming workgroup spends about 10 us on its B operand and its first stages before it multiplies, which a launch of 20 us does not get
- * back, and the tile engine's pipeline is longer than these rows. Here a workgroup owns one tile of 64 or 128 rows and columns and walks
+ * back, and the tile engine's pipeline is longer than these rows. Here a workgroup owns one tile of 64 to 128 rows and 64 to 192 columns and walks
  * K in pieces of 128 bytes through two LDS slots; two to four workgroups share a compute unit and cover one another's round trips, and
  * the grid hands out tiles as they finish. 32x32 MFMA blocks in the order of K of the other engines: bit-identical to them, so that a
  * position's result does not depend on its batch.
@@ -68,7 +68,8 @@ namespace mlhip
 	 * 192 channels, 32 rows (216) 10.7 / 11.6, 64 (432) 13.8 / 12.2.
 	 * Not beyond a number of bytes where the streaming kernel, which fetches A once, or for 64 and 128 bytes the kernels that store more at
 	 * a time are level or ahead: fp16 256-byte rows 57 MB 32.2 / 28.8, 75 35.3 / 33.7, but with three calls per layer 23.6 / 24.0 and 94 MB 28.3 / 29.5; 512: 94 MB 53.3 / 53.3, 113 59.1 / 61.4, 302 127 / 143; 768, of
-	 * which the streaming kernel holds only 128 columns: 226 MB 132 / 120, with three calls per layer 280 MB 150 / 160; fp32 512-byte rows 151 MB 82.4 / 79.9, 227
+	 * which the streaming kernel holds only 128 columns (whole networks of 8 blocks, 384 channels): 239 MB 2352 / 2083, 292 2706 / 2499, but with three
+	 * calls per layer 265 MB 2435 / 2472; fp32 512-byte rows 151 MB 82.4 / 79.9, 227
 	 * 117 / 123; 64-byte rows (the stem, alone) 170 MB 32.4 / 29.3, 340 89.8 / 101; fp32 128-byte rows 85 MB 25.3 / 26.2, 149 31.0 / 33.6, 255 49.1 / 65.0.
 	 */
 	inline bool plain_gemm_tiles_apply(const StreamGemmArgs &g, int element_size)
@@ -100,7 +101,7 @@ namespace mlhip
 				break;
 			case 768:
 				fewest = fp16 ? 3 : 1;
-				megabytes = fp16 ? 220 : megabytes;
+				megabytes = fp16 ? 240 : megabytes;
 				break;
 			default:
 				fewest = (fp16 || g.k_bytes < 384) ? 0 : 1;

@@ -84,9 +84,10 @@ def test_gemm_batched_nt_streaming_other_row_lengths(ctx, dtype, K, shape):
 
 @pytest.mark.parametrize("dtype", ["float32", "float16"])
 @pytest.mark.parametrize("shape", [(36, 1, 8, 32), (36, 65, 72, 96), (36, 191, 40, 160), (36, 192, 136, 32), (8, 257, 264, 224), (7, 700, 392, 384), (36, 300, 384, 384),
-                                   (36, 130, 128, 192), (36, 520, 256, 256), (36, 1300, 264, 256), (36, 1040, 128, 128), (9, 4100, 72, 128)])
+                                   (36, 130, 128, 192), (36, 520, 256, 256), (36, 1300, 264, 256), (36, 1040, 128, 128), (9, 4100, 72, 128),
+                                   (36, 1501, 328, 384), (36, 2300, 192, 192)])
 def test_gemm_batched_nt_tiles(ctx, dtype, shape):
-    """Plain batched products between the direct and the streaming kernel: one row, ragged rows and columns of 64 and 128-wide tiles, K rows
+    """Plain batched products between the direct and the streaming kernel: one row, ragged rows and columns of 64, 128 and 192-wide tiles, K rows
     of whole and half 128-byte pieces, grids by matrix and (at least 8 matrices of 192 rows) by rows."""
     bt, M, N, K = shape
     rng = np.random.default_rng(sum(shape))
@@ -99,9 +100,10 @@ def test_gemm_batched_nt_tiles(ctx, dtype, shape):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "float16"])
-@pytest.mark.parametrize("shape", [(7200, 256, 256), (2701, 776, 96), (14401, 264, 128), (7300, 392, 384), (9000, 200, 192), (2750, 264, 512), (130, 8192, 1024), (14500, 260, 256)])
+@pytest.mark.parametrize("shape", [(7200, 256, 256), (2701, 776, 96), (14401, 264, 128), (7300, 392, 384), (9000, 200, 192), (2750, 264, 512), (130, 8192, 1024), (14500, 260, 256),
+                                   (14401, 192, 192), (7301, 328, 384), (21000, 136, 96)])
 def test_gemm_ex_tiles(ctx, dtype, shape):
-    """Dense layers between few rows and many (tiles of 64x64, 128x64 and 128x128; ragged rows and columns; a width that is no multiple of 16 bytes
+    """Dense layers between few rows and many (tiles of 64x64, 128x64, 128x128 and 128x192; ragged rows and columns; a width that is no multiple of 16 bytes
     in fp16, which goes on to the other kernels), with bias, ReLU or linear, with and without a residual; a prefix of the rows, which takes
     another kernel, gives the same bits."""
     M, N, K = shape
