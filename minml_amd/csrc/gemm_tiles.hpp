@@ -38,6 +38,16 @@ namespace mlhip
 		return static_cast<unsigned long long>(g.batch) * g.M * (static_cast<unsigned long long>(g.k_bytes) + static_cast<unsigned long long>(g.N) * element_size);
 	}
 	/*
+	 * Whether the transforms before and after a batch may divide its rows among the XCDs: the 36 matrices of their 6x6 tiles. Any other batch gains nothing
+	 * from the order by rows and pays for it, each XCD fetching all of B; and so do 36 matrices with many more columns than rows. Alone, fp16, us by
+	 * matrix / by rows: 16 x 512 x 2048, 128-byte K rows (streaming kernel) 11.5 / 16.6, 64 x 192 x 1024 9.8 / 13.5; 64 x 192 x 1024, 256 bytes 13.4 / 14.6, 512
+	 * 16.6 / 20.9; 16 x 1024 x 1024, 512 bytes 17.0 / 20.9; 36 x 192 x 1024, 384 bytes 10.8 / 11.5.
+	 */
+	inline bool between_transforms(const StreamGemmArgs &g)
+	{
+		return g.batch == 36 && g.N <= 2LL * g.M;
+	}
+	/*
 	 * By rows (header) while A and C fit the L2s of the XCDs and there are enough rows to divide among them. us per product + transform, 64x64
 	 * tiles by matrix / by rows: fp16 256 channels 128 rows 11.0 / 11.0, 192 12.9 / 12.8, 256 15.5 / 15.2, 384 19.5 / 18.0; 128 channels 256 rows 10.1 / 9.8, 1024
 	 * 21.0 / 15.5, 2048 (38 MB) 23.2 / 22.0; tiles of 128x64: 256 channels 960 rows (35 MB) 27.9 / 27.1, 1152 (42 MB) 31.8 / 31.7, 1408 35.5 / 35.0, 2304 52.2 / 51.8;
@@ -46,7 +56,7 @@ namespace mlhip
 	 */
 	inline bool products_meet_in_l2(const StreamGemmArgs &g, int element_size)
 	{
-		return g.batch >= 8 && g.M >= 192 && exchanged_bytes(g, element_size) <= (40ULL << 20);
+		return between_transforms(g) && g.M >= 192 && exchanged_bytes(g, element_size) <= (40ULL << 20);
 	}
 	/*
 	 * And beyond where all of B takes a small part of each L2, while the transforms divide the images like that (matrices_stay_cached in
@@ -57,7 +67,7 @@ namespace mlhip
 	{
 		const unsigned long long b_bytes = static_cast<unsigned long long>(g.batch) * g.N * g.k_bytes;
 		return products_meet_in_l2(g, element_size)
-				|| (g.batch >= 8 && g.M >= 8 * static_cast<long long>(g.N) && 2 * b_bytes <= (5ULL << 20) && exchanged_bytes(g, element_size) <= (112ULL << 20));
+				|| (between_transforms(g) && g.M >= 8 * static_cast<long long>(g.N) && 2 * b_bytes <= (5ULL << 20) && exchanged_bytes(g, element_size) <= (112ULL << 20));
 	}
 	/*
 	 * Whether these tiles take a batch of plain products, by the number of 32x32 tiles and the bytes of A and C (figures as above, other

@@ -1,0 +1,25 @@
+/*
+ * Prints what the dispatch rules of the products decide on a card of 256 compute units, without a device: one line per line of the input,
+ *   plain <element size> <matrices> <rows> <columns> <bytes of a K row>      "<tiles 0|1> <by rows 0|1> <direct kernel 0|1>"
+ */
+#include "gemm_direct.hpp"
+
+#include <cstdio>
+
+namespace mlhip
+{
+	int device_compute_units()
+	{
+		return 256;
+	}
+}
+
+int main()
+{
+	char kind[16];
+	int element_size;
+	mlhip::StreamGemmArgs g { };
+	while (std::scanf("%15s %d %d %d %d %d", kind, &element_size, &g.batch, &g.M, &g.N, &g.k_bytes) == 6)
+		std::printf("%d %d %d\n", mlhip::plain_gemm_tiles_apply(g, element_size), mlhip::products_go_by_rows(g, element_size), element_size == 2 && mlhip::gemm_direct_applies(g));
+	return 0;
+}

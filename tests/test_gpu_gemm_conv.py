@@ -88,7 +88,7 @@ def test_gemm_batched_nt_streaming_other_row_lengths(ctx, dtype, K, shape):
                                    (36, 1501, 328, 384), (36, 2300, 192, 192)])
 def test_gemm_batched_nt_tiles(ctx, dtype, shape):
     """Plain batched products between the direct and the streaming kernel: one row, ragged rows and columns of 64, 128 and 192-wide tiles, K rows
-    of whole and half 128-byte pieces, grids by matrix and (at least 8 matrices of 192 rows) by rows."""
+    of whole and half 128-byte pieces, grids by matrix and (36 matrices of 192 rows and more) by rows."""
     bt, M, N, K = shape
     rng = np.random.default_rng(sum(shape))
     A = random_tensor(rng, (bt, M, K), dtype, 0.5)

@@ -1,0 +1,41 @@
+"""No-GPU checks of the rules that choose a kernel for a product (csrc/gemm_tiles.hpp, csrc/gemm_direct.hpp): compiled for the host alone and asked
+for the sides of their lines that measurements stand beside."""
+import os
+import subprocess
+
+import pytest
+
+from minml_amd.build import CSRC, hipcc
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+SIZE = {"float16": 2, "float32": 4}
+
+
+@pytest.fixture(scope="module")
+def decide(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("routes") / "product_routes")
+    subprocess.run([hipcc(), "--offload-arch=gfx950", "--cuda-host-only", "-std=c++17", "-O0", "-I" + CSRC, "-x", "hip", os.path.join(HERE, "product_routes.cpp"),
+                    "-o", exe], check=True, capture_output=True)
+
+    def ask(kind, dtype, matrices, rows, columns, K):
+        line = "%s %d %d %d %d %d\n" % (kind, SIZE[dtype], matrices, rows, columns, K * SIZE[dtype])
+        return subprocess.run([exe], input=line, check=True, capture_output=True, text=True).stdout.split()
+
+    return ask
+
+
+@pytest.mark.parametrize("dtype,matrices,rows,columns,K,by_rows", [
+    # the 36 products between two transforms, which divide the images in the same way
+    ("float16", 36, 192, 256, 256, True), ("float16", 36, 1024, 64, 64, True), ("float32", 36, 512, 128, 128, True), ("float16", 36, 640, 384, 384, True),
+    ("float16", 36, 191, 256, 256, False), ("float16", 36, 2304, 384, 384, False),
+    # any other batch has no such neighbours, and more columns than rows make every XCD fetch more of B than it saves of A and C
+    ("float16", 16, 512, 2048, 64, False), ("float16", 64, 192, 1024, 64, False), ("float16", 64, 192, 1024, 128, False), ("float16", 8, 1024, 1024, 256, False),
+    ("float16", 36, 192, 1024, 192, False), ("float32", 16, 1024, 256, 64, False)])
+def test_order_of_batched_products(decide, dtype, matrices, rows, columns, K, by_rows):
+    assert decide("plain", dtype, matrices, rows, columns, K)[1] == str(int(by_rows))
+
+
+def test_direct_kernel_takes_more_tiles_only_in_the_order_by_rows(decide):
+    assert decide("plain", "float16", 36, 2048, 64, 64)[2] == "1"
+    assert decide("plain", "float16", 16, 512, 2048, 64)[2] == "0"
+    assert decide("plain", "float16", 64, 192, 256, 64)[2] == "1"
