@@ -249,18 +249,6 @@ namespace
 				g.a_row_bytes != 0 ? g.a_row_bytes : static_cast<size_t>(g.k_bytes), epilogue);
 		return true;
 	}
-	/*
-	 * Larger tiles, which fetch less, once there are enough of them. fp16 by rows, 64x64 / 128x64: 256 channels 448 rows (1008 tiles of 64x64) 18.6 / 19.2, 512
-	 * (1152) 19.8 / 19.1; 128 channels 896... 960 rows (1080) 16.1 / 16.0; 384 channels 192 rows (648) 18.9 / 19.4, 256 (864) 21.6 / 20.6. By matrix, 128x64 / 128x128:
-	 * 192 channels 2304 rows 32.8 / 35.5; 256 channels 1616 rows 37.8 / 36.7, 2304 52.2 / 51.2; 384 channels 1408 rows 58.4 / 55.1, 3072 97.5 / 95.6. fp32 stays at
-	 * 64x64: 128 channels 2048 rows 45.6 / 46.0, 256 channels 960 63.0 / 65.5, 640 46.7 / 45.8 (128x64).
-	 * By matrix tiles of 128x192 wherever they pad the columns no more than 64 would: A is fetched once for 192 columns and twice for 384, in place of
-	 * three times by either of the others, and nothing is multiplied for padding as by 128x128 at 192. Whole networks, the tile before / this one, us: 192
-	 * channels, 10 blocks, 1616 rows 640 / 599, 4800 1401 / 1383, with three calls per layer (8 blocks) 1616 564 / 538, 6400 1540 / 1435; 384 channels, 1024 rows
-	 * 856 / 827, 1616 1225 / 1200, 2880 1957 / 1898, with three calls per layer 3248 1734 / 1679. By rows they are level or behind, with too few of
-	 * them for two rounds (8 blocks: 192 channels 768 rows 333.5 / 337.2, 384 channels 256 rows 352.2 / 356.5), and as a dense layer with its epilogue, whose
-	 * side inputs do not fit the registers beside three blocks (192 channels with residual, 184832 rows 57.7 / 67.0, 384 channels 27797 21.1 / 21.9).
-	 */
 	template<typename T>
 	bool try_launch_plain(hipStream_t stream, const StreamGemmArgs &g)
 	{
@@ -268,33 +256,33 @@ namespace
 			return false;
 		const bool by_rows = products_go_by_rows(g, sizeof(T));
 		if constexpr (sizeof(T) == 2)
-		{
-			const long long tiles = static_cast<long long>(ceil_div(g.M, 64)) * ceil_div(g.N, 64) * g.batch;
-			if (tiles >= (g.k_bytes >= 768 ? 3 : 4) * device_compute_units())
+			switch (tile_of_plain(g, sizeof(T)))
 			{
-				if (!by_rows && ceil_div(g.N, 64) % 3 == 0)
-					return launch_as<T, 1, 3, 4, 2>(stream, g, false, PlainStore { });
-				if (!by_rows && g.k_bytes >= 512)
-					return launch_as<T, 2, 1, 2, 4>(stream, g, false, PlainStore { });
-				return launch_as<T, 2, 1, 2, 2>(stream, g, by_rows, PlainStore { });
+				case GemmTile::T128x192:
+					return launch_as<T, 1, 3, 4, 2>(stream, g, by_rows, PlainStore { });
+				case GemmTile::T128x128:
+					return launch_as<T, 2, 1, 2, 4>(stream, g, by_rows, PlainStore { });
+				case GemmTile::T128x64:
+					return launch_as<T, 2, 1, 2, 2>(stream, g, by_rows, PlainStore { });
+				default:
+					break;
 			}
-		}
 		return launch_as<T, 1, 1, 2, 2>(stream, g, by_rows, PlainStore { });
 	}
 
-	/*
-	 * fp16: 128x128 tiles from 3.5 of 64x64 per unit on (256 x 256, 14400 rows (900): 8.0 / 7.3 us; 384 x 256, 7200 rows (452) 6.5 / 7.7, 14400 9.7 / 8.7), 128x64
-	 * where 128 pads the columns more (192 x 192, 57600 rows 15.3 / 14.1).
-	 */
 	template<typename T, typename Epilogue>
 	bool launch_fixed(hipStream_t stream, const StreamGemmArgs &g, const Epilogue &epilogue)
 	{
 		if constexpr (sizeof(T) == 2)
-		{
-			const long long tiles = static_cast<long long>(ceil_div(g.M, 64)) * ceil_div(g.N, 64) * g.batch;
-			if (g.k_bytes <= 1024 && 2 * tiles >= 7 * device_compute_units())
-				return (ceil_div(g.N, 64) % 2 != 0) ? launch_as<T, 2, 1, 2, 2>(stream, g, false, epilogue) : launch_as<T, 2, 1, 2, 4>(stream, g, false, epilogue);
-		}
+			switch (tile_with_epilogue(g, sizeof(T)))
+			{
+				case GemmTile::T128x128:
+					return launch_as<T, 2, 1, 2, 4>(stream, g, false, epilogue);
+				case GemmTile::T128x64:
+					return launch_as<T, 2, 1, 2, 2>(stream, g, false, epilogue);
+				default:
+					break;
+			}
 		return launch_as<T, 1, 1, 2, 2>(stream, g, false, epilogue);
 	}
 	template<typename T>

@@ -150,6 +150,54 @@ namespace mlhip
 		const unsigned long long bytes = exchanged_bytes(g, element_size) + (reads_c ? static_cast<unsigned long long>(g.batch) * g.M * g.N * element_size : 0);
 		return 4 * tiles >= (g.k_bytes <= 512 ? 7 : g.k_bytes <= 768 ? 4 : 2) * units && !(streams && bytes > ((g.N > 128 ? 96ULL : 180ULL) << 20));
 	}
+	/* rows x columns of the tile that a workgroup owns */
+	enum class GemmTile
+	{
+		T64x64, T128x64, T128x128, T128x192
+	};
+	/*
+	 * Whether 128 rows to a tile pad at most a quarter more than 64 do. Short matrices of a batch, or a few rows and many columns, would be multiplied twice:
+	 * fp16, us, 64x64 / 128x64 / 128x128: 64 x 16 x 1024, 256-byte K rows 5.1 / 6.6 / 5.8; 48 x 22 x 2000, 384 bytes 9.5 / 10.7 / 10.6 (direct kernel
+	 * 8.9); 64 x 64 x 1024 7.1 / 9.2 / 8.1 (7.7); 32 x 190 x 2048, 256 bytes 11.9 / 13.3 / 11.8 (12.8); 64 x 70 x 1024, 512 bytes, which both pad to
+	 * 128, 11.5 / 10.9 / 9.9; one of 40 x 60000 with ReLU, 384 bytes 6.7 / 9.4 / 7.9 (6.6).
+	 */
+	inline bool fills_128_rows(const StreamGemmArgs &g)
+	{
+		return 8LL * ceil_div(g.M, 128) <= 5LL * ceil_div(g.M, 64);
+	}
+	/*
+	 * Plain products: larger tiles, which fetch less, once there are enough of them and M fills them. fp16 by rows, 64x64 / 128x64: 256 channels 448 rows (1008 tiles of 64x64) 18.6 / 19.2, 512
+	 * (1152) 19.8 / 19.1; 128 channels 896... 960 rows (1080) 16.1 / 16.0; 384 channels 192 rows (648) 18.9 / 19.4, 256 (864) 21.6 / 20.6. By matrix, 128x64 / 128x128:
+	 * 192 channels 2304 rows 32.8 / 35.5; 256 channels 1616 rows 37.8 / 36.7, 2304 52.2 / 51.2; 384 channels 1408 rows 58.4 / 55.1, 3072 97.5 / 95.6. fp32 stays at
+	 * 64x64: 128 channels 2048 rows 45.6 / 46.0, 256 channels 960 63.0 / 65.5, 640 46.7 / 45.8 (128x64).
+	 * By matrix tiles of 128x192 wherever they pad the columns no more than 64 would: A is fetched once for 192 columns and twice for 384, in place of
+	 * three times by either of the others, and nothing is multiplied for padding as by 128x128 at 192. Whole networks, the tile before / this one, us: 192
+	 * channels, 10 blocks, 1616 rows 640 / 599, 4800 1401 / 1383, with three calls per layer (8 blocks) 1616 564 / 538, 6400 1540 / 1435; 384 channels, 1024 rows
+	 * 856 / 827, 1616 1225 / 1200, 2880 1957 / 1898, with three calls per layer 3248 1734 / 1679. By rows they are level or behind, with too few of
+	 * them for two rounds (8 blocks: 192 channels 768 rows 333.5 / 337.2, 384 channels 256 rows 352.2 / 356.5), and as a dense layer with its epilogue, whose
+	 * side inputs do not fit the registers beside three blocks (192 channels with residual, 184832 rows 57.7 / 67.0, 384 channels 27797 21.1 / 21.9).
+	 */
+	inline GemmTile tile_of_plain(const StreamGemmArgs &g, int element_size)
+	{
+		const long long tiles = static_cast<long long>(ceil_div(g.M, 64)) * ceil_div(g.N, 64) * g.batch;
+		if (element_size != 2 || tiles < (g.k_bytes >= 768 ? 3 : 4) * device_compute_units() || !fills_128_rows(g))
+			return GemmTile::T64x64;
+		const bool by_rows = products_go_by_rows(g, element_size);
+		if (!by_rows && ceil_div(g.N, 64) % 3 == 0)
+			return GemmTile::T128x192;
+		return (!by_rows && g.k_bytes >= 512) ? GemmTile::T128x128 : GemmTile::T128x64;
+	}
+	/*
+	 * With the epilogue, fp16: 128x128 tiles from 3.5 of 64x64 per unit on (256 x 256, 14400 rows (900): 8.0 / 7.3 us; 384 x 256, 7200 rows (452) 6.5 / 7.7, 14400 9.7 / 8.7), 128x64
+	 * where 128 pads the columns more (192 x 192, 57600 rows 15.3 / 14.1).
+	 */
+	inline GemmTile tile_with_epilogue(const StreamGemmArgs &g, int element_size)
+	{
+		const long long tiles = static_cast<long long>(ceil_div(g.M, 64)) * ceil_div(g.N, 64) * g.batch;
+		if (element_size != 2 || g.k_bytes > 1024 || 2 * tiles < 7 * device_compute_units() || !fills_128_rows(g))
+			return GemmTile::T64x64;
+		return (ceil_div(g.N, 64) % 2 != 0) ? GemmTile::T128x64 : GemmTile::T128x128;
+	}
 	/* false: nothing was launched. Plain batched products of fp16 or fp32; and products with bias (+ beta * C), linear or ReLU */
 	bool try_launch_gemm_tiles(hipStream_t stream, mlDataType_t dtype, const StreamGemmArgs &g);
 	bool try_launch_gemm_tiles(hipStream_t stream, const StreamGemmArgs &g, const FloatEpilogue<half_t> &epilogue);

@@ -1,10 +1,12 @@
 /*
  * Prints what the dispatch rules of the products decide on a card of 256 compute units, without a device: one line per line of the input,
- *   plain <element size> <matrices> <rows> <columns> <bytes of a K row>      "<tiles 0|1> <by rows 0|1> <direct kernel 0|1>"
+ *   plain <element size> <matrices> <rows> <columns> <bytes of a K row>      "<tiles 0|1> <by rows 0|1> <direct kernel 0|1> <tile>"
+ *   dense ...                                                                "<tiles 0|1> 0 <direct kernel 0|1> <tile>"   (bias, no C)
  */
 #include "gemm_direct.hpp"
 
 #include <cstdio>
+#include <cstring>
 
 namespace mlhip
 {
@@ -20,6 +22,12 @@ int main()
 	int element_size;
 	mlhip::StreamGemmArgs g { };
 	while (std::scanf("%15s %d %d %d %d %d", kind, &element_size, &g.batch, &g.M, &g.N, &g.k_bytes) == 6)
-		std::printf("%d %d %d\n", mlhip::plain_gemm_tiles_apply(g, element_size), mlhip::products_go_by_rows(g, element_size), element_size == 2 && mlhip::gemm_direct_applies(g));
+	{
+		const bool plain = std::strcmp(kind, "plain") == 0;
+		const mlhip::GemmTile tile = plain ? mlhip::tile_of_plain(g, element_size) : mlhip::tile_with_epilogue(g, element_size);
+		const char *names[] = { "64x64", "128x64", "128x128", "128x192" };
+		std::printf("%d %d %d %s\n", plain ? mlhip::plain_gemm_tiles_apply(g, element_size) : mlhip::gemm_tiles_apply(g, element_size, false),
+				plain && mlhip::products_go_by_rows(g, element_size), element_size == 2 && mlhip::gemm_direct_applies(g), names[static_cast<int>(tile)]);
+	}
 	return 0;
 }

@@ -39,3 +39,12 @@ def test_direct_kernel_takes_more_tiles_only_in_the_order_by_rows(decide):
     assert decide("plain", "float16", 36, 2048, 64, 64)[2] == "1"
     assert decide("plain", "float16", 16, 512, 2048, 64)[2] == "0"
     assert decide("plain", "float16", 64, 192, 256, 64)[2] == "1"
+
+
+@pytest.mark.parametrize("kind,matrices,rows,columns,K,tile", [
+    ("plain", 64, 64, 1024, 192, "64x64"), ("plain", 48, 22, 2000, 192, "64x64"), ("plain", 32, 190, 2048, 128, "64x64"), ("dense", 1, 40, 60000, 192, "64x64"),
+    ("dense", 64, 40, 1024, 512, "64x64"), ("plain", 64, 70, 1024, 192, "128x64"), ("plain", 64, 70, 1024, 256, "128x128"), ("plain", 64, 300, 384, 384, "128x192"),
+    ("plain", 36, 2304, 256, 256, "128x128"), ("plain", 36, 500, 256, 256, "128x64"), ("dense", 1, 14400, 256, 256, "128x128"), ("dense", 1, 57600, 192, 192, "128x64")])
+def test_tiles_of_128_rows_where_the_matrix_fills_them(decide, kind, matrices, rows, columns, K, tile):
+    taken, _, _, chosen = decide(kind, "float16", matrices, rows, columns, K)
+    assert (taken, chosen) == ("1", tile)
