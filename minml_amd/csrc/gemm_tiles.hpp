@@ -75,7 +75,10 @@ namespace mlhip
 	 * Not where the direct kernel's 32x32 tiles are few enough to be ahead: 256-byte rows, 128 channels, 448 rows (2016 tiles) 13.0 / 14.1 us, 512 (2304) 12.9 /
 	 * 12.1; 512: 256 channels, 96 rows (864) 10.4 / 10.7, 128 (1152) 11.3 / 11.0; 384: 192 channels, 96 rows (648) 9.0 / 9.4, 160 (1080) 10.6 / 10.5; 768: 384
 	 * channels, 32 rows (432) 10.5 / 11.2, 64 (864) 13.0 / 12.2; and fp32 rows of 384 bytes and more but 512, for which the small tiles of conv_tiles.hpp stand:
-	 * 192 channels, 32 rows (216) 10.7 / 11.6, 64 (432) 13.8 / 12.2.
+	 * 192 channels, 32 rows (216) 10.7 / 11.6, 64 (432) 13.8 / 12.2. From 1024 bytes on they stand to two per unit, the most that conv_tiles.hpp gives them, and
+	 * the more K the further they are ahead (alone): 36 x 16 x 256 (288) 8.0 / 8.6, 36 x 16 x 384, 1536 bytes (432) 10.9 / 12.0, 9 x 776 x 56, 2048 bytes
+	 * (450) 13.5 / 14.8, 8 x 64 x 512, 4096 bytes (256) 17.0 / 25.2, 8192 (256) 30.1 / 46.4, 8 x 128 x 512 (512) 41.9 / 46.8, 16384 78.3 / 89.6; above, 36 x 64 x 256 (576, in a
+	 * network) 18.5 / 14.9.
 	 * Not beyond a number of bytes where the streaming kernel, which fetches A once, or for 64 and 128 bytes the kernels that store more at
 	 * a time are level or ahead: fp16 256-byte rows 57 MB 32.2 / 28.8, 75 35.3 / 33.7, but with three calls per layer 23.6 / 24.0 and 94 MB 28.3 / 29.5; 512: 94 MB 53.3 / 53.3, 113 59.1 / 61.4, 302 127 / 143; 768, of
 	 * which the streaming kernel holds only 128 columns (whole networks of 8 blocks, 384 channels): 239 MB 2352 / 2083, 292 2706 / 2499, but with three
@@ -117,6 +120,8 @@ namespace mlhip
 				fewest = (fp16 || g.k_bytes < 384) ? 0 : 1;
 				break;
 		}
+		if (!fp16 && g.k_bytes >= 1024 && tiles <= 2LL * device_compute_units())
+			return false;
 		return tiles >= fewest * device_compute_units() && exchanged_bytes(g, element_size) <= (megabytes << 20);
 	}
 	/*
