@@ -83,7 +83,10 @@ namespace mlhip
 	 * a time are level or ahead: fp16 256-byte rows 57 MB 32.2 / 28.8, 75 35.3 / 33.7, but with three calls per layer 23.6 / 24.0 and 94 MB 28.3 / 29.5; 512: 94 MB 53.3 / 53.3, 113 59.1 / 61.4, 302 127 / 143; 768, of
 	 * which the streaming kernel holds only 128 columns (whole networks of 8 blocks, 384 channels): 239 MB 2352 / 2083, 292 2706 / 2499, but with three
 	 * calls per layer 265 MB 2435 / 2472; fp32 512-byte rows 151 MB 82.4 / 79.9, 227
-	 * 117 / 123; 64-byte rows (the stem, alone) 170 MB 32.4 / 29.3, 340 89.8 / 101; fp32 128-byte rows 85 MB 25.3 / 26.2, 149 31.0 / 33.6, 255 49.1 / 65.0.
+	 * 117 / 123; 64-byte rows (the stem, alone) 170 MB 32.4 / 29.3, 340 89.8 / 101; fp32 128-byte rows, the stem, with the
+	 * input from memory 24 MB 11.9 / 10.1, 47 16.6 / 16.4, 57 16.6 / 17.7, 85 23.3 / 27.6, 94 23.3 / 27.6; whole networks of one block 128 channels 9 MB 67.2 / 63.9, 38
+	 * 125.3 / 125.3, 47 144.9 / 144.5, 66 184.3 / 185.4, 94 241.3 / 245.6, 256 channels 42 MB 195.3 / 194.6, 67 276.8 / 280.6, 64 channels, for
+	 * which A is fetched once, 57 MB 124.8 / 123.6, 111 200.3 / 204.6.
 	 */
 	inline bool plain_gemm_tiles_apply(const StreamGemmArgs &g, int element_size)
 	{
@@ -99,7 +102,7 @@ namespace mlhip
 				megabytes = 270;
 				break;
 			case 128:
-				megabytes = 100;
+				megabytes = (g.N <= 64) ? 60 : 48;
 				break;
 			case 256:
 				fewest = fp16 ? 8 : 0;
