@@ -82,7 +82,10 @@ namespace mlhip
 	 * Not beyond a number of bytes where the streaming kernel, which fetches A once, or for 64 and 128 bytes the kernels that store more at
 	 * a time are level or ahead: fp16 256-byte rows 57 MB 32.2 / 28.8, 75 35.3 / 33.7, but with three calls per layer 23.6 / 24.0 and 94 MB 28.3 / 29.5; 512: 94 MB 53.3 / 53.3, 113 59.1 / 61.4, 302 127 / 143; 768, of
 	 * which the streaming kernel holds only 128 columns (whole networks of 8 blocks, 384 channels): 239 MB 2352 / 2083, 292 2706 / 2499, but with three
-	 * calls per layer 265 MB 2435 / 2472; fp32 512-byte rows 151 MB 82.4 / 79.9, 227
+	 * calls per layer 265 MB 2435 / 2472, where three or five column tiles leave its slices of 128 columns padded or some compute units idle; other widths, alone
+	 * (12 and 36 matrices, this one's time over the other's): 256 columns 150 MB 0.96, 200 1.05, 245 1.16, 512 150 0.96, 200 0.99, 245 1.13, 1024 90 0.85, 120 0.95, 200 1.04, 245 1.20 (64 matrices 108 1.06),
+	 * 2048 150 1.03, 245 1.18; 320 245 0.88, 640 0.90); fp32 256-byte rows, where those slices are not padded by more than an eighth: 128 columns 250 MB 0.94, 300 1.00,
+	 * 450 1.06, 256 columns 250 0.98, 300 1.08, 450 1.13, 512 250 1.03, 300 1.09, 600 1.18 (64 columns 600 MB 0.92, 192 0.88); fp32 512-byte rows 151 MB 82.4 / 79.9, 227
 	 * 117 / 123; 64-byte rows (the stem, alone) 170 MB 32.4 / 29.3, 340 89.8 / 101; fp32 128-byte rows, the stem, with the
 	 * input from memory 24 MB 11.9 / 10.1, 47 16.6 / 16.4, 57 16.6 / 17.7, 85 23.3 / 27.6, 94 23.3 / 27.6; whole networks of one block 128 channels 9 MB 67.2 / 63.9, 38
 	 * 125.3 / 125.3, 47 144.9 / 144.5, 66 184.3 / 185.4, 94 241.3 / 245.6, 256 channels 42 MB 195.3 / 194.6, 67 276.8 / 280.6, 64 channels, for
@@ -106,7 +109,10 @@ namespace mlhip
 				break;
 			case 256:
 				fewest = fp16 ? 8 : 0;
-				megabytes = fp16 ? 64 : megabytes;
+				if (fp16)
+					megabytes = 64;
+				else if (g.N > 64 && 8 * (ceil_div(g.N, 128) * 128LL - g.N) <= g.N)
+					megabytes = 256;
 				break;
 			case 384:
 				fewest = fp16 ? 4 : 1;
@@ -117,7 +123,8 @@ namespace mlhip
 				break;
 			case 768:
 				fewest = fp16 ? 3 : 1;
-				megabytes = fp16 ? 240 : megabytes;
+				if (fp16)
+					megabytes = (ceil_div(g.N, 64) % 3 == 0 || ceil_div(g.N, 64) % 5 == 0) && g.N <= 1024 ? 240 : g.N <= 512 ? 160 : 100;
 				break;
 			default:
 				fewest = (fp16 || g.k_bytes < 384) ? 0 : 1;
