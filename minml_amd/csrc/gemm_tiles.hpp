@@ -43,9 +43,10 @@ namespace mlhip
 	 * matrix / by rows: 16 x 512 x 2048, 128-byte K rows (streaming kernel) 11.5 / 16.6, 64 x 192 x 1024 9.8 / 13.5; 64 x 192 x 1024, 256 bytes 13.4 / 14.6, 512
 	 * 16.6 / 20.9; 16 x 1024 x 1024, 512 bytes 17.0 / 20.9; 36 x 192 x 1024, 384 bytes 10.8 / 11.5.
 	 */
+	constexpr int TRANSFORM_MATRICES = 36;
 	inline bool between_transforms(const StreamGemmArgs &g)
 	{
-		return g.batch == 36 && g.N <= 2LL * g.M;
+		return g.batch == TRANSFORM_MATRICES && g.N <= 2LL * g.M;
 	}
 	/*
 	 * By rows (header) while A and C fit the L2s of the XCDs and there are enough rows to divide among them. us per product + transform, 64x64
@@ -74,7 +75,9 @@ namespace mlhip
 	 * kernel / this one).
 	 * Not where the direct kernel's 32x32 tiles are few enough to be ahead: 256-byte rows, 128 channels, 448 rows (2016 tiles) 13.0 / 14.1 us, 512 (2304) 12.9 /
 	 * 12.1; 512: 256 channels, 96 rows (864) 10.4 / 10.7, 128 (1152) 11.3 / 11.0; 384: 192 channels, 96 rows (648) 9.0 / 9.4, 160 (1080) 10.6 / 10.5; 768: 384
-	 * channels, 32 rows (432) 10.5 / 11.2, 64 (864) 13.0 / 12.2; and fp32 rows of 384 bytes and more but 512, for which the small tiles of conv_tiles.hpp stand:
+	 * channels, 32 rows (432) 10.5 / 11.2, 64 (864) 13.0 / 12.2. Other batches than the 36 of a network gain nothing around the product (alone): 512 bytes,
+	 * 8 x 400 x 400 (1352) 4.5 / 5.0, 100 x 128 x 128 (1600) 4.8 / 5.1, 16 x 400 x 400 (2704) 6.6 / 6.6, 24 x 512 x 256 (3072) 6.8 / 6.2; 768, 16 x 192 x 256 (768) 4.7 / 5.2,
+	 * 64 x 128 x 128 (1024) 5.5 / 5.0. And fp32 rows of 384 bytes and more but 512, for which the small tiles of conv_tiles.hpp stand:
 	 * 192 channels, 32 rows (216) 10.7 / 11.6, 64 (432) 13.8 / 12.2. From 1024 bytes on they stand to two per unit, the most that conv_tiles.hpp gives them, and
 	 * the more K the further they are ahead (alone): 36 x 16 x 256 (288) 8.0 / 8.6, 36 x 16 x 384, 1536 bytes (432) 10.9 / 12.0, 9 x 776 x 56, 2048 bytes
 	 * (450) 13.5 / 14.8, 8 x 64 x 512, 4096 bytes (256) 17.0 / 25.2, 8192 (256) 30.1 / 46.4, 8 x 128 x 512 (512) 41.9 / 46.8, 16384 78.3 / 89.6; above, 36 x 64 x 256 (576, in a
@@ -118,11 +121,11 @@ namespace mlhip
 				fewest = fp16 ? 4 : 1;
 				break;
 			case 512:
-				fewest = fp16 ? 4 : 0;
+				fewest = fp16 ? (g.batch == TRANSFORM_MATRICES ? 4 : 8) : 0;
 				megabytes = fp16 ? 90 : 200;
 				break;
 			case 768:
-				fewest = fp16 ? 3 : 1;
+				fewest = fp16 ? (g.batch == TRANSFORM_MATRICES ? 3 : 4) : 1;
 				if (fp16)
 					megabytes = (ceil_div(g.N, 64) % 3 == 0 || ceil_div(g.N, 64) % 5 == 0) && g.N <= 1024 ? 240 : g.N <= 512 ? 160 : 100;
 				break;
