@@ -144,6 +144,9 @@ namespace mlhip
 	 *   (516) 5.9 / 5.2), 1 up to 768 bytes (384 x 256: 7200 (452) 11.0 / 6.5; x 384: 2700 (258) 6.2 / 6.0), 0.5 up to 1024 (512 x 256: 2700 (172) 7.0 / 6.0). Rows of
 	 *   2048 bytes, for which a tile of 256 rows is the better one where there are enough, from 1 to 4 (eight experts of 1024 x 256: 912 rows
 	 *   (480) 13.4 / 10.6, 3648 (1824) 25.4 / 30.7); 1024 with a batch to 8 (512 x 1024: 912 rows (1920) 18.5 / 15.9, 3648 (7296) 43.5 / 46.4).
+	 *   Half a tile of padding is not for them: at most 32 columns where the streaming or direct kernel take the rows, from 3.5 tiles per unit (28800 x 32: 256-byte
+	 *   rows (450) 3.9 / 4.4, 512 4.7 / 5.1, 768 5.5 / 5.9; 57600 (900) 5.2 / 5.3, 7.4 / 7.3, 14.1 / 11.0); 384 bytes, whose direct kernel has no upper limit,
+	 *   from 64 columns (114119 x 32 10.8 / 11.9, 230400 x 24 17.3 / 18.9, 57600 x 40 from memory 8.6 / 9.2).
 	 *   Not beyond 96 MB of A, C and what is read of it where the streaming kernel takes the rows (256 x 256: 57600 rows, 88 MB with residual, 26.4 / 23.8,
 	 *   115200 (177) 41.7 / 41.7, 230400 81.5 / 105; 256 x 1024: 27797 (71) 28.7 / 28.1, 57600 (147) 48.8 / 55.1; 384 x 384 with residual: 27797 (64) 25.2 / 22.2, 57600
 	 *   (133) 39.7 / 40.1; eight experts of 256 x 1024: 3648 rows (75) 36.7 / 29.4, 7296 (149) 57.1 / 55.4, 14592 89 / 127), 180 with one column tile
@@ -166,6 +169,8 @@ namespace mlhip
 			return false;
 		const bool streams = g.k_bytes == 256 || g.k_bytes == 512 || g.k_bytes == 768;
 		const unsigned long long bytes = exchanged_bytes(g, element_size) + (reads_c ? static_cast<unsigned long long>(g.batch) * g.M * g.N * element_size : 0);
+		if ((g.k_bytes == 384 && g.N < 64) || (streams && g.N <= 32 && 2 * tiles < 7 * units))
+			return false;
 		return 4 * tiles >= (g.k_bytes <= 512 ? 7 : g.k_bytes <= 768 ? 4 : 2) * units && !(streams && bytes > ((g.N > 128 ? 96ULL : 180ULL) << 20));
 	}
 	/* rows x columns of the tile that a workgroup owns */

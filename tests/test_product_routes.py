@@ -65,3 +65,11 @@ def test_tiles_of_128_rows_where_the_matrix_fills_them(decide, kind, matrices, r
     ("float16", 16, 192, 256, 384, False), ("float16", 64, 128, 128, 384, True)])
 def test_plain_batches_on_the_tiles(decide, dtype, matrices, rows, columns, K, taken):
     assert decide("plain", dtype, matrices, rows, columns, K)[0] == str(int(taken))
+
+
+@pytest.mark.parametrize("dtype,matrices,rows,columns,K,taken", [
+    # few columns: half of a tile would be padding
+    ("float16", 1, 28800, 32, 256, False), ("float16", 1, 57600, 32, 256, True), ("float16", 1, 114119, 32, 192, False), ("float16", 1, 57600, 40, 192, False),
+    ("float16", 1, 114119, 64, 192, True), ("float16", 1, 28800, 32, 96, True), ("float16", 1, 28800, 40, 256, True)])
+def test_dense_layers_on_the_tiles(decide, dtype, matrices, rows, columns, K, taken):
+    assert decide("dense", dtype, matrices, rows, columns, K)[0] == str(int(taken))
