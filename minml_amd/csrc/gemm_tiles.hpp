@@ -141,7 +141,9 @@ namespace mlhip
 	 * The same for products with bias (+ beta * C), linear or ReLU: dense layers, 1x1 convolutions, the experts' layers. Alone, other kernel / this one, us, and
 	 * the number of 64x64 tiles:
 	 *   fp16, from 1.75 tiles per unit with rows up to 512 bytes (256 x 256: 2700 rows (172) 4.3 / 4.8, 7200 (452) 5.7 / 5.6; 128 to 768: 2700
-	 *   (516) 5.9 / 5.2), 1 up to 768 bytes (384 x 256: 7200 (452) 11.0 / 6.5; x 384: 2700 (258) 6.2 / 6.0), 0.5 up to 1024 (512 x 256: 2700 (172) 7.0 / 6.0). Rows of
+	 *   (516) 5.9 / 5.2), 1 up to 768 bytes (384 x 256: 7200 (452) 11.0 / 6.5; x 384: 2700 (258) 6.2 / 6.0), 0.5 up to 1024, where the 32x32 tiles of
+	 *   conv_tiles.hpp end (512 x 256: 2048 (128) 5.5 / 5.7, from memory 5.2 / 5.9, 2300 (144) 6.9 / 5.8, 2700 (172) 7.0 / 6.0; eight experts 228 rows (128) 5.3 / 5.7, 300
+	 *   (160) 6.5 / 5.8). Rows of
 	 *   2048 bytes, for which a tile of 256 rows is the better one where there are enough, from 1 to 4 (eight experts of 1024 x 256: 912 rows
 	 *   (480) 13.4 / 10.6, 3648 (1824) 25.4 / 30.7); 1024 with a batch to 8 (512 x 1024: 912 rows (1920) 18.5 / 15.9, 3648 (7296) 43.5 / 46.4).
 	 *   Half a tile of padding is not for them: at most 32 columns where the streaming or direct kernel take the rows, from 3.5 tiles per unit (28800 x 32: 256-byte
@@ -157,6 +159,7 @@ namespace mlhip
 	inline bool gemm_tiles_apply(const StreamGemmArgs &g, int element_size, bool reads_c)
 	{
 		const long long tiles = static_cast<long long>(ceil_div(g.M, 64)) * ceil_div(g.N, 64) * g.batch, units = device_compute_units();
+		const long long small_tiles = static_cast<long long>(ceil_div(g.M, 32)) * ceil_div(g.N, 32) * g.batch;
 		if (g.k_bytes % 64 != 0)
 			return false;
 		if (element_size == 4)
@@ -164,6 +167,8 @@ namespace mlhip
 		if (g.k_bytes == 2048)
 			return tiles >= units && tiles <= 4 * units;
 		if (g.k_bytes < 192 || g.k_bytes > 1024)
+			return false;
+		if (g.k_bytes > 768 && g.k_bytes % 128 == 0 && small_tiles <= 2 * units)
 			return false;
 		if (g.k_bytes > 768 && g.batch > 1 && tiles > 8 * units)
 			return false;

@@ -70,6 +70,9 @@ def test_plain_batches_on_the_tiles(decide, dtype, matrices, rows, columns, K, t
 @pytest.mark.parametrize("dtype,matrices,rows,columns,K,taken", [
     # few columns: half of a tile would be padding
     ("float16", 1, 28800, 32, 256, False), ("float16", 1, 57600, 32, 256, True), ("float16", 1, 114119, 32, 192, False), ("float16", 1, 57600, 40, 192, False),
-    ("float16", 1, 114119, 64, 192, True), ("float16", 1, 28800, 32, 96, True), ("float16", 1, 28800, 40, 256, True)])
+    ("float16", 1, 114119, 64, 192, True), ("float16", 1, 28800, 32, 96, True), ("float16", 1, 28800, 40, 256, True),
+    # 1024-byte K rows: from where the 32x32 tiles of conv_tiles.hpp end, two per compute unit
+    ("float16", 1, 2048, 256, 512, False), ("float16", 1, 2300, 256, 512, True), ("float16", 8, 228, 256, 512, False), ("float16", 8, 300, 256, 512, True),
+    ("float16", 1, 2048, 256, 480, True)])
 def test_dense_layers_on_the_tiles(decide, dtype, matrices, rows, columns, K, taken):
     assert decide("dense", dtype, matrices, rows, columns, K)[0] == str(int(taken))
