@@ -143,9 +143,11 @@ namespace mlhip
 	 *   fp16, from 1.75 tiles per unit with rows up to 512 bytes (256 x 256: 2700 rows (172) 4.3 / 4.8, 7200 (452) 5.7 / 5.6; 128 to 768: 2700
 	 *   (516) 5.9 / 5.2), 1 up to 768 bytes (384 x 256: 7200 (452) 11.0 / 6.5; x 384: 2700 (258) 6.2 / 6.0), 0.5 up to 1024, where the 32x32 tiles of
 	 *   conv_tiles.hpp end (512 x 256: 2048 (128) 5.5 / 5.7, from memory 5.2 / 5.9, 2300 (144) 6.9 / 5.8, 2700 (172) 7.0 / 6.0; eight experts 228 rows (128) 5.3 / 5.7, 300
-	 *   (160) 6.5 / 5.8). Rows of
-	 *   2048 bytes, for which a tile of 256 rows is the better one where there are enough, from 1 to 4 (eight experts of 1024 x 256: 912 rows
-	 *   (480) 13.4 / 10.6, 3648 (1824) 25.4 / 30.7); 1024 with a batch to 8 (512 x 1024: 912 rows (1920) 18.5 / 15.9, 3648 (7296) 43.5 / 46.4).
+	 *   (160) 6.5 / 5.8). Longer
+	 *   rows, for which a tile of 256 rows is the better one where there are enough, to 4 per unit and 8192 bytes of K rows per unit (eight experts of 576 to 2048 x 256,
+	 *   from L2: 300 rows (160) 1152 bytes 6.9 / 6.2, 2048 9.7 / 8.9, 4096 15.6 / 13.9; 912 (480) 9.4 / 8.0, 13.2 / 10.7, 21.1 / 17.6; 1824 (928) 13.3 / 12.1, 18.5 /
+	 *   17.6, 30.4 / 32.1, from memory 14.3 / 14.5, 21.8 / 22.1, 37.4 / 39.3; 2100 (1056) 14.0 / 14.7, 20.2 / 22.2, 33.6 / 37.1; 3072 bytes 1200 (608) 22.1 / 18.1, 1824 from
+	 *   memory 30.2 / 31.7; single layers of 256 columns, whose other kernel has its epilogue at run time, 1536 bytes 10800 rows (676) 13.6 / 10.6, 14400 (900) 15.7 / 14.1). 1024 with a batch to 8 (512 x 1024: 912 rows (1920) 18.5 / 15.9, 3648 (7296) 43.5 / 46.4).
 	 *   Half a tile of padding is not for them: at most 32 columns where the streaming or direct kernel take the rows, from 3.5 tiles per unit (28800 x 32: 256-byte
 	 *   rows (450) 3.9 / 4.4, 512 4.7 / 5.1, 768 5.5 / 5.9; 57600 (900) 5.2 / 5.3, 7.4 / 7.3, 14.1 / 11.0); 384 bytes, whose direct kernel has no upper limit,
 	 *   from 64 columns (114119 x 32 10.8 / 11.9, 230400 x 24 17.3 / 18.9, 57600 x 40 from memory 8.6 / 9.2).
@@ -164,12 +166,10 @@ namespace mlhip
 			return false;
 		if (element_size == 4)
 			return g.k_bytes == 256 || g.k_bytes == 512 || (g.k_bytes <= 4096 && 8 * tiles >= 5 * units);
-		if (g.k_bytes == 2048)
-			return tiles >= units && tiles <= 4 * units;
-		if (g.k_bytes < 192 || g.k_bytes > 1024)
+		if (g.k_bytes < 192 || (g.k_bytes > 768 && g.k_bytes % 128 == 0 && small_tiles <= 2 * units))
 			return false;
-		if (g.k_bytes > 768 && g.k_bytes % 128 == 0 && small_tiles <= 2 * units)
-			return false;
+		if (g.k_bytes > 1024)
+			return g.k_bytes <= 4096 && small_tiles > 2 * units && tiles <= 4 * units && tiles * g.k_bytes <= 8192 * units;
 		if (g.k_bytes > 768 && g.batch > 1 && tiles > 8 * units)
 			return false;
 		const bool streams = g.k_bytes == 256 || g.k_bytes == 512 || g.k_bytes == 768;

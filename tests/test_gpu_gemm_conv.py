@@ -101,7 +101,7 @@ def test_gemm_batched_nt_tiles(ctx, dtype, shape):
 
 @pytest.mark.parametrize("dtype", ["float32", "float16"])
 @pytest.mark.parametrize("shape", [(7200, 256, 256), (2701, 776, 96), (14401, 264, 128), (7300, 392, 384), (9000, 200, 192), (2750, 264, 512), (130, 8192, 1024), (14500, 260, 256),
-                                   (14401, 192, 192), (7301, 328, 384), (21000, 136, 96)])
+                                   (14401, 192, 192), (7301, 328, 384), (21000, 136, 96), (3700, 264, 576), (2500, 264, 544), (2400, 392, 2048)])
 def test_gemm_ex_tiles(ctx, dtype, shape):
     """Dense layers between few rows and many (tiles of 64x64, 128x64, 128x128 and 128x192; ragged rows and columns; a width that is no multiple of 16 bytes
     in fp16, which goes on to the other kernels), with bias, ReLU or linear, with and without a residual; a prefix of the rows, which takes

@@ -73,6 +73,10 @@ def test_plain_batches_on_the_tiles(decide, dtype, matrices, rows, columns, K, t
     ("float16", 1, 114119, 64, 192, True), ("float16", 1, 28800, 32, 96, True), ("float16", 1, 28800, 40, 256, True),
     # 1024-byte K rows: from where the 32x32 tiles of conv_tiles.hpp end, two per compute unit
     ("float16", 1, 2048, 256, 512, False), ("float16", 1, 2300, 256, 512, True), ("float16", 8, 228, 256, 512, False), ("float16", 8, 300, 256, 512, True),
-    ("float16", 1, 2048, 256, 480, True)])
+    ("float16", 1, 2048, 256, 480, True),
+    # longer ones: to four 64x64 tiles and 8192 bytes of K rows per unit
+    ("float16", 8, 912, 256, 576, True), ("float16", 8, 1824, 256, 768, True), ("float16", 8, 1824, 256, 1024, True), ("float16", 8, 2100, 256, 1024, False),
+    ("float16", 8, 1200, 256, 1536, True), ("float16", 8, 1824, 256, 1536, False), ("float16", 8, 912, 256, 2048, True), ("float16", 8, 1200, 256, 2048, False),
+    ("float16", 8, 912, 256, 2080, False), ("float16", 8, 228, 256, 1024, False)])
 def test_dense_layers_on_the_tiles(decide, dtype, matrices, rows, columns, K, taken):
     assert decide("dense", dtype, matrices, rows, columns, K)[0] == str(int(taken))
