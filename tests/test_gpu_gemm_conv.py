@@ -103,7 +103,7 @@ def test_gemm_batched_nt_tiles(ctx, dtype, shape):
 @pytest.mark.parametrize("shape", [(7200, 256, 256), (2701, 776, 96), (14401, 264, 128), (7300, 392, 384), (9000, 200, 192), (2750, 264, 512), (130, 8192, 1024), (14500, 260, 256),
                                    (14401, 192, 192), (7301, 328, 384), (21000, 136, 96), (3700, 264, 576), (2500, 264, 544), (2400, 392, 2048)])
 def test_gemm_ex_tiles(ctx, dtype, shape):
-    """Dense layers between few rows and many (tiles of 64x64, 128x64, 128x128 and 128x192; ragged rows and columns; a width that is no multiple of 16 bytes
+    """Dense layers between few rows and many (tiles of 64x64, 128x64 and 128x128; ragged rows and columns; a width that is no multiple of 16 bytes
     in fp16, which goes on to the other kernels), with bias, ReLU or linear, with and without a residual; a prefix of the rows, which takes
     another kernel, gives the same bits."""
     M, N, K = shape
@@ -123,7 +123,7 @@ def test_gemm_ex_tiles(ctx, dtype, shape):
 
 
 @pytest.mark.parametrize("dtype,K,N", [("float16", 32, 256), ("float16", 64, 64), ("float16", 96, 96), ("float16", 128, 128), ("float16", 192, 192), ("float16", 256, 256),
-                                       ("float16", 384, 384), ("float32", 32, 64), ("float32", 64, 64), ("float32", 128, 128), ("float32", 192, 192)])
+                                       ("float16", 384, 384), ("float32", 32, 64), ("float32", 64, 64), ("float32", 128, 128), ("float32", 192, 192), ("float32", 256, 256)])
 def test_gemm_batched_rows_do_not_depend_on_their_number(ctx, dtype, K, N):
     """Every kernel and grid order that a Winograd product may take by its number of rows gives the same bits for the same row."""
     rng = np.random.default_rng(K + N)
@@ -762,11 +762,12 @@ def test_group_gemm(ctx, dtype, case):
 
 @pytest.mark.parametrize("dtype,chunk", [("float16", 64), ("float32", 32)])
 @pytest.mark.parametrize("chunks", [1, 2, 3, 4, 5, 8])
-def test_group_gemm_wide_tiles(ctx, dtype, chunk, chunks):
+@pytest.mark.parametrize("N", [250, 252, 256, 260])
+def test_group_gemm_wide_tiles(ctx, dtype, chunk, chunks, N):
     """Every length of the 256-wide tile's pipeline (its head, the steady part, both parities of its two slots, its tail), with whole and
-    ragged tiles of rows and columns; the last bits do not depend on where in a tile a row or column lies. The operands and their sums are
-    small whole numbers, exact in every precision used: the tolerance is 0."""
-    M, N, K, groups = 300, 260, chunk * chunks, 2
+    ragged tiles of rows; 250 and 252 columns pad the tile (without and with stores of four), 260 are one tile and four columns on narrow ones.
+    The operands and their sums are small whole numbers, exact in every precision used: the tolerance is 0."""
+    M, K, groups = 300, chunk * chunks, 2
     rng = np.random.default_rng(chunks)
     stored = O.to_half if dtype == "float16" else (lambda t: t)
     a, b, c = (rng.integers(-1, 2, s).astype(np.float32) for s in ((M, K * groups), (N, K * groups), (M, N * groups)))

@@ -25,7 +25,8 @@ def init_for_test_int8(shape, shift):
 
 
 @pytest.mark.parametrize("shape", [(75, 44, 36), (1716, 44, 36), (130, 70, 64), (300, 256, 2304), (33, 5, 20), (64, 64, 16),
-                                   (33001, 256, 256), (40000, 72, 128), (32900, 132, 512)])
+                                   (33001, 256, 256), (40000, 72, 128), (32900, 132, 512),
+                                   (33001, 252, 384), (33001, 250, 640), (16600, 516, 768)])  # the last three on 256-wide tiles
 def test_int8_gemm_exact(ctx, shape):
     M, N, K = shape
     rng = np.random.default_rng(M)
@@ -112,6 +113,26 @@ def test_int8_convolution_of_few_positions(ctx, shape, cout, k):
             assert np.abs(dy.copyToHost(ctx).astype(np.int32) - want.astype(np.int32)).max() <= 1
         else:
             assert mismatches(dy.copyToHost(ctx), want) == 0
+
+
+@pytest.mark.parametrize("shape,cout", [((203, 19, 19, 16), 128), ((131, 19, 19, 32), 202)])
+def test_int8_convolution_short_k_many_pixels(ctx, shape, cout):
+    """3x3 with K rows of at most 512 bytes that straddle taps, more than 1024 tiles of 128x64: the register-staged tiles with every form of their
+    epilogue, bit for bit; 202 columns are no multiple of 4."""
+    b, h, w, cin = shape
+    rng = np.random.default_rng(cout)
+    x = rng.integers(-128, 128, shape).astype(np.int8)
+    wt = rng.integers(-127, 128, (cout, 3, 3, cin)).astype(np.int8)
+    scales = (rng.random(cout) * 0.002 + 0.0005).astype(np.float32)
+    bias = rng.standard_normal(cout).astype(np.float32)
+    ext = rng.integers(-128, 128, (b, h, w, cout)).astype(np.int8)
+    dx, dw, ds, db, de = (ml.toDevice(ctx, a) for a in (x, wt, scales, bias, ext))
+    O.set_num_threads(8)
+    for code, act, use_ext in ((O.INT8, "relu", True), (O.INT8, "linear", True), (O.INT8, "linear", False), (O.FLOAT32, "linear", True), (O.FLOAT32, "relu", False)):
+        want = O.int8_conv2d_forward(x, IN_QD, wt, scales, bias, code, OUT_QD, ext if use_ext else None, EXT_QD, ml.act_of(act))
+        dy = ml.Tensor((b, h, w, cout), code)
+        ml.quantizedConvForward(ctx, dx, IN_QD, dw, ds, db, dy, OUT_QD, de if use_ext else None, EXT_QD, act)
+        assert mismatches(dy.copyToHost(ctx), want) == 0
 
 
 def test_quantized_network_layer_config3(ctx):

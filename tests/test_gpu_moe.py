@@ -179,6 +179,28 @@ def test_expert_layers(ctx, dtype, dims):
     assert max_abs_rel(dy.copyToHost(ctx), M.moe_forward(x, w, bias, O.LINEAR, beta=0.5, y=y0)) <= TOL[dtype]
 
 
+@pytest.mark.parametrize("dtype", ["float32", "float16"])
+@pytest.mark.parametrize("rows,c,n", [(907, 256, 1024), (912, 1024, 256), (901, 384, 200), (2403, 192, 192), (300, 512, 256), (613, 576, 264)])
+def test_expert_layers_between_few_rows_and_many(ctx, dtype, rows, c, n):
+    """Eight experts with more rows than the small tiles are for and fewer than the streaming kernel and the 256-row tiles: every expert has its own rows of
+    x and y, weights and bias, in tiles of 64x64, 128x64 and 128x128 with ragged rows and columns; both activations, and beta times the output in
+    place. The first rows alone, which take other kernels, give the same bits."""
+    experts, few = 8, 40
+    rng = np.random.default_rng(rows + c)
+    O.set_num_threads(8)
+    x = random_tensor(rng, (1, rows, experts, c), dtype)
+    w = random_tensor(rng, (experts, n, c), dtype, (1.0 / c) ** 0.5)
+    bias, y0 = random_tensor(rng, (experts, n), dtype, 0.1), random_tensor(rng, (1, rows, experts, n), dtype)
+    dx, dw, db, first = ml.toDevice(ctx, x), ml.toDevice(ctx, w), ml.toDevice(ctx, bias), ml.toDevice(ctx, x[:, :few])
+    for act, beta in (("relu", 0.0), ("linear", 0.0), ("relu", 0.5), ("linear", 0.5)):
+        y, some = ml.toDevice(ctx, y0), ml.toDevice(ctx, y0[:, :few])
+        ml.moeForward(ctx, dx, dw, db, beta, y, act)
+        ml.moeForward(ctx, first, dw, db, beta, some, act)
+        got = y.copyToHost(ctx)
+        assert max_abs_rel(got, M.moe_forward(x, w, bias, ml.act_of(act), beta=beta, y=y0)) <= TOL[dtype]
+        assert mismatches(some.copyToHost(ctx), np.ascontiguousarray(got[:, :few])) == 0
+
+
 # ---- the reference's own tests, mirrored: its device layers against the CPU baselines of test/backend/test_moe.cpp, fp32, 1e-4 -----------
 
 def _routing_table(rng, batch, tokens, experts, slots, empty=0.15):
