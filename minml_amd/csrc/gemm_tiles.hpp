@@ -155,7 +155,9 @@ namespace mlhip
 	 *   115200 (177) 41.7 / 41.7, 230400 81.5 / 105; 256 x 1024: 27797 (71) 28.7 / 28.1, 57600 (147) 48.8 / 55.1; 384 x 384 with residual: 27797 (64) 25.2 / 22.2, 57600
 	 *   (133) 39.7 / 40.1; eight experts of 256 x 1024: 3648 rows (75) 36.7 / 29.4, 7296 (149) 57.1 / 55.4, 14592 89 / 127), 180 with one column tile
 	 *   (128 x 128 with residual: 230400 rows (177) 36.4 / 34.2, 369664 (284) 50.2 / 68.8).
-	 *   fp32, rows of 256 and 512 bytes, which only the streaming kernel took: always (128 x 128: 225 rows 17.2 / 6.2, 27797 20.2 / 16.4, 230400 105 / 87).
+	 *   fp32, rows of 256 and 512 bytes, which only the streaming kernel took: always (128 x 128: 225 rows 17.2 / 6.2, 27797 20.2 / 16.4, 230400 105 / 87); those of
+	 *   experts (a_row_bytes), for which the 32x32 tiles of conv_tiles.hpp stand, from where these end (eight of 128 x 64: 64 rows 4.5 / 5.6, 512 4.7 / 5.7, 800 5.4 / 5.8; 36 of 64 x 64: 85 rows
+	 *   3.8 / 4.3, 177 4.3 / 4.4; sixteen of 128 x 256, 809 rows 16.2 / 14.2).
 	 *   Others up to 4096 bytes from 0.6 (256 x 256: 900 rows (60) 6.8 / 8.8, 2700 (172) 11.8 / 9.2, 57600 87.6 / 74.5).
 	 */
 	inline bool gemm_tiles_apply(const StreamGemmArgs &g, int element_size, bool reads_c)
@@ -164,8 +166,10 @@ namespace mlhip
 		const long long small_tiles = static_cast<long long>(ceil_div(g.M, 32)) * ceil_div(g.N, 32) * g.batch;
 		if (g.k_bytes % 64 != 0)
 			return false;
+		if (element_size == 4 && (g.k_bytes == 256 || g.k_bytes == 512))
+			return g.a_row_bytes == 0 || small_tiles > 2 * units;
 		if (element_size == 4)
-			return g.k_bytes == 256 || g.k_bytes == 512 || (g.k_bytes <= 4096 && 8 * tiles >= 5 * units);
+			return g.k_bytes <= 4096 && 8 * tiles >= 5 * units;
 		if (g.k_bytes < 192 || (g.k_bytes > 768 && g.k_bytes % 128 == 0 && small_tiles <= 2 * units))
 			return false;
 		if (g.k_bytes > 1024)
