@@ -86,6 +86,6 @@ def test_dense_layers_on_the_tiles(decide, dtype, matrices, rows, columns, K, ta
     # fp32 experts of 256 and 512-byte K rows: the 32x32 tiles of conv_tiles.hpp up to two per compute unit; a single layer has no such kernel
     ("experts", 8, 64, 64, 128, False), ("experts", 8, 800, 64, 128, False), ("experts", 8, 1100, 64, 128, True), ("experts", 36, 85, 64, 64, False),
     ("experts", 8, 200, 256, 64, False), ("experts", 1, 225, 128, 128, False), ("experts", 4, 818, 256, 128, True), ("dense", 1, 225, 128, 128, True),
-    ("experts", 4, 398, 256, 96, True), ("experts", 8, 640, 64, 192, False)])
+    ("experts", 4, 700, 256, 96, True), ("experts", 8, 640, 64, 192, False)])
 def test_fp32_experts_on_the_tiles(decide, kind, matrices, rows, columns, K, taken):
     assert decide(kind, "float32", matrices, rows, columns, K)[0] == str(int(taken))
