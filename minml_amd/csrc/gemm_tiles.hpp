@@ -151,10 +151,16 @@ namespace mlhip
 	 *   Half a tile of padding is not for them: at most 32 columns where the streaming or direct kernel take the rows, from 3.5 tiles per unit (28800 x 32: 256-byte
 	 *   rows (450) 3.9 / 4.4, 512 4.7 / 5.1, 768 5.5 / 5.9; 57600 (900) 5.2 / 5.3, 7.4 / 7.3, 14.1 / 11.0); 384 bytes, whose direct kernel has no upper limit,
 	 *   from 64 columns (114119 x 32 10.8 / 11.9, 230400 x 24 17.3 / 18.9, 57600 x 40 from memory 8.6 / 9.2).
-	 *   Not beyond 96 MB of A, C and what is read of it where the streaming kernel takes the rows (256 x 256: 57600 rows, 88 MB with residual, 26.4 / 23.8,
+	 *   Not beyond a number of bytes of A, C and what is read of it where the streaming kernel takes the rows: ahead further with the operands in the last-level
+	 *   cache than from memory (this one's time over the other's, cached / from memory), and with a residual, whose fetch the other does not hide, further than without.
+	 *   256-byte rows to 34 MB: 128 columns 32 MB 0.77 / 0.94, 40 0.87 / 1.05, 66 0.92 / 1.12; 256 columns 24 0.87 / 1.05, 32 0.85 / 1.06, 40 0.97 / 1.22, 95 1.00 / 1.38; 1024
+	 *   columns 24 0.82 / 0.99, 40 0.89 / 1.15, 80 1.04 / 1.47. 512 to 46 MB: 256 columns 40 MB 0.77 / 0.97, 52 0.91 / 1.09, 95 0.94 / 1.19; 1024 columns 40 0.85 / 1.05, 52 0.90 /
+	 *   1.18, 80 1.04 / 1.36. 768 to 67 MB: 256 columns 66 MB 0.79 / 1.02, 95 0.84 / 1.09; 1024 columns 66 0.85 / 1.04, 80 0.86 / 1.10. With a residual to 101 MB: 256-byte rows 40
+	 *   to 95 MB 0.87 to 1.04 / 0.86 to 1.11, 512 0.80 to 0.93 / 0.80 to 1.06, 768 0.80 to 0.95 / 0.87 to 1.07 (256 x 256: 57600 rows, 88 MB with residual, 26.4 / 23.8,
 	 *   115200 (177) 41.7 / 41.7, 230400 81.5 / 105; 256 x 1024: 27797 (71) 28.7 / 28.1, 57600 (147) 48.8 / 55.1; 384 x 384 with residual: 27797 (64) 25.2 / 22.2, 57600
-	 *   (133) 39.7 / 40.1; eight experts of 256 x 1024: 3648 rows (75) 36.7 / 29.4, 7296 (149) 57.1 / 55.4, 14592 89 / 127), 180 with one column tile
-	 *   (128 x 128 with residual: 230400 rows (177) 36.4 / 34.2, 369664 (284) 50.2 / 68.8).
+	 *   (133) 39.7 / 40.1; eight experts of 256 x 1024: 7296 rows (149) 57.1 / 55.4, 14592 89 / 127), to 189 with at most 128 columns
+	 *   from 512 bytes on (512: 66 to 130 MB 0.81 / 1.06 to 0.80 / 1.04, 768 130 MB 0.75 / 1.00; with residual 256 bytes 230400 rows (177) 36.4 / 34.2, 369664 (284) 50.2 / 68.8, but
+	 *   from memory 130 MB 0.95 / 1.08).
 	 *   fp32, rows of 256 and 512 bytes, which only the streaming kernel took: always (128 x 128: 225 rows 17.2 / 6.2, 27797 20.2 / 16.4, 230400 105 / 87); those of
 	 *   experts (a_row_bytes), for which the 32x32 tiles of conv_tiles.hpp stand, from where these end (eight of 128 x 64: 64 rows 4.5 / 5.6, 512 4.7 / 5.7, 800 5.4 / 5.8; 36 of 64 x 64: 85 rows
 	 *   3.8 / 4.3, 177 4.3 / 4.4; sixteen of 128 x 256, 809 rows 16.2 / 14.2).
@@ -180,7 +186,8 @@ namespace mlhip
 		const unsigned long long bytes = exchanged_bytes(g, element_size) + (reads_c ? static_cast<unsigned long long>(g.batch) * g.M * g.N * element_size : 0);
 		if ((g.k_bytes == 384 && g.N < 64) || (streams && g.N <= 32 && 2 * tiles < 7 * units))
 			return false;
-		return 4 * tiles >= (g.k_bytes <= 512 ? 7 : g.k_bytes <= 768 ? 4 : 2) * units && !(streams && bytes > ((g.N > 128 ? 96ULL : 180ULL) << 20));
+		const unsigned long long megabytes = (g.N <= 128 && g.k_bytes > 256) ? 180 : reads_c ? 96 : g.k_bytes == 256 ? 32 : g.k_bytes == 512 ? 44 : 64;
+		return 4 * tiles >= (g.k_bytes <= 512 ? 7 : g.k_bytes <= 768 ? 4 : 2) * units && !(streams && bytes > (megabytes << 20));
 	}
 	/* rows x columns of the tile that a workgroup owns */
 	enum class GemmTile

@@ -2,7 +2,8 @@
  * Prints what the dispatch rules of the products decide on a card of 256 compute units, without a device: one line per line of the input,
  *   plain <element size> <matrices> <rows> <columns> <bytes of a K row>      "<tiles 0|1> <by rows 0|1> <direct kernel 0|1> <tile>"
  *   dense ...                                                                "<tiles 0|1> 0 <direct kernel 0|1> <tile>"   (bias, no C)
- *   experts ...                                                              the same with the matrices' rows side by side
+ *   residual ...                                                             the same with C
+ *   experts ...                                                              as dense, with the matrices' rows side by side
  */
 #include "gemm_direct.hpp"
 
@@ -28,7 +29,7 @@ int main()
 		g.a_row_bytes = (std::strcmp(kind, "experts") == 0) ? static_cast<size_t>(g.batch) * g.k_bytes : 0;
 		const mlhip::GemmTile tile = plain ? mlhip::tile_of_plain(g, element_size) : mlhip::tile_with_epilogue(g, element_size);
 		const char *names[] = { "64x64", "128x64", "128x128", "128x192" };
-		std::printf("%d %d %d %s\n", plain ? mlhip::plain_gemm_tiles_apply(g, element_size) : mlhip::gemm_tiles_apply(g, element_size, false),
+		std::printf("%d %d %d %s\n", plain ? mlhip::plain_gemm_tiles_apply(g, element_size) : mlhip::gemm_tiles_apply(g, element_size, std::strcmp(kind, "residual") == 0),
 				plain && mlhip::products_go_by_rows(g, element_size), element_size == 2 && mlhip::gemm_direct_applies(g), names[static_cast<int>(tile)]);
 	}
 	return 0;

@@ -77,7 +77,11 @@ def test_plain_batches_on_the_tiles(decide, dtype, matrices, rows, columns, K, t
     # longer ones: to four 64x64 tiles and 8192 bytes of K rows per unit
     ("float16", 8, 912, 256, 576, True), ("float16", 8, 1824, 256, 768, True), ("float16", 8, 1824, 256, 1024, True), ("float16", 8, 2100, 256, 1024, False),
     ("float16", 8, 1200, 256, 1536, True), ("float16", 8, 1824, 256, 1536, False), ("float16", 8, 912, 256, 2048, True), ("float16", 8, 1200, 256, 2048, False),
-    ("float16", 8, 912, 256, 2080, False), ("float16", 8, 228, 256, 1024, False)])
+    ("float16", 8, 912, 256, 2080, False), ("float16", 8, 228, 256, 1024, False),
+    # short K rows from memory: the streaming kernel from 34, 46 and 67 MB of A and C on, with at most 128 columns later
+    ("float16", 1, 41666, 256, 128, True), ("float16", 1, 52083, 256, 128, False), ("float16", 1, 128906, 128, 128, False), ("float16", 16, 1007, 2048, 128, False),
+    ("float16", 1, 39062, 256, 256, True), ("float16", 1, 50781, 256, 256, False), ("float16", 4, 8140, 512, 256, False), ("float16", 1, 169270, 128, 256, True),
+    ("float16", 1, 50000, 256, 384, True), ("float16", 1, 74218, 256, 384, False), ("float16", 1, 126953, 128, 384, True)])
 def test_dense_layers_on_the_tiles(decide, dtype, matrices, rows, columns, K, taken):
     assert decide("dense", dtype, matrices, rows, columns, K)[0] == str(int(taken))
 
@@ -89,3 +93,10 @@ def test_dense_layers_on_the_tiles(decide, dtype, matrices, rows, columns, K, ta
     ("experts", 4, 700, 256, 96, True), ("experts", 8, 640, 64, 192, False)])
 def test_fp32_experts_on_the_tiles(decide, kind, matrices, rows, columns, K, taken):
     assert decide(kind, "float32", matrices, rows, columns, K)[0] == str(int(taken))
+
+
+@pytest.mark.parametrize("rows,columns,K,taken", [
+    # with a residual, which the streaming kernel does not hide: to 101 MB
+    (74218, 256, 128, True), (80000, 256, 128, False), (61848, 256, 256, True), (53011, 256, 384, True), (27797, 384, 384, True), (169270, 128, 128, False), (126953, 128, 256, True)])
+def test_dense_layers_with_residual_on_the_tiles(decide, rows, columns, K, taken):
+    assert decide("residual", "float16", 1, rows, columns, K)[0] == str(int(taken))
