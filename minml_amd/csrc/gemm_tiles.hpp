@@ -87,7 +87,10 @@ namespace mlhip
 	 * which the streaming kernel holds only 128 columns (whole networks of 8 blocks, 384 channels): 239 MB 2352 / 2083, 292 2706 / 2499, but with three
 	 * calls per layer 265 MB 2435 / 2472, where three or five column tiles leave its slices of 128 columns padded or some compute units idle; other widths, alone
 	 * (12 and 36 matrices, this one's time over the other's): 256 columns 150 MB 0.96, 200 1.05, 245 1.16, 512 150 0.96, 200 0.99, 245 1.13, 1024 90 0.85, 120 0.95, 200 1.04, 245 1.20 (64 matrices 108 1.06),
-	 * 2048 150 1.03, 245 1.18; 320 245 0.88, 640 0.90); fp32 256-byte rows, where those slices are not padded by more than an eighth: 128 columns 250 MB 0.94, 300 1.00,
+	 * 2048 150 1.03, 245 1.18; 320 245 0.88, 640 0.90). Other batches than the 36 of a network have their operands as often from memory (cached / from memory, 16 matrices):
+	 * 256 bytes to 34 MB, 24 MB 128 columns 0.70 / 0.92, 256 0.83 / 1.05, 512 0.78 / 0.93, 32 0.82 / 1.06, 0.82 / 1.08, 0.74 / 1.01, 54 0.83 / 1.11, 0.83 / 1.20, 0.94 / 1.36;
+	 * 512 to 67, 256 columns 66 MB 0.76 / 0.95, 80 0.82 / 1.05, 92 0.86 / 1.12, 1024 columns 66 0.74 / 0.96, 80 0.97 / 1.30; 768 to 105, 256 columns 92 0.82 / 1.05, 130 0.87 / 1.10, 512 92 0.74 / 0.96,
+	 * 130 0.83 / 1.07, beyond 512 columns to 84, 1024 80 0.76 / 0.96, 92 0.96 / 1.22, in three or five column tiles to 210, 384 200 0.76 / 0.97, 250 0.85 / 1.07, 640 200 0.92 / 1.10, 250 1.02 / 1.14. fp32 256-byte rows, where those slices are not padded by more than an eighth: 128 columns 250 MB 0.94, 300 1.00,
 	 * 450 1.06, 256 columns 250 0.98, 300 1.08, 450 1.13, 512 250 1.03, 300 1.09, 600 1.18 (64 columns 600 MB 0.92, 192 0.88); fp32 512-byte rows 151 MB 82.4 / 79.9, 227
 	 * 117 / 123; 64-byte rows (the stem, alone) 170 MB 32.4 / 29.3, 340 89.8 / 101; fp32 128-byte rows, the stem, with the
 	 * input from memory 24 MB 11.9 / 10.1, 47 16.6 / 16.4, 57 16.6 / 17.7, 85 23.3 / 27.6, 94 23.3 / 27.6; whole networks of one block 128 channels 9 MB 67.2 / 63.9, 38
@@ -96,7 +99,7 @@ namespace mlhip
 	 */
 	inline bool plain_gemm_tiles_apply(const StreamGemmArgs &g, int element_size)
 	{
-		const bool fp16 = element_size == 2;
+		const bool fp16 = element_size == 2, between = g.batch == TRANSFORM_MATRICES;
 		if (g.k_bytes % 64 != 0 || (fp16 && (g.k_bytes == 128 || g.k_bytes > 768)))
 			return false;
 		const long long tiles = static_cast<long long>(ceil_div(g.M, 32)) * ceil_div(g.N, 32) * g.batch;
@@ -113,7 +116,7 @@ namespace mlhip
 			case 256:
 				fewest = fp16 ? 8 : 0;
 				if (fp16)
-					megabytes = 64;
+					megabytes = between ? 64 : 32;
 				else if (g.N > 64 && 8 * (ceil_div(g.N, 128) * 128LL - g.N) <= g.N)
 					megabytes = 256;
 				break;
@@ -121,13 +124,15 @@ namespace mlhip
 				fewest = fp16 ? 4 : 1;
 				break;
 			case 512:
-				fewest = fp16 ? (g.batch == TRANSFORM_MATRICES ? 4 : 8) : 0;
-				megabytes = fp16 ? 90 : 200;
+				fewest = fp16 ? (between ? 4 : 8) : 0;
+				megabytes = fp16 ? (between ? 90 : 64) : 200;
 				break;
 			case 768:
-				fewest = fp16 ? (g.batch == TRANSFORM_MATRICES ? 3 : 4) : 1;
-				if (fp16)
-					megabytes = (ceil_div(g.N, 64) % 3 == 0 || ceil_div(g.N, 64) % 5 == 0) && g.N <= 1024 ? 240 : g.N <= 512 ? 160 : 100;
+				fewest = fp16 ? (between ? 3 : 4) : 1;
+				if (fp16 && (ceil_div(g.N, 64) % 3 == 0 || ceil_div(g.N, 64) % 5 == 0) && g.N <= 1024)
+					megabytes = between ? 240 : 200;
+				else if (fp16)
+					megabytes = (g.N <= 512) ? (between ? 160 : 100) : (between ? 100 : 80);
 				break;
 			default:
 				fewest = (fp16 || g.k_bytes < 384) ? 0 : 1;

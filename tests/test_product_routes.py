@@ -57,12 +57,16 @@ def test_tiles_of_128_rows_where_the_matrix_fills_them(decide, kind, matrices, r
     # fp32, 128-byte K rows (32 planes): to 50 MB of A and C, 63 with one column tile
     ("float32", 36, 4096, 64, 32, True), ("float32", 36, 8000, 64, 32, False),
     ("float32", 36, 1616, 128, 32, True), ("float32", 36, 4096, 128, 32, False), ("float32", 36, 1616, 256, 32, False), ("float32", 36, 1024, 256, 32, True),
-    # wide columns that fill the streaming kernel's slices: 768-byte fp16 rows to 168 or 105 MB, 256-byte fp32 rows to 268 MB; other widths further
-    ("float16", 64, 1024, 1024, 384, False), ("float16", 64, 800, 1024, 384, False), ("float16", 64, 500, 1024, 384, True), ("float16", 64, 1400, 512, 384, True), ("float16", 36, 4300, 384, 384, True), ("float16", 36, 3300, 640, 384, True),
+    # wide columns that fill the streaming kernel's slices: 768-byte fp16 rows of a network's batch to 168 or 105 MB, 256-byte fp32 rows to 268 MB; other widths further
+    ("float16", 64, 1024, 1024, 384, False), ("float16", 64, 800, 1024, 384, False), ("float16", 64, 450, 1024, 384, True), ("float16", 36, 2400, 512, 384, True), ("float16", 36, 4300, 384, 384, True), ("float16", 36, 3300, 640, 384, True),
     ("float16", 36, 4300, 256, 384, False), ("float32", 64, 1024, 1024, 64, False), ("float32", 36, 16384, 64, 64, True), ("float32", 36, 9000, 192, 64, True),
     # few tiles: the direct kernel further in batches that are not between transforms
     ("float16", 36, 128, 256, 256, True), ("float16", 8, 400, 400, 256, False), ("float16", 24, 512, 256, 256, True), ("float16", 36, 64, 384, 384, True),
-    ("float16", 16, 192, 256, 384, False), ("float16", 64, 128, 128, 384, True)])
+    ("float16", 16, 192, 256, 384, False), ("float16", 64, 128, 128, 384, True),
+    # and the streaming kernel earlier, whose lead is larger with the operands from memory
+    ("float16", 36, 2300, 256, 128, True), ("float16", 16, 2500, 256, 128, True), ("float16", 16, 3417, 256, 128, False), ("float16", 36, 2400, 256, 256, True),
+    ("float16", 16, 4028, 256, 256, True), ("float16", 16, 5615, 256, 256, False), ("float16", 64, 442, 1024, 256, False), ("float16", 16, 3208, 512, 384, True),
+    ("float16", 64, 1400, 512, 384, False), ("float16", 16, 2041, 1024, 384, False), ("float16", 16, 8138, 384, 384, True), ("float16", 16, 10172, 384, 384, False)])
 def test_plain_batches_on_the_tiles(decide, dtype, matrices, rows, columns, K, taken):
     assert decide("plain", dtype, matrices, rows, columns, K)[0] == str(int(taken))
 
