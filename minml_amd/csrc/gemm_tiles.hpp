@@ -77,8 +77,9 @@ namespace mlhip
 	 * 12.1; 512: 256 channels, 96 rows (864) 10.4 / 10.7, 128 (1152) 11.3 / 11.0; 384: 192 channels, 96 rows (648) 9.0 / 9.4, 160 (1080) 10.6 / 10.5; 768: 384
 	 * channels, 32 rows (432) 10.5 / 11.2, 64 (864) 13.0 / 12.2. Other batches than the 36 of a network gain nothing around the product (alone): 512 bytes,
 	 * 8 x 400 x 400 (1352) 4.5 / 5.0, 100 x 128 x 128 (1600) 4.8 / 5.1, 16 x 400 x 400 (2704) 6.6 / 6.6, 24 x 512 x 256 (3072) 6.8 / 6.2; 768, 16 x 192 x 256 (768) 4.7 / 5.2,
-	 * 64 x 128 x 128 (1024) 5.5 / 5.0. And fp32 rows of 384 bytes and more but 512, for which the small tiles of conv_tiles.hpp stand:
-	 * 192 channels, 32 rows (216) 10.7 / 11.6, 64 (432) 13.8 / 12.2. From 1024 bytes on they stand to two per unit, the most that conv_tiles.hpp gives them, and
+	 * 64 x 128 x 128 (1024) 5.5 / 5.0. And fp32 rows of 384 bytes and more but 512, for which the small tiles of conv_tiles.hpp stand,
+	 * resident at once to one per unit: 192 channels, 32 rows (216) 10.7 / 11.6, 64 (432) 13.8 / 12.2; alone, 8 x 512 x 64 (256) 640 bytes 5.5 / 6.2, 768 5.5 / 6.9, 896 6.3 / 7.5, 8 x 600 x 64 (304)
+	 * 6.5 / 6.2, 6.5 / 6.9, 7.6 / 7.6, to 512 the same, then 8.3 / 6.4, 9.1 / 7.0, 10.0 / 7.7. From 1024 bytes on they stand to two per unit, the most that conv_tiles.hpp gives them, and
 	 * the more K the further they are ahead (alone): 36 x 16 x 256 (288) 8.0 / 8.6, 36 x 16 x 384, 1536 bytes (432) 10.9 / 12.0, 9 x 776 x 56, 2048 bytes
 	 * (450) 13.5 / 14.8, 8 x 64 x 512, 4096 bytes (256) 17.0 / 25.2, 8192 (256) 30.1 / 46.4, 8 x 128 x 512 (512) 41.9 / 46.8, 16384 78.3 / 89.6; above, 36 x 64 x 256 (576, in a
 	 * network) 18.5 / 14.9.
@@ -138,7 +139,7 @@ namespace mlhip
 				fewest = (fp16 || g.k_bytes < 384) ? 0 : 1;
 				break;
 		}
-		if (!fp16 && g.k_bytes >= 1024 && tiles <= 2LL * device_compute_units())
+		if (!fp16 && g.k_bytes >= 384 && g.k_bytes % 128 == 0 && g.k_bytes != 512 && tiles <= (g.k_bytes >= 1024 ? 2LL : 1LL) * device_compute_units())
 			return false;
 		return tiles >= fewest * device_compute_units() && exchanged_bytes(g, element_size) <= (megabytes << 20);
 	}

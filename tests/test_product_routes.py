@@ -54,6 +54,9 @@ def test_tiles_of_128_rows_where_the_matrix_fills_them(decide, kind, matrices, r
     # fp32, long K rows: the small tiles of conv_tiles.hpp up to two 32x32 tiles per compute unit
     ("float32", 36, 16, 256, 256, False), ("float32", 8, 64, 512, 2048, False), ("float32", 8, 128, 512, 4096, False), ("float32", 9, 776, 56, 512, False),
     ("float32", 36, 64, 256, 256, True), ("float32", 8, 256, 512, 1024, True), ("float32", 36, 4096, 256, 256, True),
+    # up to one per unit below that
+    ("float32", 8, 512, 64, 160, False), ("float32", 8, 600, 64, 160, True), ("float32", 8, 512, 64, 192, False), ("float32", 8, 128, 256, 224, False), ("float32", 8, 150, 256, 224, True),
+    ("float32", 8, 512, 64, 144, True), ("float32", 8, 512, 64, 128, True),
     # fp32, 128-byte K rows (32 planes): to 50 MB of A and C, 63 with one column tile
     ("float32", 36, 4096, 64, 32, True), ("float32", 36, 8000, 64, 32, False),
     ("float32", 36, 1616, 128, 32, True), ("float32", 36, 4096, 128, 32, False), ("float32", 36, 1616, 256, 32, False), ("float32", 36, 1024, 256, 32, True),
