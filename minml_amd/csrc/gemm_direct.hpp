@@ -199,7 +199,9 @@ namespace mlhip
 	/*
 	 * Whether this kernel takes a product: the 64 x 64 tiles per compute unit up to which it is not behind the kernel that would take it
 	 * otherwise. Every tile fetches its rows of A and B anew (KB * 128 bytes) where the streaming kernel fetches A once. Single products
-	 * alone; batched ones between a network's transforms, where those that are plain go to gemm_tiles.hpp first. Streaming kernel / this one, and the
+	 * alone; batched ones between a network's transforms. Of both, gemm_tiles.hpp takes its ranges first: plain batches of 256 to 768-byte rows from one or two such tiles
+	 * per unit on, products with bias from 1 to 1.75. What its limits in bytes leave has many tiles and goes on to the streaming kernel; the limits here
+	 * are for the rest: alpha or activations that have no fixed epilogue, columns that are no multiple of 16 bytes, few columns. Streaming kernel / this one, and the
 	 * number of tiles:
 	 *   128-byte rows  single 4: 14400 x 256 (900) 7.2 / 6.8, 20000 x 256 (1252) 7.5 / 7.9; batched 3: 15x15 1280 rows x 36 (720)
 	 *                  17.9 / 17.8, 1536 (864) 19.1 / 19.7; by rows as long as that order is for (with transforms of the same order: 1024 rows of
@@ -211,7 +213,7 @@ namespace mlhip
 	 *                  18.7 / 16.5; batched 7: 15x15 640 rows x 36 (1440) 27.0 / 26.6, 768 (1728) 28.0 / 29.7, 896 (2016) 28.7 / 30.9,
 	 *                  19x19 625 (1440) 31.2 / 29.5, 750 (1728) 32.9 / 31.0, 875 (2016) 34.2 / 34.2
 	 *   768-byte rows  3: 15x15 192 rows x 36 (648) 24.0 / 21.9, 256 (864) 24.3 / 24.8; single products cross at 768 to 1024
-	 *   384-byte rows  every size: the streaming kernel does not take them, and the tile engine, for whose pipeline 3 pieces of K are
+	 *   384-byte rows  whatever gemm_tiles.hpp has left: the streaming kernel does not take them, and the tile engine, for whose pipeline 3 pieces of K are
 	 *                  short, is behind or level throughout (1280 rows x 36 39.4 / 28.9; alone 32768 x 36 391 / 352, single products of
 	 *                  2000 to 92000 tiles 0.55 to 0.95 of its time, below 2000 level)
 	 */

@@ -32,7 +32,8 @@
 
 namespace mlhip
 {
-	/* what the products read once and write: all of A and C */
+	/* what the products read once and write: all of A and C. Limits and figures in MB of 10^6 bytes */
+	constexpr unsigned long long MB = 1000 * 1000;
 	inline unsigned long long exchanged_bytes(const StreamGemmArgs &g, int element_size)
 	{
 		return static_cast<unsigned long long>(g.batch) * g.M * (static_cast<unsigned long long>(g.k_bytes) + static_cast<unsigned long long>(g.N) * element_size);
@@ -57,7 +58,7 @@ namespace mlhip
 	 */
 	inline bool products_meet_in_l2(const StreamGemmArgs &g, int element_size)
 	{
-		return between_transforms(g) && g.M >= 192 && exchanged_bytes(g, element_size) <= (40ULL << 20);
+		return between_transforms(g) && g.M >= 192 && exchanged_bytes(g, element_size) <= 42 * MB;
 	}
 	/*
 	 * And beyond where all of B takes a small part of each L2, while the transforms divide the images like that (matrices_stay_cached in
@@ -68,7 +69,7 @@ namespace mlhip
 	{
 		const unsigned long long b_bytes = static_cast<unsigned long long>(g.batch) * g.N * g.k_bytes;
 		return products_meet_in_l2(g, element_size)
-				|| (between_transforms(g) && g.M >= 8 * static_cast<long long>(g.N) && 2 * b_bytes <= (5ULL << 20) && exchanged_bytes(g, element_size) <= (112ULL << 20));
+				|| (between_transforms(g) && g.M >= 8 * static_cast<long long>(g.N) && 5 * b_bytes <= 13 * MB && exchanged_bytes(g, element_size) <= 117 * MB);
 	}
 	/*
 	 * Whether these tiles take a batch of plain products, by the number of 32x32 tiles and the bytes of A and C (figures as above, other
@@ -83,6 +84,9 @@ namespace mlhip
 	 * the more K the further they are ahead (alone): 36 x 16 x 256 (288) 8.0 / 8.6, 36 x 16 x 384, 1536 bytes (432) 10.9 / 12.0, 9 x 776 x 56, 2048 bytes
 	 * (450) 13.5 / 14.8, 8 x 64 x 512, 4096 bytes (256) 17.0 / 25.2, 8192 (256) 30.1 / 46.4, 8 x 128 x 512 (512) 41.9 / 46.8, 16384 78.3 / 89.6; above, 36 x 64 x 256 (576, in a
 	 * network) 18.5 / 14.9.
+	 * Other K rows have no limit in bytes: what else would take them is behind throughout (other kernel / this one): fp16 36 x 11815 x 64, 576 bytes (299 MB) 72.1 / 60.4, 36 x 16113 x 512,
+	 * 640 (965) 564 / 355, 16 x 5255 x 384, 704 (124) 45.6 / 36.4, 64 x 698 x 1024, 192 (100) 39.0 / 27.6, 36 x 6688 x 512, 384 (339) 137 / 133; fp32 64 x 3512 x 256, 768 (403) 284 /
+	 * 202, 8 x 4741 x 512, 1024 (117) 169 / 92, 36 x 3425 x 384, 1536 (379) 334 / 316, 36 x 7479 x 128 (551) 288 / 235, 4 x 15450 x 1024 (348) 485 / 417, 64 x 4248 x 192, 2048 (766) 529 / 458.
 	 * Not beyond a number of bytes where the streaming kernel, which fetches A once, or for 64 and 128 bytes the kernels that store more at
 	 * a time are level or ahead: fp16 256-byte rows 57 MB 32.2 / 28.8, 75 35.3 / 33.7, but with three calls per layer 23.6 / 24.0 and 94 MB 28.3 / 29.5; 512: 94 MB 53.3 / 53.3, 113 59.1 / 61.4, 302 127 / 143; 768, of
 	 * which the streaming kernel holds only 128 columns (whole networks of 8 blocks, 384 channels): 239 MB 2352 / 2083, 292 2706 / 2499, but with three
@@ -105,35 +109,35 @@ namespace mlhip
 			return false;
 		const long long tiles = static_cast<long long>(ceil_div(g.M, 32)) * ceil_div(g.N, 32) * g.batch;
 		long long fewest = 0; /* 32x32 tiles per compute unit */
-		unsigned long long megabytes = ~0ULL >> 20; /* most of A and C together */
+		unsigned long long megabytes = ~0ULL / MB; /* most of A and C together */
 		switch (g.k_bytes)
 		{
 			case 64:
-				megabytes = 270;
+				megabytes = 283;
 				break;
 			case 128:
-				megabytes = (g.N <= 64) ? 60 : 48;
+				megabytes = (g.N <= 64) ? 63 : 50;
 				break;
 			case 256:
 				fewest = fp16 ? 8 : 0;
 				if (fp16)
-					megabytes = between ? 64 : 32;
+					megabytes = between ? 67 : 34;
 				else if (g.N > 64 && 8 * (ceil_div(g.N, 128) * 128LL - g.N) <= g.N)
-					megabytes = 256;
+					megabytes = 268;
 				break;
 			case 384:
 				fewest = fp16 ? 4 : 1;
 				break;
 			case 512:
 				fewest = fp16 ? (between ? 4 : 8) : 0;
-				megabytes = fp16 ? (between ? 90 : 64) : 200;
+				megabytes = fp16 ? (between ? 94 : 67) : 210;
 				break;
 			case 768:
 				fewest = fp16 ? (between ? 3 : 4) : 1;
 				if (fp16 && (ceil_div(g.N, 64) % 3 == 0 || ceil_div(g.N, 64) % 5 == 0) && g.N <= 1024)
-					megabytes = between ? 240 : 200;
+					megabytes = between ? 252 : 210;
 				else if (fp16)
-					megabytes = (g.N <= 512) ? (between ? 160 : 100) : (between ? 100 : 80);
+					megabytes = (g.N <= 512) ? (between ? 168 : 105) : (between ? 105 : 84);
 				break;
 			default:
 				fewest = (fp16 || g.k_bytes < 384) ? 0 : 1;
@@ -141,7 +145,7 @@ namespace mlhip
 		}
 		if (!fp16 && g.k_bytes >= 384 && g.k_bytes % 128 == 0 && g.k_bytes != 512 && tiles <= (g.k_bytes >= 1024 ? 2LL : 1LL) * device_compute_units())
 			return false;
-		return tiles >= fewest * device_compute_units() && exchanged_bytes(g, element_size) <= (megabytes << 20);
+		return tiles >= fewest * device_compute_units() && exchanged_bytes(g, element_size) <= megabytes * MB;
 	}
 	/*
 	 * The same for products with bias (+ beta * C), linear or ReLU: dense layers, 1x1 convolutions, the experts' layers. Alone, other kernel / this one, us, and
@@ -192,8 +196,8 @@ namespace mlhip
 		const unsigned long long bytes = exchanged_bytes(g, element_size) + (reads_c ? static_cast<unsigned long long>(g.batch) * g.M * g.N * element_size : 0);
 		if ((g.k_bytes == 384 && g.N < 64) || (streams && g.N <= 32 && 2 * tiles < 7 * units))
 			return false;
-		const unsigned long long megabytes = (g.N <= 128 && g.k_bytes > 256) ? 180 : reads_c ? 96 : g.k_bytes == 256 ? 32 : g.k_bytes == 512 ? 44 : 64;
-		return 4 * tiles >= (g.k_bytes <= 512 ? 7 : g.k_bytes <= 768 ? 4 : 2) * units && !(streams && bytes > (megabytes << 20));
+		const unsigned long long megabytes = (g.N <= 128 && g.k_bytes > 256) ? 189 : reads_c ? 101 : g.k_bytes == 256 ? 34 : g.k_bytes == 512 ? 46 : 67;
+		return 4 * tiles >= (g.k_bytes <= 512 ? 7 : g.k_bytes <= 768 ? 4 : 2) * units && !(streams && bytes > megabytes * MB);
 	}
 	/* rows x columns of the tile that a workgroup owns */
 	enum class GemmTile

@@ -162,8 +162,8 @@ namespace
 
 	/*
 	 * Whether what a transform reads and writes stays in the last-level cache (256 MB) between the launches of a network: both sets of matrices
-	 * within 112 MB, which leaves room for the activations and weights beside them. Then nothing is marked non-temporal, and every XCD transforms one contiguous
-	 * eighth of the images, the rows that the product's tiles by rows read and write through the same L2 (gemm_tiles.hpp); beyond, the products
+	 * within 117 MB, which leaves room for the activations and weights beside them. Then the output transform and the fused one mark nothing non-temporal (the
+	 * input transform's stores keep the hint: below), and every XCD transforms one contiguous eighth of the images, the rows that the product's tiles by rows read and write through the same L2 (gemm_tiles.hpp); beyond, the products
 	 * stream and the orders and hints beside the kernels below are ahead. Fused transform + product, us, images round the XCDs and non-temporal /
 	 * contiguous / contiguous and cached: fp16 128 channels 500 rows of 19x19 18.6 / 15.5 / 15.6, 1275 26.7 / 24.4 / 22.9; 256 channels 15x15 128 rows 13.2 / 12.2 /
 	 * 12.2, 640 23.9 / 22.9 / 22.9, 1616 37.3 / 37.1 / 35.9, 3072 (113 MB) 60.4 / 59.5 / 58.4, 4096 (151 MB) 72.0 / 72.0 / 75.5; with the streaming product 8192
@@ -171,7 +171,7 @@ namespace
 	 */
 	inline bool matrices_stay_cached(size_t tiles, int channels, size_t element_size)
 	{
-		return 2 * 36 * tiles * channels * element_size <= (static_cast<size_t>(112) << 20);
+		return 2 * 36 * tiles * channels * element_size <= static_cast<size_t>(117) * 1000 * 1000;
 	}
 
 	/*
