@@ -99,6 +99,15 @@ def timed_passes(ctx, forward, steps, warmup):
     ctx.synchronize()
     return (time.perf_counter() - t0) / steps
 
+
+def winograd_product_kernel(tiles, channels, esize):
+    """which kernel gemm.hip runs for a network's 36 products of many rows (the limits of gemm_tiles.hpp; below about 100 rows of tiles fp16 takes
+    kernel_gemm_direct_nt)"""
+    megabytes = 2 * 36 * tiles * channels * esize / 1e6
+    streams_from = {2: {64: 0, 128: 67, 256: 94, 384: 252}, 4: {128: 210}}[esize].get(channels, float("inf"))
+    return "kernel_gemm_stream_wide_nt" if megabytes > streams_from else "kernel_gemm_tiles_nt"
+
+
 def measured_gemm_traffic_bytes(config):
     """HBM bytes of one launch of the block-convolution GEMM kernel, from rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE (two runs, each counter
     scaled by its reading for a 256 MiB copy kernel in the same run), as recorded in profiles/hbm_traffic_<config>.md together with the
@@ -577,7 +586,7 @@ def main():
         if n_t:
             transforms["%s@%s" % (entry, label)] = {"kernel": kernel, "launches_timed": n_t, "avg_launch_us": t_t * 1e6, "algorithmic_bytes": nbytes,
                                                    "gbs": nbytes / t_t / 1e9, "frac_hbm": nbytes / t_t / 1e9 / PEAK_HBM_GBS}
-    kernel_name = "kernel_gemm_stream_wide_nt" if channels * esize in (128, 256, 512) else "kernel_gemm_dma"
+    kernel_name = winograd_product_kernel(tiles, channels, esize)
     # the roofline that bounds the dominant kernel: whichever of its algorithmic bytes and flops takes longer at the chip's peaks
     hbm_bound = gemm_bytes / (PEAK_HBM_GBS * 1e9) >= gemm_flops / (PEAK_MFMA_TFLOPS[dtype] * 1e12)
     if hbm_bound:
