@@ -414,11 +414,21 @@ namespace mlhip
 		return true;
 	}
 	/*
-	 * Convolutions whose 128-byte pieces straddle taps. The register-staged 128 x 128 tiles (gemm_core.hpp) remain for K of at most 512
-	 * bytes and many tiles, where storing is most of the work and the wider tile reads its input once per 128 columns (int8, 32 -> 256
-	 * channels 3x3, 230400 pixels: 88 against 94 us; 14400 pixels: 12.6 against 9.4), and beyond 2^32 threads of these tiles, the most
-	 * that a launch can have: theirs are a quarter as many.
+	 * Convolutions whose 128-byte pieces straddle taps. The register-staged 128 x 128 tiles (gemm_core.hpp) remain for pixels of 16 bytes of int8, more than 64
+	 * columns and more than 8 tiles per unit, where storing is most of the work and the wider tile gathers every pixel, which one 16-byte load per tap is, once per
+	 * 128 columns; and beyond 2^32 threads of these tiles, the most that a launch can have: theirs are a quarter as many. us, these / register-staged:
+	 *   int8 3x3 without residual, 16 -> 128 channels: 115200 pixels (1800 tiles) 20.2 / 20.5, 159975 (2500) 24.2 / 23.0; 16 -> 256: 79875 (2500) 24.4 / 23.0, 230400 (7200)
+	 *   60.5 / 55.3 (with residual 75.7 / 68.7, from memory 83.2 / 90.3); 5x5 16 -> 256: 230400 82.2 / 75.7; but 16 -> 64: 230400 20.2 / 27.9; 32 -> 256: 39825 14.6 / 16.8, 79875 25.4 /
+	 *   27.0, 230400 63.8 / 65.6 (with residual from memory 90.1 / 101.0); 48 -> 256: 230400 72.4 / 76.3
+	 *   fp16 3x3, 8 -> 64: 230400 20.2 / 33.9; 8 -> 256: 39825 15.2 / 18.1, 460800 111 / 133; 24 -> 256: 230400 70.7 / 90.4; fp32 4 -> 256: 39825 24.2 / 25.4, 460800 208 / 227;
+	 *   12 -> 128: 230400 89 / 98; with residual 1.2 to 2.1 times as long throughout
 	 */
+	inline bool stays_register_staged(const ConvTileArgs &g, int element_size)
+	{
+		const long long tiles = tiles_of(g, 128, 64);
+		return (element_size == 1 && g.c_bytes <= 16 && g.k_bytes <= 512 && g.N > 64 && tiles > 8LL * device_compute_units())
+				|| tiles * 64 * ConvTile128x64::WAVES > 0xffffffffLL;
+	}
 	template<typename T, typename Epilogue>
 	inline bool try_launch_straddling(hipStream_t stream, const ConvTileArgs &g, const Epilogue &epilogue)
 	{
@@ -426,8 +436,7 @@ namespace mlhip
 			return false;
 		if (try_launch_small_tiles<T>(stream, g, epilogue))
 			return true;
-		const long long tiles = tiles_of(g, 128, 64);
-		if ((g.k_bytes <= 512 && tiles > 4LL * device_compute_units()) || tiles * 64 * ConvTile128x64::WAVES > 0xffffffffLL)
+		if (stays_register_staged(g, sizeof(T)))
 			return false;
 		launch_conv_tiles_as<T, ConvTile128x64, false>(stream, g, epilogue);
 		return true;

@@ -241,8 +241,8 @@ namespace
 			const uint32_t z = static_cast<uint32_t>(input_zero) & 0xffu;
 			a_loader.fill = z | (z << 8) | (z << 16) | (z << 24);
 			const int tiles_m = ceil_div(M, Cfg::BM), tiles_n = ceil_div(filters_out, Cfg::BN);
-			/* with so short a K the epilogue is most of the work: its common cases are fixed at compile time (the stem of the int8 network, 32 -> 256
-			 * channels 3x3, 230400 pixels: 93 -> 72 us) */
+			/* with so short a K the epilogue is most of the work: its common cases are fixed at compile time (32 -> 256 channels 3x3, 230400 pixels:
+			 * 93 -> 72 us) */
 			specialise_epilogue(ep, [&](const auto &fixed)
 			{
 				typedef typename std::decay<decltype(fixed)>::type Fixed;

@@ -4,7 +4,9 @@
  *   dense ...                                                                "<tiles 0|1> 0 <direct kernel 0|1> <tile>"   (bias, no C)
  *   residual ...                                                             the same with C
  *   experts ...                                                              as dense, with the matrices' rows side by side
+ *   straddling <element size> <bytes of a pixel> <pixels> <columns> <bytes of a K row>      "<register-staged 0|1>"
  */
+#include "conv_tiles.hpp"
 #include "gemm_direct.hpp"
 
 #include <cstdio>
@@ -25,6 +27,16 @@ int main()
 	mlhip::StreamGemmArgs g { };
 	while (std::scanf("%15s %d %d %d %d %d", kind, &element_size, &g.batch, &g.M, &g.N, &g.k_bytes) == 6)
 	{
+		if (std::strcmp(kind, "straddling") == 0)
+		{
+			mlhip::ConvTileArgs c { };
+			c.c_bytes = g.batch;
+			c.M = g.M;
+			c.N = g.N;
+			c.k_bytes = g.k_bytes;
+			std::printf("%d\n", mlhip::stays_register_staged(c, element_size));
+			continue;
+		}
 		const bool plain = std::strcmp(kind, "plain") == 0;
 		g.a_row_bytes = (std::strcmp(kind, "experts") == 0) ? static_cast<size_t>(g.batch) * g.k_bytes : 0;
 		const mlhip::GemmTile tile = plain ? mlhip::tile_of_plain(g, element_size) : mlhip::tile_with_epilogue(g, element_size);

@@ -115,10 +115,10 @@ def test_int8_convolution_of_few_positions(ctx, shape, cout, k):
             assert mismatches(dy.copyToHost(ctx), want) == 0
 
 
-@pytest.mark.parametrize("shape,cout", [((203, 19, 19, 16), 128), ((131, 19, 19, 32), 202)])
+@pytest.mark.parametrize("shape,cout", [((203, 19, 19, 16), 128), ((131, 19, 19, 32), 202), ((203, 19, 19, 16), 256), ((203, 19, 19, 16), 202)])
 def test_int8_convolution_short_k_many_pixels(ctx, shape, cout):
-    """3x3 with K rows of at most 512 bytes that straddle taps, more than 1024 tiles of 128x64: the register-staged tiles with every form of their
-    epilogue, bit for bit; 202 columns are no multiple of 4."""
+    """3x3 with K rows of at most 512 bytes that straddle taps and many pixels, with every form of the epilogue, bit for bit: 128x64 tiles, and from 2048 of them
+    and 16 channels the register-staged ones; 202 columns are no multiple of 4."""
     b, h, w, cin = shape
     rng = np.random.default_rng(cout)
     x = rng.integers(-128, 128, shape).astype(np.int8)

@@ -8,7 +8,7 @@ import pytest
 from minml_amd.build import CSRC, hipcc
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-SIZE = {"float16": 2, "float32": 4}
+SIZE = {"float16": 2, "float32": 4, "int8": 1}
 
 
 @pytest.fixture(scope="module")
@@ -107,3 +107,12 @@ def test_fp32_experts_on_the_tiles(decide, kind, matrices, rows, columns, K, tak
     (74218, 256, 128, True), (80000, 256, 128, False), (61848, 256, 256, True), (53011, 256, 384, True), (27797, 384, 384, True), (169270, 128, 128, False), (126953, 128, 256, True)])
 def test_dense_layers_with_residual_on_the_tiles(decide, rows, columns, K, taken):
     assert decide("residual", "float16", 1, rows, columns, K)[0] == str(int(taken))
+
+
+@pytest.mark.parametrize("dtype,channels,kernel,pixels,columns,staged", [
+    # 16-byte pixels of int8, more than one column tile and 8 tiles of 128x64 per compute unit; and beyond 2^32 threads of those
+    ("int8", 16, 3, 230400, 256, True), ("int8", 16, 3, 79875, 256, True), ("int8", 16, 3, 39825, 256, False), ("int8", 16, 3, 460800, 64, False),
+    ("int8", 16, 5, 230400, 256, True), ("int8", 32, 3, 230400, 256, False), ("int8", 48, 3, 460800, 128, False), ("float16", 8, 3, 460800, 256, False),
+    ("float16", 16, 3, 115200, 128, False), ("float32", 4, 3, 460800, 256, False), ("float32", 12, 3, 230400, 64, False), ("float16", 8, 3, 1074790400, 65, True)])
+def test_convolutions_with_straddling_pieces(decide, dtype, channels, kernel, pixels, columns, staged):
+    assert decide("straddling", dtype, channels * SIZE[dtype], pixels, columns, kernel * kernel * channels) == [str(int(staged))]
