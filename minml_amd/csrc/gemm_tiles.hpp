@@ -154,8 +154,8 @@ namespace mlhip
 	 *   (516) 5.9 / 5.2), 1 up to 768 bytes (384 x 256: 7200 (452) 11.0 / 6.5; x 384: 2700 (258) 6.2 / 6.0), 0.5 up to 1024, where the 32x32 tiles of
 	 *   conv_tiles.hpp end (512 x 256: 2048 (128) 5.5 / 5.7, from memory 5.2 / 5.9, 2300 (144) 6.9 / 5.8, 2700 (172) 7.0 / 6.0; eight experts 228 rows (128) 5.3 / 5.7, 300
 	 *   (160) 6.5 / 5.8). Longer
-	 *   rows, for which a tile of 256 rows is the better one where there are enough, to 4 per unit (3 with at most 128 columns: eight experts of 768 x 128, 3072 rows 13.4 / 11.5, from
-	 *   memory 17.7 / 17.3, 3584 19.9 / 20.9, of 1024 x 128 15.7 / 13.8 and 20.8 / 20.2, 17.3 / 17.3 and 23.1 / 24.6) and 8192 bytes of K rows per unit (eight experts of 576 to 2048 x 256,
+	 *   rows, for which a tile of 256 rows is the better one where there are enough, to 4 per unit (3 for experts of 2048 bytes and at most 128 columns: eight of 1024 x 128, 3072 rows 15.7 / 13.8, from
+	 *   memory 20.8 / 20.2, 3584 17.3 / 17.3 and 23.1 / 24.6; of 768 x 128 16.1 / 14.0 and 19.9 / 20.9; one of 1024 x 128, 28672 rows 20.9 / 17.0 and 25.6 / 24.6) and 8192 bytes of K rows per unit (eight experts of 576 to 2048 x 256,
 	 *   from L2: 300 rows (160) 1152 bytes 6.9 / 6.2, 2048 9.7 / 8.9, 4096 15.6 / 13.9; 912 (480) 9.4 / 8.0, 13.2 / 10.7, 21.1 / 17.6; 1824 (928) 13.3 / 12.1, 18.5 /
 	 *   17.6, 30.4 / 32.1, from memory 14.3 / 14.5, 21.8 / 22.1, 37.4 / 39.3; 2100 (1056) 14.0 / 14.7, 20.2 / 22.2, 33.6 / 37.1; 3072 bytes 1200 (608) 22.1 / 18.1, 1824 from
 	 *   memory 30.2 / 31.7; single layers of 256 columns, whose other kernel has its epilogue at run time, 1536 bytes 10800 rows (676) 13.6 / 10.6, 14400 (900) 15.7 / 14.1). 1024 with a batch to 8 (512 x 1024: 912 rows (1920) 18.5 / 15.9, 3648 (7296) 43.5 / 46.4).
@@ -190,7 +190,7 @@ namespace mlhip
 		if (g.k_bytes < 192 || (g.k_bytes > 768 && g.k_bytes % 128 == 0 && small_tiles <= 2 * units))
 			return false;
 		if (g.k_bytes > 1024)
-			return g.k_bytes <= 4096 && small_tiles > 2 * units && tiles <= (g.N > 128 ? 4 : 3) * units && tiles * g.k_bytes <= 8192 * units;
+			return g.k_bytes <= 4096 && small_tiles > 2 * units && tiles <= ((g.batch > 1 && g.N <= 128 && g.k_bytes >= 2048) ? 3 : 4) * units && tiles * g.k_bytes <= 8192 * units;
 		if (g.k_bytes > 768 && g.batch > 1 && tiles > 8 * units)
 			return false;
 		const bool streams = g.k_bytes == 256 || g.k_bytes == 512 || g.k_bytes == 768;

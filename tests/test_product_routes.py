@@ -84,7 +84,7 @@ def test_plain_batches_on_the_tiles(decide, dtype, matrices, rows, columns, K, t
     # longer ones: to four 64x64 tiles and 8192 bytes of K rows per unit
     ("float16", 8, 912, 256, 576, True), ("float16", 8, 1824, 256, 768, True), ("float16", 8, 1824, 256, 1024, True), ("float16", 8, 2100, 256, 1024, False),
     ("float16", 8, 1200, 256, 1536, True), ("float16", 8, 1824, 256, 1536, False), ("float16", 8, 912, 256, 2048, True), ("float16", 8, 1200, 256, 2048, False),
-    ("float16", 8, 912, 256, 2080, False), ("float16", 8, 228, 256, 1024, False), ("float16", 8, 3072, 128, 768, True), ("float16", 8, 3584, 128, 768, False),
+    ("float16", 8, 912, 256, 2080, False), ("float16", 8, 228, 256, 1024, False), ("float16", 8, 3072, 128, 1024, True), ("float16", 8, 3584, 128, 1024, False), ("float16", 8, 3584, 128, 768, True), ("float16", 1, 28672, 128, 1024, True),
     # short K rows from memory: the streaming kernel from 34, 46 and 67 MB of A and C on, with at most 128 columns later
     ("float16", 1, 41666, 256, 128, True), ("float16", 1, 52083, 256, 128, False), ("float16", 1, 128906, 128, 128, False), ("float16", 16, 1007, 2048, 128, False),
     ("float16", 1, 39062, 256, 256, True), ("float16", 1, 50781, 256, 256, False), ("float16", 4, 8140, 512, 256, False), ("float16", 1, 169270, 128, 256, True),
