@@ -84,8 +84,11 @@ namespace mlhip
 	 * the more K the further they are ahead (alone): 36 x 16 x 256 (288) 8.0 / 8.6, 36 x 16 x 384, 1536 bytes (432) 10.9 / 12.0, 9 x 776 x 56, 2048 bytes
 	 * (450) 13.5 / 14.8, 8 x 64 x 512, 4096 bytes (256) 17.0 / 25.2, 8192 (256) 30.1 / 46.4, 8 x 128 x 512 (512) 41.9 / 46.8, 16384 78.3 / 89.6; above, 36 x 64 x 256 (576, in a
 	 * network) 18.5 / 14.9.
-	 * Other K rows have no limit in bytes: what else would take them is behind throughout (other kernel / this one): fp16 36 x 11815 x 64, 576 bytes (299 MB) 72.1 / 60.4, 36 x 16113 x 512,
-	 * 640 (965) 564 / 355, 16 x 5255 x 384, 704 (124) 45.6 / 36.4, 64 x 698 x 1024, 192 (100) 39.0 / 27.6, 36 x 6688 x 512, 384 (339) 137 / 133; fp32 64 x 3512 x 256, 768 (403) 284 /
+	 * fp16 rows of one, two or three pieces and a half beyond 252 MB only with one or three column tiles (this one's time over the other's, 36 matrices): 192 bytes 256 columns 200 MB 0.88, 300 1.06, 700 1.06,
+	 * 128 columns 0.76, 1.08, 1.06, 384 columns 0.79, 0.97, 0.99, 64 0.73, 0.79, 0.81; 320 bytes 256 columns 0.86, 1.06, 1.07, 512 0.90, 1.02, 1.04, 384 0.79, 0.94, 0.88; 448 bytes 256 columns 0.87,
+	 * 1.02, 1.03, 512 0.91, 1.04, 1.02, 128 0.84, 0.96, 0.98.
+	 * Other K rows have no limit in bytes: what else would take them is behind throughout (other kernel / this one): fp16 36 x 11815 x 64, 576 bytes (299 MB) 72.1 / 60.4, 36 x 17871 x 256 (700)
+	 * 236 / 209, 36 x 16113 x 512, 640 (965) 564 / 355, 36 x 15990 x 256, 704 (700) 242 / 212, 36 x 21701 x 256, 384 (700) 260 / 210; fp32 64 x 3512 x 256, 768 (403) 284 /
 	 * 202, 8 x 4741 x 512, 1024 (117) 169 / 92, 36 x 3425 x 384, 1536 (379) 334 / 316, 36 x 7479 x 128 (551) 288 / 235, 4 x 15450 x 1024 (348) 485 / 417, 64 x 4248 x 192, 2048 (766) 529 / 458.
 	 * Not beyond a number of bytes where the streaming kernel, which fetches A once, or for 64 and 128 bytes the kernels that store more at
 	 * a time are level or ahead: fp16 256-byte rows 57 MB 32.2 / 28.8, 75 35.3 / 33.7, but with three calls per layer 23.6 / 24.0 and 94 MB 28.3 / 29.5; 512: 94 MB 53.3 / 53.3, 113 59.1 / 61.4, 302 127 / 143; 768, of
@@ -138,6 +141,13 @@ namespace mlhip
 					megabytes = between ? 252 : 210;
 				else if (fp16)
 					megabytes = (g.N <= 512) ? (between ? 168 : 105) : (between ? 105 : 84);
+				break;
+			case 192:
+			case 320:
+			case 448:
+				fewest = (fp16 || g.k_bytes < 384) ? 0 : 1;
+				if (fp16 && g.N > 64 && ceil_div(g.N, 64) % 3 != 0)
+					megabytes = 252;
 				break;
 			default:
 				fewest = (fp16 || g.k_bytes < 384) ? 0 : 1;

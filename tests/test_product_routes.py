@@ -63,6 +63,10 @@ def test_tiles_of_128_rows_where_the_matrix_fills_them(decide, kind, matrices, r
     # wide columns that fill the streaming kernel's slices: 768-byte fp16 rows of a network's batch to 168 or 105 MB, 256-byte fp32 rows to 268 MB; other widths further
     ("float16", 64, 1024, 1024, 384, False), ("float16", 64, 800, 1024, 384, False), ("float16", 64, 450, 1024, 384, True), ("float16", 36, 2400, 512, 384, True), ("float16", 36, 4300, 384, 384, True), ("float16", 36, 3300, 640, 384, True),
     ("float16", 36, 4300, 256, 384, False), ("float32", 64, 1024, 1024, 64, False), ("float32", 36, 16384, 64, 64, True), ("float32", 36, 9000, 192, 64, True),
+    # fp16 rows of one to three pieces and a half: to 252 MB, with one or three column tiles at any size; other lengths at any size
+    ("float16", 36, 7891, 256, 96, True), ("float16", 36, 11837, 256, 96, False), ("float16", 36, 10016, 256, 160, False), ("float16", 64, 11505, 256, 160, False),
+    ("float16", 36, 8491, 512, 224, False), ("float16", 36, 43402, 64, 160, True), ("float16", 36, 17871, 384, 160, True), ("float16", 36, 21701, 256, 192, True),
+    ("float16", 36, 17871, 256, 288, True), ("float32", 16, 20000, 256, 80, True),
     # few tiles: the direct kernel further in batches that are not between transforms
     ("float16", 36, 128, 256, 256, True), ("float16", 8, 400, 400, 256, False), ("float16", 24, 512, 256, 256, True), ("float16", 36, 64, 384, 384, True),
     ("float16", 16, 192, 256, 384, False), ("float16", 64, 128, 128, 384, True),
