@@ -270,6 +270,41 @@ namespace mlhip
 		return (id % XCDS) * (full / XCDS) + id / XCDS;
 	}
 	/*
+	 * The tiles of a launch of many matrices, the column tiles of one row tile (or, by_columns, the row tiles of one column tile) next to one another on one XCD and
+	 * the matrix changing slowest or, by_rows, faster than the rows. A launch of few positions is a few microseconds long and its first loads wait for these numbers, so
+	 * what divides them is prepared on the host: two divisions by run-time values are about 60 dependent scalar instructions.
+	 */
+	struct TileOrder
+	{
+			FastDivisor inner, outer;
+			uint32_t tiles;
+			enum Kind : uint32_t
+			{
+				ROWS_INNERMOST, /* matrix, column tile, row tile */
+				COLUMNS_INNERMOST, /* matrix, row tile, column tile */
+				MATRICES_BETWEEN /* row tile, matrix, column tile */
+			} kind;
+			struct Tile
+			{
+					uint32_t matrix, row, column;
+			};
+			__device__ __forceinline__ Tile tile_of(uint32_t block) const
+			{
+				const uint32_t full = tiles & ~7u;
+				const uint32_t id = (block < full) ? (block & 7u) * (full >> 3) + (block >> 3) : block;
+				uint32_t innermost, middle;
+				const uint32_t slowest = fast_divide(fast_divide(id, inner, innermost), outer, middle);
+				return Tile { (kind == MATRICES_BETWEEN) ? middle : slowest, (kind == ROWS_INNERMOST) ? innermost : (kind == COLUMNS_INNERMOST) ? middle : slowest,
+						(kind == ROWS_INNERMOST) ? middle : innermost };
+			}
+	};
+	inline TileOrder make_tile_order(TileOrder::Kind kind, uint32_t tiles_m, uint32_t tiles_n, uint32_t matrices)
+	{
+		return TileOrder { make_fast_divisor(kind == TileOrder::ROWS_INNERMOST ? tiles_m : tiles_n),
+				make_fast_divisor(kind == TileOrder::ROWS_INNERMOST ? tiles_n : kind == TileOrder::COLUMNS_INNERMOST ? tiles_m : matrices), tiles_m * tiles_n * matrices, kind };
+	}
+
+	/*
 	 * The other way to keep neighbouring work in one L2: runs of `run` consecutive logical ids go to one XCD, and the runs go round
 	 * the 8 XCDs, so that the whole chip works on one dense window of the logical range at any moment. Ids beyond the last whole
 	 * group of 8 runs keep their value.

@@ -14,6 +14,10 @@
  * loads in flight: 4 wavefronts of 32 x 32 take 7.05 instead of 6.66 us at 256 rows), and 32 x 32 by 4 wavefronts of 16 x 16 where
  * 64 x 64 leaves compute units without a tile. Consecutive tiles (same matrix, same columns) lie on one XCD and share its L2.
  *
+ * The first loads wait for the workgroup's tile: its numbers come from divisors prepared on the host (TileOrder), rows of A and B are different loads, so that no
+ * lane chooses between them, and everything else is asked for with one set of scalar loads. 344 -> 193 instructions, 162 -> 90 of them before the first load;
+ * from a workgroup's start until its loads are out 0.9 -> 0.5 us, the launch 2.6 -> 2.2 us (timestamps in the kernel, one 15x15 position of 256 channels).
+ *
  * Measured, 36 products of M rows, 8 launches replayed as one graph, us per launch, streaming kernel (384-byte rows: tile engine) ->
  * this one: 64 -> 64 channels: M = 16 (one 15x15 position) 4.6 -> 3.4, 1024 6.0 -> 5.5; 128 -> 128: 16 6.0 -> 3.4, 512 7.2 -> 5.7;
  * 192 -> 192: 16 4.4 -> 3.5, 256 6.5 -> 5.1, 1024 20.0 -> 11.1, 2048 39.2 -> 20.5, 16384 202 -> 163; 256 -> 256: 16 9.8 -> 4.0,
@@ -31,34 +35,22 @@ namespace mlhip
 {
 	template<int KB, int BLOCKS_M, int BLOCKS_N, int WAVES_M, int WAVES_N, typename Epilogue>
 	__global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void kernel_gemm_direct_nt(const half_t *A, const half_t *B, half_t *C, int M, int N, size_t stride_a,
-			size_t stride_b, size_t stride_c, unsigned int tiles_m, unsigned int tiles_n, unsigned int matrices, int by_rows, size_t a_row_bytes, Epilogue epilogue)
+			size_t stride_b, size_t stride_c, TileOrder order, uint32_t a_row_bytes, Epilogue epilogue)
 	{
 		constexpr bool PLAIN = std::is_same<Epilogue, PlainStore>::value;
 		constexpr int PIECES = KB / 128; /* 128-byte pieces of a K row */
 		constexpr int BM = 16 * BLOCKS_M * WAVES_M, BN = 16 * BLOCKS_N * WAVES_N, WAVES = WAVES_M * WAVES_N;
-		constexpr int ROW_BLOCKS = (BM + BN) / 8, PIECE_LOADS = ROW_BLOCKS / WAVES; /* 8-row blocks of a piece, all and per wavefront */
-		static_assert(KB % 128 == 0 && ROW_BLOCKS % WAVES == 0, "K rows of whole 128-byte pieces, the same number of loads for every wavefront");
-		const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+		constexpr int ROW_BLOCKS = (BM + BN) / 8; /* 8-row blocks of a piece */
+		constexpr int A_LOADS = BM / 8 / WAVES, B_LOADS = BN / 8 / WAVES, PIECE_LOADS = A_LOADS + B_LOADS; /* of them per wavefront */
+		static_assert(KB % 128 == 0 && BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "K rows of whole 128-byte pieces, the same loads for every wavefront");
+		static_assert(WAVES % 2 == 0, "the swizzle of a lane is then the same in all its loads");
+		const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 		const int wave_m = wave / WAVES_N, wave_n = wave % WAVES_N;
 		const int frag_row = lane & 15, quarter = lane >> 4;
 
-		const unsigned int id = xcd_contiguous_block_id(blockIdx.x, gridDim.x);
-		unsigned int matrix;
-		int m_tile, n_tile;
-		if (by_rows)
-		{ /* every XCD has rows of all matrices (gemm_tiles.hpp) */
-			const unsigned int row_tile = id / tiles_n, slow = row_tile / matrices;
-			matrix = row_tile - slow * matrices;
-			m_tile = slow * BM;
-			n_tile = (id - row_tile * tiles_n) * BN;
-		}
-		else
-		{
-			const unsigned int column_tiles = id / tiles_m; /* matrix * tiles_n + n_tile */
-			matrix = column_tiles / tiles_n;
-			m_tile = (id - column_tiles * tiles_m) * BM;
-			n_tile = (column_tiles - matrix * tiles_n) * BN;
-		}
+		const TileOrder::Tile tile = order.tile_of(blockIdx.x);
+		const unsigned int matrix = tile.matrix;
+		const int m_tile = tile.row * BM, n_tile = tile.column * BN;
 		const int m0 = m_tile + wave_m * 16 * BLOCKS_M, n0 = n_tile + wave_n * 16 * BLOCKS_N;
 
 		/* lane l, register r of block (i, j): m = 16 i + l % 16, n = 16 j + 4 (l / 16) + r */
@@ -104,16 +96,19 @@ namespace mlhip
 		extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
 		const uint8_t *a_base = reinterpret_cast<const uint8_t*>(A + matrix * stride_a);
 		const uint8_t *b_base = reinterpret_cast<const uint8_t*>(B + matrix * stride_b);
+		const int sub_row = lane >> 3, chunk = ((lane & 7) ^ ((4 * wave + (sub_row >> 1)) & 7)) * 16;
+		const uint8_t *src[PIECE_LOADS];
 #pragma unroll
-		for (int u = 0; u < PIECES * PIECE_LOADS; u++)
-		{
-			const int block = wave + WAVES * (u % PIECE_LOADS), piece = u / PIECE_LOADS;
-			const int row = block * 8 + (lane >> 3);
-			const int chunk = ((lane & 7) ^ ((row >> 1) & 7)) * 16;
-			const uint8_t *src = (row < BM) ? a_base + static_cast<size_t>(min(m_tile + row, M - 1)) * a_row_bytes
-					: b_base + static_cast<size_t>(min(n_tile + row - BM, N - 1)) * KB;
-			__builtin_amdgcn_global_load_lds((global_ptr_t) (src + piece * 128 + chunk), (lds_ptr_t) (lds + (piece * ROW_BLOCKS + block) * 1024), 16, 0, 0);
-		}
+		for (int u = 0; u < A_LOADS; u++)
+			src[u] = a_base + static_cast<uint64_t>(static_cast<uint32_t>(min(m_tile + (wave + WAVES * u) * 8 + sub_row, M - 1))) * a_row_bytes + chunk;
+#pragma unroll
+		for (int u = 0; u < B_LOADS; u++)
+			src[A_LOADS + u] = b_base + static_cast<uint64_t>(static_cast<uint32_t>(min(n_tile + (wave + WAVES * u) * 8 + sub_row, N - 1))) * KB + chunk;
+#pragma unroll
+		for (int piece = 0; piece < PIECES; piece++)
+#pragma unroll
+			for (int u = 0; u < PIECE_LOADS; u++)
+				__builtin_amdgcn_global_load_lds((global_ptr_t) (src[u] + piece * 128), (lds_ptr_t) (lds + (piece * ROW_BLOCKS + wave + WAVES * u) * 1024), 16, 0, 0);
 		float4_t acc[BLOCKS_M][BLOCKS_N];
 #pragma unroll
 		for (int i = 0; i < BLOCKS_M; i++)
@@ -192,9 +187,10 @@ namespace mlhip
 		auto kernel = kernel_gemm_direct_nt<KB, BLOCKS_M, BLOCKS_N, WAVES_M, WAVES_N, Epilogue>;
 		if (LDS > 64 * 1024)
 			ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), LDS);
-		hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned int>(tiles_m) * tiles_n * g.batch), dim3(64 * WAVES_M * WAVES_N), LDS, stream, reinterpret_cast<const half_t*>(g.A),
-				reinterpret_cast<const half_t*>(g.B), reinterpret_cast<half_t*>(g.C), g.M, g.N, g.stride_a, g.stride_b, g.stride_c, tiles_m, tiles_n, g.batch, products_meet_in_l2(g, sizeof(half_t)),
-				g.a_row_bytes != 0 ? g.a_row_bytes : static_cast<size_t>(KB), epilogue);
+		const TileOrder order = make_tile_order(products_meet_in_l2(g, sizeof(half_t)) ? TileOrder::MATRICES_BETWEEN : TileOrder::ROWS_INNERMOST, tiles_m, tiles_n, g.batch);
+		hipLaunchKernelGGL(kernel, dim3(order.tiles), dim3(64 * WAVES_M * WAVES_N), LDS, stream, reinterpret_cast<const half_t*>(g.A),
+				reinterpret_cast<const half_t*>(g.B), reinterpret_cast<half_t*>(g.C), g.M, g.N, g.stride_a, g.stride_b, g.stride_c, order,
+				g.a_row_bytes != 0 ? static_cast<uint32_t>(g.a_row_bytes) : static_cast<uint32_t>(KB), epilogue);
 	}
 	/*
 	 * Whether this kernel takes a product: the 64 x 64 tiles per compute unit up to which it is not behind the kernel that would take it
@@ -221,6 +217,8 @@ namespace mlhip
 	{
 		const long long tiles = static_cast<long long>(ceil_div(g.M, 64)) * ceil_div(g.N, 64) * g.batch, units = device_compute_units();
 		const bool batched = g.batch > 1;
+		if (g.a_row_bytes > 0xffffffffULL)
+			return false;
 		switch (g.k_bytes)
 		{
 			case 128:
