@@ -19,6 +19,7 @@
 #include "device_utils.hpp"
 #include "gemm_stream.hpp"
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 
@@ -698,7 +699,7 @@ namespace
 	}
 
 	/*
-	 * The same launch for few images. One workgroup per image and 64 channels leaves most of the chip idle there, and it is slow by itself:
+	 * The same launch for few images of fp32 (boards of up to four tiles a row; the form after this one is ahead elsewhere). One workgroup per image and 64 channels leaves most of the chip idle there, and it is slow by itself:
 	 * a compute unit moves about one 64-byte piece per 3 clocks whatever the width of the instruction, so the 36 loads and 36 stores of 16
 	 * tiles x 128 bytes take 7000 clocks, and its four wavefronts issue the arithmetic of 16 tiles back to back (another 10000). Here a
 	 * workgroup owns ONE ROW of tiles of an image (a strip of 4 pixel rows) and 16 channels, one channel per lane. The strip's input
@@ -878,6 +879,232 @@ namespace
 					plane += matrix_stride;
 				}
 			}
+		}
+	}
+
+	/*
+	 * The same launch for few images, one lane per LINE of a tile: 16 channels (two to a lane) of the tiles of one row or of a whole image to a workgroup, a
+	 * wavefront to a tile. A launch over few images takes as long as one lane's chain of instructions, and a lane that owns a tile has 36 loads, 22 one-dimensional
+	 * transforms and 36 stores in it. Here lane (line, channels) of a wavefront loads one COLUMN of the tile's products (6 loads), transforms it, hands the results to the
+	 * wavefront's other lanes through LDS, takes one ROW, finishes the outputs into the workgroup's pixels in LDS (zeros around the image, so that windows are read
+	 * at constant offsets), and after the workgroup's one barrier does the same for the input transform: 6 reads, a column, LDS, a row, 6 stores.
+	 * Where one tile row is all that a workgroup owns, further wavefronts repeat the output transform of the tiles above and below for the one pixel row that the
+	 * windows need of each; neighbours then read one another's product rows and residual, so nothing that is read may be written by the same launch. With whole
+	 * images a workgroup reads and writes its own part only. Results are bit-identical to the other forms (the same expressions).
+	 * Timestamps in the kernel, one 15x15 position of 256 channels: 3.5 us with a lane per tile and channel (0.8 us until 36 loads are out, 0.8 in the output and 1.0 in
+	 * the input transform) against 2.9 us; a chain of such launches costs 1.65 us each for the launch itself. us per layer (transform + product) of
+	 * networks, a lane per tile / this, 15x15, 256 channels: 1 position 8.8 / 8.4, 4 9.7 / 9.3, 8 11.7 / 11.5, 12 13.4 / 12.7, 16 14.5 / 13.7, 32 19.3 / 18.4;
+	 * 128 channels: 1 7.6 / 7.2, 32 11.7 / 11.0; 19x19, 256 channels: 1 10.4 / 8.9, 8 16.4 / 15.3, 32 26.4 / 23.6; 20x20, 128 channels: 64 23.1 / 20.2; 9x9: 64 14.2 / 12.3.
+	 */
+	constexpr int LINES_CHANNELS = 16, LINES_VEC = 2, LINES_MAX_WAVES = 16;
+	template<typename T>
+	struct LinesArgs
+	{
+			const T *matrices;
+			T *next_matrices;
+			const T *ext, *bias;
+			T *output;
+			uint32_t matrix_stride, image_elements; /* elements between two matrices; of one image of the activations */
+			int height, width, channels, tiles_h, tiles_w;
+			int strips; /* tile rows of an image that one workgroup owns: all of them, or one */
+			int waves, contiguous;
+			uint32_t workgroups;
+			FastDivisor by_slices, by_strips, by_tiles_w; /* slices per strip, workgroups per slice of an image, tiles per row */
+	};
+	/* what this wavefront's lanes have written to its own part of LDS is there for its other lanes */
+	__device__ __forceinline__ void wait_lds()
+	{
+		asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+		__builtin_amdgcn_wave_barrier();
+	}
+	template<typename T, int ACT, bool HAS_EXT>
+	__global__ __launch_bounds__(64 * LINES_MAX_WAVES) void kernel_output_input_transform_lines(LinesArgs<T> g)
+	{
+		constexpr int SLICE = LINES_CHANNELS, VEC = LINES_VEC, LANES = SLICE / VEC;
+		typedef typename RawVec<T, VEC>::type raw_t;
+		typedef float line_t __attribute__((ext_vector_type(VEC)));
+		extern __shared__ __attribute__((aligned(16))) uint8_t lds_bytes[];
+		const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+		const int index = lane / LANES, channel = (lane % LANES) * VEC; /* which line of the tile; the lane's channels */
+		const int pitch = 4 * g.tiles_w + 2;
+		float *lines = reinterpret_cast<float*>(lds_bytes) + wave * 36 * SLICE; /* this wavefront's [6][6][SLICE] */
+		T *pixels = reinterpret_cast<T*>(lds_bytes + g.waves * 36 * SLICE * sizeof(float)); /* [4 * strips + 2][pitch][SLICE], zeros outside the image */
+
+		uint32_t lin = blockIdx.x;
+		if (g.contiguous)
+		{
+			const uint32_t full = g.workgroups & ~7u;
+			if (lin < full)
+				lin = (lin & 7u) * (full >> 3) + (lin >> 3);
+		}
+		else
+			lin = xcd_run_block_id(lin, g.workgroups, 4);
+		uint32_t slice, strip_of_image;
+		const uint32_t batch = fast_divide(fast_divide(lin, g.by_slices, slice), g.by_strips, strip_of_image);
+		const int first_strip = strip_of_image * g.strips, tiles = g.tiles_h * g.tiles_w;
+		const T *product = g.matrices + static_cast<size_t>(batch * tiles) * g.channels + slice * SLICE;
+		T *next = g.next_matrices + static_cast<size_t>(batch * tiles) * g.channels + slice * SLICE;
+		const size_t first_pixel = static_cast<size_t>(batch) * g.image_elements + slice * SLICE;
+		const uint32_t in_plane = (index * g.matrix_stride + channel) * sizeof(T);
+
+		const bool above = first_strip > 0, below = first_strip + g.strips < g.tiles_h;
+		/* the zeros around the image: the columns left and right of it, and whole rows above and below */
+		const auto fill_border = [&]() __attribute__((always_inline))
+		{
+			Vec<T, VEC> zero;
+			zero.zero();
+			for (int row = threadIdx.x / LANES; row < 4 * g.strips + 2; row += g.waves * LANES)
+			{
+				zero.store(pixels + row * pitch * SLICE + channel);
+				zero.store(pixels + (row * pitch + pitch - 1) * SLICE + channel);
+			}
+			if (!above)
+				for (int y = threadIdx.x / LANES; y < pitch; y += g.waves * LANES)
+					zero.store(pixels + y * SLICE + channel);
+			if (!below)
+				for (int y = threadIdx.x / LANES; y < pitch; y += g.waves * LANES)
+					zero.store(pixels + ((4 * g.strips + 1) * pitch + y) * SLICE + channel);
+		};
+		/* read in any case and kept as it is until it is needed: a load in a block of its own would be waited for there */
+		const bool has_bias = g.bias != nullptr;
+		raw_t bias;
+
+		/* output transform of the strips' tiles, and of those above and below for the one pixel row that the windows need of each */
+		const int own = g.strips * g.tiles_w, halo_above = above ? g.tiles_w : 0, tasks = own + halo_above + (below ? g.tiles_w : 0);
+#pragma clang loop unroll(disable)
+		for (int task = wave; task < tasks; task += g.waves)
+		{
+			const bool is_own = task < own, is_above = !is_own && task < own + halo_above;
+			/* number of the tile from the first of the strips; halo tiles lie before and behind */
+			const int place = is_own ? task : is_above ? task - own - g.tiles_w : task - halo_above;
+			uint32_t tile_y;
+			const int tile_x = static_cast<int>(fast_divide(place + g.tiles_w, g.by_tiles_w, tile_y)) - 1; /* from the first strip */
+			const T *plane = product + static_cast<size_t>(first_strip * g.tiles_w + place) * g.channels;
+			raw_t raw[6];
+			if (index < 6)
+#pragma unroll
+				for (int row = 0; row < 6; row++)
+				{
+					raw[row] = *reinterpret_cast<const raw_t*>(reinterpret_cast<const uint8_t*>(plane) + in_plane);
+					plane += 6 * static_cast<size_t>(g.matrix_stride);
+				}
+			const int x = 4 * tile_x + (index & 3), x_image = 4 * first_strip + x, y0 = 4 * tile_y; /* of the output row that this lane makes after the column pass */
+			raw_t residual[4];
+			if constexpr (HAS_EXT)
+#pragma unroll
+				for (int col = 0; col < 4; col++)
+				{
+					const uint32_t pixel = min(x_image, g.height - 1) * g.width + min(y0 + col, g.width - 1);
+					residual[col] = *reinterpret_cast<const raw_t*>(g.ext + first_pixel + pixel * static_cast<uint32_t>(g.channels) + channel);
+				}
+			if (task == wave)
+			{
+				bias = *reinterpret_cast<const raw_t*>((has_bias ? g.bias : g.matrices) + slice * SLICE + channel);
+				fill_border();
+			}
+			if (index < 6)
+			{
+				float line[6][VEC], res[4][VEC];
+#pragma unroll
+				for (int row = 0; row < 6; row++)
+#pragma unroll
+					for (int c = 0; c < VEC; c++)
+						line[row][c] = RawVec<T, VEC>::get(raw[row], c);
+				output_transform_1d<VEC>(line, res);
+#pragma unroll
+				for (int row = 0; row < 4; row++)
+					*reinterpret_cast<line_t*>(lines + (row * 6 + index) * SLICE + channel) = line_t { res[row][0], res[row][1] };
+			}
+			wait_lds();
+			if (is_own ? index < 4 : index == (is_above ? 3 : 0))
+			{
+				float line[6][VEC], res[4][VEC];
+#pragma unroll
+				for (int col = 0; col < 6; col++)
+				{
+					const line_t v = *reinterpret_cast<const line_t*>(lines + (index * 6 + col) * SLICE + channel);
+#pragma unroll
+					for (int c = 0; c < VEC; c++)
+						line[col][c] = v[c];
+				}
+				output_transform_1d<VEC>(line, res);
+				const bool row_inside = x_image < g.height;
+				T *in_lds = pixels + ((x + 1) * pitch + 1 + y0) * SLICE + channel;
+				T *y = g.output + first_pixel + static_cast<uint32_t>((x_image * g.width + y0) * g.channels) + channel;
+#pragma unroll
+				for (int col = 0; col < 4; col++)
+				{
+					const bool inside = row_inside && y0 + col < g.width;
+					Vec<T, VEC> out;
+#pragma unroll
+					for (int c = 0; c < VEC; c++)
+					{
+						float t = res[col][c] + (has_bias ? RawVec<T, VEC>::get(bias, c) : 0.0f);
+						if constexpr (HAS_EXT)
+							t = t + RawVec<T, VEC>::get(residual[col], c);
+						if constexpr (ACT == 1)
+							t = fmaxf(t, 0.0f);
+						out.v[c] = inside ? t : 0.0f;
+					}
+					out.store(in_lds + col * SLICE);
+					if (g.output != nullptr && is_own && inside)
+						out.store(y + static_cast<uint32_t>(col * g.channels));
+				}
+			}
+			wait_lds();
+		}
+		__syncthreads();
+
+		/* input transform of the next layer out of the LDS image */
+#pragma clang loop unroll(disable)
+		for (int task = wave; task < own; task += g.waves)
+		{
+			uint32_t tile_y;
+			const int tile_x = fast_divide(task, g.by_tiles_w, tile_y);
+			if (index < 6)
+			{
+				const T *window = pixels + (4 * tile_x * pitch + 4 * static_cast<int>(tile_y) + index) * SLICE + channel;
+				float line[6][VEC], res[6][VEC];
+#pragma unroll
+				for (int row = 0; row < 6; row++)
+				{
+					const raw_t raw = *reinterpret_cast<const raw_t*>(window + row * pitch * SLICE);
+#pragma unroll
+					for (int c = 0; c < VEC; c++)
+						line[row][c] = RawVec<T, VEC>::get(raw, c);
+				}
+				input_transform_1d<VEC>(line, res);
+#pragma unroll
+				for (int row = 0; row < 6; row++)
+					*reinterpret_cast<line_t*>(lines + (row * 6 + index) * SLICE + channel) = line_t { res[row][0], res[row][1] };
+			}
+			wait_lds();
+			if (index < 6)
+			{
+				float line[6][VEC], res[6][VEC];
+#pragma unroll
+				for (int col = 0; col < 6; col++)
+				{
+					const line_t v = *reinterpret_cast<const line_t*>(lines + (index * 6 + col) * SLICE + channel);
+#pragma unroll
+					for (int c = 0; c < VEC; c++)
+						line[col][c] = v[c];
+				}
+				input_transform_1d<VEC>(line, res);
+				T *plane = next + static_cast<size_t>(first_strip * g.tiles_w + task) * g.channels;
+				const uint32_t in_next = (6 * index * g.matrix_stride + channel) * sizeof(T);
+#pragma unroll
+				for (int col = 0; col < 6; col++)
+				{
+					Vec<T, VEC> out;
+#pragma unroll
+					for (int c = 0; c < VEC; c++)
+						out.v[c] = res[col][c];
+					out.store(reinterpret_cast<T*>(reinterpret_cast<uint8_t*>(plane) + in_next));
+					plane += g.matrix_stride;
+				}
+			}
+			wait_lds();
 		}
 	}
 
@@ -1250,13 +1477,7 @@ namespace
 	}
 	/* fused output + next input transform: channels must be a multiple of 64 and 4-element accesses aligned; COMMON_ACT_ONLY / RESIDUAL: what
 	 * the caller has made sure of (activation linear or ReLU; a residual given or not), other forms are not instantiated */
-	enum
-	{
-		RESIDUAL_NEVER = 0,
-		RESIDUAL_ALWAYS = 1,
-		RESIDUAL_OR_NOT = 2
-	};
-	template<typename T, int SLICE, int VEC, int THREADS, bool COMMON_ACT_ONLY, int RESIDUAL>
+	template<typename T, int SLICE, int VEC, int THREADS, bool COMMON_ACT_ONLY, bool RESIDUAL>
 	void launch_output_input(hipStream_t stream, const mlTensor_t &matrices, const mlTensor_t &bias, const mlTensor_t &ext, const mlShape_t &shape, void *output,
 			mlActivationType_t act, mlTensor_t &next)
 	{
@@ -1281,7 +1502,7 @@ namespace
 				ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), static_cast<int>(lds)); \
 			hipLaunchKernelGGL(kernel, grid, block, lds, stream, in, out, b, e, a, nxt, batch, height, width, channels, tiles_h, tiles_w); \
 		} while (0)
-		if constexpr (RESIDUAL != RESIDUAL_NEVER)
+		if constexpr (RESIDUAL)
 		{
 			if (e != nullptr)
 			{
@@ -1293,19 +1514,83 @@ namespace
 					MLHIP_LAUNCH_FUSED(2, true);
 			}
 		}
-		if constexpr (RESIDUAL != RESIDUAL_ALWAYS)
+		if (e == nullptr)
 		{
-			if (e == nullptr)
-			{
-				if (mode == 0)
-					MLHIP_LAUNCH_FUSED(0, false);
-				else if (mode == 1)
-					MLHIP_LAUNCH_FUSED(1, false);
-				else if constexpr (!COMMON_ACT_ONLY)
-					MLHIP_LAUNCH_FUSED(2, false);
-			}
+			if (mode == 0)
+				MLHIP_LAUNCH_FUSED(0, false);
+			else if (mode == 1)
+				MLHIP_LAUNCH_FUSED(1, false);
+			else if constexpr (!COMMON_ACT_ONLY)
+				MLHIP_LAUNCH_FUSED(2, false);
 		}
 #undef MLHIP_LAUNCH_FUSED
+		MLHIP_CHECK(hipGetLastError());
+	}
+	/* one tile row of an image to a workgroup, or all of them */
+	struct LinesShape
+	{
+			int strips, waves;
+			size_t lds;
+	};
+	inline LinesShape lines_shape(int height, int width, size_t element_size, bool one_strip)
+	{
+		const int tiles_h = ceil_div(height, 4), tiles_w = ceil_div(width, 4);
+		LinesShape r;
+		r.strips = one_strip ? 1 : tiles_h;
+		r.waves = std::min(LINES_MAX_WAVES, (one_strip ? std::min(3, tiles_h) : tiles_h) * tiles_w);
+		r.lds = static_cast<size_t>(r.waves) * 36 * LINES_CHANNELS * sizeof(float) + static_cast<size_t>(4 * r.strips + 2) * (4 * tiles_w + 2) * LINES_CHANNELS * element_size;
+		return r;
+	}
+	/* linear or ReLU activation; one_strip: nothing the launch reads may overlap what it writes */
+	template<typename T>
+	void launch_output_input_lines(hipStream_t stream, const mlTensor_t &matrices, const mlTensor_t &bias, const mlTensor_t &ext, const mlShape_t &shape,
+			void *output, mlActivationType_t act, mlTensor_t &next, bool one_strip)
+	{
+		const int batch = shape.dim[0], height = shape.dim[1], width = shape.dim[2], channels = shape.dim[3];
+		const LinesShape form = lines_shape(height, width, sizeof(T), one_strip);
+		LinesArgs<T> g;
+		g.matrices = ptr<const T>(matrices);
+		g.next_matrices = ptr<T>(next);
+		g.ext = ptr<const T>(ext);
+		g.bias = ptr<const T>(bias);
+		g.output = reinterpret_cast<T*>(output);
+		g.height = height;
+		g.width = width;
+		g.channels = channels;
+		g.tiles_h = ceil_div(height, 4);
+		g.tiles_w = ceil_div(width, 4);
+		g.matrix_stride = static_cast<uint32_t>(batch * g.tiles_h * g.tiles_w * channels);
+		g.image_elements = static_cast<uint32_t>(height * width * channels);
+		g.strips = form.strips;
+		g.waves = form.waves;
+		g.contiguous = batch >= 4;
+		g.by_slices = make_fast_divisor(channels / LINES_CHANNELS);
+		g.by_strips = make_fast_divisor(g.tiles_h / form.strips);
+		g.by_tiles_w = make_fast_divisor(g.tiles_w);
+		g.workgroups = static_cast<uint32_t>(batch) * (g.tiles_h / form.strips) * (channels / LINES_CHANNELS);
+		const bool relu = (act == ACTIVATION_RELU);
+#define MLHIP_LAUNCH_LINES(ACT, EXT) \
+		do { \
+			auto kernel = kernel_output_input_transform_lines<T, ACT, EXT>; \
+			if (form.lds > 64 * 1024) \
+				ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), static_cast<int>(form.lds)); \
+			hipLaunchKernelGGL(kernel, dim3(g.workgroups), dim3(64 * form.waves), form.lds, stream, g); \
+		} while (0)
+		if (g.ext != nullptr)
+		{
+			if (relu)
+				MLHIP_LAUNCH_LINES(1, true);
+			else
+				MLHIP_LAUNCH_LINES(0, true);
+		}
+		else
+		{
+			if (relu)
+				MLHIP_LAUNCH_LINES(1, false);
+			else
+				MLHIP_LAUNCH_LINES(0, false);
+		}
+#undef MLHIP_LAUNCH_LINES
 		MLHIP_CHECK(hipGetLastError());
 	}
 	/* linear or ReLU activation; nothing the launch reads may overlap what it writes */
@@ -1582,8 +1867,14 @@ extern "C"
 		 *         32 channels              23.2 / 28.3  22.6 / 30.6  27.1 / 35.0  28.0 / 35.7  37.7 / 46.5  51.0 / 60.3  64.5 / 75.2  76.1 / 87.6
 		 *         16 channels              22.9 / 23.5  22.9 / 23.5  27.1 / 28.2  28.5 / 30.0  38.5 / 40.1  52.0 / 55.0  65.8 / 70.1  78.5 / 83.3
 		 *         strips of 16 channels    20.7 / 21.0  20.8 / 21.7  25.5 / 26.8  26.9 / 28.2  37.7 / 40.1  51.0 / 55.0  65.1 / 70.1  77.7 / 83.3
-		 * A launch over few images is bound by what one workgroup must issue, a launch over many by memory, which wants whole 128-byte lines.
-		 * Strips to 85 slices in fp16 (at 96, 64 to 384 channels, -2 to +5 %) and to 96 in fp32 (-2 to -9 %; behind at 128): their repeated rows
+		 * A launch over few images is bound by what one lane must issue, a launch over many by memory, which wants whole 128-byte lines.
+		 * Lines, fp16: a tile row to a workgroup while there is one for every compute unit at most (us per layer, a row / an image: 256 channels 15x15 4 images (256) 9.3 / 9.8,
+		 * 8 (512) 11.6 / 11.5, 12 15.0 / 12.7; 128 channels 9x9 16 (384) 8.9 / 8.4; 64 channels 9x9 16 (192) 7.4 / 7.7; 192 channels 20x20 4 (240) 9.6 / 10.9, 8 (480) 13.3 / 13.0),
+		 * images to three per unit (the other forms / this: 256 channels 15x15 48 images (768) 23.6 / 23.2, 64 (1024) 26.2 / 27.7; 192 channels 20x20 64 (768) 28.7 / 27.2;
+		 * 128 channels 12x12 96 (768) 16.4 / 14.8, 9x9 128 (1024) 17.7 / 17.6; 64 channels 9x9 256 (1024) 17.0 / 17.4). fp32 the same for a tile row of more than four tiles
+		 * (strips / lines: 64 channels 19x19 1 image 9.9 / 9.0, 8 11.5 / 10.9, 32 (128 images of 16 channels) 15.0 / 14.6; 192 channels 20x20 1 12.5 / 11.7, 8 20.1 / 19.8), not for
+		 * narrower ones, whose loads of 64 bytes the strips issue as fast (128 channels 15x15 1 10.5 / 10.6, 16 14.7 / 15.2).
+		 * Strips in fp32 to 96 slices (-2 to -9 %; behind at 128): their repeated rows
 		 * come from the L2 of their XCD, which has the neighbouring strips. 32 channels to 320 slices (without residual 4 to 10 % ahead of 64
 		 * there, with residual -7 to +1 %; at 404 -4 to +6 %). With residual the fp32 form of 32 channels keeps 54 registers per lane in scratch
 		 * memory and is not built: 16 channels, 5 to 14 % ahead of 64 at 160 and 192 slices while the matrices stay cached, 20 % behind where
@@ -1608,14 +1899,27 @@ extern "C"
 			const bool strips_fit = static_cast<size_t>(6) * (4 * ceil_div(output_shape.dim[2], 4) + 2) * STRIP_CHANNELS * sizeof(T) <= 64 * 1024;
 			constexpr bool fp32 = sizeof(T) == 4;
 			const bool residual = ext.data != nullptr, cached = matrices_stay_cached(tiles, channels, sizeof(T));
-			if (common_act && separate && strips_fit && (fp32 ? 8 * slices <= 3 * units : 3 * slices <= units))
-				launch_output_input_strips<T>(stream, matrices, bias, ext, output_shape, output, act, next);
-			else if (common_act && (residual || fp32) && 4 * slices <= (residual && fp32 ? (cached ? 3 : 2) : 1) * units)
-				launch_output_input<T, 16, 1, 256, true, fp32 ? RESIDUAL_OR_NOT : RESIDUAL_ALWAYS>(stream, matrices, bias, ext, output_shape, output, act, next);
+			const long long images_of_16 = 4 * slices, rows_of_16 = images_of_16 * ceil_div(output_shape.dim[1], 4);
+			const auto lines_fit = [&](bool one_strip) { return common_act && m_bytes <= 0xffffffffu && lines_shape(output_shape.dim[1], output_shape.dim[2], sizeof(T), one_strip).lds <= 160 * 1024; };
+			const bool narrow = fp32 && output_shape.dim[2] <= 16; /* strips */
+			if (!narrow && separate && rows_of_16 <= units && lines_fit(true))
+				launch_output_input_lines<T>(stream, matrices, bias, ext, output_shape, output, act, next, true);
+			else if (!narrow && images_of_16 <= (fp32 ? 1 : 3) * units && lines_fit(false))
+				launch_output_input_lines<T>(stream, matrices, bias, ext, output_shape, output, act, next, false);
+			else if (fp32 && common_act && separate && strips_fit && 8 * slices <= 3 * units)
+			{
+				if constexpr (fp32)
+					launch_output_input_strips<T>(stream, matrices, bias, ext, output_shape, output, act, next);
+			}
+			else if (fp32 && common_act && 4 * slices <= (residual ? (cached ? 3 : 2) : 1) * units)
+			{
+				if constexpr (fp32)
+					launch_output_input<T, 16, 1, 256, true, true>(stream, matrices, bias, ext, output_shape, output, act, next);
+			}
 			else if (common_act && !(residual && fp32) && 4 * slices <= 5 * units)
-				launch_output_input<T, 32, 2, 256, true, fp32 ? RESIDUAL_NEVER : RESIDUAL_OR_NOT>(stream, matrices, bias, ext, output_shape, output, act, next);
+				launch_output_input<T, 32, 2, 256, true, !fp32>(stream, matrices, bias, ext, output_shape, output, act, next);
 			else
-				launch_output_input<T, 64, 4, 256, false, RESIDUAL_OR_NOT>(stream, matrices, bias, ext, output_shape, output, act, next);
+				launch_output_input<T, 64, 4, 256, false, true>(stream, matrices, bias, ext, output_shape, output, act, next);
 		};
 		if (matrices.dtype == DTYPE_FLOAT16)
 			launch(half_t(0));

@@ -229,6 +229,31 @@ def test_fused_output_input_transform_forms(ctx, dtype, shape):
             de = ml.toDevice(ctx, ext)
 
 
+@pytest.mark.parametrize("dtype", ["float32", "float16"])
+@pytest.mark.parametrize("shape", [(16, 4, 17, 256), (17, 4, 18, 256), (1, 4, 66, 64), (2, 70, 4, 64), (48, 5, 6, 256), (49, 5, 6, 256), (3, 20, 19, 128), (1, 35, 35, 64),
+                                   (20, 18, 17, 64), (64, 3, 20, 64), (65, 3, 20, 64)])
+def test_fused_transform_lines(ctx, dtype, shape):
+    """The form with one lane per line of a tile: a tile row to a workgroup (256 of them at most) and whole images (768; fp32 256), more tiles than
+    wavefronts, boards that end inside a tile, the next matrices written over the product, y over the residual, no bias. Bit for bit against the oracle."""
+    rng = np.random.default_rng(sum(shape))
+    b, h, w, c = shape
+    tiles = b * ((h + 3) // 4) * ((w + 3) // 4)
+    m, bias, ext = random_tensor(rng, (36, tiles, c), dtype), random_tensor(rng, (c,), dtype), random_tensor(rng, shape, dtype)
+    for with_bias, with_ext, keep, in_place in ((True, True, True, False), (False, False, False, False), (True, True, True, True)):
+        if not keep and (h * w + 1) * 64 * (2 if dtype == "float16" else 4) > 160 * 1024:
+            continue  # the entry point's two-kernel route
+        want_y = O.winograd_output_transform(m, shape, bias if with_bias else None, ext if with_ext else None, O.RELU)
+        dm, db, de = ml.toDevice(ctx, m), ml.toDevice(ctx, bias), ml.toDevice(ctx, ext)
+        y = de if in_place else ml.Tensor(shape, dtype)
+        dv = ml.Tensor((36, tiles, c), dtype)
+        dv.setall(ctx, float("nan"))
+        nxt = dm if in_place else dv
+        ml.winogradOutputInputTransform(ctx, (c, 3, 3, c), dm, shape, y if keep else None, db if with_bias else None, de if with_ext else None, O.RELU, nxt)
+        assert mismatches(nxt.copyToHost(ctx), O.winograd_input_transform(want_y)) == 0
+        if keep:
+            assert mismatches(y.copyToHost(ctx), want_y) == 0
+
+
 @pytest.mark.parametrize("dtype,shape", [("float16", (157, 33, 33, 64)), ("float32", (75, 33, 33, 64)), ("float32", (111, 33, 33, 64)), ("float16", (203, 19, 19, 256)),
                                          ("float16", (61, 19, 19, 128))]
                          + [(dtype, (slices, 7, 6, 64)) for dtype in ("float16", "float32") for slices in (85, 86, 96, 97, 192, 193, 320, 321)])
