@@ -257,7 +257,7 @@ namespace
 				const bool windowed = conv_dma_window_applies(c_bytes, filters_out, kernel_h, kernel_w, height, width);
 				specialise_epilogue(make_epilogue(), [&](const auto &ep)
 				{
-					launched = windowed ? try_launch_small_tiles<T, true>(stream, tile_args, ep) : try_launch_fewer_rows<T>(stream, a_loader, b_loader, tile_args, ep);
+					launched = windowed ? try_launch_small_tiles<T, ConvOrder::SLICES>(stream, tile_args, ep) : try_launch_fewer_rows<T>(stream, a_loader, b_loader, tile_args, ep);
 					if (windowed && !launched)
 					{
 						launch_conv_dma_window<T>(stream, input, weights, M, filters_out, height, width, kernel_h, static_cast<int>(c_bytes), 0u, ep);

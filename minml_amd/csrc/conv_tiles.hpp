@@ -126,19 +126,39 @@ namespace mlhip
 			static_assert((DISTANCE - 1) * LOADS <= 63 && LDS_BYTES <= 160 * 1024, "queue depth and LDS");
 	};
 
-	/* SLICES_FIRST: K in the order of gemm_dma_window.hpp (128 bytes of the channels over all taps, then the next 128; c_bytes a multiple of
-	 * 128) instead of tap by tap */
-	template<typename T, typename Cfg, bool SLICES_FIRST, typename Epilogue>
-	__global__ __launch_bounds__(64 * Cfg::WAVES) void kernel_conv_tiles(ConvTileArgs g, unsigned int tiles_n, Epilogue epilogue)
+	/* how a launch walks K */
+	enum class ConvOrder
+	{
+		STRADDLING, /* tap by tap, any channel count of whole 16-byte chunks: the tap of every chunk is a lane's own */
+		TAPS, /* tap by tap, c_bytes a multiple of 128: a piece of K lies in one tap, which is the same for all lanes */
+		SLICES /* the order of gemm_dma_window.hpp: 128 bytes of the channels over all taps, then the next 128; c_bytes a multiple of 128 */
+	};
+	/* what the kernel divides by, prepared on the host */
+	struct ConvTileDivisors
+	{
+			FastDivisor tiles_n, pixels, width;
+			unsigned int tiles;
+	};
+	/*
+	 * A launch over few rows is as long as one wavefront's chain of instructions, so a piece's addresses are few of them: where its tap is the same for all
+	 * lanes, a lane keeps the address of its row's first tap, and a load is an addition of the tap's place and
+	 * a choice between that address and the padding; nothing is divided by run-time values. Timestamps in the kernel, int8, 9 15x15 positions
+	 * of 128 channels, 32 x 32 tiles, per-lane taps / this: until the addresses' parts are there 0.5 us / 0.2, until 12 loads are out 1.2 / 0.6; the network's
+	 * launches 4.9 / 4.2 us, of which a launch without work takes 1.65.
+	 */
+	template<typename T, typename Cfg, ConvOrder ORDER, typename Epilogue>
+	__global__ __launch_bounds__(64 * Cfg::WAVES) void kernel_conv_tiles(ConvTileArgs g, ConvTileDivisors by, Epilogue epilogue)
 	{
 		typedef Mfma16Traits<T> Traits;
 		constexpr int DISTANCE = Cfg::DISTANCE;
+		constexpr bool UNIFORM = ORDER != ConvOrder::STRADDLING;
 		extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
-		const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+		const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 		const int frag_row = lane & 15, quarter = lane >> 4;
-		const unsigned int id = xcd_contiguous_block_id(blockIdx.x, gridDim.x);
-		const unsigned int tile_m = id / tiles_n;
-		const int m_tile = static_cast<int>(tile_m) * Cfg::BM, n_tile = static_cast<int>(id - tile_m * tiles_n) * Cfg::BN;
+		const unsigned int full = by.tiles & ~7u;
+		const unsigned int id = (blockIdx.x < full) ? (blockIdx.x & 7u) * (full >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+		uint32_t column_tile;
+		const int m_tile = static_cast<int>(fast_divide(id, by.tiles_n, column_tile)) * Cfg::BM, n_tile = static_cast<int>(column_tile) * Cfg::BN;
 		const int wave_m = wave / Cfg::WAVES_N, wave_n = wave % Cfg::WAVES_N;
 		const size_t matrix = blockIdx.y;
 		epilogue.D += matrix * g.stride_out;
@@ -149,25 +169,26 @@ namespace mlhip
 				epilogue.bias += matrix * epilogue.bias_batch_stride;
 		}
 
-		/* this lane's rows of the operands, and its place in them: 16 bytes at kb, which lie in tap (i, j) at byte c */
-		const uint8_t *image[Cfg::A_LOADS], *filter[Cfg::B_LOADS];
+		/* this lane's rows of the operands, and its place in them: 16 bytes at kb, which lie in tap (i, j) at byte c (for all lanes alike: of the piece) */
+		const int chunk = ((lane & 7) ^ dma_swizzle(wave * 8 + (lane >> 3))) * 16;
+		const uint8_t *image[Cfg::A_LOADS], *filter[Cfg::B_LOADS]; /* UNIFORM: the address of the chunk in the row's first tap */
 		int row_h[Cfg::A_LOADS], row_w[Cfg::A_LOADS];
 #pragma unroll
 		for (int u = 0; u < Cfg::A_LOADS; u++)
 		{
-			const int m = m_tile + (wave + Cfg::WAVES * u) * 8 + (lane >> 3);
-			const int pixels = g.height * g.width;
-			const int b = min(m, g.M - 1) / pixels;
-			const int rest = min(m, g.M - 1) - b * pixels;
-			row_h[u] = rest / g.width;
-			row_w[u] = rest - row_h[u] * g.width - (g.kernel_w - 1) / 2;
-			row_h[u] -= (g.kernel_h - 1) / 2;
-			image[u] = g.input + matrix * g.stride_input + static_cast<size_t>(b) * pixels * g.pixel_bytes;
+			const int m = min(m_tile + (wave + Cfg::WAVES * u) * 8 + (lane >> 3), g.M - 1);
+			uint32_t rest, w;
+			const uint32_t b = fast_divide(m, by.pixels, rest);
+			row_h[u] = static_cast<int>(fast_divide(rest, by.width, w)) - (g.kernel_h - 1) / 2;
+			row_w[u] = static_cast<int>(w) - (g.kernel_w - 1) / 2;
+			image[u] = g.input + matrix * g.stride_input + static_cast<size_t>(b) * by.pixels.divisor * g.pixel_bytes;
+			if constexpr (UNIFORM)
+				image[u] += static_cast<ptrdiff_t>(row_h[u] * g.width + row_w[u]) * static_cast<ptrdiff_t>(g.pixel_bytes) + chunk;
 		}
 #pragma unroll
 		for (int u = 0; u < Cfg::B_LOADS; u++)
-			filter[u] = g.weights + matrix * g.stride_weights + static_cast<size_t>(min(n_tile + (wave + Cfg::WAVES * u) * 8 + (lane >> 3), g.N - 1)) * g.k_bytes;
-		int kb = ((lane & 7) ^ dma_swizzle(wave * 8 + (lane >> 3))) * 16;
+			filter[u] = g.weights + matrix * g.stride_weights + static_cast<size_t>(min(n_tile + (wave + Cfg::WAVES * u) * 8 + (lane >> 3), g.N - 1)) * g.k_bytes + (UNIFORM ? chunk : 0);
+		int kb = UNIFORM ? 0 : chunk;
 		int tap_i = 0, tap_j = 0, c = kb;
 		const auto settle = [&]()
 		{
@@ -181,20 +202,44 @@ namespace mlhip
 				}
 			}
 		};
-		settle();
+		if constexpr (!UNIFORM)
+			settle();
+		/* UNIFORM: bytes from the first tap to the piece's */
+		ptrdiff_t place = 0;
+		const ptrdiff_t pixel = static_cast<ptrdiff_t>(g.pixel_bytes), next_row = static_cast<ptrdiff_t>(g.width - g.kernel_w) * pixel;
 		const auto next_piece = [&]()
 		{
-			if constexpr (SLICES_FIRST)
+			if constexpr (ORDER == ConvOrder::SLICES)
 			{
 				kb += g.c_bytes;
+				place += pixel;
 				if (++tap_j == g.kernel_w)
 				{
 					tap_j = 0;
+					place += next_row;
 					if (++tap_i == g.kernel_h)
 					{
 						tap_i = 0;
 						kb += 128 - g.k_bytes;
 						c += 128;
+						place = c;
+					}
+				}
+			}
+			else if constexpr (ORDER == ConvOrder::TAPS)
+			{
+				kb += 128;
+				c += 128;
+				place += 128;
+				if (c == g.c_bytes)
+				{
+					c = 0;
+					place += pixel - g.c_bytes;
+					if (++tap_j == g.kernel_w)
+					{
+						tap_j = 0;
+						tap_i++;
+						place += next_row;
 					}
 				}
 			}
@@ -206,35 +251,53 @@ namespace mlhip
 			}
 		};
 		const int steps = (g.k_bytes + Cfg::PIECES * 128 - 1) / (Cfg::PIECES * 128);
+		const uint8_t *const fill = &dma_pad_table.bytes[g.fill][0], *const zeros = &dma_pad_table.bytes[0][0];
 		const auto request = [&](int step)
 		{
 			uint8_t *slot = lds + (step % Cfg::SLOTS) * Cfg::SLOT_BYTES;
 #pragma unroll
 			for (int p = 0; p < Cfg::PIECES; p++)
 			{
-				const bool in_k = SLICES_FIRST ? c < g.c_bytes : kb < g.k_bytes; /* past the end of K both operands read zeros */
-				const uint8_t *padding = &dma_pad_table.bytes[in_k ? g.fill : 0][0];
-#pragma unroll
-				for (int u = 0; u < Cfg::A_LOADS; u++)
+				uint8_t *const a_slot = slot + p * Cfg::PIECE_BYTES + wave * 1024, *const b_slot = a_slot + Cfg::BM * 128;
+				const auto load = [](const uint8_t *src, uint8_t *dst) __attribute__((always_inline))
 				{
-					const int x = row_h[u] + tap_i, y = row_w[u] + tap_j;
-					const bool inside = in_k && static_cast<unsigned int>(x) < static_cast<unsigned int>(g.height)
-							&& static_cast<unsigned int>(y) < static_cast<unsigned int>(g.width);
-					const uint8_t *src = inside ? image[u] + static_cast<size_t>(x * g.width + y) * g.pixel_bytes + c : padding;
-					__builtin_amdgcn_global_load_lds((global_ptr_t) src, (lds_ptr_t) (slot + p * Cfg::PIECE_BYTES + (wave + Cfg::WAVES * u) * 1024), 16, 0, 0);
+					__builtin_amdgcn_global_load_lds((global_ptr_t) src, (lds_ptr_t) dst, 16, 0, 0);
+				};
+				const bool in_k = (ORDER == ConvOrder::SLICES) ? c < g.c_bytes : kb < g.k_bytes;
+				if (!UNIFORM || in_k)
+				{
+#pragma unroll
+					for (int u = 0; u < Cfg::A_LOADS; u++)
+					{
+						const int x = row_h[u] + tap_i, y = row_w[u] + tap_j;
+						const bool inside = static_cast<unsigned int>(x) < static_cast<unsigned int>(g.height)
+								&& static_cast<unsigned int>(y) < static_cast<unsigned int>(g.width);
+						if constexpr (UNIFORM)
+							load(inside ? image[u] + place : fill, a_slot + Cfg::WAVES * u * 1024);
+						else
+							load(!in_k ? zeros : inside ? image[u] + static_cast<size_t>(x * g.width + y) * g.pixel_bytes + c : fill, a_slot + Cfg::WAVES * u * 1024);
+					}
+#pragma unroll
+					for (int u = 0; u < Cfg::B_LOADS; u++)
+						load((UNIFORM || in_k) ? filter[u] + kb : zeros, b_slot + Cfg::WAVES * u * 1024);
 				}
+				else
+				{ /* past the end of K both operands read zeros */
 #pragma unroll
-				for (int u = 0; u < Cfg::B_LOADS; u++)
-				{
-					const uint8_t *src = in_k ? filter[u] + kb : padding;
-					__builtin_amdgcn_global_load_lds((global_ptr_t) src,
-							(lds_ptr_t) (slot + p * Cfg::PIECE_BYTES + Cfg::BM * 128 + (wave + Cfg::WAVES * u) * 1024), 16, 0, 0);
+					for (int u = 0; u < Cfg::A_LOADS; u++)
+						load(zeros, a_slot + Cfg::WAVES * u * 1024);
+#pragma unroll
+					for (int u = 0; u < Cfg::B_LOADS; u++)
+						load(zeros, b_slot + Cfg::WAVES * u * 1024);
 				}
 				next_piece();
 			}
 		};
-		for (int s = 0; s < DISTANCE && s < steps; s++)
-			request(s);
+		static_for<DISTANCE>([&](auto s)
+		{
+			if (decltype(s)::value < steps)
+				request(decltype(s)::value);
+		});
 
 		int a_first[Cfg::BLOCKS_M], b_first[Cfg::BLOCKS_N]; /* this lane's fragment of a piece's first k step, of the others by XOR */
 #pragma unroll
@@ -335,14 +398,15 @@ namespace mlhip
 			}
 	}
 
-	template<typename T, typename Cfg, bool SLICES_FIRST, typename Epilogue>
+	template<typename T, typename Cfg, ConvOrder ORDER, typename Epilogue>
 	inline void launch_conv_tiles_as(hipStream_t stream, const ConvTileArgs &g, const Epilogue &epilogue)
 	{
-		auto kernel = kernel_conv_tiles<T, Cfg, SLICES_FIRST, Epilogue>;
+		auto kernel = kernel_conv_tiles<T, Cfg, ORDER, Epilogue>;
 		ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), Cfg::LDS_BYTES);
 		const int tiles_m = ceil_div(g.M, Cfg::BM), tiles_n = ceil_div(g.N, Cfg::BN);
-		hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned int>(tiles_m) * tiles_n, g.batch), dim3(64 * Cfg::WAVES), Cfg::LDS_BYTES, stream, g,
-				static_cast<unsigned int>(tiles_n), epilogue);
+		const ConvTileDivisors by { make_fast_divisor(tiles_n), make_fast_divisor(static_cast<uint32_t>(g.height) * g.width), make_fast_divisor(g.width),
+				static_cast<unsigned int>(tiles_m) * tiles_n };
+		hipLaunchKernelGGL(kernel, dim3(by.tiles, g.batch), dim3(64 * Cfg::WAVES), Cfg::LDS_BYTES, stream, g, by, epilogue);
 	}
 
 	typedef ConvTileConfig<1, 1, 2, 2, 2, 4> ConvTile32; /* 64 KB of LDS: two workgroups per compute unit */
@@ -369,14 +433,14 @@ namespace mlhip
 	 * chain: 552 tiles of 32 x 32 for 1444 x 384 at K = 6912 take 27.6 us, 138 of 64 x 64 take 21.8; 512 of them for 2025 x 256 take 7.3
 	 * against 9.8; 900 tiles of 64 x 64 for 14400 x 256 at K = 2304 take 25 against 18 us of 128 x 128 tiles, 724 of them level).
 	 */
-	template<typename T, bool SLICES_FIRST = false, typename Epilogue>
+	template<typename T, ConvOrder ORDER = ConvOrder::TAPS, typename Epilogue>
 	inline bool try_launch_small_tiles(hipStream_t stream, const ConvTileArgs &g, const Epilogue &epilogue)
 	{
 		const int units = device_compute_units();
 		if (tiles_of(g, 32, 32) <= 2LL * units)
-			launch_conv_tiles_as<T, ConvTile32, SLICES_FIRST>(stream, g, epilogue);
+			launch_conv_tiles_as<T, ConvTile32, ORDER>(stream, g, epilogue);
 		else if (tiles_of(g, 64, 64) <= 3LL * units)
-			launch_conv_tiles_as<T, ConvTile64, SLICES_FIRST>(stream, g, epilogue);
+			launch_conv_tiles_as<T, ConvTile64, ORDER>(stream, g, epilogue);
 		else
 			return false;
 		return true;
@@ -402,7 +466,7 @@ namespace mlhip
 		{
 			if (tiles_of(g, 256, g.N > 128 ? 256 : g.N > 64 ? 128 : 64) * 4 > units * 3LL)
 				return false;
-			launch_conv_tiles_as<T, ConvTile128x64, false>(stream, g, epilogue);
+			launch_conv_tiles_as<T, ConvTile128x64, ConvOrder::TAPS>(stream, g, epilogue);
 			return true;
 		}
 		if constexpr (sizeof(T) < 4)
@@ -434,11 +498,11 @@ namespace mlhip
 	{
 		if (g.k_bytes == 0) /* as above */
 			return false;
-		if (try_launch_small_tiles<T>(stream, g, epilogue))
+		if (try_launch_small_tiles<T, ConvOrder::STRADDLING>(stream, g, epilogue))
 			return true;
 		if (stays_register_staged(g, sizeof(T)))
 			return false;
-		launch_conv_tiles_as<T, ConvTile128x64, false>(stream, g, epilogue);
+		launch_conv_tiles_as<T, ConvTile128x64, ConvOrder::STRADDLING>(stream, g, epilogue);
 		return true;
 	}
 } /* namespace mlhip */

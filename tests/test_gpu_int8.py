@@ -85,6 +85,23 @@ def test_int8_convolution_bit_exact(ctx, shape, cout, k, act):
         assert mismatches(dy.copyToHost(ctx), want) == 0
 
 
+@pytest.mark.parametrize("shape,cout,k", [((2, 5, 6, 256), 40, 4),  # two pieces to a tap, an even kernel
+                                          ((1, 3, 4, 128), 36, 35),  # taps far beyond the board on every side
+                                          ((1, 6, 5, 384), 33, 2),  # three pieces to a tap, the last slot half empty
+                                          ((41, 9, 9, 256), 200, 2), ((400, 7, 6, 128), 132, 2)])  # 64 x 64 and 256-row tiles
+def test_int8_convolution_taps_of_whole_pieces(ctx, shape, cout, k):
+    """Pieces of K that lie in one tap, whose place is the same for all lanes, against the oracle, bit for bit; the zero point is not 0."""
+    b, h, w, cin = shape
+    rng = np.random.default_rng(cout * k + b)
+    x, wt = rng.integers(-128, 128, shape).astype(np.int8), rng.integers(-127, 128, (cout, k, k, cin)).astype(np.int8)
+    scales, bias = (rng.random(cout) * 0.002 + 0.0005).astype(np.float32), rng.standard_normal(cout).astype(np.float32)
+    want = O.int8_conv2d_forward(x, IN_QD, wt, scales, bias, O.INT8, OUT_QD, None, EXT_QD, O.RELU)
+    dx, dw, ds, db = (ml.toDevice(ctx, a) for a in (x, wt, scales, bias))
+    dy = ml.Tensor((b, h, w, cout), O.INT8)
+    ml.quantizedConvForward(ctx, dx, IN_QD, dw, ds, db, dy, OUT_QD, None, EXT_QD, O.RELU)
+    assert mismatches(dy.copyToHost(ctx), want) == 0
+
+
 @pytest.mark.parametrize("shape,cout,k", [((1, 1, 3, 16), 4, 3),  # one tile, K shorter than a ring slot, taps of one 16-byte chunk
                                           ((1, 11, 3, 32), 33, 3),  # 33 rows and columns: one past the 32 x 32 tile; not a multiple of 4
                                           ((5, 9, 7, 144), 100, 3),  # pieces that straddle taps, K not a whole slot
