@@ -114,23 +114,32 @@ namespace
 		}
 		for (size_t first = (static_cast<size_t>(blockIdx.x) * 4 + (threadIdx.x >> 6)) * UNROLL; first < rows; first += stride)
 		{
-			Vec<T, VEC> x[UNROLL][ITEMS];
+			/* every row is requested before the first is used, from clamped places and kept as it is: a load under a test would be in a block of its own, and waited for there */
+			typedef T raw_t __attribute__((ext_vector_type(VEC)));
+			raw_t raw[UNROLL][ITEMS];
 #pragma unroll
 			for (int u = 0; u < UNROLL; u++)
 			{
-				const T *src = input + (first + u) * columns;
+				const T *src = input + (first + u < rows ? first + u : rows - 1) * columns;
 #pragma unroll
 				for (int i = 0; i < ITEMS; i++)
 				{
 					const int j = (lane + 64 * i) * VEC;
-					x[u][i].zero();
-					if (j < columns && first + u < rows)
-						x[u][i].load(src + j);
+					raw[u][i] = *reinterpret_cast<const raw_t*>(src + (j < columns ? j : 0));
 				}
 			}
+			Vec<T, VEC> x[UNROLL][ITEMS];
 #pragma unroll
 			for (int u = 0; u < UNROLL; u++)
 			{
+#pragma unroll
+				for (int i = 0; i < ITEMS; i++)
+				{
+					const bool inside = (lane + 64 * i) * VEC < columns;
+#pragma unroll
+					for (int e = 0; e < VEC; e++)
+						x[u][i].v[e] = inside ? static_cast<float>(raw[u][i][e]) : 0.0f;
+				}
 				float sum_square = 0.0f;
 #pragma unroll
 				for (int i = 0; i < ITEMS; i++)

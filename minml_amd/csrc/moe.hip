@@ -356,33 +356,53 @@ namespace
 			int channels, FastDivisor by_pieces, FastDivisor by_experts, FastDivisor by_capacity)
 	{
 		const uint32_t experts = by_experts.divisor, capacity = by_capacity.divisor;
-		for (uint64_t g64 = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; g64 < groups; g64 += static_cast<uint64_t>(gridDim.x) * blockDim.x)
+		constexpr int UNROLL = 4;
+		typedef T raw_t __attribute__((ext_vector_type(VEC)));
+		const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
+		for (uint64_t first = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; first < groups; first += UNROLL * stride)
 		{
-			uint32_t piece, e, k;
-			const uint32_t row = fast_divide(static_cast<uint32_t>(g64), by_pieces, piece); /* (b * K + k) * E + e */
-			const uint32_t bk = fast_divide(row, by_experts, e);
-			const uint32_t b = fast_divide(bk, by_capacity, k);
-			const int c = static_cast<int>(piece) * VEC;
-			const int token = static_cast<int>(Storage<T>::load(indices_and_values + (static_cast<size_t>(b * 2u) * experts + e) * capacity + k));
-			Vec<T, VEC> out;
-			out.zero();
-			T *y_piece = y + static_cast<size_t>(row) * channels + c;
-			if constexpr (WITH_BETA)
+			uint32_t row[UNROLL], image[UNROLL];
+			int c[UNROLL];
+			T index[UNROLL];
+#pragma unroll
+			for (int u = 0; u < UNROLL; u++)
 			{
-				out.load(y_piece);
+				uint32_t piece, e, k;
+				const uint64_t g = first + u * stride;
+				row[u] = fast_divide(static_cast<uint32_t>(g < groups ? g : first), by_pieces, piece); /* (b * K + k) * E + e */
+				const uint32_t bk = fast_divide(row[u], by_experts, e);
+				image[u] = fast_divide(bk, by_capacity, k);
+				c[u] = static_cast<int>(piece) * VEC;
+				index[u] = indices_and_values[(static_cast<size_t>(image[u] * 2u) * experts + e) * capacity + k];
+			}
+			raw_t in[UNROLL];
+#pragma unroll
+			for (int u = 0; u < UNROLL; u++)
+			{ /* an empty slot reads the image's first token and drops it */
+				const int token = static_cast<int>(static_cast<float>(index[u]));
+				in[u] = *reinterpret_cast<const raw_t*>(x + (static_cast<size_t>(image[u]) * tokens + (token >= 0 ? token : 0)) * channels + c[u]);
+			}
+#pragma unroll
+			for (int u = 0; u < UNROLL; u++)
+			{
+				if (u > 0 && first + u * stride >= groups)
+					break;
+				const bool filled = static_cast<int>(static_cast<float>(index[u])) >= 0;
+				Vec<T, VEC> out;
+				out.zero();
+				T *y_piece = y + static_cast<size_t>(row[u]) * channels + c[u];
+				if constexpr (WITH_BETA)
+				{
+					out.load(y_piece);
+#pragma unroll
+					for (int i = 0; i < VEC; i++)
+						out.v[i] *= beta;
+				}
 #pragma unroll
 				for (int i = 0; i < VEC; i++)
-					out.v[i] *= beta;
+					out.v[i] = filled ? static_cast<float>(in[u][i]) + out.v[i] : out.v[i];
+				out.store(y_piece);
 			}
-			if (token >= 0)
-			{
-				Vec<T, VEC> in;
-				in.load(x + (static_cast<size_t>(b) * tokens + token) * channels + c);
-#pragma unroll
-				for (int i = 0; i < VEC; i++)
-					out.v[i] = in.v[i] + out.v[i];
-			}
-			out.store(y_piece);
 		}
 	}
 
@@ -547,7 +567,7 @@ namespace
 	}
 	template<typename T, int VEC, bool WITH_BETA>
 	__global__ __launch_bounds__(256) void kernel_scatter_tokens_by_image(const T *x, const T *indices_and_values, T *y, float beta, int tokens, int channels,
-			int experts, int capacity, int splits)
+			int experts, int capacity, int splits, int gates_in_lds)
 	{
 #pragma clang fp contract(off)
 		extern __shared__ int scatter_lds[];
@@ -559,6 +579,7 @@ namespace
 		int *inverse = scatter_lds; /* [per_part][experts] */
 		int *lists = inverse + per_part * experts; /* [per_part][experts][2]: row of the image's expert outputs, gate as fp32 bits */
 		int *count = lists + per_part * experts * 2; /* [per_part] */
+		float *gates = reinterpret_cast<float*>(count + per_part); /* [experts][capacity], where they fit: fetched beside the indexes, not one latency later */
 		const T *index_plane = indices_and_values + (b * 2 + 0) * experts * capacity;
 		const T *gate_plane = indices_and_values + (b * 2 + 1) * experts * capacity;
 		for (int i = threadIdx.x; i < mine * experts; i += blockDim.x)
@@ -566,8 +587,11 @@ namespace
 		__syncthreads();
 		for (int i = threadIdx.x; i < experts * capacity; i += blockDim.x)
 		{
+			const T index = index_plane[i], gate = gate_plane[i];
 			const int e = i / capacity, k = i - e * capacity;
-			const int token = static_cast<int>(Storage<T>::load(index_plane + i)) - first;
+			const int token = static_cast<int>(static_cast<float>(index)) - first;
+			if (gates_in_lds)
+				gates[i] = static_cast<float>(gate);
 			if (token >= 0 && token < mine)
 				atomicMin(&inverse[token * experts + e], k); /* of duplicates in a hand-made table the lowest slot counts */
 		}
@@ -581,7 +605,7 @@ namespace
 				if (slot != SCATTER_NONE)
 				{
 					lists[(t * experts + n) * 2 + 0] = slot * experts + e;
-					lists[(t * experts + n) * 2 + 1] = __builtin_bit_cast(int, Storage<T>::load(gate_plane + e * capacity + slot));
+					lists[(t * experts + n) * 2 + 1] = __builtin_bit_cast(int, gates_in_lds ? gates[e * capacity + slot] : Storage<T>::load(gate_plane + e * capacity + slot));
 					n++;
 				}
 			}
@@ -797,10 +821,10 @@ extern "C"
 				const FastDivisor by_pieces = make_fast_divisor(static_cast<uint32_t>(channels / VEC)), by_experts = make_fast_divisor(static_cast<uint32_t>(experts)), \
 						by_capacity = make_fast_divisor(static_cast<uint32_t>(capacity)); \
 				if (beta != 0.0f) \
-					hipLaunchKernelGGL((kernel_gather_tokens_fast<T, VEC, true>), dim3(grid_for(groups)), dim3(256), 0, stream, ptr<const T>(x), \
+					hipLaunchKernelGGL((kernel_gather_tokens_fast<T, VEC, true>), dim3(grid_for((groups + 3) / 4)), dim3(256), 0, stream, ptr<const T>(x), \
 							ptr<const T>(indices_and_values), ptr<T>(y), beta, static_cast<uint32_t>(groups), tokens, channels, by_pieces, by_experts, by_capacity); \
 				else \
-					hipLaunchKernelGGL((kernel_gather_tokens_fast<T, VEC, false>), dim3(grid_for(groups)), dim3(256), 0, stream, ptr<const T>(x), \
+					hipLaunchKernelGGL((kernel_gather_tokens_fast<T, VEC, false>), dim3(grid_for((groups + 3) / 4)), dim3(256), 0, stream, ptr<const T>(x), \
 							ptr<const T>(indices_and_values), ptr<T>(y), beta, static_cast<uint32_t>(groups), tokens, channels, by_pieces, by_experts, by_capacity); \
 			} \
 			else \
@@ -847,6 +871,8 @@ extern "C"
 		 * one image within reach of a buffer descriptor's 32-bit offsets */
 		const int splits = std::max(1, std::min(8, tokens / 16));
 		const size_t lds_bytes = scatter_by_image_lds_bytes((tokens + splits - 1) / splits, experts);
+		const size_t gate_bytes = static_cast<size_t>(capacity) * experts * sizeof(float);
+		const bool gates_in_lds = lds_bytes + gate_bytes <= 64 * 1024;
 		const size_t image_bytes = static_cast<size_t>(capacity) * experts * channels * size_of(x.dtype);
 		const bool by_image = experts > 0 && capacity > 0 && lds_bytes <= 48 * 1024 && static_cast<size_t>(batch) * splits <= 0x7fffffffu
 				&& image_bytes < 0x40000000u;
@@ -855,11 +881,11 @@ extern "C"
 			if (by_image) \
 			{ \
 				if (beta != 0.0f) \
-					hipLaunchKernelGGL((kernel_scatter_tokens_by_image<T, VEC, true>), dim3(static_cast<unsigned int>(batch) * splits), dim3(256), lds_bytes, \
-							stream, ptr<const T>(x), ptr<const T>(indices_and_values), ptr<T>(y), beta, tokens, channels, experts, capacity, splits); \
+					hipLaunchKernelGGL((kernel_scatter_tokens_by_image<T, VEC, true>), dim3(static_cast<unsigned int>(batch) * splits), dim3(256), lds_bytes + (gates_in_lds ? gate_bytes : 0), \
+							stream, ptr<const T>(x), ptr<const T>(indices_and_values), ptr<T>(y), beta, tokens, channels, experts, capacity, splits, gates_in_lds); \
 				else \
-					hipLaunchKernelGGL((kernel_scatter_tokens_by_image<T, VEC, false>), dim3(static_cast<unsigned int>(batch) * splits), dim3(256), lds_bytes, \
-							stream, ptr<const T>(x), ptr<const T>(indices_and_values), ptr<T>(y), beta, tokens, channels, experts, capacity, splits); \
+					hipLaunchKernelGGL((kernel_scatter_tokens_by_image<T, VEC, false>), dim3(static_cast<unsigned int>(batch) * splits), dim3(256), lds_bytes + (gates_in_lds ? gate_bytes : 0), \
+							stream, ptr<const T>(x), ptr<const T>(indices_and_values), ptr<T>(y), beta, tokens, channels, experts, capacity, splits, gates_in_lds); \
 				break; \
 			} \
 			const size_t wavefronts = total_tokens * ((channels + 64 * VEC - 1) / (64 * VEC)); \
