@@ -26,7 +26,7 @@ namespace
 	/* Epilogue: PlainStore, or a functor on 4 consecutive n whose forms are fixed at compile time (epilogues.hpp) */
 	template<typename T, typename Shape, typename Epilogue>
 	__global__ __launch_bounds__(Shape::THREADS, Shape::RESIDENT * Shape::WAVES / 4) void kernel_gemm_tiles_nt(const T *A, const T *B, T *C, int M, int N, int k_bytes,
-			size_t stride_a, size_t stride_b, size_t stride_c, unsigned int tiles_m, unsigned int tiles_n, unsigned int matrices, int by_rows, size_t a_row_bytes, Epilogue epilogue)
+			size_t stride_a, size_t stride_b, size_t stride_c, unsigned int tiles_m, unsigned int tiles_n, unsigned int matrices, int by_rows, size_t a_row_bytes, int write_through, Epilogue epilogue)
 	{
 		typedef MfmaTraits<T> Traits;
 		typedef typename Traits::acc_vec acc_vec;
@@ -226,7 +226,12 @@ namespace
 				const uint4_t v = *reinterpret_cast<const uint4_t*>(slab + row * Shape::SLAB_STRIDE + col * sizeof(T));
 				const int m = m0 + 32 * i + row;
 				if (m < M && n0 + col < N)
-					*reinterpret_cast<uint4_t*>(out + m * out_stride + n0 + col) = v;
+				{
+					if (PLAIN && write_through)
+						store_through_l2(out + m * out_stride + n0 + col, v);
+					else
+						*reinterpret_cast<uint4_t*>(out + m * out_stride + n0 + col) = v;
+				}
 			}
 			wait_lgkmcnt_zero();
 			__builtin_amdgcn_wave_barrier();
@@ -246,7 +251,7 @@ namespace
 			ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), Shape::LDS_BYTES);
 		hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned int>(tiles)), dim3(Shape::THREADS), Shape::LDS_BYTES, stream, reinterpret_cast<const T*>(g.A),
 				reinterpret_cast<const T*>(g.B), reinterpret_cast<T*>(g.C), g.M, g.N, g.k_bytes, g.stride_a, g.stride_b, g.stride_c, tiles_m, tiles_n, g.batch, by_rows,
-				g.a_row_bytes != 0 ? g.a_row_bytes : static_cast<size_t>(g.k_bytes), epilogue);
+				g.a_row_bytes != 0 ? g.a_row_bytes : static_cast<size_t>(g.k_bytes), products_write_through(g, sizeof(T)), epilogue);
 		return true;
 	}
 	template<typename T>

@@ -248,6 +248,20 @@ namespace mlhip
 		return (!by_rows && g.k_bytes >= 512) ? GemmTile::T128x128 : GemmTile::T128x64;
 	}
 	/*
+	 * Whether the 36 products between transforms write through the L2 (store_through_l2 in device_utils.hpp), so that the transform after them does not wait until they are
+	 * written back. Networks of 20 blocks, us, written back / through: fp16 256 channels 15x15 12 positions 492 / 469, 16 535 / 520 (with weights that come from memory 560 / 564), 32 755 / 735, 19x19 8 609 / 590, 32 993 / 974; 128
+	 * channels 32 424 / 413, 64 600 / 576, 101 827 / 832, 19x19 100 1186 / 1142; 192 channels 16 448 / 433, 64 884 / 874; 64 channels 64 405 / 405; 384 channels 8 583 / 574, 64 1623 / 1608; fp32 64 channels
+	 * 32 444 / 441, 128 channels 32 751 / 713, 64 1124 / 1080, 256 3325 / 3318, 256 channels 16 1060 / 1019. Not where the launch itself is short of bandwidth to memory: tiles of
+	 * 128x128 (256 channels 64 1116 / 1134, 101 1526 / 1574), and orders by rows, in which every XCD fetches all of B, with a large B (384 channels, 10.6 MB, 16 802 / 816, 32 1161 / 1200).
+	 */
+	inline bool products_write_through(const StreamGemmArgs &g, int element_size)
+	{
+		if (g.batch != TRANSFORM_MATRICES || element_size == 4)
+			return g.batch == TRANSFORM_MATRICES;
+		const unsigned long long b_bytes = static_cast<unsigned long long>(g.batch) * g.N * g.k_bytes;
+		return tile_of_plain(g, element_size) != GemmTile::T128x128 && !(products_go_by_rows(g, element_size) && b_bytes > 6 * MB);
+	}
+	/*
 	 * With the epilogue, fp16: 128x128 tiles from 3.5 of 64x64 per unit on (256 x 256, 14400 rows (900): 8.0 / 7.3 us; 384 x 256, 7200 rows (452) 6.5 / 7.7, 14400 9.7 / 8.7), 128x64
 	 * where 128 pads the columns more (192 x 192, 57600 rows 15.3 / 14.1).
 	 */
