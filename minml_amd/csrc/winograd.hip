@@ -1394,15 +1394,39 @@ namespace
 		return static_cast<unsigned int>(blocks);
 	}
 
+	/*
+	 * A stand-alone transform over few images is as long as one lane's chain of instructions and leaves most compute units idle: fewer channels to a lane while there is not a
+	 * wavefront for every unit (one position of 256 channels: 4 workgroups of 4 wavefronts before, 64 of one now), one wavefront to a workgroup up to three per unit. Networks of 8
+	 * blocks as three calls per layer, us, four channels and 256 threads throughout / this: fp16 256 channels 15x15 1 position 233 / 173, 4 250 / 187, 12 285 / 238, 16 310 / 291, 32 370 / 365, 64
+	 * 494 / 494; 128 channels 1 212 / 152, 32 261 / 241, 64 292 / 288 (101, 3.2 wavefronts per unit: 408 / 420 with one to a workgroup); 192 channels 19x19 8 277 / 227; fp32 128 channels 1 265 /
+	 * 216, 64 515 / 506; the first and last layers of a fused network, 256 channels 1 143 / 137, 16 227 / 225.
+	 */
+	struct TransformLaunch
+	{
+			int vec, threads;
+			unsigned int workgroups;
+	};
+	inline TransformLaunch transform_launch(size_t tiles, int channels, int widest)
+	{
+		const size_t lanes = 64 * static_cast<size_t>(device_compute_units());
+		TransformLaunch r { widest, 256, 0u };
+		while (r.vec > 1 && tiles * (channels / r.vec) < lanes)
+			r.vec /= 2;
+		const size_t items = tiles * (channels / r.vec);
+		if (items < 3 * lanes)
+			r.threads = 64;
+		r.workgroups = static_cast<unsigned int>((items + r.threads - 1) / r.threads);
+		return r;
+	}
 	template<typename T>
 	void launch_input(hipStream_t stream, const mlTensor_t &x, mlTensor_t &matrices)
 	{
 		const int batch = x.dim[0], height = x.dim[1], width = x.dim[2], channels = x.dim[3];
 		const int tiles_h = ceil_div(height, 4), tiles_w = ceil_div(width, 4);
 		const size_t tiles = static_cast<size_t>(batch) * tiles_h * tiles_w;
-		const int vec = pick_vec(channels, x.data, matrices.data, nullptr, nullptr, sizeof(T));
-		const dim3 block(256);
-		const dim3 grid(grid_for(tiles * (channels / vec)));
+		const TransformLaunch shape = transform_launch(tiles, channels, pick_vec(channels, x.data, matrices.data, nullptr, nullptr, sizeof(T)));
+		const int vec = shape.vec;
+		const dim3 grid(shape.workgroups), block(shape.threads);
 		const T *in = ptr<const T>(x);
 		T *out = ptr<T>(matrices);
 		switch (vec)
@@ -1420,10 +1444,9 @@ namespace
 		MLHIP_CHECK(hipGetLastError());
 	}
 	template<typename T, int VEC>
-	void launch_output_vec(hipStream_t stream, dim3 grid, const T *in, T *out, const T *b, const T *e, int act, int batch, int height, int width,
+	void launch_output_vec(hipStream_t stream, dim3 grid, dim3 block, const T *in, T *out, const T *b, const T *e, int act, int batch, int height, int width,
 			int channels, int tiles_h, int tiles_w)
 	{
-		const dim3 block(256);
 		const int mode = (act == ACTIVATION_LINEAR) ? 0 : ((act == ACTIVATION_RELU) ? 1 : 2);
 		const bool cached = matrices_stay_cached(static_cast<size_t>(batch) * tiles_h * tiles_w, channels, sizeof(T));
 #define MLHIP_LAUNCH_OUTPUT(MODE, EXT) \
@@ -1454,8 +1477,9 @@ namespace
 		const int batch = y.dim[0], height = y.dim[1], width = y.dim[2], channels = y.dim[3];
 		const int tiles_h = ceil_div(height, 4), tiles_w = ceil_div(width, 4);
 		const size_t tiles = static_cast<size_t>(batch) * tiles_h * tiles_w;
-		const int vec = pick_vec(channels, matrices.data, y.data, bias.data, ext.data, sizeof(T));
-		const dim3 grid(grid_for(tiles * (channels / vec)));
+		const TransformLaunch shape = transform_launch(tiles, channels, pick_vec(channels, matrices.data, y.data, bias.data, ext.data, sizeof(T)));
+		const int vec = shape.vec;
+		const dim3 grid(shape.workgroups), block(shape.threads);
 		const T *in = ptr<const T>(matrices);
 		T *out = ptr<T>(y);
 		const T *b = ptr<const T>(bias);
@@ -1464,13 +1488,13 @@ namespace
 		switch (vec)
 		{
 			case 4:
-				launch_output_vec<T, 4>(stream, grid, in, out, b, e, a, batch, height, width, channels, tiles_h, tiles_w);
+				launch_output_vec<T, 4>(stream, grid, block, in, out, b, e, a, batch, height, width, channels, tiles_h, tiles_w);
 				break;
 			case 2:
-				launch_output_vec<T, 2>(stream, grid, in, out, b, e, a, batch, height, width, channels, tiles_h, tiles_w);
+				launch_output_vec<T, 2>(stream, grid, block, in, out, b, e, a, batch, height, width, channels, tiles_h, tiles_w);
 				break;
 			default:
-				launch_output_vec<T, 1>(stream, grid, in, out, b, e, a, batch, height, width, channels, tiles_h, tiles_w);
+				launch_output_vec<T, 1>(stream, grid, block, in, out, b, e, a, batch, height, width, channels, tiles_h, tiles_w);
 				break;
 		}
 		MLHIP_CHECK(hipGetLastError());

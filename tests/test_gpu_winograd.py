@@ -51,6 +51,24 @@ def test_transforms_bit_exact(ctx, dtype, shape, cout):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "float16"])
+@pytest.mark.parametrize("batch", [511, 512, 1023, 1024, 3071, 3072])
+def test_transforms_at_the_limits_of_their_launches(ctx, dtype, batch):
+    """One, two or four channels to a lane and one or four wavefronts to a workgroup, by the number of tiles: both sides of each limit for 256 compute
+    units (boards of one ragged tile, 64 channels), bit for bit against the oracle."""
+    rng = np.random.default_rng(batch)
+    shape = (batch, 3, 4, 64)
+    x, m, bias = random_tensor(rng, shape, dtype), random_tensor(rng, (36, batch, 64), dtype), random_tensor(rng, (64,), dtype)
+    dv, dy = ml.Tensor((36, batch, 64), dtype), ml.Tensor(shape, dtype)
+    dv.setall(ctx, float("nan"))
+    ml.winogradInputTransform(ctx, (64, 3, 3, 64), ml.toDevice(ctx, x), dv)
+    assert mismatches(dv.copyToHost(ctx), O.winograd_input_transform(x)) == 0
+    for ext in (None, x):
+        dy.setall(ctx, float("nan"))
+        ml.winogradOutputTransform(ctx, (64, 3, 3, 64), ml.toDevice(ctx, m), dy, ml.toDevice(ctx, bias), None if ext is None else ml.toDevice(ctx, ext), O.RELU)
+        assert mismatches(dy.copyToHost(ctx), O.winograd_output_transform(m, shape, bias, ext, O.RELU)) == 0
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float16"])
 @pytest.mark.parametrize("act", [O.SIGMOID, O.TANH, O.LEAKY_RELU, O.EXP])
 def test_output_transform_other_activations(ctx, dtype, act):
     rng = np.random.default_rng(act)
