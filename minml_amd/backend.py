@@ -28,15 +28,12 @@ class mlTensor_t(ctypes.Structure):
     _fields_ = [("data", ctypes.c_void_p), ("dtype", ctypes.c_int), ("rank", ctypes.c_int), ("dim", ctypes.c_int * 6)]
 
 
-_Dims = ctypes.c_int * 6
-
-
 def make_shape(dims):
-    return mlShape_t(len(dims), _Dims(*map(int, dims)))
+    return mlShape_t(len(dims), tuple(map(int, dims)))
 
 
 def make_tensor(ptr, dtype, dims):
-    return mlTensor_t(ptr, dtype, len(dims), _Dims(*map(int, dims))) if ptr else mlTensor_t(ptr, dtype, 0, _Dims())
+    return mlTensor_t(ptr, dtype, len(dims), tuple(map(int, dims))) if ptr else mlTensor_t(ptr, dtype, 0)
 
 
 _vp, _sz, _i, _f, _b, _c = ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int, ctypes.c_float, ctypes.c_bool, ctypes.c_char

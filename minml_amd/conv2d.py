@@ -143,15 +143,20 @@ class Conv2D:
         return output
 
     # ---- the three stages of the Winograd path, separately callable so that a runner can fuse across layers -------------------
+    def _input_matrices(self, batch, workspace):
+        """The view at element 0 of the workspace (Conv2D.cpp:365-367)."""
+        return workspace.view(get_matrices_shape(self.kernel_size, self.winograd_tile_size, (batch,) + self.input_shape[1:]))
+
+    def _output_matrices(self, batch, workspace):
+        """The view behind the input matrices, at element 36*T*Cin."""
+        squared, tiles, filters_in = get_matrices_shape(self.kernel_size, self.winograd_tile_size, (batch,) + self.input_shape[1:])
+        return workspace.view((squared, tiles, self.output_shape[3]), squared * tiles * filters_in)
+
     def _winograd_views(self, batch, workspace):
-        """(input matrices, output matrices): views at element 0 and 36*T*Cin of the workspace (Conv2D.cpp:365-367)."""
-        in_shape = get_matrices_shape(self.kernel_size, self.winograd_tile_size, (batch,) + self.input_shape[1:])
-        out_shape = get_matrices_shape(self.kernel_size, self.winograd_tile_size, (batch,) + self.output_shape[1:])
-        return workspace.view(in_shape), workspace.view(out_shape, math.prod(in_shape))
+        return self._input_matrices(batch, workspace), self._output_matrices(batch, workspace)
 
     def winograd_input(self, x, workspace):
-        input_matrices, _ = self._winograd_views(x.shape[0], workspace)
-        ml.winogradInputTransform(self.context, self.weight_shape, x, input_matrices)
+        ml.winogradInputTransform(self.context, self.weight_shape, x, self._input_matrices(x.shape[0], workspace))
 
     def winograd_gemm(self, batch, workspace):
         """36 batched products of the input matrices already in the workspace with the cached transformed weights."""
@@ -163,15 +168,14 @@ class Conv2D:
         ml.gemmBatched(ctx, "n", "t", output_matrices, input_matrices, self.transformed_weights, 1.0, 0.0)
 
     def winograd_output(self, output, add, workspace):
-        _, output_matrices = self._winograd_views(output.shape[0], workspace)
-        ml.winogradOutputTransform(self.context, self.weight_shape, output_matrices, output, self.bias, add, self.activation)
+        ml.winogradOutputTransform(self.context, self.weight_shape, self._output_matrices(output.shape[0], workspace), output, self.bias, add, self.activation)
 
     def winograd_output_into(self, next_layer, batch, output, add, workspace):
         """Output transform of this layer fused with the input transform of `next_layer` (a Winograd layer on this layer's output,
         sharing the workspace): the next layer's input matrices land at element 0, where this layer's are no longer needed.
         `output` may be None when nothing else reads this layer's result."""
         input_matrices, output_matrices = self._winograd_views(batch, workspace)
-        next_input, _ = next_layer._winograd_views(batch, workspace)
+        next_input = next_layer._input_matrices(batch, workspace)
         if next_input.volume() > input_matrices.volume():
             raise ValueError("the next layer's input matrices would overlap this layer's output matrices in the workspace")
         out_shape = (batch,) + self.output_shape[1:]
@@ -186,7 +190,7 @@ class Conv2D:
             self.transformed_weights = ml.Tensor(get_weight_matrices_shape(self.weight_shape, self.winograd_tile_size), self.dtype, ctx.device_index)
             ml.winogradWeightTransform(ctx, self.weights, self.transformed_weights, False)
         input_matrices, output_matrices = self._winograd_views(batch, workspace)
-        next_input, _ = next_layer._winograd_views(batch, workspace)
+        next_input = next_layer._input_matrices(batch, workspace)
         if next_input.volume() > input_matrices.volume():
             raise ValueError("the next layer's input matrices would overlap this layer's output matrices in the workspace")
         out_shape = (batch,) + self.output_shape[1:]

@@ -164,7 +164,8 @@ class Tensor:
         return self.shape[i]
 
     def volume(self):
-        return math.prod(self.shape) if self.shape else 0
+        shape = self.shape
+        return math.prod(shape) if shape else 0
 
     def firstDim(self):
         return self.shape[0]
@@ -176,7 +177,7 @@ class Tensor:
         return self.volume() * B.DTYPE_SIZE[self.dtype]
 
     def isEmpty(self):
-        return self.volume() == 0
+        return not self.shape or 0 in self.shape
 
     def view(self, shape, offset=0):
         """Non-owning tensor over the same memory, `offset` in elements (reference: Tensor::view; hip_create_view is the same sum of
@@ -245,16 +246,18 @@ class Tensor:
 
     def __del__(self):
         try:
-            self.free()
+            if self._owning:  # a view has nothing to give back, and a pass makes hundreds of them
+                self.free()
         except Exception:
             pass
 
     # ---- descriptors
     def desc(self):
-        return B.make_tensor(self.ptr, self.dtype, self.shape)
+        # the shape is a tuple of whole numbers from the start
+        return B.mlTensor_t(self.ptr, self.dtype, len(self.shape), self.shape) if self.ptr else B.make_tensor(self.ptr, self.dtype, self.shape)
 
     def shape_desc(self):
-        return B.make_shape(self.shape)
+        return B.mlShape_t(len(self.shape), self.shape)
 
 
 def toDevice(context, array, dtype=None):
@@ -338,8 +341,14 @@ def _launch(name, *args):
 
 
 def _same_dtype(*tensors):
-    ts = [t for t in tensors if t is not None and not t.isEmpty()]
-    return all(t.dtype == ts[0].dtype for t in ts)
+    dtype = None
+    for t in tensors:
+        if t is not None and not t.isEmpty():
+            if dtype is None:
+                dtype = t.dtype
+            elif t.dtype != dtype:
+                return False
+    return True
 
 
 def get_winograd_tile(weight_shape, matrices_shape):
