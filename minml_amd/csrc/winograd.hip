@@ -924,6 +924,10 @@ namespace
 		typedef typename RawVec<T, VEC>::type raw_t;
 		typedef float line_t __attribute__((ext_vector_type(VEC)));
 		extern __shared__ __attribute__((aligned(16))) uint8_t lds_bytes[];
+		/* all arguments at once: left to itself the compiler asks for them in six rounds, each where its first field is used, and waits for each (0.1 us a round) */
+		asm volatile("" :: "s"(g.matrices), "s"(g.next_matrices), "s"(g.ext), "s"(g.bias), "s"(g.output), "s"(g.matrix_stride), "s"(g.image_elements), "s"(g.height), "s"(g.width),
+				"s"(g.channels), "s"(g.tiles_h), "s"(g.tiles_w), "s"(g.strips), "s"(g.waves), "s"(g.contiguous), "s"(g.workgroups), "s"(g.by_slices.divisor), "s"(g.by_slices.magic),
+				"s"(g.by_slices.shift), "s"(g.by_strips.divisor), "s"(g.by_strips.magic), "s"(g.by_strips.shift), "s"(g.by_tiles_w.divisor), "s"(g.by_tiles_w.magic), "s"(g.by_tiles_w.shift));
 		const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 		const int index = lane / LANES, channel = (lane % LANES) * VEC; /* which line of the tile; the lane's channels */
 		const int pitch = 4 * g.tiles_w + 2;
