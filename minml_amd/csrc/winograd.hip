@@ -1895,7 +1895,8 @@ extern "C"
 		 *         32 channels              23.2 / 28.3  22.6 / 30.6  27.1 / 35.0  28.0 / 35.7  37.7 / 46.5  51.0 / 60.3  64.5 / 75.2  76.1 / 87.6
 		 *         16 channels              22.9 / 23.5  22.9 / 23.5  27.1 / 28.2  28.5 / 30.0  38.5 / 40.1  52.0 / 55.0  65.8 / 70.1  78.5 / 83.3
 		 *         strips of 16 channels    20.7 / 21.0  20.8 / 21.7  25.5 / 26.8  26.9 / 28.2  37.7 / 40.1  51.0 / 55.0  65.1 / 70.1  77.7 / 83.3
-		 * A launch over few images is bound by what one lane must issue, a launch over many by memory, which wants whole 128-byte lines.
+		 * A launch over few images is bound by what one lane must issue, a launch over many by memory, which wants whole 128-byte lines. The last two fp16 rows
+		 * are forms that the lines replaced and that are no longer built in fp16.
 		 * Lines, fp16: a tile row to a workgroup while there is one for every compute unit at most (us per layer, a row / an image: 256 channels 15x15 4 images (256) 9.3 / 9.8,
 		 * 8 (512) 11.6 / 11.5, 12 15.0 / 12.7; 128 channels 9x9 16 (384) 8.9 / 8.4; 64 channels 9x9 16 (192) 7.4 / 7.7; 192 channels 20x20 4 (240) 9.6 / 10.9, 8 (480) 13.3 / 13.0),
 		 * images to three per unit (the other forms / this: 256 channels 15x15 48 images (768) 23.6 / 23.2, 64 (1024) 26.2 / 27.7; 192 channels 20x20 64 (768) 28.7 / 27.2;
