@@ -253,11 +253,18 @@ namespace mlhip
 	 * channels 32 424 / 413, 64 600 / 576, 101 827 / 832, 19x19 100 1186 / 1142; 192 channels 16 448 / 433, 64 884 / 874; 64 channels 64 405 / 405; 384 channels 8 583 / 574, 64 1623 / 1608; fp32 64 channels
 	 * 32 444 / 441, 128 channels 32 751 / 713, 64 1124 / 1080, 256 3325 / 3318, 256 channels 16 1060 / 1019. Not where the launch itself is short of bandwidth to memory: tiles of
 	 * 128x128 (256 channels 64 1116 / 1134, 101 1526 / 1574), and orders by rows, in which every XCD fetches all of B, with a large B (384 channels, 10.6 MB, 16 802 / 816, 32 1161 / 1200).
+	 * Rows of C that are not whole lines of 128 bytes leave the L2 in parts: no matter while there are few of them (18 blocks of 96 channels, C of 1.8 MB 430 / 415, 3.5 446 / 440,
+	 * 7.1 586 / 583), more traffic than the wait costs after that (19x19, 11 MB 758 / 815; 14 MB 813 / 880, 24 MB 1179 / 1229).
 	 */
 	inline bool products_write_through(const StreamGemmArgs &g, int element_size)
 	{
-		if (g.batch != TRANSFORM_MATRICES || element_size == 4)
-			return g.batch == TRANSFORM_MATRICES;
+		if (g.batch != TRANSFORM_MATRICES)
+			return false;
+		const unsigned long long c_row = static_cast<unsigned long long>(g.N) * element_size;
+		if (c_row % 128 != 0 && g.batch * g.M * c_row > 8 * MB)
+			return false;
+		if (element_size == 4)
+			return true;
 		const unsigned long long b_bytes = static_cast<unsigned long long>(g.batch) * g.N * g.k_bytes;
 		return tile_of_plain(g, element_size) != GemmTile::T128x128 && !(products_go_by_rows(g, element_size) && b_bytes > 6 * MB);
 	}
