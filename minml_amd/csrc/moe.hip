@@ -816,7 +816,7 @@ extern "C"
 #define MLHIP_GATHER(T, VEC) \
 		do { \
 			const size_t groups = rows * (channels / VEC); \
-			if (groups <= 0xffffffffu) \
+			if (groups <= 0xffffffffu && tokens > 0) /* an empty board has no first token, which the fast form reads for an empty slot */ \
 			{ \
 				const FastDivisor by_pieces = make_fast_divisor(static_cast<uint32_t>(channels / VEC)), by_experts = make_fast_divisor(static_cast<uint32_t>(experts)), \
 						by_capacity = make_fast_divisor(static_cast<uint32_t>(capacity)); \

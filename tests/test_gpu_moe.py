@@ -159,6 +159,22 @@ def test_gather_and_scatter(ctx, dtype, shape, experts, capacity):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "float16"])
+@pytest.mark.parametrize("channels", [16, 5])
+def test_gather_from_an_empty_board(ctx, dtype, channels):
+    """No tokens: the routers' tables hold -1 alone, nothing of x may be read (it has no first token), the slots become 0 or keep beta * y."""
+    x, iv = ml.Tensor((2, 0, 0, channels), dtype), ml.Tensor((2, 2, 3, 4), dtype)
+    ml.hashRouting(ctx, ml.Tensor((2, 0, 0, 3), dtype), iv)
+    table = iv.copyToHost(ctx)
+    assert (index_plane(table) == -1).all()
+    y0 = random_tensor(np.random.default_rng(channels), (2, 4, 3, channels), dtype)
+    for beta in (0.0, 0.5):
+        y = ml.toDevice(ctx, y0)
+        ml.gatherTokensForward(ctx, x, iv, beta, y)
+        want = M.gather_tokens(np.zeros((2, 0, 0, channels), y0.dtype), table, beta, y0)
+        assert max_abs_rel(y.copyToHost(ctx), want) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float16"])
 @pytest.mark.parametrize("dims", [(2, 56, 8, 256, 1024), (2, 56, 8, 1024, 256), (3, 7, 3, 20, 12), (1, 5, 2, 64, 36), (4, 56, 8, 64, 128)])
 def test_expert_layers(ctx, dtype, dims):
     b, k, e, c, n = dims
