@@ -259,12 +259,20 @@ namespace mlhip
 
 	/*
 	 * A 16-byte store that writes through the L2 (which keeps the line): what a launch leaves dirty in the L2s is written back between it and the next one, and the
-	 * launch that follows waits for that (3.0 us from the end of a product of 4.7 MB to the first workgroup after it, 1.7 us where it wrote 0.3 MB). Whole lines
-	 * only: pieces of 32 bytes written through cost more than they save (fused transform of few images, +6 % of the layer). No builtin has this form.
+	 * launch that follows waits for that (3.0 us from the end of a product of 4.7 MB to the first workgroup after it, 1.7 us where it wrote 0.3 MB). For wavefronts whose
+	 * stores cover whole or half lines of 128 bytes (the product tiles with one 32-column block per wavefront store halves, the other half comes from another wavefront):
+	 * pieces of 32 bytes written through cost more than they save (fused transform of few images, +6 % of the layer). The buffer form is the one
+	 * that has a builtin: a store of more than 8 bytes must not be followed within two wait states by a vector write of its data registers, which the compiler sees
+	 * to only for stores that it knows as such.
 	 */
-	__device__ __forceinline__ void store_through_l2(void *dst, const uint4_t &value)
+	constexpr int STORE_THROUGH_L2 = 16; /* sc1, among the builtin's auxiliary bits */
+	__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(void *base)
 	{
-		asm volatile("global_store_dwordx4 %0, %1, off sc1" :: "v"(dst), "v"(value) : "memory");
+		return __builtin_amdgcn_make_buffer_rsrc(base, 0, 0x7fffffff, 0x00020000);
+	}
+	__device__ __forceinline__ void store_through_l2(__amdgpu_buffer_rsrc_t buffer, int byte_offset, const uint4_t &value)
+	{
+		__builtin_amdgcn_raw_buffer_store_b128(value, buffer, byte_offset, 0, STORE_THROUGH_L2);
 	}
 
 	/*

@@ -190,6 +190,7 @@ namespace
 		constexpr int E = 16 / sizeof(T), PER_ROW = 32 * BLOCKS_N / E;
 		static_assert(PER_ROW % 2 == 0, "whole passes of 64 lanes over 32 rows");
 		uint8_t *slab = lds + wave * 32 * Shape::SLAB_STRIDE;
+		const __amdgpu_buffer_rsrc_t through = buffer_of(out + static_cast<size_t>(m_tile) * out_stride + n_tile); /* products_write_through: a tile within 2^31 bytes */
 #pragma unroll
 		for (int i = 0; i < BLOCKS_M; i++)
 		{
@@ -228,7 +229,7 @@ namespace
 				if (m < M && n0 + col < N)
 				{
 					if (PLAIN && write_through)
-						store_through_l2(out + m * out_stride + n0 + col, v);
+						store_through_l2(through, static_cast<int>(((m - m_tile) * static_cast<int>(out_stride) + n0 - n_tile + col) * sizeof(T)), v);
 					else
 						*reinterpret_cast<uint4_t*>(out + m * out_stride + n0 + col) = v;
 				}

@@ -261,7 +261,7 @@ namespace mlhip
 		if (g.batch != TRANSFORM_MATRICES)
 			return false;
 		const unsigned long long c_row = static_cast<unsigned long long>(g.N) * element_size;
-		if (c_row % 128 != 0 && g.batch * g.M * c_row > 8 * MB)
+		if (c_row >= (1ULL << 24) || (c_row % 128 != 0 && c_row * g.batch * g.M > 8 * MB)) /* 128 rows lie within a buffer's 2^31 bytes */
 			return false;
 		if (element_size == 4)
 			return true;

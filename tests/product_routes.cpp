@@ -4,6 +4,7 @@
  *   dense ...                                                                "<tiles 0|1> 0 <direct kernel 0|1> <tile>"   (bias, no C)
  *   residual ...                                                             the same with C
  *   experts ...                                                              as dense, with the matrices' rows side by side
+ *   through ...                                                              "<write-through 0|1>" of a batch of plain products
  *   straddling <element size> <bytes of a pixel> <pixels> <columns> <bytes of a K row>      "<register-staged 0|1>"
  */
 #include "conv_tiles.hpp"
@@ -35,6 +36,12 @@ int main()
 			c.N = g.N;
 			c.k_bytes = g.k_bytes;
 			std::printf("%d\n", mlhip::stays_register_staged(c, element_size));
+			continue;
+		}
+		if (std::strcmp(kind, "through") == 0)
+		{
+			g.a_row_bytes = 0;
+			std::printf("%d\n", mlhip::products_write_through(g, element_size));
 			continue;
 		}
 		const bool plain = std::strcmp(kind, "plain") == 0;

@@ -120,3 +120,13 @@ def test_dense_layers_with_residual_on_the_tiles(decide, rows, columns, K, taken
     ("float16", 16, 3, 115200, 128, False), ("float32", 4, 3, 460800, 256, False), ("float32", 12, 3, 230400, 64, False), ("float16", 8, 3, 1074790400, 65, True)])
 def test_convolutions_with_straddling_pieces(decide, dtype, channels, kernel, pixels, columns, staged):
     assert decide("straddling", dtype, channels * SIZE[dtype], pixels, columns, kernel * kernel * channels) == [str(int(staged))]
+
+
+@pytest.mark.parametrize("dtype,matrices,rows,columns,K,through", [
+    # the products between transforms; rows that end inside a line of 128 bytes to 8 MB, tiles of 128x128 and large weights by rows never
+    ("float16", 36, 192, 256, 256, True), ("float16", 36, 1616, 256, 256, False), ("float16", 36, 256, 384, 384, False), ("float16", 36, 2304, 384, 384, True),
+    ("float16", 36, 1024, 96, 96, True), ("float16", 36, 1600, 96, 96, False), ("float32", 36, 4096, 256, 256, True), ("float16", 16, 192, 256, 256, False),
+    # what a buffer's 32-bit offsets reach of 128 rows
+    ("float32", 36, 1, (1 << 22) - 32, 8, True), ("float32", 36, 1, 1 << 22, 8, False)])
+def test_products_that_write_through(decide, dtype, matrices, rows, columns, K, through):
+    assert decide("through", dtype, matrices, rows, columns, K) == [str(int(through))]
