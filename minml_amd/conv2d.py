@@ -144,8 +144,11 @@ class Conv2D:
 
     # ---- the three stages of the Winograd path, separately callable so that a runner can fuse across layers -------------------
     def _input_matrices(self, batch, workspace):
-        """The view at element 0 of the workspace (Conv2D.cpp:365-367)."""
-        return workspace.view(get_matrices_shape(self.kernel_size, self.winograd_tile_size, (batch,) + self.input_shape[1:]))
+        """The view at element 0 of the workspace (Conv2D.cpp:365-367), which must have room for the output matrices behind it."""
+        shape = get_matrices_shape(self.kernel_size, self.winograd_tile_size, (batch,) + self.input_shape[1:])
+        if shape[0] * shape[1] * (shape[2] + self.output_shape[3]) > workspace.volume():
+            raise ValueError("the workspace is too small for the layer's input and output matrices")
+        return workspace.view(shape)
 
     def _output_matrices(self, batch, workspace):
         """The view behind the input matrices, at element 36*T*Cin."""

@@ -99,6 +99,26 @@ def test_conv2d_algorithm_choice_and_workspace_contract():
     assert get_matrices_shape(3, 4, (2, 19, 19, 8)) == (36, 2 * 25, 8)
 
 
+def test_a_workspace_without_room_for_the_output_matrices_is_refused_by_every_winograd_stage(monkeypatch):
+    """Also by the stages that fill the input matrices alone (36 * 16 tiles * 8 channels), before the library is called."""
+    def called(*args):
+        raise AssertionError("called %s" % args[0])
+
+    monkeypatch.setattr(ml, "_launch", called)
+    layer, narrow = (Conv2D(None, (1, 15, 15, 8), filters, 3, "relu", True, "float32") for filters in (16, 8))
+    layer.transformed_weights, narrow.transformed_weights = (ml.Tensor((36, filters, 8), "float32", _ptr=0x9000) for filters in (16, 8))
+    layer.context = narrow.context = type("Context", (), dict(handle=None))()
+    x, y = ml.Tensor((1, 15, 15, 8), "float32", _ptr=0x7000), ml.Tensor((1, 15, 15, 16), "float32", _ptr=0x8000)
+    needed = 36 * 16 * (8 + 16)
+    small = ml.Tensor((needed - 1,), "float32", _ptr=0x100000)
+    for stage in (lambda: layer.winograd_input(x, small), lambda: layer.winograd_gemm(1, small), lambda: layer.winograd_output(y, None, small),
+                  lambda: narrow.winograd_output_into(layer, 1, None, None, small), lambda: narrow.winograd_layer_into(layer, 1, None, None, small)):
+        with pytest.raises(ValueError):
+            stage()
+    with pytest.raises(AssertionError, match="called winograd_input_transform"):
+        layer.winograd_input(x, ml.Tensor((needed,), "float32", _ptr=0x100000))
+
+
 def test_winograd_tile_is_derived_from_the_matrices():
     """src/core/math.cpp:107-118."""
     assert ml.get_winograd_tile((8, 3, 3, 8), (36, 10, 8)) == 4
