@@ -28,12 +28,21 @@ class mlTensor_t(ctypes.Structure):
     _fields_ = [("data", ctypes.c_void_p), ("dtype", ctypes.c_int), ("rank", ctypes.c_int), ("dim", ctypes.c_int * 6)]
 
 
+MAX_RANK = 6
+
+
+def _dims(dims):
+    if len(dims) > MAX_RANK:
+        raise IndexError("a descriptor holds at most %d dimensions" % MAX_RANK)
+    return tuple(map(int, dims))
+
+
 def make_shape(dims):
-    return mlShape_t(len(dims), tuple(map(int, dims)))
+    return mlShape_t(len(dims), _dims(dims))
 
 
 def make_tensor(ptr, dtype, dims):
-    return mlTensor_t(ptr, dtype, len(dims), tuple(map(int, dims))) if ptr else mlTensor_t(ptr, dtype, 0)
+    return mlTensor_t(ptr, dtype, len(dims), _dims(dims)) if ptr else mlTensor_t(ptr, dtype, 0)
 
 
 _vp, _sz, _i, _f, _b, _c = ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int, ctypes.c_float, ctypes.c_bool, ctypes.c_char

@@ -254,10 +254,11 @@ class Tensor:
     # ---- descriptors
     def desc(self):
         # the shape is a tuple of whole numbers from the start
-        return B.mlTensor_t(self.ptr, self.dtype, len(self.shape), self.shape) if self.ptr else B.make_tensor(self.ptr, self.dtype, self.shape)
+        shape = self.shape
+        return B.mlTensor_t(self.ptr, self.dtype, len(shape), shape) if self.ptr and len(shape) <= B.MAX_RANK else B.make_tensor(self.ptr, self.dtype, shape)
 
     def shape_desc(self):
-        return B.mlShape_t(len(self.shape), self.shape)
+        return B.make_shape(self.shape)
 
 
 def toDevice(context, array, dtype=None):

@@ -57,6 +57,15 @@ def test_descriptor_layout_matches_the_reference():
     assert (B.ACTIVATION_LINEAR, B.ACTIVATION_RELU, B.ACTIVATION_EXP) == (0, 3, 5)
 
 
+def test_more_dimensions_than_a_descriptor_holds_are_an_index_error():
+    most = ml.Tensor((1, 2, 3, 4, 5, 6), "float32", _ptr=0x7000)
+    assert list(most.desc().dim) == list(most.shape_desc().dim) == list(B.make_tensor(0x7000, most.dtype, most.shape).dim) == [1, 2, 3, 4, 5, 6]
+    more = ml.Tensor((1,) * 7, "float32", _ptr=0x7000)
+    for describe in (more.desc, more.shape_desc, lambda: B.make_shape(more.shape), lambda: B.make_tensor(0x7000, more.dtype, more.shape)):
+        with pytest.raises(IndexError):
+            describe()
+
+
 def test_cabi_error_behaviour(tmp_path):
     exe = str(tmp_path / "cabi_errors")
     libdir = os.path.join(ROOT, "minml_amd")
