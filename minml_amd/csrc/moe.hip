@@ -349,59 +349,65 @@ namespace
 		}
 	}
 
-	/* the same for fewer than 2^32 groups: the flat index is split by multiplications instead of 64-bit divisions, which were most of
-	 * the instructions of a thread that moves 16 bytes; whether the old value takes part is fixed at compile time */
-	template<typename T, int VEC, bool WITH_BETA>
+	/*
+	 * The same for fewer than 2^32 groups and boards with a token: the flat index is split by multiplications instead of 64-bit divisions, which were most of
+	 * the instructions of a thread that moves 16 bytes; whether the old value takes part is fixed at compile time. A thread owns PIECES pieces a workgroup's width
+	 * apart and requests their indexes, then their rows (and old values), before it uses the first: a launch over much memory keeps more of it in flight, a
+	 * launch over little is as long as one thread. us, one piece to a thread / this (two of 16 bytes), operands in the last-level cache and from memory, 15x15 with eight experts of 57 slots,
+	 * fp16: 256 channels 16 images (234 thousand pieces) 3.3 / 3.2, 4.3 / 4.3, 32 (467) 4.2 / 4.2, 5.3 / 5.3, 64 (934) 5.9 / 5.9, 8.2 / 7.7, 128 10.5 / 10.0, 14.6 / 12.8, 256 18.4 / 18.1, 24.8 /
+	 * 20.4; fp32: 4 2.7 / 2.8, 3.4 / 3.7, 32 (934) 5.5 / 5.7, 8.0 / 8.0, 64 10.5 / 10.3, 14.1 / 13.3, 256 33.2 / 33.8, 42.3 / 36.9; with beta 64 fp32 14.2 / 14.2, 17.9 / 17.5.
+	 * Single elements (33 channels), one / four to a thread: 64 images of 16 experts (980) 3.9 / 4.3, 5.4 / 5.3, 256 9.2 / 8.7, 12.1 / 9.9, 600 23.0 / 16.7, 30.8 / 19.0. Four pieces of 16 bytes
+	 * are behind two with the operands in the cache (256 images fp32 35.0 us).
+	 */
+	template<typename T, int VEC, bool WITH_BETA, int PIECES>
 	__global__ __launch_bounds__(256) void kernel_gather_tokens_fast(const T *x, const T *indices_and_values, T *y, float beta, uint32_t groups, int tokens,
 			int channels, FastDivisor by_pieces, FastDivisor by_experts, FastDivisor by_capacity)
 	{
 		const uint32_t experts = by_experts.divisor, capacity = by_capacity.divisor;
-		constexpr int UNROLL = 4;
 		typedef T raw_t __attribute__((ext_vector_type(VEC)));
-		const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-		for (uint64_t first = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; first < groups; first += UNROLL * stride)
+		for (uint64_t first = static_cast<uint64_t>(blockIdx.x) * blockDim.x * PIECES + threadIdx.x; first < groups; first += static_cast<uint64_t>(gridDim.x) * blockDim.x * PIECES)
 		{
-			uint32_t row[UNROLL], image[UNROLL];
-			int c[UNROLL];
-			T index[UNROLL];
+			uint32_t row[PIECES], image[PIECES];
+			int c[PIECES];
+			T index[PIECES];
+			raw_t in[PIECES], old[PIECES];
 #pragma unroll
-			for (int u = 0; u < UNROLL; u++)
+			for (int u = 0; u < PIECES; u++)
 			{
 				uint32_t piece, e, k;
-				const uint64_t g = first + u * stride;
+				const uint64_t g = first + u * blockDim.x;
 				row[u] = fast_divide(static_cast<uint32_t>(g < groups ? g : first), by_pieces, piece); /* (b * K + k) * E + e */
 				const uint32_t bk = fast_divide(row[u], by_experts, e);
 				image[u] = fast_divide(bk, by_capacity, k);
 				c[u] = static_cast<int>(piece) * VEC;
 				index[u] = indices_and_values[(static_cast<size_t>(image[u] * 2u) * experts + e) * capacity + k];
 			}
-			raw_t in[UNROLL];
+			if constexpr (WITH_BETA)
 #pragma unroll
-			for (int u = 0; u < UNROLL; u++)
+				for (int u = 0; u < PIECES; u++)
+					old[u] = *reinterpret_cast<const raw_t*>(y + static_cast<size_t>(row[u]) * channels + c[u]);
+#pragma unroll
+			for (int u = 0; u < PIECES; u++)
 			{ /* an empty slot reads the image's first token and drops it */
 				const int token = static_cast<int>(static_cast<float>(index[u]));
 				in[u] = *reinterpret_cast<const raw_t*>(x + (static_cast<size_t>(image[u]) * tokens + (token >= 0 ? token : 0)) * channels + c[u]);
 			}
 #pragma unroll
-			for (int u = 0; u < UNROLL; u++)
+			for (int u = 0; u < PIECES; u++)
 			{
-				if (u > 0 && first + u * stride >= groups)
+				if (u > 0 && first + u * blockDim.x >= groups)
 					break;
 				const bool filled = static_cast<int>(static_cast<float>(index[u])) >= 0;
 				Vec<T, VEC> out;
 				out.zero();
-				T *y_piece = y + static_cast<size_t>(row[u]) * channels + c[u];
 				if constexpr (WITH_BETA)
-				{
-					out.load(y_piece);
 #pragma unroll
 					for (int i = 0; i < VEC; i++)
-						out.v[i] *= beta;
-				}
+						out.v[i] = static_cast<float>(old[u][i]) * beta;
 #pragma unroll
 				for (int i = 0; i < VEC; i++)
 					out.v[i] = filled ? static_cast<float>(in[u][i]) + out.v[i] : out.v[i];
-				out.store(y_piece);
+				out.store(y + static_cast<size_t>(row[u]) * channels + c[u]);
 			}
 		}
 	}
@@ -813,6 +819,9 @@ extern "C"
 			return;
 		MLHIP_REQUIRE(x.data != nullptr && y.data != nullptr && indices_and_values.data != nullptr, "gather_tokens_forward: null tensor");
 		const hipStream_t stream = stream_of(context);
+#define MLHIP_GATHER_FAST(T, VEC, BETA, PIECES) \
+		hipLaunchKernelGGL((kernel_gather_tokens_fast<T, VEC, BETA, PIECES>), dim3(grid_for((groups + PIECES - 1) / PIECES)), dim3(256), 0, stream, ptr<const T>(x), \
+				ptr<const T>(indices_and_values), ptr<T>(y), beta, static_cast<uint32_t>(groups), tokens, channels, by_pieces, by_experts, by_capacity)
 #define MLHIP_GATHER(T, VEC) \
 		do { \
 			const size_t groups = rows * (channels / VEC); \
@@ -820,12 +829,16 @@ extern "C"
 			{ \
 				const FastDivisor by_pieces = make_fast_divisor(static_cast<uint32_t>(channels / VEC)), by_experts = make_fast_divisor(static_cast<uint32_t>(experts)), \
 						by_capacity = make_fast_divisor(static_cast<uint32_t>(capacity)); \
-				if (beta != 0.0f) \
-					hipLaunchKernelGGL((kernel_gather_tokens_fast<T, VEC, true>), dim3(grid_for((groups + 3) / 4)), dim3(256), 0, stream, ptr<const T>(x), \
-							ptr<const T>(indices_and_values), ptr<T>(y), beta, static_cast<uint32_t>(groups), tokens, channels, by_pieces, by_experts, by_capacity); \
+				constexpr int PIECES = (VEC == 1) ? 4 : 2; \
+				const bool many = groups >= (1u << 20); \
+				if (many && beta != 0.0f) \
+					MLHIP_GATHER_FAST(T, VEC, true, PIECES); \
+				else if (many) \
+					MLHIP_GATHER_FAST(T, VEC, false, PIECES); \
+				else if (beta != 0.0f) \
+					MLHIP_GATHER_FAST(T, VEC, true, 1); \
 				else \
-					hipLaunchKernelGGL((kernel_gather_tokens_fast<T, VEC, false>), dim3(grid_for((groups + 3) / 4)), dim3(256), 0, stream, ptr<const T>(x), \
-							ptr<const T>(indices_and_values), ptr<T>(y), beta, static_cast<uint32_t>(groups), tokens, channels, by_pieces, by_experts, by_capacity); \
+					MLHIP_GATHER_FAST(T, VEC, false, 1); \
 			} \
 			else \
 				hipLaunchKernelGGL((kernel_gather_tokens<T, VEC>), dim3(grid_for(groups)), dim3(256), 0, stream, ptr<const T>(x), \
@@ -846,6 +859,7 @@ extern "C"
 				MLHIP_GATHER(float, 1);
 		}
 #undef MLHIP_GATHER
+#undef MLHIP_GATHER_FAST
 		MLHIP_CHECK(hipGetLastError());
 	}
 	catch (...)

@@ -8,7 +8,7 @@ import pytest
 import oracle as O
 from oracle import moe as M
 from minml_amd import core as ml
-from util import TOL, max_abs_rel, mismatches, random_tensor
+from util import TOL, max_abs_rel, mismatches, random_tensor, storage
 
 pytestmark = pytest.mark.gpu
 
@@ -156,6 +156,25 @@ def test_gather_and_scatter(ctx, dtype, shape, experts, capacity):
     dg = ml.toDevice(ctx, g0)
     ml.gatherTokensForward(ctx, d_x, d_iv, 2.0, dg)
     assert max_abs_rel(dg.copyToHost(ctx), M.gather_tokens(x, iv, beta=2.0, y=g0)) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float16"])
+@pytest.mark.parametrize("rows,channels", [((1 << 19) - 1, 8), (1 << 19, 8), ((1 << 19) + 65, 8), ((1 << 20) - 1, 8), (1 << 20, 8), ((1 << 20) + 129, 8),  # one piece to a row in fp16, two in fp32
+                                           (149796, 7), (149797, 7), (299593, 7)])  # seven, of single elements
+def test_gather_of_one_and_of_several_pieces_to_a_thread(ctx, dtype, rows, channels):
+    """Numbers of pieces on both sides of 2^20 and of a workgroup's share; slots of random tokens and empty ones, bit for bit."""
+    rng = np.random.default_rng(rows)
+    x = random_tensor(rng, (1, 3, 5, channels), dtype)
+    tokens = rng.integers(-1, 15, rows)
+    table = storage(np.stack([tokens, np.ones(rows)]).astype(np.float32).reshape(1, 2, 1, rows), dtype)
+    want = np.where((tokens >= 0)[:, None], x.reshape(15, channels)[np.maximum(tokens, 0)], 0).astype(x.dtype).reshape(1, rows, 1, channels)
+    dx, iv, y = ml.toDevice(ctx, x), ml.toDevice(ctx, table), ml.Tensor((1, rows, 1, channels), dtype)
+    for beta in (0.0, 1.0):
+        y.setall(ctx, 0.0)
+        ml.gatherTokensForward(ctx, dx, iv, beta, y)
+        assert mismatches(y.copyToHost(ctx), want) == 0
+    ml.gatherTokensForward(ctx, dx, iv, 2.0, y)  # x + 2 x, one rounding
+    assert mismatches(y.copyToHost(ctx), storage(3.0 * O.as_float(want), dtype)) == 0
 
 
 @pytest.mark.parametrize("dtype", ["float32", "float16"])
