@@ -566,6 +566,22 @@ namespace
 				acc.v[v] = acc.v[v] + scaled;
 			}
 	}
+	/*
+	 * Whether the gates lie in LDS too, where they arrive with the indexes instead of one latency later: not where so few workgroups fit a compute unit then that the
+	 * grid takes more rounds. us, gates from memory / in LDS, fp16: 256 images 15x15, eight experts of 57 slots, 256 channels (3 + 2 KB) 20.6 / 18.7; 19x19,
+	 * 64 channels, 20 experts: 73 slots (11 + 6 KB) 32.2 / 27.2; 361 slots (11 + 28 KB, 4 workgroups in the place of 8) 87.7 / 115, 128 images, which have 4 for each unit,
+	 * 63.9 / 59.2; 12 experts of 361 (7 + 17 KB, 6 for 8) 192 images 45.6 / 43.6, 256 54.9 / 70.4, 512 133 / 142; 14 (8 + 20 KB, 5 for 8) 160 images 50.3 / 48.2, 192 53.4 /
+	 * 81.8; 20x20, 48 experts: 34 slots (28 + 6 KB, 4 for 5) 256 images, two rounds either way, 71.8 / 54.3.
+	 */
+	inline bool scatter_gates_in_lds(size_t lds_bytes, size_t gate_bytes, size_t workgroups, size_t units)
+	{
+		const auto rounds = [=](size_t bytes)
+		{
+			const size_t at_once = units * std::min<size_t>(8, 160 * 1024 / std::max<size_t>(bytes, 1));
+			return (workgroups + at_once - 1) / at_once;
+		};
+		return lds_bytes + gate_bytes <= 64 * 1024 && 7 * rounds(lds_bytes + gate_bytes) <= 8 * rounds(lds_bytes);
+	}
 	/* dynamic LDS of kernel_scatter_tokens_by_image for `per_part` tokens per workgroup: inverse table, lists of (row, gate), counts */
 	inline size_t scatter_by_image_lds_bytes(int per_part, int experts)
 	{
@@ -886,7 +902,7 @@ extern "C"
 		const int splits = std::max(1, std::min(8, tokens / 16));
 		const size_t lds_bytes = scatter_by_image_lds_bytes((tokens + splits - 1) / splits, experts);
 		const size_t gate_bytes = static_cast<size_t>(capacity) * experts * sizeof(float);
-		const bool gates_in_lds = lds_bytes + gate_bytes <= 64 * 1024;
+		const bool gates_in_lds = scatter_gates_in_lds(lds_bytes, gate_bytes, static_cast<size_t>(batch) * splits, device_compute_units());
 		const size_t image_bytes = static_cast<size_t>(capacity) * experts * channels * size_of(x.dtype);
 		const bool by_image = experts > 0 && capacity > 0 && lds_bytes <= 48 * 1024 && static_cast<size_t>(batch) * splits <= 0x7fffffffu
 				&& image_bytes < 0x40000000u;

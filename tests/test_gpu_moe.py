@@ -159,6 +159,28 @@ def test_gather_and_scatter(ctx, dtype, shape, experts, capacity):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "float16"])
+@pytest.mark.parametrize("shape,experts,capacity", [((1, 38, 38, 8), 20, 267), ((1, 38, 38, 8), 20, 268),  # 44 KB of lists: with the gates just within 64 KB, and beyond
+                                                    ((640, 6, 6, 4), 16, 400), ((641, 6, 6, 4), 16, 400)])  # 28 KB, 5 workgroups a unit instead of 8: all at once, and not
+def test_scatter_with_the_gates_in_lds_and_in_memory(ctx, dtype, shape, experts, capacity):
+    """Both places that kernel_scatter_tokens_by_image takes the gates from, on both sides of the limit in bytes and of the one in workgroups (256 units)."""
+    b, h, w, c = shape
+    rng = np.random.default_rng(b + capacity)
+    table = np.full((b, 2, experts, capacity), -1, np.float32)
+    slots = min(capacity, h * w)
+    for e in range(experts):  # the last slots are filled: the end of the gates' array counts
+        table[:, 0, e, capacity - slots:] = rng.permutation(h * w)[:slots]
+    table[:, 1] = rng.random((experts, capacity))
+    iv, x, y0 = storage(table, dtype), random_tensor(rng, (b, capacity, experts, c), dtype), random_tensor(rng, shape, dtype)
+    d_iv, d_x = ml.toDevice(ctx, iv), ml.toDevice(ctx, x)
+    for beta in (0.0, 0.5):
+        y = ml.toDevice(ctx, y0)
+        ml.scatterTokensForward(ctx, d_x, d_iv, beta, y)
+        got, picked = y.copyToHost(ctx), [0, b - 1]
+        want = M.scatter_tokens(x[picked], iv[picked], (len(picked), h, w, c), beta=beta, y=y0[picked])
+        assert max_abs_rel(got[picked], want) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float16"])
 @pytest.mark.parametrize("rows,channels", [((1 << 19) - 1, 8), (1 << 19, 8), ((1 << 19) + 65, 8), ((1 << 20) - 1, 8), (1 << 20, 8), ((1 << 20) + 129, 8),  # one piece to a row in fp16, two in fp32
                                            (149796, 7), (149797, 7), (299593, 7)])  # seven, of single elements
 def test_gather_of_one_and_of_several_pieces_to_a_thread(ctx, dtype, rows, channels):
