@@ -114,32 +114,46 @@ namespace
 		}
 		for (size_t first = (static_cast<size_t>(blockIdx.x) * 4 + (threadIdx.x >> 6)) * UNROLL; first < rows; first += stride)
 		{
-			/* every row is requested before the first is used, from clamped places and kept as it is: a load under a test would be in a block of its own, and waited for there */
+			/*
+			 * fp16, and fp32 rows of more than one vector to a lane: every row is requested before the first is used, from clamped places and kept as it is. A load and its conversion under a test
+			 * would be in a block of their own, and waited for there (fp16, 57600 rows of 256 elements 13.8 -> 12.2 us). fp32 needs no conversion, and its short rows are behind
+			 * with clamped loads (us, under a test / clamped, from the last-level cache and from memory: 230400 rows of 64 elements 24.2 / 25.5, 28.0 / 33.0, of 32 23.7 / 25.1, 26.1 / 29.8, 57600 of 192 14.7 /
+			 * 15.0, 18.8 / 20.0; but 14400 of 512 10.4 / 10.1, 15.6 / 14.3).
+			 */
+			constexpr bool CLAMPED = sizeof(T) == 2 || ITEMS > 1;
 			typedef T raw_t __attribute__((ext_vector_type(VEC)));
 			raw_t raw[UNROLL][ITEMS];
-#pragma unroll
-			for (int u = 0; u < UNROLL; u++)
-			{
-				const T *src = input + (first + u < rows ? first + u : rows - 1) * columns;
-#pragma unroll
-				for (int i = 0; i < ITEMS; i++)
-				{
-					const int j = (lane + 64 * i) * VEC;
-					raw[u][i] = *reinterpret_cast<const raw_t*>(src + (j < columns ? j : 0));
-				}
-			}
 			Vec<T, VEC> x[UNROLL][ITEMS];
 #pragma unroll
 			for (int u = 0; u < UNROLL; u++)
 			{
+				const T *src = input + (CLAMPED && first + u >= rows ? rows - 1 : first + u) * columns;
 #pragma unroll
 				for (int i = 0; i < ITEMS; i++)
 				{
-					const bool inside = (lane + 64 * i) * VEC < columns;
-#pragma unroll
-					for (int e = 0; e < VEC; e++)
-						x[u][i].v[e] = inside ? static_cast<float>(raw[u][i][e]) : 0.0f;
+					const int j = (lane + 64 * i) * VEC;
+					if constexpr (CLAMPED)
+						raw[u][i] = *reinterpret_cast<const raw_t*>(src + (j < columns ? j : 0));
+					else
+					{
+						x[u][i].zero();
+						if (j < columns && first + u < rows)
+							x[u][i].load(src + j);
+					}
 				}
+			}
+#pragma unroll
+			for (int u = 0; u < UNROLL; u++)
+			{
+				if constexpr (CLAMPED)
+#pragma unroll
+					for (int i = 0; i < ITEMS; i++)
+					{
+						const bool inside = (lane + 64 * i) * VEC < columns;
+#pragma unroll
+						for (int e = 0; e < VEC; e++)
+							x[u][i].v[e] = inside ? static_cast<float>(raw[u][i][e]) : 0.0f;
+					}
 				float sum_square = 0.0f;
 #pragma unroll
 				for (int i = 0; i < ITEMS; i++)

@@ -49,6 +49,19 @@ def test_rmsnorm_shapes(ctx, dtype, shape):
     assert max_abs_rel(rmsnorm(ctx, x), O.rmsnorm_forward(x)) <= TOL[dtype]
 
 
+@pytest.mark.parametrize("dtype", ["float32", "float16"])
+@pytest.mark.parametrize("columns", [16, 128, 132, 136, 256, 260, 264, 512, 520, 1024, 1032])  # each form's shortest and longest rows in either type
+def test_rmsnorm_forms_with_ragged_rows(ctx, dtype, columns):
+    """Wavefronts with one to four rows, in place as well: no row but their own is written, and the last one is read again by nobody else."""
+    rng = np.random.default_rng(columns)
+    for rows in (1, 3, 4, 17, 18):
+        x, gamma = random_tensor(rng, (rows, columns), dtype, 2.0), random_tensor(rng, (columns,), dtype)
+        got, in_place = rmsnorm(ctx, x, gamma), ml.toDevice(ctx, x)
+        assert max_abs_rel(got, O.rmsnorm_forward(x, gamma)) <= TOL[dtype]
+        ml.rmsnormForward(ctx, in_place, in_place, ml.toDevice(ctx, gamma))
+        assert mismatches(in_place.copyToHost(ctx), got) == 0
+
+
 def test_rmsnorm_in_place_and_zero_rows(ctx):
     rng = np.random.default_rng(1)
     x = random_tensor(rng, (37, 256), "float16", 3.0)
