@@ -16,7 +16,6 @@ One difference by design: kernel sizes other than 1 and 3 use the fused implicit
 point only on cuDNN builds, Conv2D.cpp:478-485) because on this backend it needs no im2row workspace; `algorithm=` overrides the choice.
 The int8 path has the reference's three-call sequence ("reference") and the single fused launch ("fused").
 """
-import math
 
 import numpy as np
 

@@ -288,9 +288,9 @@ namespace mlhip
 		return (id % XCDS) * (full / XCDS) + id / XCDS;
 	}
 	/*
-	 * The tiles of a launch of many matrices, the column tiles of one row tile (or, by_columns, the row tiles of one column tile) next to one another on one XCD and
-	 * the matrix changing slowest or, by_rows, faster than the rows. A launch of few positions is a few microseconds long and its first loads wait for these numbers, so
-	 * what divides them is prepared on the host: two divisions by run-time values are about 60 dependent scalar instructions.
+	 * The tiles of a launch of many matrices, in one of two orders; consecutive tiles lie on one XCD and share its L2. A launch of few positions is a few
+	 * microseconds long and its first loads wait for these numbers, so what divides them is prepared on the host: two divisions by run-time values are about 60
+	 * dependent scalar instructions.
 	 */
 	struct TileOrder
 	{
@@ -298,9 +298,8 @@ namespace mlhip
 			uint32_t tiles;
 			enum Kind : uint32_t
 			{
-				ROWS_INNERMOST, /* matrix, column tile, row tile */
-				COLUMNS_INNERMOST, /* matrix, row tile, column tile */
-				MATRICES_BETWEEN /* row tile, matrix, column tile */
+				ROWS_INNERMOST, /* matrix (slowest), column tile, row tile (fastest) */
+				MATRICES_BETWEEN /* row tile, matrix, column tile: every XCD has rows of all matrices (gemm_tiles.hpp) */
 			} kind;
 			struct Tile
 			{
@@ -312,14 +311,13 @@ namespace mlhip
 				const uint32_t id = (block < full) ? (block & 7u) * (full >> 3) + (block >> 3) : block;
 				uint32_t innermost, middle;
 				const uint32_t slowest = fast_divide(fast_divide(id, inner, innermost), outer, middle);
-				return Tile { (kind == MATRICES_BETWEEN) ? middle : slowest, (kind == ROWS_INNERMOST) ? innermost : (kind == COLUMNS_INNERMOST) ? middle : slowest,
-						(kind == ROWS_INNERMOST) ? middle : innermost };
+				return (kind == ROWS_INNERMOST) ? Tile { slowest, innermost, middle } : Tile { middle, slowest, innermost };
 			}
 	};
 	inline TileOrder make_tile_order(TileOrder::Kind kind, uint32_t tiles_m, uint32_t tiles_n, uint32_t matrices)
 	{
-		return TileOrder { make_fast_divisor(kind == TileOrder::ROWS_INNERMOST ? tiles_m : tiles_n),
-				make_fast_divisor(kind == TileOrder::ROWS_INNERMOST ? tiles_n : kind == TileOrder::COLUMNS_INNERMOST ? tiles_m : matrices), tiles_m * tiles_n * matrices, kind };
+		const bool rows_innermost = (kind == TileOrder::ROWS_INNERMOST);
+		return TileOrder { make_fast_divisor(rows_innermost ? tiles_m : tiles_n), make_fast_divisor(rows_innermost ? tiles_n : matrices), tiles_m * tiles_n * matrices, kind };
 	}
 
 	/*
