@@ -699,7 +699,7 @@ namespace
 	}
 
 	/*
-	 * The same launch for few images of fp32 (boards of up to four tiles a row; the form after this one is ahead elsewhere). One workgroup per image and 64 channels leaves most of the chip idle there, and it is slow by itself:
+	 * The same launch for few images, mostly of fp32 (boards of up to four tiles a row; the form after this one is ahead elsewhere). One workgroup per image and 64 channels leaves most of the chip idle there, and it is slow by itself:
 	 * a compute unit moves about one 64-byte piece per 3 clocks whatever the width of the instruction, so the 36 loads and 36 stores of 16
 	 * tiles x 128 bytes take 7000 clocks, and its four wavefronts issue the arithmetic of 16 tiles back to back (another 10000). Here a
 	 * workgroup owns ONE ROW of tiles of an image (a strip of 4 pixel rows) and 16 channels, one channel per lane. The strip's input
@@ -1895,14 +1895,18 @@ extern "C"
 		 *         32 channels              23.2 / 28.3  22.6 / 30.6  27.1 / 35.0  28.0 / 35.7  37.7 / 46.5  51.0 / 60.3  64.5 / 75.2  76.1 / 87.6
 		 *         16 channels              22.9 / 23.5  22.9 / 23.5  27.1 / 28.2  28.5 / 30.0  38.5 / 40.1  52.0 / 55.0  65.8 / 70.1  78.5 / 83.3
 		 *         strips of 16 channels    20.7 / 21.0  20.8 / 21.7  25.5 / 26.8  26.9 / 28.2  37.7 / 40.1  51.0 / 55.0  65.1 / 70.1  77.7 / 83.3
-		 * A launch over few images is bound by what one lane must issue, a launch over many by memory, which wants whole 128-byte lines. The last two fp16 rows
-		 * are forms that the lines replaced and that are no longer built in fp16.
+		 * A launch over few images is bound by what one lane must issue, a launch over many by memory, which wants whole 128-byte lines. In fp16 the form of 16
+		 * channels is no longer built and the strips are what one step of the lines' rule leaves them.
 		 * Lines, fp16: a tile row to a workgroup while there is one for every compute unit at most (us per layer, a row / an image: 256 channels 15x15 4 images (256) 9.3 / 9.8,
 		 * 8 (512) 11.6 / 11.5, 12 15.0 / 12.7; 128 channels 9x9 16 (384) 8.9 / 8.4; 64 channels 9x9 16 (192) 7.4 / 7.7; 192 channels 20x20 4 (240) 9.6 / 10.9, 8 (480) 13.3 / 13.0),
 		 * images to three per unit (the other forms / this: 256 channels 15x15 48 images (768) 23.6 / 23.2, 64 (1024) 26.2 / 27.7; 192 channels 20x20 64 (768) 28.7 / 27.2;
 		 * 128 channels 12x12 96 (768) 16.4 / 14.8, 9x9 128 (1024) 17.7 / 17.6; 64 channels 9x9 256 (1024) 17.0 / 17.4). fp32 the same for a tile row of more than four tiles
 		 * (strips / lines: 64 channels 19x19 1 image 9.9 / 9.0, 8 11.5 / 10.9, 32 (128 images of 16 channels) 15.0 / 14.6; 192 channels 20x20 1 12.5 / 11.7, 8 20.1 / 19.8), not for
 		 * narrower ones, whose loads of 64 bytes the strips issue as fast (128 channels 15x15 1 10.5 / 10.6, 16 14.7 / 15.2).
+		 * Strips in fp16: images of 4 x 4 tiles are workgroups of 16 wavefronts, and as soon as some compute units have two of them the launch in lines takes a third longer
+		 * (256 of them 5.0 us, 288 6.7, 512 7.5), so strips are ahead from there to a quarter more images (two layers, without and with residual, and an input transform, us, lines / strips:
+		 * 192 channels 15x15 22 images (264) 31.4 / 29.4, 384 12 (288) 38.5 / 36.8, 64 80 (320) 28.3 / 26.9; 64 85 (340) 30.3 / 30.3, 256 24 (384) 38.3 / 39.3; 16x16 and 13x13 the
+		 * same). Not with other numbers of tiles (288, the launch alone, without / with residual, lines and strips: 9x9 4.9 / 5.2 and 4.9 / 5.4, 19x19 8.6 / 10.6 and 10.1 / 13.0).
 		 * Strips in fp32 to 96 slices (-2 to -9 %; behind at 128): their repeated rows
 		 * come from the L2 of their XCD, which has the neighbouring strips. 32 channels to 320 slices (without residual 4 to 10 % ahead of 64
 		 * there, with residual -7 to +1 %; at 404 -4 to +6 %). With residual the fp32 form of 32 channels keeps 54 registers per lane in scratch
@@ -1931,15 +1935,15 @@ extern "C"
 			const long long images_of_16 = 4 * slices, rows_of_16 = images_of_16 * ceil_div(output_shape.dim[1], 4);
 			const auto lines_fit = [&](bool one_strip) { return common_act && m_bytes <= 0xffffffffu && lines_shape(output_shape.dim[1], output_shape.dim[2], sizeof(T), one_strip).lds <= 160 * 1024; };
 			const bool narrow = fp32 && output_shape.dim[2] <= 16; /* strips */
+			const bool four_by_four = ceil_div(output_shape.dim[1], 4) == 4 && ceil_div(output_shape.dim[2], 4) == 4;
 			if (!narrow && separate && rows_of_16 <= units && lines_fit(true))
 				launch_output_input_lines<T>(stream, matrices, bias, ext, output_shape, output, act, next, true);
+			else if (!fp32 && common_act && separate && strips_fit && four_by_four && images_of_16 > units && 4 * images_of_16 <= 5 * units)
+				launch_output_input_strips<T>(stream, matrices, bias, ext, output_shape, output, act, next);
 			else if (!narrow && images_of_16 <= (fp32 ? 1 : 3) * units && lines_fit(false))
 				launch_output_input_lines<T>(stream, matrices, bias, ext, output_shape, output, act, next, false);
 			else if (fp32 && common_act && separate && strips_fit && 8 * slices <= 3 * units)
-			{
-				if constexpr (fp32)
-					launch_output_input_strips<T>(stream, matrices, bias, ext, output_shape, output, act, next);
-			}
+				launch_output_input_strips<T>(stream, matrices, bias, ext, output_shape, output, act, next);
 			else if (fp32 && common_act && 4 * slices <= (residual ? (cached ? 3 : 2) : 1) * units)
 			{
 				if constexpr (fp32)

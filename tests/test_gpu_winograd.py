@@ -272,6 +272,27 @@ def test_fused_transform_lines(ctx, dtype, shape):
             assert mismatches(y.copyToHost(ctx), want_y) == 0
 
 
+@pytest.mark.parametrize("shape", [(64, 15, 15, 64), (65, 15, 15, 64), (22, 16, 13, 192), (80, 13, 16, 64), (81, 13, 16, 64)])
+def test_fused_transform_of_half_on_both_sides_of_the_strips(ctx, shape):
+    """fp16 images of 4 x 4 tiles: a compute unit's worth of workgroups in lines (256 images of 16 channels), strips to a quarter more, lines again; with
+    the output in the residual's place the lines throughout. Bit for bit against the oracle."""
+    rng = np.random.default_rng(sum(shape))
+    b, h, w, c = shape
+    m, bias, ext = random_tensor(rng, (36, b * 16, c), "float16"), random_tensor(rng, (c,), "float16"), random_tensor(rng, shape, "float16")
+    db = ml.toDevice(ctx, bias)
+    for act, with_ext, keep, in_place in ((O.RELU, True, True, False), (O.LINEAR, False, False, False), (O.RELU, True, True, True)):
+        want_y = O.winograd_output_transform(m, shape, bias, ext if with_ext else None, act)
+        dm, de = ml.toDevice(ctx, m), ml.toDevice(ctx, ext)
+        y = de if in_place else ml.Tensor(shape, "float16")
+        dv = ml.Tensor((36, b * 16, c), "float16")
+        dv.setall(ctx, float("nan"))
+        nxt = dm if in_place else dv
+        ml.winogradOutputInputTransform(ctx, (c, 3, 3, c), dm, shape, y if keep else None, db, de if with_ext else None, act, nxt)
+        assert mismatches(nxt.copyToHost(ctx), O.winograd_input_transform(want_y)) == 0
+        if keep:
+            assert mismatches(y.copyToHost(ctx), want_y) == 0
+
+
 @pytest.mark.parametrize("dtype,shape", [("float16", (157, 33, 33, 64)), ("float32", (75, 33, 33, 64)), ("float32", (111, 33, 33, 64)), ("float16", (203, 19, 19, 256)),
                                          ("float16", (61, 19, 19, 128))]
                          + [(dtype, (slices, 7, 6, 64)) for dtype in ("float16", "float32") for slices in (85, 86, 96, 97, 192, 193, 320, 321)])
