@@ -15,10 +15,16 @@ LIB = os.path.join(HERE, "libminml_hip.so")
 
 SOURCES = ["runtime.hip", "winograd.hip", "gemm.hip", "gemm_tiles.hip", "conv.hip", "quantized.hip", "elementwise.hip", "heads.hip", "attention.hip", "moe.hip", "cuda_stubs.cpp"]
 # packed fp32 VALU forms are switched off for all device code; the host pass does not know the feature and says so (harmless)
-# the leading kernel arguments arrive in scalar registers with the wavefront instead of being loaded by it (0.25 us from a workgroup's start until
-# they are there): 20 x 256 channels, us per layer of two launches, 1 position 9.1 -> 8.9, 16 14.8 -> 14.6, 32 19.5 -> 19.2; fp32 128 channels 10.7 -> 10.4
 COMMON = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
-          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-mllvm", "-amdgpu-kernarg-preload-count=16"]
+          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+# the leading kernel arguments arrive in scalar registers with the wavefront instead of being loaded by it (0.25 us from a workgroup's start until
+# they are there): 20 x 256 channels, us per layer of two launches, 1 position 9.1 -> 8.9, 16 14.8 -> 14.6, 32 19.5 -> 19.2; fp32 128 channels 10.7 -> 10.4.
+# The launch itself waits for them, up to 0.15 us, so that kernels of a few instructions are behind: element-wise calls on one or 16 boards take as much longer
+# (us, without / with: conversion of 225 x 256 elements 1.68 / 1.84, sum of two tensors 1.79 / 1.94, bias and ReLU 2.16 / 2.25), on 256 they gain less (256
+# channels 15.8 / 15.4, 11.0 / 11.1, 11.1 / 11.2). Gathers and products of the same length do too (1.81 / 1.88), but their files' longer kernels gain more (routing
+# 2 to 7 %, products of the networks 1 %)
+PRELOAD = ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
+WITHOUT_PRELOAD = {"elementwise.hip"}
 # the transforms reproduce the reference's expression trees exactly: no contraction beyond the explicit fma calls
 PER_FILE = {"winograd.hip": ["-ffp-contract=off"]}
 
@@ -45,7 +51,7 @@ def build(verbose=False, jobs=None):
 
     def compile_one(src):
         obj = os.path.join(OBJ, os.path.splitext(src)[0] + ".o")
-        cmd = [cc] + COMMON + PER_FILE.get(src, []) + ["-c", os.path.join(CSRC, src), "-o", obj]
+        cmd = [cc] + COMMON + ([] if src in WITHOUT_PRELOAD else PRELOAD) + PER_FILE.get(src, []) + ["-c", os.path.join(CSRC, src), "-o", obj]
         if src.endswith(".cpp"):
             cmd = [cc, "-O2", "-std=c++17", "-fPIC", "-Wall", "-x", "c++", "-c", os.path.join(CSRC, src), "-o", obj]
         out = _run(cmd)
