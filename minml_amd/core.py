@@ -253,9 +253,11 @@ class Tensor:
 
     # ---- descriptors
     def desc(self):
-        # the shape is a tuple of whole numbers from the start
+        # a tuple of whole numbers unless it was assigned: no conversion then
         shape = self.shape
-        return B.mlTensor_t(self.ptr, self.dtype, len(shape), shape) if self.ptr and len(shape) <= B.MAX_RANK else B.make_tensor(self.ptr, self.dtype, shape)
+        if self.ptr and type(shape) is tuple and len(shape) <= B.MAX_RANK:
+            return B.mlTensor_t(self.ptr, self.dtype, len(shape), shape)
+        return B.make_tensor(self.ptr, self.dtype, shape)
 
     def shape_desc(self):
         return B.make_shape(self.shape)

@@ -66,6 +66,15 @@ def test_more_dimensions_than_a_descriptor_holds_are_an_index_error():
             describe()
 
 
+def test_descriptors_of_a_shape_that_was_assigned():
+    """A list or whole numbers of numpy, which the constructor would have made a tuple of ints."""
+    t = ml.Tensor((6,), "float32", _ptr=0x7000)
+    for shape in ([2, 3], (np.int64(2), np.int32(3))):
+        t.shape = shape
+        assert t.desc().rank == t.shape_desc().rank == 2
+        assert list(t.desc().dim) == list(t.shape_desc().dim) == [2, 3, 0, 0, 0, 0]
+
+
 def test_cabi_error_behaviour(tmp_path):
     exe = str(tmp_path / "cabi_errors")
     libdir = os.path.join(ROOT, "minml_amd")
