@@ -102,6 +102,22 @@ def test_int8_convolution_taps_of_whole_pieces(ctx, shape, cout, k):
     assert mismatches(dy.copyToHost(ctx), want) == 0
 
 
+@pytest.mark.parametrize("batch", [390, 391, 780, 782])
+def test_int8_convolution_at_the_limits_of_the_tiles(ctx, batch):
+    """Both sides of the limits at which a convolution of whole pieces leaves the 64 x 64 tiles (768 of them on 256 compute units: 390 boards of 7x6) and the
+    128 x 128 tiles (512: 780 boards; the test above has 400, which is in between) for the 256-row engine, bit for bit against the oracle."""
+    rng = np.random.default_rng(batch)
+    shape, cout, k = (batch, 7, 6, 128), 132, 2
+    x, wt = rng.integers(-128, 128, shape).astype(np.int8), rng.integers(-127, 128, (cout, k, k, 128)).astype(np.int8)
+    scales, bias = (rng.random(cout) * 0.002 + 0.0005).astype(np.float32), rng.standard_normal(cout).astype(np.float32)
+    O.set_num_threads(8)
+    want = O.int8_conv2d_forward(x, IN_QD, wt, scales, bias, O.INT8, OUT_QD, x[..., :1].repeat(cout, -1), EXT_QD, O.RELU)
+    dx, dw, ds, db, de = (ml.toDevice(ctx, a) for a in (x, wt, scales, bias, np.ascontiguousarray(x[..., :1].repeat(cout, -1))))
+    dy = ml.Tensor((batch, 7, 6, cout), O.INT8)
+    ml.quantizedConvForward(ctx, dx, IN_QD, dw, ds, db, dy, OUT_QD, de, EXT_QD, O.RELU)
+    assert mismatches(dy.copyToHost(ctx), want) == 0
+
+
 @pytest.mark.parametrize("shape,cout,k", [((1, 1, 3, 16), 4, 3),  # one tile, K shorter than a ring slot, taps of one 16-byte chunk
                                           ((1, 11, 3, 32), 33, 3),  # 33 rows and columns: one past the 32 x 32 tile; not a multiple of 4
                                           ((5, 9, 7, 144), 100, 3),  # pieces that straddle taps, K not a whole slot
