@@ -326,10 +326,11 @@ namespace
 
 		/*
 		 * ---- stage keys, transposed values, key places and the head's table ----
-		 * With few images the launch is one workgroup's chain. In the AHEAD form the table, the first query block and two rounds of keys and values are requested
-		 * before any of them is used, from clamped places, and the next query block before the work of the present one. 6 images of 15x15, 8 heads of 32, in a
-		 * network with 4 of these launches: 321 -> 313 us. Only where a query row is 2 chunks: longer rows pay for the registers (fp16, 64 images of 19x19, 4 heads
-		 * of 64: 28 -> 32 us; fp32, heads of 32: 126 -> 135).
+		 * A workgroup's chain begins with these loads. In the AHEAD form the table, the first query block and two rounds of keys and values are requested
+		 * before any of them is used, from clamped places, and the next query block before the work of the present one. us, each load waited for where it is used / this,
+		 * fp16, 8 heads of 32 with a table: 15x15 6 images 7.34 / 7.24, 9 7.71 / 7.50, 24 9.79 / 9.58, 100 34.0 / 32.3, 512 110.2 / 108.6; 19x19 16 12.75 / 12.42, 256 133.2 / 129.8; 9x9 256
+		 * 15.28 / 14.32, up to 32 level. Without a table 19x19 16 10.69 / 10.24, 20x20 9 10.92 / 10.27; 15x15 6 level, 64 16.1 / 16.5. Only where a query row is 2 chunks: longer rows pay for
+		 * the registers (fp16, 64 images of 19x19, 4 heads of 64: 28 -> 32 us; fp32, heads of 32: 126 -> 135).
 		 */
 		constexpr bool AHEAD = (Q_CHUNKS <= 2);
 		constexpr int TABLE_AHEAD = AHEAD ? 1024 / THREADS : 1;

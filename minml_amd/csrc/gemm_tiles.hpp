@@ -252,7 +252,8 @@ namespace mlhip
 	 * written back. Networks of 20 blocks, us, written back / through: fp16 256 channels 15x15 12 positions 492 / 469, 16 535 / 520 (with weights that come from memory 560 / 564), 32 755 / 735, 19x19 8 609 / 590, 32 993 / 974; 128
 	 * channels 32 424 / 413, 64 600 / 576, 101 827 / 832, 19x19 100 1186 / 1142; 192 channels 16 448 / 433, 64 884 / 874; 64 channels 64 405 / 405; 384 channels 8 583 / 574, 64 1623 / 1608; fp32 64 channels
 	 * 32 444 / 441, 128 channels 32 751 / 713, 64 1124 / 1080, 256 3325 / 3318, 256 channels 16 1060 / 1019. Not where the launch itself is short of bandwidth to memory: tiles of
-	 * 128x128 (256 channels 64 1116 / 1134, 101 1526 / 1574), and orders by rows, in which every XCD fetches all of B, with a large B (384 channels, 10.6 MB, 16 802 / 816, 32 1161 / 1200).
+	 * 128x128 (256 channels 64 1116 / 1134, 101 1526 / 1574), and orders by rows, in which every XCD fetches all of B, with a large B (384 channels, 10.6 MB, 16 802 / 816, 32 1161 / 1200; the line lies
+	 * between 256 and 320 channels, 4.7 and 7.4 MB: two layers of 320, 15x15 12 30.0 / 29.6, 32 50.2 / 50.5, 48 62.6 / 63.6, 19x19 24 55.5 / 56.3).
 	 * Rows of C that are not whole lines of 128 bytes leave the L2 in parts: no matter while there are few of them (18 blocks of 96 channels, C of 1.8 MB 430 / 415, 3.5 446 / 440,
 	 * 7.1 586 / 583), more traffic than the wait costs after that (19x19, 11 MB 758 / 815; 14 MB 813 / 880, 24 MB 1179 / 1229).
 	 */
