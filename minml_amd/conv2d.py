@@ -143,11 +143,11 @@ class Conv2D:
 
     # ---- the three stages of the Winograd path, separately callable so that a runner can fuse across layers -------------------
     def _input_matrices(self, batch, workspace):
-        """The view at element 0 of the workspace (Conv2D.cpp:365-367), which must have room for the output matrices behind it."""
+        """The view at element 0 of the workspace (Conv2D.cpp:365-367), which must have room for the output matrices behind it: a view of both, cut to the first."""
         shape = get_matrices_shape(self.kernel_size, self.winograd_tile_size, (batch,) + self.input_shape[1:])
-        if shape[0] * shape[1] * (shape[2] + self.output_shape[3]) > workspace.volume():
-            raise ValueError("the workspace is too small for the layer's input and output matrices")
-        return workspace.view(shape)
+        matrices = workspace.view((shape[0], shape[1], shape[2] + self.output_shape[3]))
+        matrices.shape = shape
+        return matrices
 
     def _output_matrices(self, batch, workspace):
         """The view behind the input matrices, at element 36*T*Cin."""
@@ -155,7 +155,10 @@ class Conv2D:
         return workspace.view((squared, tiles, self.output_shape[3]), squared * tiles * filters_in)
 
     def _winograd_views(self, batch, workspace):
-        return self._input_matrices(batch, workspace), self._output_matrices(batch, workspace)
+        """Both, which end where the second does."""
+        shape = get_matrices_shape(self.kernel_size, self.winograd_tile_size, (batch,) + self.input_shape[1:])
+        squared, tiles, filters_in = shape
+        return workspace.view(shape), workspace.view((squared, tiles, self.output_shape[3]), squared * tiles * filters_in)
 
     def winograd_input(self, x, workspace):
         ml.winogradInputTransform(self.context, self.weight_shape, x, self._input_matrices(x.shape[0], workspace))

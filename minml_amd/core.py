@@ -253,14 +253,19 @@ class Tensor:
 
     # ---- descriptors
     def desc(self):
-        # a tuple of whole numbers unless it was assigned: no conversion then
+        # the shape is a tuple of whole numbers that fits, unless it was assigned: what the structure does not take is converted, or refused, there
         shape = self.shape
-        if self.ptr and type(shape) is tuple and len(shape) <= B.MAX_RANK:
-            return B.mlTensor_t(self.ptr, self.dtype, len(shape), shape)
-        return B.make_tensor(self.ptr, self.dtype, shape)
+        try:
+            return B.mlTensor_t(self.ptr, self.dtype, len(shape), shape) if self.ptr else B.make_tensor(self.ptr, self.dtype, shape)
+        except (RuntimeError, TypeError):
+            return B.make_tensor(self.ptr, self.dtype, shape)
 
     def shape_desc(self):
-        return B.make_shape(self.shape)
+        shape = self.shape
+        try:
+            return B.mlShape_t(len(shape), shape)
+        except (RuntimeError, TypeError):
+            return B.make_shape(shape)
 
 
 def toDevice(context, array, dtype=None):
